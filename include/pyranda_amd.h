@@ -16,8 +16,9 @@
  *  - Errors return a nonzero status; pyr_last_error() gives the message
  *    (replaces the reference's print + STOP, compact_d1.f90:65-72).
  *  - `_f64` entry points compute like the reference in FP64. `_r32` entry
- *    points read/write FP32 fields, sweep in FP32 and refine once with an
- *    FP64 residual against the same banded operator.
+ *    points read/write FP32 fields; bounded lines are solved in FP32 and
+ *    refined once with an FP64 residual against the same banded operator,
+ *    periodic lines in FP64 registers with one rounding of each result.
  */
 #ifndef PYRANDA_AMD_H
 #define PYRANDA_AMD_H
@@ -68,20 +69,21 @@ int pyr_destroy(pyr_ctx* ctx);
 int pyr_set_stream(pyr_ctx* ctx, void* stream);
 
 /* Solver of periodic implicit lines. No counterpart in the reference, which
- * always uses the bordered cyclic LU (pentadiagonal.f90:64-131, 654-825):
- * PYR_PSOLVE_CIRCULANT (default) factors the circulant LHS as c Q^T Q and
- * runs constant-coefficient recurrences; PYR_PSOLVE_LU uses the chunked LU
- * of bounded lines with the cyclic coupling in its reduced system. Both give
- * the same solution to rounding. */
+ * always uses the bordered cyclic LU (pentadiagonal.f90:64-131, 654-825).
+ * Periodic lines are solved through the circulant factorization c Q^T Q of
+ * their left-hand side in either mode: a chunked LU of them gave the same
+ * solution to rounding and was slower. The setting is kept, and members of a
+ * group still have to agree on it. */
 enum { PYR_PSOLVE_CIRCULANT = 0, PYR_PSOLVE_LU = 1 };
 int pyr_set_periodic_solver(pyr_ctx* ctx, int mode);
 
 /* Arithmetic of the solves on FP32 fields (PYR_R32 entry points and
  * pyr_apply with PYR_R32). No counterpart in the reference (FP64 only):
- * PYR_R32_SOLVE_REFINED (default) solves in FP32 and applies one FP64-residual
- * refinement; PYR_R32_SOLVE_FP64 forms the RHS and solves in FP64 registers
+ * PYR_R32_SOLVE_REFINED (default) solves bounded lines in FP32 and applies one
+ * FP64-residual refinement; PYR_R32_SOLVE_FP64 solves them in FP64 registers
  * and rounds once to FP32 (on gfx950 FP32 and FP64 vector FMAs issue at the
- * same rate, so this is the cheaper of the two). */
+ * same rate, so this is the cheaper and the more accurate of the two).
+ * Periodic lines take the FP64 solve in both modes. */
 enum { PYR_R32_SOLVE_REFINED = 0, PYR_R32_SOLVE_FP64 = 1 };
 int pyr_set_r32_solve(pyr_ctx* ctx, int mode);
 /* The same choice for one operator (PYR_OP_*) along one direction, over the
@@ -124,7 +126,7 @@ int pyr_grads_f64(pyr_ctx* ctx, const double* val, double* v1, double* v2,
 int pyr_divergence_f64(pyr_ctx* ctx, const double* fx, const double* fy, const double* fz,
                        double* val);                                 /* parcop.f90:202 divergence */
 
-/* --- FP32 fields, FP32 sweeps + one FP64-residual refinement ------------ */
+/* --- FP32 fields (arithmetic: pyr_set_r32_solve) ------------------------- */
 int pyr_ddx_r32(pyr_ctx* ctx, const float* val, float* dval);
 int pyr_ddy_r32(pyr_ctx* ctx, const float* val, float* dval);
 int pyr_ddz_r32(pyr_ctx* ctx, const float* val, float* dval);
@@ -192,16 +194,15 @@ int pyr_rk_update_dt(pyr_ctx* ctx, int prec, long long n, const void* F, double*
                      const void* U_in, void* U_out, double* U64, const double* dt, double A,
                      double B);
 
-/* Tuning of one operator along one direction at one precision (for FP32
- * fields: in the context's current FP32 solve mode): x_lds_kb is the LDS
- * budget of an x-line workgroup (8..160 KB; it sets the lines per
- * workgroup), yz_pipe switches the pipelined kernels (0/1; on x also 2: the
- * next group of lines prefetched into registers, used by the explicit
- * filter; on y/z also 3: the plain kernel with runtime row counts, fewer
- * registers), yz_lines the
- * lines per plain y/z workgroup (16, 32 or 64); -1 keeps the context default.
- * Set by pyranda_amd's autotuner (ParcopContext.autotune), which times the
- * candidates on the device. No counterpart in the reference. */
+/* Tuning of one operator along one direction at one precision: yz_lines is
+ * the lines per y/z workgroup (16, 32 or 64), yz_pipe 3 (y/z) selects the
+ * kernel with runtime row counts also where whole chunks would allow
+ * compile-time ones; -1 keeps the default. The x lines have one kernel and
+ * one shape: x_lds_kb (8..160 KB) and the other values of yz_pipe (0/1, on x
+ * also 2) are checked and change nothing. The refined FP32 solve of bounded
+ * lines has one shape, too. Results do not depend on any of them. Set by
+ * pyranda_amd's autotuner (ParcopContext.autotune), which times the candidates
+ * on the device. No counterpart in the reference. */
 int pyr_set_tuning(pyr_ctx* ctx, int op, int dir, int prec, int x_lds_kb, int yz_pipe,
                    int yz_lines);
 
@@ -212,7 +213,7 @@ int pyr_set_tuning(pyr_ctx* ctx, int op, int dir, int prec, int x_lds_kb, int yz
  * member m's (nx,ny,nz) block at offsets[m] elements; offsets that are
  * multiples of 16 elements keep the 16-byte row copies. pyr_group_apply is
  * pyr_apply on every member at once: one launch for all members' lines of
- * the direction (any lengths 8..512), plus a null-operator pass for members
+ * the direction (any lengths 8..1024), plus a null-operator pass for members
  * whose direction has fewer than 4 points. The epilogue constant of member m is
  * epi_scale * d_m^mesh_power (d_m its mesh spacing d1..d3 along the
  * direction: mesh_power 2 gives the ring scaling of operators.f90:615-643).

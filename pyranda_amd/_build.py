@@ -5,9 +5,9 @@ import subprocess
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRCS = [os.path.join(HERE, "csrc", "pyr_core.hip"), os.path.join(HERE, "csrc", "pyr_mlp.hip"),
         os.path.join(HERE, "csrc", "pyr_fuse.cpp")]
-# compile units: pyr_core.hip builds as four parts (host code and C-ABI; the
-# line kernels of each solve mode), compiled in parallel
-UNITS = [(SRCS[0], ["PYR_PART=%d" % k]) for k in range(4)] + [(SRCS[1], []), (SRCS[2], [])]
+# compile units: pyr_core.hip builds as eight parts (host code and C-ABI; the
+# line kernels by solve, width and grouping), compiled in parallel
+UNITS = [(SRCS[0], ["PYR_PART=%d" % k]) for k in range(8)] + [(SRCS[1], []), (SRCS[2], [])]
 OUT = os.path.join(HERE, "libpyranda_amd.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 

@@ -3,11 +3,11 @@
 // One launch applies one compact operator along one direction to a whole
 // (nx,ny,nz) field. Each thread owns one chunk of one line (pyr_plan.hpp):
 //   y/z lines: lanes of a wave are adjacent lines, i.e. adjacent x, so every
-//     row load/store of a wave is one contiguous 256-512 B segment;
-//   x lines:   a workgroup stages LX contiguous lines in LDS with coalesced
-//     copies, threads then read their chunk window from LDS.
-// The reduced system couples the chunks of a line through LDS within the
-// workgroup, so every field element is read once and written once from HBM.
+//     row load/store of a wave is made of 128-512 B segments; the chunks of a
+//     line are in one workgroup and exchange their carries through LDS;
+//   x lines:   a wave owns a few whole lines, moves them through its own LDS
+//     tile with 16-byte accesses, and needs no workgroup barrier at all.
+// Every field element is read once and written once from HBM.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -25,6 +25,7 @@
 
 #include "../../include/pyranda_amd.h"
 #include "pyr_line.hpp"
+#include "pyr_refined.hpp"
 
 using namespace pyr;
 
@@ -32,9 +33,10 @@ using namespace pyr;
 // error reporting
 // ---------------------------------------------------------------------------
 // The file compiles as several translation units that build in parallel:
-// PYR_PART 0 holds the host code and the C-ABI, parts 1-3 the line kernels
-// of one solve mode each (FP64, FP32-refined, FP32 fields with FP64 solves),
-// through explicit instantiations of the launch functions.
+// PYR_PART 0 holds the host code and the C-ABI, the others the line kernels
+// (1, 2: periodic lines of FP64 and FP32 fields; 3, 4: bounded lines and the
+// explicit filter; 5, 6: grouped launches; 7: the refined FP32 solve) through
+// explicit instantiations of the launch functions.
 #ifndef PYR_PART
 #define PYR_PART 0
 #endif
@@ -64,264 +66,23 @@ static int fail(const std::string& m) { return pyr::report_error(m); }
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-template <int MODE> struct SolveT { using type = double; };
-template <> struct SolveT<MODE_R32> { using type = float; };  // MODE_S32 solves in double
+enum Solve { SOLVE_NONE = 0, SOLVE_BND = 1, SOLVE_CIRC = 2 };
 
-constexpr int WG_MAX = 512;
+// What the epilogue of a y/z row needs besides the solution, in registers
+// before the solve so that no store waits on a load: the input value (filters
+// add v back) or the current output (accumulating epilogues).
+enum Pre { PRE_NONE = 0, PRE_V = 1, PRE_OLD = 2 };
 
-// Coefficient tables of one operator, as the solve reads them (LDS copies on
-// the device, plan vectors in the host emulation).
-struct Tabs {
-  const double* lu = nullptr;
-  const double* rc = nullptr;
-  const double* gsel = nullptr;
-  const float* lu32 = nullptr;
-  const float* rc32 = nullptr;
-  const float* gsel32 = nullptr;
-  const double* band = nullptr;
-};
+constexpr int WG_MAX = 1024;
 
-__host__ __device__ inline size_t align16(size_t b) { return (b + 15) & ~(size_t)15; }
-
-// bytes of the staged tables: FP64 lu|rc|gsel, or FP32 lu|rc|gsel + FP64 band
-template <int MODE>
-__host__ __device__ inline size_t stage_bytes(int ntab, int N) {
-  return MODE != MODE_R32 ? align16((size_t)ntab * sizeof(double))
-                          : align16((size_t)ntab * sizeof(float)) + align16((size_t)5 * N * sizeof(double));
-}
-
-template <int MODE>
-__device__ __forceinline__ Tabs stage_tables(const LineArgs& a, unsigned char* dst, int tid, int nthr) {
-  Tabs t;
-  if (MODE != MODE_R32) {
-    double* d = reinterpret_cast<double*>(dst);
-    for (int e = tid; e < a.ntab; e += nthr) d[e] = a.tab64[e];
-    t.lu = d;
-    t.rc = d + 5 * a.N;
-    t.gsel = d + 9 * a.N;
-  } else {
-    float* f = reinterpret_cast<float*>(dst);
-    for (int e = tid; e < a.ntab; e += nthr) f[e] = a.tab32[e];
-    double* bd = reinterpret_cast<double*>(dst + align16((size_t)a.ntab * sizeof(float)));
-    for (int e = tid; e < 5 * a.N; e += nthr) bd[e] = a.band[e];
-    t.lu32 = f;
-    t.rc32 = f + 5 * a.N;
-    t.gsel32 = f + 9 * a.N;
-    t.band = bd;
-  }
-  return t;
-}
-
-// The tables as the solve reads them from global memory (lines whose tables
-// exceed the LDS budget, grouped launches).
-template <int MODE>
-__device__ __forceinline__ Tabs global_tables(const LineArgs& a) {
-  Tabs t;
-  t.lu = a.lu;
-  t.rc = a.rc;
-  t.gsel = a.gsel;
-  t.lu32 = a.lu32;
-  t.rc32 = a.rc32;
-  t.gsel32 = a.gsel32;
-  t.band = a.band;
-  return t;
-}
-
-template <int MODE>
-__device__ __forceinline__ Tabs get_tables(const LineArgs& a, unsigned char* dst, int tid, int nthr) {
-  return a.gtab ? global_tables<MODE>(a) : stage_tables<MODE>(a, dst, tid, nthr);
-}
-
-// staged tables above this size are read from global memory instead
-constexpr size_t STAGE_MAX_BYTES = 64 * 1024;
-
-enum Solve { SOLVE_NONE = 0, SOLVE_LU = 1, SOLVE_CIRC = 2 };
-
-// Solve one chunk given its RHS with the chunked LU; the LDS exchange of edge
-// values goes through Y (4P x ly entries of the solve type), column `col`
-// belongs to this line. The solution replaces the RHS in `rhs`.
-// act: the thread's chunk exists (a grouped launch shapes its workgroups for
-// the member with the most chunks; other threads only take the barriers).
-template <int MODE, typename CS>
-__device__ __forceinline__ void solve_chunk_lu(const LineArgs& a, const Tabs& t, int p, int s, int m,
-                                               CS* Y, int ly, int col, double* rhs, bool act = true) {
-  auto yr = [&](int c) { return Y[c * ly + col]; };
-  if (MODE != MODE_R32) {
-    double* x = rhs;  // solve in place
-    double e4[4];
-    if (act) {
-      local_solve<double>(t.lu, s, m, x);
-      edges(x, m, e4);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) Y[(4 * p + q) * ly + col] = (CS)e4[q];
-    }
-    __syncthreads();
-    if (act) {
-      double z[4];
-      neighbours<double>(t.gsel, p, a.P, yr, z);
-      spike_correct(t.rc, s, m, z, x);
-    }
-  } else {
-    float x[CHUNK];
-    float z[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < CHUNK; ++k) x[k] = (float)rhs[k];
-    if (act) {
-      local_solve<float>(t.lu32, s, m, x);
-      float e4[4];
-      edges(x, m, e4);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) Y[(4 * p + q) * ly + col] = (CS)e4[q];
-    }
-    __syncthreads();
-    float d[CHUNK];
-    if (act) {
-      neighbours<float>(t.gsel32, p, a.P, yr, z);
-      spike_correct(t.rc32, s, m, z, x);
-      // one refinement step: FP64 residual against the same banded operator
-      residual64([&](int k) { return t.band + 5 * (s + k); }, m, rhs, x, z, rhs);
-#pragma unroll
-      for (int k = 0; k < CHUNK; ++k) d[k] = (float)rhs[k];
-      local_solve<float>(t.lu32, s, m, d);
-    }
-    __syncthreads();
-    if (act) {
-      float f4[4];
-      edges(d, m, f4);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) Y[(4 * p + q) * ly + col] = (CS)f4[q];
-    }
-    __syncthreads();
-    if (act) {
-      float zd[4];
-      neighbours<float>(t.gsel32, p, a.P, yr, zd);
-      spike_correct(t.rc32, s, m, zd, d);
-#pragma unroll
-      for (int k = 0; k < CHUNK; ++k) rhs[k] = (double)x[k] + (double)d[k];
-    }
-  }
-}
-
-// One circulant solve A y = r of the chunk (without the 1/c): forward
-// recurrence with its carry through Xa, backward recurrence with its carry
-// through Xb; the rows of the result go to sink(k, y_k). Two barriers. A
-// thread whose chunk index p is not below P (a workgroup shaped for a longer
-// line of another member of a grouped launch) only takes the barriers.
-template <bool GRP, typename C, typename Sink>
-__device__ __forceinline__ void circ_solve(const C* kf, const C* kb, C p1, C p2, int p, int P,
-                                           int m, C* Xa, C* Xb, int ly, int col, C* x, Sink sink) {
-  const bool act = !GRP || p < P;
-  C e0 = 0, e1 = 0;
-  if (act) {
-    circ_fwd_exit(x, m, p1, p2, e0, e1);
-    Xa[(2 * p) * ly + col] = e0;
-    Xa[(2 * p + 1) * ly + col] = e1;
-  }
-  __syncthreads();
-  if (act) {
-    circ_carry(kf, p, P, [&](int c) { return Xa[c * ly + col]; }, e0, e1);
-    circ_fwd(x, m, p1, p2, e0, e1);
-    circ_bwd_exit(x, m, p1, p2, e0, e1);
-    Xb[(2 * p) * ly + col] = e0;
-    Xb[(2 * p + 1) * ly + col] = e1;
-  }
-  __syncthreads();
-  if (act) {
-    circ_carry(kb, p, P, [&](int c) { return Xb[c * ly + col]; }, e0, e1);
-    circ_bwd_sink(x, m, p1, p2, e0, e1, sink);
-  }
-}
-
-// Circulant solve of one chunk; X0 and X1 hold 4P x ly entries each. Every
-// buffer is written only after a barrier that follows its last read. The
-// solution rows go to emit(k, y_k) in FP64 (before the metric scale).
-// carry rows of the circulant solve in the solve type: 0 forward, 1 backward
-template <int MODE>
-__device__ __forceinline__ const typename SolveT<MODE>::type* kmat(const LineArgs& a, int which) {
-  if constexpr (MODE == MODE_R32) return which ? a.kb32 : a.kf32;
-  else return which ? a.kb : a.kf;
-}
-
-// Entries per chunk of each of the two exchange buffers of solve_chunk_circ
-// (per line): the forward and backward carries take 2; the refined FP32 solve
-// also exchanges the 4 edge values of its first solution.
-template <int MODE>
-constexpr int circ_words() { return MODE == MODE_R32 ? 4 : 2; }
-
-// kf/kb: the carry rows in the solve type (global memory or an LDS copy)
-template <int MODE, typename CS, bool GRP = false, typename Emit>
-__device__ __forceinline__ void solve_chunk_circ(const LineArgs& a, const CS* kf, const CS* kb, int p,
-                                                 int m, CS* X0, CS* X1, int ly, int col, double* rhs,
-                                                 Emit emit) {
-  const int P = a.P;
-  if constexpr (MODE != MODE_R32) {
-    circ_solve<GRP, double>(kf, kb, a.p1, a.p2, p, P, m, X0, X1, ly, col, rhs,
-                       [&](int k, double v) { emit(k, v * a.invc); });
-  } else {
-    float y[CHUNK];
-#pragma unroll
-    for (int k = 0; k < CHUNK; ++k) y[k] = (float)rhs[k];
-    circ_solve<GRP, float>(kf, kb, a.p1f, a.p2f, p, P, m, X0, X1, ly, col, y,
-                      [&](int k, float v) { y[k] = v * a.invcf; });
-    // neighbour values of the FP32 solution for the residual
-    const bool act = !GRP || p < P;
-    if (act) {
-      float e4[4];
-      edges(y, m, e4);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) X0[(4 * p + q) * ly + col] = e4[q];
-    }
-    __syncthreads();
-    if (act) {
-      const int pm = p == 0 ? P - 1 : p - 1, pp = p == P - 1 ? 0 : p + 1;
-      const float z[4] = {X0[(4 * pm + 2) * ly + col], X0[(4 * pm + 3) * ly + col],
-                          X0[(4 * pp) * ly + col], X0[(4 * pp + 1) * ly + col]};
-      const double row[5] = {a.bd[0], a.bd[1], a.bd[2], a.bd[1], a.bd[0]};
-      residual64([&](int) { return row; }, m, rhs, y, z, rhs);
-    }
-    float d[CHUNK];
-#pragma unroll
-    for (int k = 0; k < CHUNK; ++k) d[k] = (float)rhs[k];
-    circ_solve<GRP, float>(kf, kb, a.p1f, a.p2f, p, P, m, X1, X0, ly, col, d,
-                      [&](int k, float v) { emit(k, (double)y[k] + (double)(v * a.invcf)); });
-  }
-}
-
-// y/z lines. block = (LY lanes, P chunks). With LY = 64 the chunk index is
-// wave-uniform; with LY = 32 a wave holds two chunks of 32 lines each.
-// What the epilogue of a y/z row needs besides the solution, fetched into
-// registers before the solve so that no store waits on a load: the input
-// value (filters add v back) or the current output (accumulating epilogues).
-// PRE_LATE loads them in the epilogue instead (fewer registers, a wait per row).
-enum Pre { PRE_NONE = 0, PRE_V = 1, PRE_OLD = 2, PRE_LATE = 3 };
-
-// Build-time tuning knobs (register pressure against latency hiding):
-//   PYR_FULL_CHUNKS  compile-time row counts when CHUNK divides N
-//   PYR_PREFETCH     PRE_V / PRE_OLD (1) or PRE_LATE (0)
-//   PYR_YZ_WAVES_PER_EU, PYR_X_WAVES_PER_EU  minimum waves per SIMD the y/z
-//                    and x kernels are built for
-//   XU               copies in flight per thread in the x-tile loads and stores
-//                    (8; 16 measured 0.7% faster on the FP64 Taylor-Green step
-//                    at 256^3 and 1.3% slower on the FP32-refined one)
-#ifndef PYR_FULL_CHUNKS
-#define PYR_FULL_CHUNKS 1
-#endif
-#ifndef PYR_PREFETCH
-#define PYR_PREFETCH 1
-#endif
-#ifndef PYR_YZ_WAVES_PER_EU
-#define PYR_YZ_WAVES_PER_EU 1
-#endif
-#ifndef PYR_X_WAVES_PER_EU
-#define PYR_X_WAVES_PER_EU 1
-#endif
-
-// Raw buffer access to one field: a wave's row of 64 adjacent lines is one
-// load/store whose lane part sits in a VGPR and whose row part (uniform across
-// the wave) sits in an SGPR, so no per-row 64-bit address is formed. Fields
-// are below 2 GiB (at most 512^3 FP64). dword3 0x00020000: 32-bit data format,
-// the raw (untyped) configuration of gfx9-family buffer descriptors.
+// Raw buffer access to one field: the lane part of an address sits in a VGPR
+// and the row part (uniform across the wave) in an SGPR, so no per-row 64-bit
+// address is formed, and an access at OOB reads 0 or stores nothing without a
+// branch. Fields are below 2 GiB (at most 512^3 FP64). dword3 0x00020000:
+// 32-bit data format, the raw (untyped) configuration of gfx9-family buffer
+// descriptors.
 constexpr int BUF_DWORD3 = 0x00020000;
+constexpr int OOB = (int)0x80000000;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, int nbytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, nbytes, BUF_DWORD3);
@@ -340,699 +101,404 @@ __device__ __forceinline__ void buf_store(float v, __amdgpu_buffer_rsrc_t r, int
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, voff, soff, 0);
 }
 
-// Occupancy the y/z kernels are built for (waves per SIMD). Measured on
-// gfx950 at 256^3: capping the FP64-solve circulant kernels without epilogue
-// prefetch and the FP32 explicit filter at 128 VGPRs (4 waves) is faster
-// despite a few spilled registers (d1 y 39 -> 33 us, gbar y 62 -> 54 us);
-// for every other instance the spills cost more than the occupancy gains.
-template <typename TS, int SOLVE, int MODE, int PRE>
-struct YzWaves {
-  static constexpr int v =
-      PYR_YZ_WAVES_PER_EU > 1 ? PYR_YZ_WAVES_PER_EU
-      : (((MODE == MODE_S32 && SOLVE == SOLVE_CIRC && PRE == PRE_NONE) ||
-          (SOLVE == SOLVE_NONE && sizeof(TS) == 4 && PRE == PRE_NONE)) ? 4 : 1);
-};
+// A pair of FP64 values moved as one 16-byte LDS or global access.
+using D2 = double __attribute__((ext_vector_type(2)));
 
+// Carry matrix of term j for chunk p (periodic lines of equal chunks share one
+// per term: kp = 1, which FULL lines know at compile time).
+template <bool SHARED>
+__device__ __forceinline__ const double* carry_row(const double* K, const LineArgs& a, int j, int p) {
+  return SHARED ? K + 4 * j : K + 4 * (j * a.kp + (a.kp > 1 ? p : 0));
+}
+
+// Entry state of chunk p: its carry matrices times the exit states of the
+// chunks that follow in direction `step` (-1: p-1, p-2, ...; +1: p+1, ...).
+// exit_of(q) reads the exit pair of chunk q.
+template <bool CYCLIC, bool SHARED, int STEP, typename ExitOf>
+__device__ __forceinline__ void carry_in(const LineArgs& a, const double* K, int p, ExitOf exit_of, double& e0,
+                                         double& e1) {
+  e0 = e1 = 0.0;
+  int q = p;
+  for (int j = 0; j < a.W; ++j) {
+    q += STEP;
+    if (CYCLIC) {
+      if (q < 0) q = a.P - 1;
+      if (q >= a.P) q = 0;
+    }
+    if (CYCLIC || (q >= 0 && q < a.P)) {
+      const D2 u = exit_of(q);
+      if (SHARED) {
+        const double* k = carry_row<SHARED>(K, a, j, p);
+        carry_add(k, u.x, u.y, e0, e1);
+      } else {
+        // the matrix rows as two 16-byte loads
+        const D2* k = reinterpret_cast<const D2*>(carry_row<SHARED>(K, a, j, p));
+        const D2 r0 = k[0], r1 = k[1];
+        const double kk[4] = {r0.x, r0.y, r1.x, r1.y};
+        carry_add(kk, u.x, u.y, e0, e1);
+      }
+    }
+  }
+}
+
+// The chunks of one wave that need the line's own factors (the wave then
+// takes them for all of its chunks: converged rows give the same bits).
+__device__ __forceinline__ bool wave_needs_tables(const LineArgs& a, int p) {
+  return __ballot(p < a.tlo || p == a.P - 1) != 0;
+}
+
+// The passes of one chunk around its two exchanges. `rows` are ConstRows or
+// TableRows; the bounded solve picks one per wave.
+template <int SOLVE, typename F>
+__device__ __forceinline__ void with_rows(const LineArgs& a, bool tab, int p, F f) {
+  if (SOLVE == SOLVE_BND && tab) f(TableRows{a.tf, a.tb, a.tg, a.P, p});
+  else f(ConstRows{a.p1, a.p2});
+}
+
+// y/z lines. Thread (lane, p): line blk * lines + lane, chunk p; a.lines
+// (a power of two) adjacent lines per workgroup. Bound by HBM: 16 rows a
+// thread keep the kernel at 75-110 VGPRs, so that the load, solve and store
+// phases of two or more workgroups overlap on a CU.
 // FULL: every chunk has CHUNK rows (N a multiple of CHUNK), so the row
-// predicates vanish at compile time. The circulant solve implies periodic lines.
+// predicates vanish at compile time.
+// GRP: a workgroup shaped for other members of a grouped launch; threads
+// without a chunk only take the barriers.
 // The body takes the workgroup's line-group index `blk` (blockIdx.x for one
 // field, the member-local index for a grouped launch over several fields).
-template <typename TS, int KIND, int SOLVE, int MODE, int LY, bool FULL, int PRE, bool GRP = false>
+template <typename TS, int KIND, int SOLVE, bool FULL, int PRE, bool GRP = false>
 __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, const TS* __restrict__ in,
                                              TS* __restrict__ out) {
   constexpr int R = Halo<KIND>::R;
-  constexpr bool PER = SOLVE == SOLVE_CIRC;
-  using CS = typename SolveT<MODE>::type;
   extern __shared__ __align__(16) unsigned char smem[];
-  const int lane = threadIdx.x;
-  int p = threadIdx.y;
-  if (LY == 64) p = __builtin_amdgcn_readfirstlane(p);
-  const int tid = threadIdx.x + LY * threadIdx.y;
-  const int nthr = LY * blockDim.y;
-  CS* Y = reinterpret_cast<CS*>(smem);
-  Tabs t;
-  if (SOLVE == SOLVE_LU) t = get_tables<MODE>(a, smem + align16((size_t)4 * a.P * LY * sizeof(CS)), tid, nthr);
+  const int LY = a.lines;
+  const int lane = threadIdx.x & (LY - 1);
+  const int p = (int)threadIdx.x >> __builtin_ctz(LY);
+  const bool act = !GRP || p < a.P;
   const long long L = blk * LY + lane;
-  const bool valid = L < a.nlines;
-  const long long Lc = valid ? L : (long long)a.nlines - 1;
-  const long long base = (Lc % a.A) + a.B * (Lc / a.A);
-  // act: this thread's chunk exists (a grouped launch shapes its workgroups
-  // for the member with the most chunks)
-  const bool act = FULL || !GRP || p < a.P;
-  const int s = FULL ? p * CHUNK : (act ? a.cstart[p] : 0);
-  const int m = FULL ? CHUNK : (act ? a.cstart[p + 1] - s : 0);
+  const bool valid = act && L < a.nlines;
+  const long long Lc = L < a.nlines ? L : (long long)a.nlines - 1;
+  const int lane_off = (int)(((Lc % a.A) + a.B * (Lc / a.A)) * (long long)sizeof(TS));
+  const int rb = (int)(a.stride * (long long)sizeof(TS));
+  const int s = FULL ? p * CHUNK : chunk_start(a, p);
+  const int m = FULL ? CHUNK : a.mb + (p < a.mx ? 1 : 0);
+  const bool last = p == a.P - 1;
+  const bool wrap = SOLVE == SOLVE_CIRC || (SOLVE == SOLVE_NONE && a.periodic);
   const __amdgpu_buffer_rsrc_t rin = buf_rsrc(in, a.nbytes), rout = buf_rsrc(out, a.nbytes);
   // the FP32 copy of an FP64 result (LineArgs::out32), half the bytes per element
   [[maybe_unused]] const __amdgpu_buffer_rsrc_t rout32 = buf_rsrc(a.out32, a.nbytes / 2);
-  const int lane_off = (int)(base * (long long)sizeof(TS));
-  const int row_bytes = (int)(a.stride * (long long)sizeof(TS));
-  // row `row` of this line; the row offset is wave-uniform when LY == 64
-  auto ld = [&](__amdgpu_buffer_rsrc_t r, int row) -> TS {
-    if constexpr (LY == 64) return buf_load(TS(), r, lane_off, row * row_bytes);
-    else return buf_load(TS(), r, lane_off + row * row_bytes, 0);
-  };
-  auto st = [&](TS v, int row) {
-    if constexpr (LY == 64) buf_store(v, rout, lane_off, row * row_bytes);
-    else buf_store(v, rout, lane_off + row * row_bytes, 0);
-  };
-  // With fewer than 64 lines per workgroup a wave holds several chunks, so a
-  // row index is not wave-uniform; for whole chunks the row offset splits
-  // into a per-lane base (the chunk's first row, or the first row of a halo)
-  // and a wave-uniform row count, one VGPR in all instead of one per row.
-  constexpr bool SPLIT = LY != 64 && FULL;
-  const int vmid = lane_off + s * row_bytes;
-  // row s + k of this line (0 <= k < CHUNK)
-  auto ldk = [&](__amdgpu_buffer_rsrc_t r, int k) -> TS {
-    if constexpr (SPLIT) return buf_load(TS(), r, vmid, k * row_bytes);
-    else return ld(r, s + k);
-  };
-  auto stk = [&](TS v, int k) {
-    if constexpr (SPLIT) buf_store(v, rout, vmid, k * row_bytes);
-    else st(v, s + k);
-  };
-  TS pre[CHUNK];
+  // rows s .. s+m-1; the halo rows wrap around a periodic line and are 0
+  // beyond the ends of a bounded one
+  const int vmid = act ? lane_off + s * rb : OOB;
+  const int vlo = !act ? OOB : (p > 0 ? vmid - R * rb : (wrap ? lane_off + (a.N - R) * rb : OOB));
+  const int vhi = !act ? OOB : (!last ? vmid + CHUNK * rb : (wrap ? lane_off : OOB));  // FULL only
+  auto row_off = [&](int k) { return (int)((unsigned)vmid + (unsigned)k * (unsigned)rb); };
+  TS pre[PRE == PRE_OLD ? CHUNK : 1];
   if constexpr (PRE == PRE_OLD) {
 #pragma unroll
-    for (int k = 0; k < CHUNK; ++k) pre[k] = k < m ? ldk(rout, k) : (TS)0;
+    for (int k = 0; k < CHUNK; ++k)
+      pre[k] = FULL ? buf_load(TS(), rout, vmid, k * rb) : buf_load(TS(), rout, k < m ? row_off(k) : OOB, 0);
   }
-
   TS win[CHUNK + 2 * R];
-  if constexpr (SPLIT) {
-    // rows s-R .. s-1 (wrapped to N-R .. N-1 for the first chunk of a
-    // periodic line), s .. s+CHUNK-1, s+CHUNK .. s+CHUNK+R-1 (wrapped to
-    // 0 .. R-1 for the last chunk); a bounded line's missing halo rows are 0
-    const bool wrap = PER || a.periodic;
-    const int vlo = lane_off + (s >= R ? s - R : a.N - R) * row_bytes;
-    const int vhi = lane_off + (s + CHUNK < a.N ? s + CHUNK : 0) * row_bytes;
-    const bool lo_ok = act && (wrap || s >= R);
-    const bool hi_ok = act && (wrap || s + CHUNK < a.N);
 #pragma unroll
-    for (int w = 0; w < CHUNK + 2 * R; ++w) {
-      TS v = (TS)0;
-      if (w < R) {
-        if (lo_ok) v = buf_load(TS(), rin, vlo, w * row_bytes);
-      } else if (w < CHUNK + R) {
-        if (act) v = buf_load(TS(), rin, vmid, (w - R) * row_bytes);
-      } else {
-        if (hi_ok) v = buf_load(TS(), rin, vhi, (w - CHUNK - R) * row_bytes);
-      }
-      win[w] = v;
-    }
-  } else {
-#pragma unroll
-    for (int w = 0; w < CHUNK + 2 * R; ++w) {
-      int row = s - R + w;
-      TS v = (TS)0;
-      if (act && w < m + 2 * R) {
-        if (PER || a.periodic) {
-          row = row < 0 ? row + a.N : (row >= a.N ? row - a.N : row);
-          v = ld(rin, row);
-        } else if (row >= 0 && row < a.N) {
-          v = ld(rin, row);
-        }
-      }
-      win[w] = v;
+  for (int w = 0; w < CHUNK + 2 * R; ++w) {
+    const int k = w - R;
+    if (w < R) {
+      win[w] = buf_load(TS(), rin, vlo, w * rb);
+    } else if (FULL) {
+      win[w] = k < CHUNK ? buf_load(TS(), rin, vmid, k * rb)
+                         : buf_load(TS(), rin, vhi, (k - CHUNK) * rb);
+    } else if (k < 2 * NB) {  // every chunk has 2 NB rows
+      win[w] = buf_load(TS(), rin, vmid, k * rb);
+    } else {
+      const bool over = s + k >= a.N;
+      int off = over ? (wrap ? lane_off + (s + k - a.N) * rb : OOB) : row_off(k);
+      if (!act || k >= m + R) off = OOB;
+      win[w] = buf_load(TS(), rin, off, 0);
     }
   }
-  // grouped launches (runtime row counts, longer register live ranges) re-read
-  // v when it is added back instead of holding the chunk across the solve
-  constexpr bool HOLDV = PRE == PRE_V && !GRP;
-  if constexpr (HOLDV) {
-#pragma unroll
-    for (int k = 0; k < CHUNK; ++k) pre[k] = win[k + R];
-  }
-  double rhs[CHUNK];
-  rhs_interior<KIND>(a, win, rhs, m);
-  if (!PER && act) rhs_boundary(a, s, m, rhs, [&](int i) { return ld(rin, i); });
+  double x[CHUNK];
+  rhs_interior<KIND>(a, win, x);
+  if (SOLVE == SOLVE_BND || (SOLVE == SOLVE_NONE && !a.periodic))
+    if (act) rhs_boundary<KIND, FULL>(a, a.wb, p, win, x);
+
   // row k of the result: metric scale, filters add v back, fused epilogue, store
   auto emit = [&](int k, double y) {
-    if (!valid) return;
     double val = y * a.scale;
-    if constexpr (HOLDV) val += (double)pre[k];
-    if constexpr (PRE == PRE_V && GRP) val += (double)ldk(rin, k);
-    if constexpr (PRE == PRE_LATE)
-      if (a.addv) val += (double)ldk(rin, k);
+    if constexpr (PRE == PRE_V) val += (double)win[k + R];
+    const int off = FULL ? vmid : row_off(k);
+    const int soff = FULL ? k * rb : 0;
     TS old = (TS)0;
     if constexpr (PRE == PRE_OLD) old = pre[k];
-    if constexpr (PRE == PRE_LATE) old = (a.epi == EPI_ADD || a.epi == EPI_MAXABS) ? ldk(rout, k) : (TS)0;
     // a filter with an accumulating epilogue (only through pyr_apply) reads
     // the output in place
-    if constexpr (PRE == PRE_V) old = (a.epi == EPI_ADD || a.epi == EPI_MAXABS) ? ldk(rout, k) : (TS)0;
+    if constexpr (PRE == PRE_V)
+      if (a.epi == EPI_ADD || a.epi == EPI_MAXABS) old = buf_load(TS(), rout, off, soff);
     const TS r = epilogue<TS>(a.epi, a.epi_c, val, old);
-    if (sizeof(TS) != 8 || GRP || !a.only32) stk(r, k);
+    if (sizeof(TS) != 8 || GRP || !a.only32) buf_store(r, rout, off, soff);
     // (store epilogues only: the accumulating variants keep their registers)
     if constexpr (sizeof(TS) == 8 && PRE != PRE_OLD && !GRP)
-      if (a.out32) {
-        if constexpr (LY == 64) buf_store((float)r, rout32, lane_off / 2, (s + k) * (row_bytes / 2));
-        else if constexpr (SPLIT) buf_store((float)r, rout32, vmid / 2, k * (row_bytes / 2));
-        else buf_store((float)r, rout32, lane_off / 2 + (s + k) * (row_bytes / 2), 0);
-      }
+      if (a.out32) buf_store((float)r, rout32, off / 2, soff / 2);
   };
-  if (SOLVE == SOLVE_CIRC) {
-    solve_chunk_circ<MODE, CS, GRP>(a, kmat<MODE>(a, 0), kmat<MODE>(a, 1), p, m, Y, Y + 4 * a.P * LY, LY, lane,
-                                    rhs, emit);
-  } else {
-    if (SOLVE == SOLVE_LU) {
-      __syncthreads();  // staged tables visible
-      solve_chunk_lu<MODE, CS>(a, t, p, s, m, Y, LY, lane, rhs, act);
-    }
+  if constexpr (SOLVE == SOLVE_NONE) {
+    if (!valid) return;
 #pragma unroll
     for (int k = 0; k < CHUNK; ++k)
-      if (k < m) emit(k, rhs[k]);
-  }
-}
-
-template <typename TS, int KIND, int SOLVE, int MODE, int LY, bool FULL, int PRE>
-__global__ void __launch_bounds__(WG_MAX) __attribute__((amdgpu_waves_per_eu(YzWaves<TS, SOLVE, MODE, PRE>::v, 8)))
-k_line_yz(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
-  line_yz_body<TS, KIND, SOLVE, MODE, LY, FULL, PRE>(a, blockIdx.x, in, out);
-}
-
-// 16-byte copy from HBM straight into LDS (global_load_lds_dwordx4): lane i's
-// bytes land at lds + 16 i. The builtin is given to the device pass only:
-// with it in a kernel body the host pass drops the kernel's launch stub.
-__device__ __forceinline__ void lds_copy16(const void* g, void* lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
-#endif
-}
-
-// y/z lines, software-pipelined. A persistent workgroup walks groups of LG
-// adjacent lines (LG lanes x P chunks). The N rows of the next group are
-// copied from HBM into one of two LDS tiles by global->LDS DMA (no registers,
-// no waits) while the current group is solved from the other tile, so HBM
-// reads overlap the solve even with few waves per CU. Results leave as
-// coalesced buffer stores. Requirements, checked on the host: periodic lines,
-// CHUNK | N, the LG lines of a group adjacent in memory (LG | A), 16-byte
-// aligned rows and both tiles within the LDS budget.
-template <typename TS, int KIND, int SOLVE, int MODE, int LG, int PRE>
-__global__ void __launch_bounds__(WG_MAX) k_line_yz_pipe(LineArgs a, const TS* __restrict__ in,
-                                                         TS* __restrict__ out) {
-  constexpr int R = Halo<KIND>::R;
-  using CS = typename SolveT<MODE>::type;
-  constexpr int VE = 16 / (int)sizeof(TS);        // elements one lane moves
-  constexpr int LPR = LG * (int)sizeof(TS) / 16;  // lanes per tile row
-  constexpr int RPI = 64 / LPR;                   // tile rows per wave instruction (1 KiB)
-  static_assert(LPR >= 1 && 64 % LPR == 0, "tile row must be a whole number of 16-byte pieces");
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int N = a.N, P = a.P;
-  const int lane = threadIdx.x;
-  const int p = threadIdx.y;
-  const int flat = threadIdx.x + LG * threadIdx.y;
-  const int wave = __builtin_amdgcn_readfirstlane(flat >> 6);
-  const int nwaves = (LG * (int)blockDim.y) >> 6;
-  const int lane64 = flat & 63;
-  // tile rows: R wrapped rows, the N rows of the lines, R wrapped rows, and
-  // up to RPI-1 surplus rows (copies are issued in runs of RPI rows)
-  const int NT = ((N + 2 * R + RPI - 1) / RPI) * RPI;
-  TS* tiles = reinterpret_cast<TS*>(smem);
-  const int tile_elems = NT * LG;
-  CS* X0 = reinterpret_cast<CS*>(smem + align16(2 * (size_t)tile_elems * sizeof(TS)));
-  CS* X1 = X0 + 4 * P * LG;
-  CS* Kl = X1 + 4 * P * LG;  // carry rows, forward then backward (4P^2 each)
-  if constexpr (SOLVE == SOLVE_CIRC) {
-    const CS* kf = kmat<MODE>(a, 0);
-    const CS* kb = kmat<MODE>(a, 1);
-    const int nk = 4 * P * P;
-    for (int e = flat; e < nk; e += LG * (int)blockDim.y) {
-      Kl[e] = kf[e];
-      Kl[nk + e] = kb[e];
+      if (FULL || k < m) emit(k, x[k]);
+  } else {
+    constexpr bool CYC = SOLVE == SOLVE_CIRC;
+    constexpr bool SHARED = CYC && FULL;
+    const int nex = GRP ? (int)blockDim.x : a.P * LY;
+    D2* X0 = reinterpret_cast<D2*>(smem);
+    D2* X1 = X0 + nex;
+    int* bad = reinterpret_cast<int*>(X1 + nex);
+    const bool tab = SOLVE == SOLVE_BND && wave_needs_tables(a, p);
+    if (p == 0) bad[lane] = 0;
+    double e0 = 0.0, e1 = 0.0;
+    if (act) {
+      with_rows<SOLVE>(a, tab, p, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
+      X0[p * LY + lane] = D2{e0, e1};
     }
-  }
-  const int ngroups = a.nlines / LG;
-  const __amdgpu_buffer_rsrc_t rout = buf_rsrc(out, a.nbytes);
-  const int row_bytes = (int)(a.stride * (long long)sizeof(TS));
-  const int s = p * CHUNK;
-  constexpr int m = CHUNK;
-
-  // tile row j (0 <= j < NT) holds line row (j - R) mod N
-  auto issue = [&](int g, int t) {
-    const long long L0 = (long long)g * LG;
-    const TS* src = in + (L0 % a.A) + a.B * (L0 / a.A);
-    TS* dst = tiles + t * tile_elems;
-    const int c = (lane64 % LPR) * VE;
-    for (int j0 = wave * RPI; j0 < NT; j0 += nwaves * RPI) {
-      int r = j0 + lane64 / LPR - R;
-      r = r < 0 ? r + N : (r >= N ? r - N : r);
-      lds_copy16(src + (long long)a.stride * r + c, dst + j0 * LG);
-    }
-  };
-
-  int t = 0;
-  if ((int)blockIdx.x < ngroups) issue(blockIdx.x, 0);
-  for (int g = blockIdx.x; g < ngroups; g += gridDim.x, t ^= 1) {
-    // this wave's copies (and last group's stores) are done; the barrier makes
-    // every wave's copies visible and retires all reads of the other tile
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const long long L = (long long)g * LG + lane;
-    const int lane_off = (int)(((L % a.A) + a.B * (L / a.A)) * (long long)sizeof(TS));
-    // accumulating epilogues read the current output before the next copies are
-    // queued, so waiting for them never waits for the copies
-    TS pre[CHUNK];
-    if constexpr (PRE == PRE_OLD) {
-#pragma unroll
-      for (int k = 0; k < CHUNK; ++k) pre[k] = buf_load(TS(), rout, lane_off + (s + k) * row_bytes, 0);
+    double b0 = 0.0, b1 = 0.0;
+    if (act) {
+      carry_in<CYC, SHARED, -1>(a, a.kf, p, [&](int q) { return X0[q * LY + lane]; }, e0, e1);
+      with_rows<SOLVE>(a, tab, p, [&](auto rows) {
+        fwd_pass<FULL, true>(rows, x, m, e0, e1);
+        bwd_exit<FULL>(rows, x, m, b0, b1);
+      });
+      X1[p * LY + lane] = D2{b0, b1};
+      // a NaN or infinity anywhere in a line spreads to all of it, as it does
+      // through a whole-line sweep; the truncated carries alone would not
+      // take it further than W chunks
+      if (!__builtin_isfinite(b0) || !__builtin_isfinite(b1)) bad[lane] = 1;
     }
-    const int gn = g + gridDim.x;
-    if (gn < ngroups) issue(gn, t ^ 1);
-    // window rows s-R .. s+CHUNK+R-1 are tile rows s .. s+CHUNK+2R-1 (no wrap)
-    const TS* col0 = tiles + t * tile_elems + s * LG + lane;
-    TS win[CHUNK + 2 * R];
-#pragma unroll
-    for (int w = 0; w < CHUNK + 2 * R; ++w) win[w] = col0[w * LG];
-    double rhs[CHUNK];
-    rhs_interior<KIND>(a, win, rhs, m);
-    auto emit = [&](int k, double y) {
-      double val = y * a.scale;
-      // filters add v back: re-read from the tile (intact until the copies
-      // of the group after next) rather than holding CHUNK values across the
-      // solve, which would spill
-      if constexpr (PRE == PRE_V) val += (double)col0[(k + R) * LG];
-      TS old = (TS)0;
-      if constexpr (PRE == PRE_OLD) old = pre[k];
-      buf_store(epilogue<TS>(a.epi, a.epi_c, val, old), rout, lane_off + (s + k) * row_bytes, 0);
-    };
-    if constexpr (SOLVE == SOLVE_CIRC) {
-      solve_chunk_circ<MODE, CS>(a, Kl, Kl + 4 * P * P, p, m, X0, X1, LG, lane, rhs, emit);
-    } else {
-#pragma unroll
-      for (int k = 0; k < CHUNK; ++k) emit(k, rhs[k]);
-    }
+    __syncthreads();
+    if (!act) return;
+    carry_in<CYC, SHARED, 1>(a, a.kb, p, [&](int q) { return X1[q * LY + lane]; }, b0, b1);
+    if (bad[lane]) b0 = b1 = __builtin_nan("");
+    if (!valid) return;
+    with_rows<SOLVE>(a, tab, p, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
   }
+}
+
+template <typename TS, int KIND, int SOLVE, bool FULL, int PRE>
+__global__ void __launch_bounds__(WG_MAX) k_line_yz(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
+  line_yz_body<TS, KIND, SOLVE, FULL, PRE>(a, blockIdx.x, in, out);
 }
 
 // 16-byte vector of the storage type
 template <typename TS> struct Vec16;
-template <> struct Vec16<double> { using type = double2; static constexpr int W = 2; };
-template <> struct Vec16<float> { using type = float4; static constexpr int W = 4; };
+template <> struct Vec16<double> { using type = double __attribute__((ext_vector_type(2))); static constexpr int W = 2; };
+template <> struct Vec16<float> { using type = float __attribute__((ext_vector_type(4))); static constexpr int W = 4; };
 
-// r <- f(r, o) per component, without taking the vectors' addresses (which
-// would move them to scratch)
-template <typename F>
-__device__ __forceinline__ void vzip(double2& r, const double2& o, F f) {
-  r.x = f(r.x, o.x);
-  r.y = f(r.y, o.y);
-}
-template <typename F>
-__device__ __forceinline__ void vzip(float4& r, const float4& o, F f) {
-  r.x = f(r.x, o.x);
-  r.y = f(r.y, o.y);
-  r.z = f(r.z, o.z);
-  r.w = f(r.w, o.w);
+// Orders the LDS accesses of one wave: its own reads and writes reach LDS in
+// program order, so only the compiler has to be held back.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-#ifndef XU
-#define XU 8  // unroll of the tile load/store loops (a build-time knob, above)
-#endif
+// Moves the lines of one wave between HBM and its LDS tile. `end` elements
+// from src on (element 0 is the first of the 16-byte vector that holds the
+// lines' first element, `sh` the offset of that element in it); CH rows per
+// chunk, at most 64 chunks. PAD: one extra vector after every CH elements of
+// the tile (lines of whole chunks), which spreads the lanes' window reads over
+// the banks; other lines sit in the tile as in memory.
+template <typename TS, int CH, bool PAD>
+struct XTile {
+  using V = typename Vec16<TS>::type;
+  static constexpr int VW = Vec16<TS>::W;
+  static constexpr int CP = PAD ? CH + VW : CH;              // tile elements per chunk
+  static constexpr int SIZE = 64 * CP + (PAD ? 0 : 2 * VW);
+  static constexpr int NV = CH / VW + (PAD ? 0 : 1);          // vectors per lane
+  static __device__ __forceinline__ int at(int i) { return PAD ? i + i / CH * VW : i; }
 
-// x lines: LX contiguous lines per workgroup staged in LDS (row pitch
-// a.pitch). Rows move between HBM and LDS as 16-byte vectors when the line
-// length and pointers allow it, XU copies in flight per thread. The tile is
-// reused for the results, which leave through the same coalesced path.
-// LU solve: the tile region also holds the tables and edge exchange once the
-// windows are in registers. Circulant solve: the carry exchange sits after
-// the tile.
-template <typename TS, int KIND, int SOLVE, int MODE, bool FULL, bool GRP = false>
+  // avail: elements from src to the end of the field
+  static __device__ __forceinline__ void load(TS* tile, const TS* src, int end, long long avail, int vec, int lane) {
+    if (!vec) {
+      for (int e = lane; e < end; e += 64) tile[at(e)] = src[e];
+      return;
+    }
+    // whole vectors that lie inside the field, then the rest one by one
+    int nv = (end + VW - 1) / VW;
+    if (!PAD && (long long)nv * VW > avail) --nv;
+    V t[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int e = lane + 64 * j;
+      t[j] = reinterpret_cast<const V*>(src)[e < nv ? e : 0];
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int e = lane + 64 * j;
+      if (e < nv) *reinterpret_cast<V*>(tile + at(e * VW)) = t[j];
+    }
+    if (!PAD && nv * VW + lane < end) tile[nv * VW + lane] = src[nv * VW + lane];
+  }
+
+  // the results, with the epilogue; dst as src, o32 (if not null) the FP32
+  // copy of FP64 results, only32 instead of them
+  static __device__ __forceinline__ void store(const TS* tile, TS* dst, int sh, int end, int vec, int lane, int epi,
+                                               double epi_c, float* o32, int only32) {
+    const bool need_old = epi == EPI_ADD || epi == EPI_MAXABS;
+    auto put = [&](int e) {
+      TS r = tile[at(e)];
+      if (epi != EPI_STORE) r = epilogue<TS>(epi, epi_c, (double)r, need_old ? dst[e] : (TS)0);
+      if (sizeof(TS) != 8 || !only32) dst[e] = r;
+      if constexpr (sizeof(TS) == 8)
+        if (o32) o32[e] = (float)r;
+    };
+    if (!vec) {
+      for (int e = sh + lane; e < end; e += 64) put(e);
+      return;
+    }
+    // whole vectors of these lines; the elements of shared vectors one by one
+    const int v0 = (sh + VW - 1) / VW, v1 = end / VW;
+    V* dv = reinterpret_cast<V*>(dst);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int e = lane + 64 * j;
+      if (e >= v0 && e < v1) {
+        V r = *reinterpret_cast<const V*>(tile + at(e * VW));
+        if (epi != EPI_STORE) {
+          const V o = need_old ? dv[e] : V{};
+#pragma unroll
+          for (int i = 0; i < VW; ++i) r[i] = epilogue<TS>(epi, epi_c, (double)r[i], o[i]);
+        }
+        if (sizeof(TS) != 8 || !only32) dv[e] = r;
+        if constexpr (sizeof(TS) == 8) {
+          using F2 = float __attribute__((ext_vector_type(2)));
+          if (o32) reinterpret_cast<F2*>(o32)[e] = F2{(float)r[0], (float)r[1]};
+        }
+      }
+    }
+    if constexpr (!PAD) {
+      if (lane >= sh && lane < v0 * VW && lane < end) put(lane);
+      const int tail = v1 * VW + lane;
+      if (lane < VW && tail >= v0 * VW && tail < end) put(tail);
+    }
+  }
+};
+
+// The lanes of line l of a wave whose lines have P lanes each.
+__device__ __forceinline__ unsigned long long line_lanes(int l, int P) {
+  return (P >= 64 ? ~0ull : (1ull << P) - 1) << ((l * P) & 63);
+}
+
+// x lines. A workgroup is one wave, which owns a.lines whole lines (64 / P):
+// their elements are contiguous, come in and leave as 16-byte vectors through
+// the wave's own LDS tile, and lane l * P + p solves chunk p of line l. The
+// chunks of a line are lanes of one wave, so the carries need no barrier and
+// the waves of a CU run independently: 14-20 of them fit its LDS, enough
+// loads and stores in flight to reach the rate of a plain copy. Measured at
+// 256^3 (64-thread workgroups with 8 lines and 32-row chunks before): FP64
+// fbar 84 -> 53 us, d1 79 -> 50 us, FP32 d1 47 -> 33 us; a copy takes 50 and
+// 25 us. A persistent variant that fetches its next lines into registers
+// while it solves measured slower (512^3 d1 408 us against 373).
+template <typename TS, int KIND, int SOLVE, bool FULL, bool GRP = false>
 __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, const TS* __restrict__ in,
                                             TS* __restrict__ out) {
   constexpr int R = Halo<KIND>::R;
-  constexpr bool PER = SOLVE == SOLVE_CIRC;
-  using CS = typename SolveT<MODE>::type;
-  using V = typename Vec16<TS>::type;
-  constexpr int VW = Vec16<TS>::W;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int N = a.N, pitch = a.pitch, LX = a.lx;
-  TS* tile = reinterpret_cast<TS*>(smem);
-  const int tid = threadIdx.x;
-  const int nthr = blockDim.x;
-  const int l = tid % LX;
-  const int p = tid / LX;
-  const long long L0 = blk * LX;
+  using T = XTile<TS, CHUNK, FULL>;
+  constexpr int CP = T::CP;
+  __shared__ __align__(16) TS tile[T::SIZE];
+  __shared__ __align__(16) D2 ex[64];
+  const int N = a.N, P = a.P;
+  const int lane = threadIdx.x;
+  const long long L0 = blk * a.lines;
   const long long rem = (long long)a.nlines - L0;
-  const int nval = (int)(rem < LX ? rem : LX);
-  const TS* src = in + L0 * N;
-  if (a.vec) {
-    const int vpl = N / VW, nvec = nval * vpl;
-    const V* sv = reinterpret_cast<const V*>(src);
-    // global and LDS never alias, so the unrolled loads issue back to back
-#pragma unroll XU
-    for (int e = tid; e < nvec; e += nthr) {
-      const int ll = e / vpl, i = e - ll * vpl;
-      *reinterpret_cast<V*>(tile + ll * pitch + i * VW) = sv[e];
-    }
-  } else {
-    const int ne = nval * N;
-#pragma unroll XU
-    for (int e = tid; e < ne; e += nthr) {
-      const int ll = e / N, i = e - ll * N;
-      tile[ll * pitch + i] = src[e];
-    }
-  }
-  __syncthreads();
-  const int lr = l < nval ? l : 0;
-  const TS* row0 = tile + lr * pitch;
-  // act: this thread's chunk exists (a grouped launch sizes its workgroups
-  // for the member with the most threads per workgroup)
-  const bool act = !GRP || p < a.P;
-  const int s = FULL ? p * CHUNK : (act ? a.cstart[p] : 0);
-  const int m = FULL ? CHUNK : (act ? a.cstart[p + 1] - s : 0);
+  const int nval = (int)(rem < a.lines ? rem : a.lines);
+  const long long E0 = L0 * N;
+  const int sh = (!FULL && a.vec) ? (int)(E0 & (T::VW - 1)) : 0;
+  const int end = sh + nval * N;
+  T::load(tile, in + (E0 - sh), end, (long long)a.nlines * N - (E0 - sh), a.vec, lane);
+  wave_fence();
+  const int l = lane / P, p = lane - l * P;
+  const bool act = l < nval;
+  const int s = FULL ? p * CHUNK : chunk_start(a, p);
+  const int m = FULL ? CHUNK : a.mb + (p < a.mx ? 1 : 0);
+  const bool last = p == P - 1;
+  const bool wrap = SOLVE == SOLVE_CIRC || (SOLVE == SOLVE_NONE && a.periodic);
+  TS* row0 = tile + (act ? (FULL ? l * P * CP : sh + l * N) : (FULL ? 0 : sh));
+  TS* mo = row0 + (FULL ? p * CP : s);
   TS win[CHUNK + 2 * R];
+  if constexpr (FULL) {
+    const TS* lo = row0 + (p == 0 ? P - 1 : p - 1) * CP;
+    const TS* hi = row0 + (last ? 0 : p + 1) * CP;
 #pragma unroll
-  for (int w = 0; w < CHUNK + 2 * R; ++w) {
-    int row = s - R + w;
-    TS v = (TS)0;
-    if (act && w < m + 2 * R) {
-      if (PER || a.periodic) {
-        row = row < 0 ? row + N : (row >= N ? row - N : row);
-        v = row0[row];
-      } else if (row >= 0 && row < N) {
-        v = row0[row];
-      }
+    for (int w = 0; w < CHUNK + 2 * R; ++w) {
+      if (w < R) win[w] = lo[CHUNK - R + w];
+      else if (w < CHUNK + R) win[w] = mo[w - R];
+      else win[w] = hi[w - CHUNK - R];
     }
-    win[w] = v;
-  }
-  double rhs[CHUNK];
-  rhs_interior<KIND>(a, win, rhs, m);
-  if (!PER && act) rhs_boundary(a, s, m, rhs, [&](int i) { return row0[i]; });
-  if (SOLVE == SOLVE_LU) {
-    __syncthreads();  // the tile is consumed; reuse its LDS
-    CS* Y = reinterpret_cast<CS*>(smem);
-    const Tabs t = get_tables<MODE>(a, smem + align16((size_t)4 * a.P * LX * sizeof(CS)), tid, nthr);
-    __syncthreads();
-    solve_chunk_lu<MODE, CS>(a, t, p, s, m, Y, LX, l, rhs, act);
-    __syncthreads();  // tables and edge values no longer read
-  } else if (SOLVE == SOLVE_NONE) {
-    __syncthreads();  // the tile is consumed
-  }
-  TS* rowo = tile + l * pitch;
-  // filters add v back here, read from the tile row before the result takes
-  // its place (the windows are in registers by now; with the LU solve the
-  // tile holds the tables instead and v is added on the way out)
-  constexpr bool VTILE = SOLVE != SOLVE_LU;
-  auto emit = [&](int k, double y) {
-    if (act && l < nval) {
-      double val = y * a.scale;
-      if (VTILE && a.addv) val += (double)rowo[s + k];
-      rowo[s + k] = (TS)val;
-    }
-  };
-  if (SOLVE == SOLVE_CIRC) {
-    // the first carry barrier also retires every read of the tile
-    CS* X0 = reinterpret_cast<CS*>(smem + align16((size_t)LX * pitch * sizeof(TS)));
-    solve_chunk_circ<MODE, CS, GRP>(a, kmat<MODE>(a, 0), kmat<MODE>(a, 1), p, m, X0,
-                                    X0 + circ_words<MODE>() * a.P * LX, LX, l, rhs, emit);
-  } else {
+    if (!wrap) {
 #pragma unroll
-    for (int k = 0; k < CHUNK; ++k)
-      if (k < m) emit(k, rhs[k]);
-  }
-  __syncthreads();
-  TS* dst = out + L0 * N;
-  const bool need_old = (a.epi == EPI_ADD || a.epi == EPI_MAXABS);
-  if constexpr (sizeof(TS) == 8 && !GRP) {
-    if (a.out32) {
-      // FP64 result rounded to FP32 (store epilogue), with or without the
-      // FP64 store
-      float* d32 = a.out32 + L0 * N;
-      const int ne = nval * N;
-#pragma unroll XU
-      for (int e = tid; e < ne; e += nthr) {
-        const int ll = e / N, i = e - ll * N;
-        double val = (double)tile[ll * pitch + i];
-        if (!VTILE && a.addv) val = (double)(TS)(val + (double)src[e]);
-        if (!a.only32) dst[e] = (TS)val;
-        d32[e] = (float)val;
+      for (int w = 0; w < R; ++w) {
+        if (p == 0) win[w] = (TS)0;
+        if (last) win[CHUNK + R + w] = (TS)0;
       }
-      return;
-    }
-  }
-  if (a.vec) {
-    const int vpl = N / VW, nvec = nval * vpl;
-    const V* sv = reinterpret_cast<const V*>(src);
-    V* dv = reinterpret_cast<V*>(dst);
-#pragma unroll XU
-    for (int e = tid; e < nvec; e += nthr) {
-      const int ll = e / vpl, i = e - ll * vpl;
-      V r = *reinterpret_cast<const V*>(tile + ll * pitch + i * VW);
-      if (!VTILE && a.addv) vzip(r, sv[e], [](TS y, TS v) { return (TS)((double)y + (double)v); });
-      if (a.epi != EPI_STORE) {
-        const V o = need_old ? dv[e] : V{};
-        vzip(r, o, [&](TS y, TS old) { return epilogue<TS>(a.epi, a.epi_c, (double)y, old); });
-      }
-      dv[e] = r;
     }
   } else {
-    const int ne = nval * N;
-#pragma unroll XU
-    for (int e = tid; e < ne; e += nthr) {
-      const int ll = e / N, i = e - ll * N;
-      double val = (double)tile[ll * pitch + i];
-      if (!VTILE && a.addv) val = (double)(TS)(val + (double)src[e]);
-      const TS old = need_old ? dst[e] : (TS)0;
-      dst[e] = epilogue<TS>(a.epi, a.epi_c, val, old);
-    }
-  }
-}
-
-template <typename TS, int KIND, int SOLVE, int MODE, bool FULL>
-__global__ void __launch_bounds__(WG_MAX) __attribute__((amdgpu_waves_per_eu(PYR_X_WAVES_PER_EU, 8)))
-k_line_x(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
-  line_x_body<TS, KIND, SOLVE, MODE, FULL>(a, blockIdx.x, in, out);
-}
-
-// x lines, software-pipelined (periodic lines of whole 32-row chunks whose
-// length is a whole number of KiB, circulant solve or explicit filter). A
-// persistent workgroup walks groups of LX lines; the next group's lines are
-// copied HBM -> LDS by global->LDS DMA into the second of two tiles while the
-// current group is solved from the first, and the results leave through the
-// current tile with coalesced vector stores. Tile row pitch: N + one 16-byte
-// vector, so the windows (lanes over lines) read conflict-free.
-template <typename TS, int KIND, int SOLVE, int MODE>
-__global__ void __launch_bounds__(WG_MAX) __attribute__((amdgpu_waves_per_eu(PYR_X_WAVES_PER_EU, 8)))
-k_line_x_pipe(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
-  constexpr int R = Halo<KIND>::R;
-  using CS = typename SolveT<MODE>::type;
-  using V = typename Vec16<TS>::type;
-  constexpr int VW = Vec16<TS>::W;
-  constexpr int EPK = 1024 / (int)sizeof(TS);  // elements of one wave's 1 KiB copy
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int N = a.N, LX = a.lx, pitch = a.pitch;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int l = tid % LX, p = tid / LX;
-  const int lane64 = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nwaves = nthr >> 6;
-  const int tile_elems = LX * pitch;
-  TS* tiles = reinterpret_cast<TS*>(smem);
-  CS* X0 = reinterpret_cast<CS*>(smem + align16(2 * (size_t)tile_elems * sizeof(TS)));
-  CS* X1 = X0 + 4 * a.P * LX;
-  const int ngroups = (a.nlines + LX - 1) / LX;
-  const int ppl = N / EPK;  // 1 KiB pieces per line
-  auto issue = [&](int g, int t) {
-    const long long L0 = (long long)g * LX;
-    const long long rem = (long long)a.nlines - L0;
-    const int nval = (int)(rem < LX ? rem : LX);
-    const TS* src = in + L0 * N;
-    TS* dst = tiles + t * tile_elems;
-    for (int j = wave; j < nval * ppl; j += nwaves) {
-      const int ll = j / ppl, q = j - ll * ppl;
-      lds_copy16(src + (long long)ll * N + q * EPK + lane64 * VW, dst + ll * pitch + q * EPK);
-    }
-  };
-  const int s = p * CHUNK;
-  constexpr int m = CHUNK;
-  const bool need_old = (a.epi == EPI_ADD || a.epi == EPI_MAXABS);
-  int t = 0;
-  if ((int)blockIdx.x < ngroups) issue(blockIdx.x, 0);
-  for (int g = blockIdx.x; g < ngroups; g += gridDim.x, t ^= 1) {
-    // this wave's copies and last group's stores are done; the barrier makes
-    // every wave's copies visible and retires all reads of the other tile
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const int gn = g + gridDim.x;
-    if (gn < ngroups) issue(gn, t ^ 1);
-    const long long L0 = (long long)g * LX;
-    const long long rem = (long long)a.nlines - L0;
-    const int nval = (int)(rem < LX ? rem : LX);
-    TS* tile = tiles + t * tile_elems;
-    const int lr = l < nval ? l : 0;
-    const TS* row0 = tile + lr * pitch;
-    TS win[CHUNK + 2 * R];
 #pragma unroll
     for (int w = 0; w < CHUNK + 2 * R; ++w) {
       int row = s - R + w;
-      row = row < 0 ? row + N : (row >= N ? row - N : row);
-      win[w] = row0[row];
-    }
-    double rhs[CHUNK];
-    rhs_interior<KIND>(a, win, rhs, m);
-    TS* rowo = tile + l * pitch;
-    auto emit = [&](int k, double y) {
-      if (l < nval) {
-        double val = y * a.scale;
-        if (a.addv) val += (double)rowo[s + k];
-        rowo[s + k] = (TS)val;
+      bool ok = w < m + 2 * R;
+      if (row < 0 || row >= N) {
+        ok = ok && wrap;
+        row = row < 0 ? row + N : row - N;
       }
-    };
-    if constexpr (SOLVE == SOLVE_CIRC) {
-      // the first carry barrier also retires every window read of the tile
-      solve_chunk_circ<MODE, CS>(a, kmat<MODE>(a, 0), kmat<MODE>(a, 1), p, m, X0, X1, LX, l, rhs, emit);
-    } else {
-      __syncthreads();  // every window read before any result lands in the tile
-#pragma unroll
-      for (int k = 0; k < CHUNK; ++k) emit(k, rhs[k]);
-    }
-    __syncthreads();
-    const int vpl = N / VW, nvec = nval * vpl;
-    V* dv = reinterpret_cast<V*>(out + L0 * N);
-#pragma unroll XU
-    for (int e = tid; e < nvec; e += nthr) {
-      const int ll = e / vpl, i = e - ll * vpl;
-      V r = *reinterpret_cast<const V*>(tile + ll * pitch + i * VW);
-      if (a.epi != EPI_STORE) {
-        const V o = need_old ? dv[e] : V{};
-        vzip(r, o, [&](TS y, TS old) { return epilogue<TS>(a.epi, a.epi_c, (double)y, old); });
-      }
-      dv[e] = r;
+      const TS v = row0[ok ? row : 0];
+      win[w] = ok ? v : (TS)0;
     }
   }
+  double x[CHUNK];
+  rhs_interior<KIND>(a, win, x);
+  if (SOLVE == SOLVE_BND || (SOLVE == SOLVE_NONE && !a.periodic)) rhs_boundary<KIND, FULL>(a, a.wb, p, win, x);
+  // filters add v back here, read from the tile before the result takes its place
+  auto emit = [&](int k, double y) {
+    if (act) {
+      double val = y * a.scale;
+      if (a.addv) val += (double)mo[k];
+      mo[k] = (TS)val;
+    }
+  };
+  if constexpr (SOLVE == SOLVE_NONE) {
+    wave_fence();  // every window is in registers
+#pragma unroll
+    for (int k = 0; k < CHUNK; ++k)
+      if (FULL || k < m) emit(k, x[k]);
+  } else {
+    constexpr bool CYC = SOLVE == SOLVE_CIRC;
+    constexpr bool SHARED = CYC && FULL;
+    // lanes past the last whole line read some exit and drop the result
+    auto exit_of = [&](int q) { return ex[l * P + q < 64 ? l * P + q : 0]; };
+    double e0 = 0.0, e1 = 0.0, b0 = 0.0, b1 = 0.0;
+    with_rows<SOLVE>(a, true, p, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
+    ex[lane] = D2{e0, e1};
+    wave_fence();
+    carry_in<CYC, SHARED, -1>(a, a.kf, p, exit_of, e0, e1);
+    with_rows<SOLVE>(a, true, p, [&](auto rows) {
+      fwd_pass<FULL, true>(rows, x, m, e0, e1);
+      bwd_exit<FULL>(rows, x, m, b0, b1);
+    });
+    // as in line_yz_body: a NaN or infinity spreads to the whole line
+    const unsigned long long bad = __ballot(act && (!__builtin_isfinite(b0) || !__builtin_isfinite(b1)));
+    wave_fence();
+    ex[lane] = D2{b0, b1};
+    wave_fence();
+    carry_in<CYC, SHARED, 1>(a, a.kb, p, exit_of, b0, b1);
+    if (bad & line_lanes(l, P)) b0 = b1 = __builtin_nan("");
+    with_rows<SOLVE>(a, true, p, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
+  }
+  wave_fence();
+  float* o32 = nullptr;
+  if constexpr (sizeof(TS) == 8 && !GRP) o32 = a.out32 ? a.out32 + (E0 - sh) : nullptr;
+  T::store(tile, out + (E0 - sh), sh, end, a.vec, lane, a.epi, a.epi_c, o32, GRP ? 0 : a.only32);
 }
 
-// x lines, software-pipelined through registers (periodic lines of whole
-// 32-row chunks, 16-byte aligned rows, circulant solve or explicit filter).
-// A persistent workgroup walks groups of LX lines through ONE LDS tile: while
-// it solves group g from the tile, the rows of its next group are already in
-// flight from HBM into registers (CHUNK elements per thread, as 16-byte
-// vectors), and they go into the tile once group g's results have left it.
-// Against k_line_x_pipe (a second LDS tile filled by DMA) this keeps the LDS
-// footprint, hence the workgroups per CU, of the one-pass kernel, and pays
-// for the prefetch in registers, which the LDS-bound occupancy leaves free.
-// Every LX * P threads move LX * N elements: CHUNK per thread exactly. The
-// prefetch is issued after the windows have been turned into right-hand
-// sides, so that it overlaps the solve and the stores.
-template <typename TS, int KIND, int SOLVE, int MODE>
-__global__ void __launch_bounds__(WG_MAX) __attribute__((amdgpu_waves_per_eu(2, 8)))
-k_line_x_rpipe(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
-  constexpr int R = Halo<KIND>::R;
-  using CS = typename SolveT<MODE>::type;
-  using V = typename Vec16<TS>::type;
-  constexpr int VW = Vec16<TS>::W;
-  constexpr int NV = CHUNK / VW;  // prefetched vectors per thread
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int N = a.N, LX = a.lx, pitch = a.pitch;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int l = tid % LX, p = tid / LX;
-  const int vpl = N / VW;
-  TS* tile = reinterpret_cast<TS*>(smem);
-  CS* X0 = reinterpret_cast<CS*>(smem + align16((size_t)LX * pitch * sizeof(TS)));
-  CS* X1 = X0 + circ_words<MODE>() * a.P * LX;
-  const int ngroups = (a.nlines + LX - 1) / LX;
-  auto nval_of = [&](int g) {
-    const long long rem = (long long)a.nlines - (long long)g * LX;
-    return (int)(rem < LX ? rem : LX);
-  };
-  V pf[NV];
-  const int s = p * CHUNK;
-  constexpr int m = CHUNK;
-  const bool need_old = (a.epi == EPI_ADD || a.epi == EPI_MAXABS);
-  int g = blockIdx.x;
-  if (g < ngroups) {
-    const int nvec = nval_of(g) * vpl;
-    const V* sv = reinterpret_cast<const V*>(in + (long long)g * LX * N);
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int e = tid + j * nthr;
-      pf[j] = e < nvec ? sv[e] : V{};
-    }
-  }
-  for (; g < ngroups; g += gridDim.x) {
-    const int nval = nval_of(g);
-    const int nvec = nval * vpl;
-    // group g's rows into the tile (the previous group's stores have read it:
-    // barrier at the end of the last iteration)
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int e = tid + j * nthr;
-      if (e < nvec) {
-        const int ll = e / vpl, i = e - ll * vpl;
-        *reinterpret_cast<V*>(tile + ll * pitch + i * VW) = pf[j];
-      }
-    }
-    __syncthreads();
-    const int lr = l < nval ? l : 0;
-    const TS* row0 = tile + lr * pitch;
-    double rhs[CHUNK];
-    {
-      TS win[CHUNK + 2 * R];
-#pragma unroll
-      for (int w = 0; w < CHUNK + 2 * R; ++w) {
-        int row = s - R + w;
-        row = row < 0 ? row + N : (row >= N ? row - N : row);
-        win[w] = row0[row];
-      }
-      rhs_interior<KIND>(a, win, rhs, m);
-    }
-    // the next group's rows travel while this group is solved and stored
-    // (issued once the windows are consumed: their registers take the rows)
-    const int gn = g + gridDim.x;
-    __builtin_amdgcn_sched_barrier(0);  // keep the prefetch below the windows
-    if (gn < ngroups) {
-      const int nvn = nval_of(gn) * vpl;
-      const V* sv = reinterpret_cast<const V*>(in + (long long)gn * LX * N);
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int e = tid + j * nthr;
-        pf[j] = e < nvn ? sv[e] : V{};
-      }
-    }
-    TS* rowo = tile + l * pitch;
-    auto emit = [&](int k, double y) {
-      if (l < nval) {
-        double val = y * a.scale;
-        if (a.addv) val += (double)rowo[s + k];
-        rowo[s + k] = (TS)val;
-      }
-    };
-    if constexpr (SOLVE == SOLVE_CIRC) {
-      // the first carry barrier also retires every window read of the tile
-      solve_chunk_circ<MODE, CS>(a, kmat<MODE>(a, 0), kmat<MODE>(a, 1), p, m, X0, X1, LX, l, rhs, emit);
-    } else {
-      __syncthreads();  // every window read before any result lands in the tile
-#pragma unroll
-      for (int k = 0; k < CHUNK; ++k) emit(k, rhs[k]);
-    }
-    __syncthreads();
-    const long long L0 = (long long)g * LX;
-    if constexpr (sizeof(TS) == 8) {
-      if (a.out32) {
-        // FP64 result rounded to FP32, with or without the FP64 store
-        double* dst = reinterpret_cast<double*>(out) + L0 * N;
-        float* d32 = a.out32 + L0 * N;
-#pragma unroll XU
-        for (int e = tid; e < nvec; e += nthr) {
-          const int ll = e / vpl, i = e - ll * vpl;
-          const double2 r = *reinterpret_cast<const double2*>(tile + ll * pitch + i * VW);
-          if (!a.only32) reinterpret_cast<double2*>(dst)[e] = r;
-          reinterpret_cast<float2*>(d32)[e] = make_float2((float)r.x, (float)r.y);
-        }
-        __syncthreads();  // every read of the tile before the next group lands
-        continue;
-      }
-    }
-    V* dv = reinterpret_cast<V*>(out + L0 * N);
-#pragma unroll XU
-    for (int e = tid; e < nvec; e += nthr) {
-      const int ll = e / vpl, i = e - ll * vpl;
-      V r = *reinterpret_cast<const V*>(tile + ll * pitch + i * VW);
-      if (a.epi != EPI_STORE) {
-        const V o = need_old ? dv[e] : V{};
-        vzip(r, o, [&](TS y, TS old) { return epilogue<TS>(a.epi, a.epi_c, (double)y, old); });
-      }
-      dv[e] = r;
-    }
-    __syncthreads();  // every read of the tile before the next group lands
-  }
+template <typename TS, int KIND, int SOLVE, bool FULL>
+__global__ void __launch_bounds__(64) k_line_x(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
+  line_x_body<TS, KIND, SOLVE, FULL>(a, blockIdx.x, in, out);
 }
 
 // Grouped launches: one launch applies the same operator to the fields of
@@ -1040,15 +506,17 @@ k_line_x_rpipe(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
 // one allocation), with lines of any lengths. Entry j covers workgroups
 // [blk0_j, blk0_{j+1}); a workgroup finds its member by binary search
 // (wave-uniform) and runs the single-field body with that member's line
-// arguments. Workgroups are shaped for the member with the most chunks (or
-// threads); the bodies leave threads without a chunk idle at the barriers.
+// arguments: every member has its own lines per workgroup (x: 64 / P, y/z: as
+// many as P chunk threads each leave room for), so one launch serves all
+// line lengths.
 struct GrpEntry {
   LineArgs a;
   long long off;
   long long blk0;
 };
 
-__device__ __forceinline__ int grp_member(const GrpEntry* __restrict__ g, int M, long long b) {
+template <typename Entry>
+__device__ __forceinline__ int grp_member(const Entry* __restrict__ g, int M, long long b) {
   int lo = 0, hi = M - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -1058,24 +526,242 @@ __device__ __forceinline__ int grp_member(const GrpEntry* __restrict__ g, int M,
   return lo;
 }
 
-template <typename TS, int KIND, int SOLVE, int MODE>
-__global__ void __launch_bounds__(WG_MAX) __attribute__((amdgpu_waves_per_eu(PYR_X_WAVES_PER_EU, 8)))
-k_line_x_grp(const GrpEntry* __restrict__ g, int M, const TS* __restrict__ in, TS* __restrict__ out) {
+template <typename TS, int KIND, int SOLVE>
+__global__ void __launch_bounds__(64) k_line_x_grp(const GrpEntry* __restrict__ g, int M, const TS* __restrict__ in,
+                                                   TS* __restrict__ out) {
   const int j = grp_member(g, M, blockIdx.x);
   // a private copy: its fields load once (wave-uniform) and no store of the
   // body can alias them
   const LineArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
-  line_x_body<TS, KIND, SOLVE, MODE, false, true>(a, (long long)blockIdx.x - b0, in + off, out + off);
+  line_x_body<TS, KIND, SOLVE, false, true>(a, (long long)blockIdx.x - b0, in + off, out + off);
 }
 
-template <typename TS, int KIND, int SOLVE, int MODE, int LY, int PRE>
-__global__ void __launch_bounds__(WG_MAX) __attribute__((amdgpu_waves_per_eu(YzWaves<TS, SOLVE, MODE, PRE>::v, 8)))
-k_line_yz_grp(const GrpEntry* __restrict__ g, int M, const TS* __restrict__ in, TS* __restrict__ out) {
+template <typename TS, int KIND, int SOLVE, int PRE>
+__global__ void __launch_bounds__(WG_MAX) k_line_yz_grp(const GrpEntry* __restrict__ g, int M,
+                                                        const TS* __restrict__ in, TS* __restrict__ out) {
   const int j = grp_member(g, M, blockIdx.x);
   const LineArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
-  line_yz_body<TS, KIND, SOLVE, MODE, LY, false, PRE, true>(a, (long long)blockIdx.x - b0, in + off, out + off);
+  line_yz_body<TS, KIND, SOLVE, false, PRE, true>(a, (long long)blockIdx.x - b0, in + off, out + off);
+}
+
+// --- refined FP32 solve of bounded lines (pyr_refined.hpp) -------------------
+// Threads are shaped as in the FP64 kernels above, with up to 32 rows each and
+// workgroups of 512 (x: four waves, each with its own lines and tile). What
+// bounds these kernels is the latency of one workgroup: the factors come from
+// the class tables in LDS (one 16-byte read per row and table quarter instead
+// of nine 4-byte loads from a whole-line table in memory), the reduced rows as
+// 16-byte loads of the chunks within reach, and the boundary rows' terms as
+// independent loads.
+constexpr int REF_THREADS = 512;
+constexpr int REF_X_WAVES = 4;
+
+// class tables into LDS
+__device__ __forceinline__ void ref_stage(const RefArgs& a, float* tab) {
+  for (int e = threadIdx.x; e < NCLS * RCHUNK * CROW / 4; e += blockDim.x)
+    reinterpret_cast<F4*>(tab)[e] = reinterpret_cast<const F4*>(a.cls)[e];
+}
+
+template <int KIND, int PRE>
+__device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, const float* __restrict__ in,
+                                            float* __restrict__ out) {
+  constexpr int R = Halo<KIND>::R;
+  __shared__ __align__(16) float tab[NCLS * RCHUNK * CROW];
+  __shared__ __align__(16) F4 Y0[REF_THREADS], Y1[REF_THREADS];
+  __shared__ float ends[2 * (ENDS + 1) * 64];
+  __shared__ int bad[64];
+  ref_stage(a, tab);
+  const int LY = a.lines;
+  const int lane = threadIdx.x & (LY - 1);
+  const int p = (int)threadIdx.x >> __builtin_ctz(LY);
+  if (p == 0) bad[lane] = 0;
+  const bool act = p < a.P;
+  const long long L = blk * LY + lane;
+  const long long Lc = L < a.nlines ? L : (long long)a.nlines - 1;
+  const int lane_off = (int)(((Lc % a.A) + a.B * (Lc / a.A)) * (long long)sizeof(float));
+  const int rb = (int)(a.stride * (long long)sizeof(float));
+  const int s = p * a.mb + (p < a.mx ? p : a.mx);
+  const int m = a.mb + (p < a.mx ? 1 : 0);
+  const __amdgpu_buffer_rsrc_t rin = buf_rsrc(in, a.nbytes), rout = buf_rsrc(out, a.nbytes);
+  auto off_of = [&](int row) { return (int)((unsigned)lane_off + (unsigned)row * (unsigned)rb); };
+  float pre[PRE == PRE_OLD ? RCHUNK : 1];
+  if constexpr (PRE == PRE_OLD) {
+#pragma unroll
+    for (int k = 0; k < RCHUNK; ++k) pre[k] = buf_load(0.0f, rout, act && k < m ? off_of(s + k) : OOB, 0);
+  }
+  // rows beyond the ends read 0
+  float win[RCHUNK + 2 * R];
+#pragma unroll
+  for (int w = 0; w < RCHUNK + 2 * R; ++w) {
+    const int row = s - R + w;
+    win[w] = buf_load(0.0f, rin, act && w < m + 2 * R && row >= 0 && row < a.N ? off_of(row) : OOB, 0);
+  }
+  double rhs[RCHUNK];
+  ref_rhs_interior<KIND>(a, win, rhs, m);
+  if (act && (p == 0 || p == a.P - 1)) {
+    // the boundary rows name any of the eight rows at their end: this thread's
+    // copy of them in LDS, indexed at run time (no other thread reads it)
+    float* mine = ends + (p == 0 ? 0 : ENDS + 1) * 64 + lane;
+    mine[ENDS * 64] = 0.0f;
+    if (p == 0) {
+#pragma unroll
+      for (int k = 0; k < ENDS / 2; ++k) mine[k * 64] = win[k + R];
+    }
+    if (p == a.P - 1) {
+#pragma unroll
+      for (int k = 0; k < RCHUNK; ++k) {
+        const int j = k - (a.mb - ENDS / 2);
+        if (j >= 0 && j < ENDS / 2) mine[(ENDS / 2 + j) * 64] = win[k + R];
+      }
+    }
+    ref_rhs_boundary(a, p, rhs, [&](int slot) { return mine[slot * 64]; });
+  }
+  __syncthreads();  // class tables visible
+  const float* t = tab + ref_class(p, a.P, a.mx) * (RCHUNK * CROW);
+  float x[RCHUNK], d[RCHUNK], z[4], e4[4];
+#pragma unroll
+  for (int k = 0; k < RCHUNK; ++k) x[k] = (float)rhs[k];
+  if (act) {
+    ref_local_solve(t, m, x);
+    ref_edges(x, m, e4);
+    Y0[p * LY + lane] = F4{e4[0], e4[1], e4[2], e4[3]};
+    // as in line_yz_body: a NaN or infinity spreads to the whole line
+    if (!__builtin_isfinite(e4[0]) || !__builtin_isfinite(e4[1])) bad[lane] = 1;
+  }
+  __syncthreads();
+  if (act) {
+    ref_neighbours(a, p, [&](int q) { return Y0[q * LY + lane]; }, z);
+    if (bad[lane]) z[0] = z[1] = z[2] = z[3] = __builtin_nanf("");
+    ref_spike(t, m, z, x);
+    ref_residual(a, p, m, rhs, x, z, d);
+    ref_local_solve(t, m, d);
+    ref_edges(d, m, e4);
+    Y1[p * LY + lane] = F4{e4[0], e4[1], e4[2], e4[3]};
+  }
+  __syncthreads();
+  if (!act || L >= a.nlines) return;
+  ref_neighbours(a, p, [&](int q) { return Y1[q * LY + lane]; }, z);
+  ref_spike(t, m, z, d);
+#pragma unroll
+  for (int k = 0; k < RCHUNK; ++k) {
+    if (k < m) {
+      double val = ((double)x[k] + (double)d[k]) * a.scale;
+      if constexpr (PRE == PRE_V) val += (double)win[k + R];
+      float old = 0.0f;
+      if constexpr (PRE == PRE_OLD) old = pre[k];
+      if constexpr (PRE == PRE_V)
+        if (a.epi == EPI_ADD || a.epi == EPI_MAXABS) old = buf_load(0.0f, rout, off_of(s + k), 0);
+      buf_store(epilogue<float>(a.epi, a.epi_c, val, old), rout, off_of(s + k), 0);
+    }
+  }
+}
+
+template <int KIND>
+__device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, const float* __restrict__ in,
+                                           float* __restrict__ out) {
+  constexpr int R = Halo<KIND>::R;
+  constexpr int NW = REF_X_WAVES;
+  using T = XTile<float, RCHUNK, false>;
+  __shared__ __align__(16) float tab[NCLS * RCHUNK * CROW];
+  __shared__ __align__(16) float tiles[NW][T::SIZE];
+  __shared__ __align__(16) F4 ex[NW][64];
+  ref_stage(a, tab);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  float* tile = tiles[wave];
+  const int N = a.N, P = a.P;
+  const long long L0 = (blk * NW + wave) * a.lines;
+  const long long rem = (long long)a.nlines - L0;
+  if (rem <= 0) return;
+  const int nval = (int)(rem < a.lines ? rem : a.lines);
+  const long long E0 = L0 * N;
+  const int sh = a.vec ? (int)(E0 & (T::VW - 1)) : 0;
+  const int end = sh + nval * N;
+  T::load(tile, in + (E0 - sh), end, (long long)a.nlines * N - (E0 - sh), a.vec, lane);
+  wave_fence();
+  const int l = lane / P, p = lane - l * P;
+  const bool act = l < nval;
+  const int s = p * a.mb + (p < a.mx ? p : a.mx);
+  const int m = a.mb + (p < a.mx ? 1 : 0);
+  float* row0 = tile + sh + (act ? l * N : 0);
+  float win[RCHUNK + 2 * R];
+#pragma unroll
+  for (int w = 0; w < RCHUNK + 2 * R; ++w) {
+    const int row = s - R + w;
+    const bool ok = w < m + 2 * R && row >= 0 && row < N;
+    const float v = row0[ok ? row : 0];
+    win[w] = ok ? v : 0.0f;
+  }
+  double rhs[RCHUNK];
+  ref_rhs_interior<KIND>(a, win, rhs, m);
+  ref_rhs_boundary(a, p, rhs, [&](int slot) { return end_value(slot, N, [&](int i) { return row0[i]; }); });
+  const float* t = tab + ref_class(p, P, a.mx) * (RCHUNK * CROW);
+  float x[RCHUNK], d[RCHUNK], z[4], e4[4];
+#pragma unroll
+  for (int k = 0; k < RCHUNK; ++k) x[k] = (float)rhs[k];
+  auto edges_of = [&](int q) { return ex[wave][l * P + q < 64 ? l * P + q : 0]; };
+  ref_local_solve(t, m, x);
+  ref_edges(x, m, e4);
+  ex[wave][lane] = F4{e4[0], e4[1], e4[2], e4[3]};
+  const unsigned long long bad = __ballot(act && (!__builtin_isfinite(e4[0]) || !__builtin_isfinite(e4[1])));
+  wave_fence();
+  ref_neighbours(a, p, edges_of, z);
+  if (bad & line_lanes(l, P)) z[0] = z[1] = z[2] = z[3] = __builtin_nanf("");
+  ref_spike(t, m, z, x);
+  ref_residual(a, p, m, rhs, x, z, d);
+  ref_local_solve(t, m, d);
+  ref_edges(d, m, e4);
+  wave_fence();
+  ex[wave][lane] = F4{e4[0], e4[1], e4[2], e4[3]};
+  wave_fence();
+  ref_neighbours(a, p, edges_of, z);
+  ref_spike(t, m, z, d);
+#pragma unroll
+  for (int k = 0; k < RCHUNK; ++k) {
+    if (act && k < m) {
+      double val = ((double)x[k] + (double)d[k]) * a.scale;
+      if (a.addv) val += (double)win[k + R];
+      row0[s + k] = (float)val;
+    }
+  }
+  wave_fence();
+  T::store(tile, out + (E0 - sh), sh, end, a.vec, lane, a.epi, a.epi_c, nullptr, 0);
+}
+
+struct RefEntry {
+  RefArgs a;
+  long long off;
+  long long blk0;
+};
+
+template <int KIND, int PRE>
+__global__ void __launch_bounds__(REF_THREADS) k_ref_yz(RefArgs a, const float* __restrict__ in,
+                                                        float* __restrict__ out) {
+  ref_yz_body<KIND, PRE>(a, blockIdx.x, in, out);
+}
+template <int KIND>
+__global__ void __launch_bounds__(64 * REF_X_WAVES) __attribute__((amdgpu_waves_per_eu(2, 8))) k_ref_x(RefArgs a, const float* __restrict__ in,
+                                                            float* __restrict__ out) {
+  ref_x_body<KIND>(a, blockIdx.x, in, out);
+}
+template <int KIND, int PRE>
+__global__ void __launch_bounds__(REF_THREADS) k_ref_yz_grp(const RefEntry* __restrict__ g, int M,
+                                                            const float* __restrict__ in, float* __restrict__ out) {
+  const int j = grp_member(g, M, blockIdx.x);
+  const RefArgs a = g[j].a;
+  const long long off = g[j].off, b0 = g[j].blk0;
+  ref_yz_body<KIND, PRE>(a, (long long)blockIdx.x - b0, in + off, out + off);
+}
+template <int KIND>
+__global__ void __launch_bounds__(64 * REF_X_WAVES) __attribute__((amdgpu_waves_per_eu(2, 8))) k_ref_x_grp(const RefEntry* __restrict__ g, int M,
+                                                                const float* __restrict__ in,
+                                                                float* __restrict__ out) {
+  const int j = grp_member(g, M, blockIdx.x);
+  const RefArgs a = g[j].a;
+  const long long off = g[j].off, b0 = g[j].blk0;
+  ref_x_body<KIND>(a, (long long)blockIdx.x - b0, in + off, out + off);
 }
 
 // null operator of a direction with fewer than 4 points (zero or copy)
@@ -1123,16 +809,16 @@ __global__ void k_rk_update(long long n, const TF* __restrict__ F, double* __res
 // ---------------------------------------------------------------------------
 // context
 // ---------------------------------------------------------------------------
+// Device addresses of a plan's tables, all inside the context's one table
+// allocation (pyr_ctx::tables).
 struct DevPlan {
-  void* mem = nullptr;  // one allocation holding every table
-  const int* cstart = nullptr;
-  const double *lu = nullptr, *rc = nullptr, *gsel = nullptr, *band = nullptr, *bcoef = nullptr;
-  const float *lu32 = nullptr, *rc32 = nullptr, *gsel32 = nullptr;
-  const short* bidx = nullptr;
-  const int* bnt = nullptr;
-  int ntab = 0;
-  const double *kf = nullptr, *kb = nullptr;
-  const float *kf32 = nullptr, *kb32 = nullptr;
+  const double *wb = nullptr, *kf = nullptr, *kb = nullptr, *tf = nullptr, *tb = nullptr, *tg = nullptr;
+};
+
+struct DevRefPlan {
+  const float *cls = nullptr, *g = nullptr;
+  const double *be = nullptr, *bcoef = nullptr;
+  const int* bidx = nullptr;
 };
 
 struct pyr_ctx {
@@ -1151,24 +837,29 @@ struct pyr_ctx {
   bool has_anti[3] = {false, false, false};
   OpPlan plan_a[NOPS][3];
   DevPlan dplan_a[NOPS][3];
+  // refined FP32 solve of the bounded implicit lines (N > 0), both members
+  RefPlan rplan[NOPS][3], rplan_a[NOPS][3];
+  DevRefPlan drplan[NOPS][3], drplan_a[NOPS][3];
+  void* tables = nullptr;  // the tables of every plan
   void* field_tmp[2] = {nullptr, nullptr};  // one field-sized temp per precision
   int periodic_solver = PYR_PSOLVE_CIRCULANT;
   int r32_solve = PYR_R32_SOLVE_REFINED;
-  int x_lds_kb = 40;                        // LDS budget of one x-line workgroup
-  int yz_pipe = 1;                           // pipelined y/z kernels where the shape allows
-  // per operator, direction and solve mode (MODE_*): tuned values of the two
-  // knobs above, -1 = the context default (pyr_set_tuning)
-  int yz_lines = 0;                          // lines per plain y/z workgroup (0: 64, or 32 past 8 chunks; 16, 32)
-  int tune_xlds[NOPS][3][3];
-  int tune_pipe[NOPS][3][3];
-  int tune_ly[NOPS][3][3];
-  // per operator and direction: FP32 solve arithmetic (PYR_R32_SOLVE_*), -1 = r32_solve
+  // launch knobs (pyr_set_tuning): lines per y/z workgroup (0: the rule of
+  // yz_lines), and the y/z kernel with runtime row counts; per operator,
+  // direction and field width (0 FP64, 1 FP32), -1 / 0 = the default
+  int yz_lines = 0;
+  int tune_ly[NOPS][3][2];
+  int tune_rt[NOPS][3][2] = {};
+  // settings that no longer change a launch, kept as group members must agree
+  // on them: the x-line LDS budget, the periodic solver (above) and the solve
+  // arithmetic of FP32 fields per operator and direction (-1 = r32_solve)
+  int x_lds_kb = 40;
   int tune_solve[NOPS][3];
   pyr_ctx() {
     for (int o = 0; o < NOPS; ++o)
       for (int d = 0; d < 3; ++d) {
         tune_solve[o][d] = -1;
-        for (int m = 0; m < 3; ++m) tune_xlds[o][d][m] = tune_pipe[o][d][m] = tune_ly[o][d][m] = -1;
+        for (int w = 0; w < 2; ++w) tune_ly[o][d][w] = -1;
       }
   }
   int ncu = 256;                             // compute units of the device
@@ -1178,104 +869,89 @@ struct pyr_ctx {
   size_t npts() const { return (size_t)n[0] * n[1] * n[2]; }
 };
 
-static int upload_plan(const OpPlan& pl, DevPlan& d) {
-  if (pl.null_op) return 0;
-  const size_t n = pl.N, P = pl.P;
-  std::vector<std::pair<const void*, size_t>> parts;
-  auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
-  size_t off = 0;
-  size_t o_cs = off; off = align(off + (P + 1) * sizeof(int));
-  // lu|rc|gsel contiguous (one block copied to LDS by the kernels)
-  size_t o_lu = off;
-  size_t o_rc = o_lu + n * 5 * sizeof(double);
-  size_t o_gs = o_rc + n * 4 * sizeof(double);
-  off = align(o_gs + P * 16 * P * sizeof(double));
-  size_t o_bd = off; off = align(off + n * 5 * sizeof(double));
-  size_t o_bc = off; off = align(off + 2 * NB * MAXT * sizeof(double));
-  size_t o_bi = off; off = align(off + 2 * NB * MAXT * 2 * sizeof(short));
-  size_t o_bn = off; off = align(off + 2 * NB * sizeof(int));
-  size_t o_lu32 = off;
-  size_t o_rc32 = o_lu32 + n * 5 * sizeof(float);
-  size_t o_gs32 = o_rc32 + n * 4 * sizeof(float);
-  off = align(o_gs32 + P * 16 * P * sizeof(float));
-  const size_t nk = pl.circ ? 4 * P * P : 0;  // 2P x 2P carry rows
-  size_t o_kf = off; off = align(off + nk * sizeof(double));
-  size_t o_kb = off; off = align(off + nk * sizeof(double));
-  size_t o_kf32 = off; off = align(off + nk * sizeof(float));
-  size_t o_kb32 = off; off = align(off + nk * sizeof(float));
-  std::vector<unsigned char> host(off, 0);
-  std::memcpy(&host[o_cs], pl.cstart.data(), (P + 1) * sizeof(int));
-  std::memcpy(&host[o_lu], pl.lu.data(), n * 5 * sizeof(double));
-  std::memcpy(&host[o_rc], pl.rc.data(), n * 4 * sizeof(double));
-  std::memcpy(&host[o_gs], pl.gsel.data(), P * 16 * P * sizeof(double));
-  std::memcpy(&host[o_bd], pl.band.data(), n * 5 * sizeof(double));
-  std::memcpy(&host[o_bc], pl.bcoef.data(), 2 * NB * MAXT * sizeof(double));
-  std::memcpy(&host[o_bi], pl.bidx.data(), 2 * NB * MAXT * 2 * sizeof(short));
-  std::memcpy(&host[o_bn], pl.bnt.data(), 2 * NB * sizeof(int));
-  float* lu32 = reinterpret_cast<float*>(&host[o_lu32]);
-  float* rc32 = reinterpret_cast<float*>(&host[o_rc32]);
-  float* gs32 = reinterpret_cast<float*>(&host[o_gs32]);
-  for (size_t i = 0; i < n * 5; ++i) lu32[i] = (float)pl.lu[i];
-  for (size_t i = 0; i < n * 4; ++i) rc32[i] = (float)pl.rc[i];
-  for (size_t i = 0; i < P * 16 * P; ++i) gs32[i] = (float)pl.gsel[i];
-  if (nk) {
-    std::memcpy(&host[o_kf], pl.kf.data(), nk * sizeof(double));
-    std::memcpy(&host[o_kb], pl.kb.data(), nk * sizeof(double));
-    float* kf32 = reinterpret_cast<float*>(&host[o_kf32]);
-    float* kb32 = reinterpret_cast<float*>(&host[o_kb32]);
-    for (size_t i = 0; i < nk; ++i) {
-      kf32[i] = (float)pl.kf[i];
-      kb32[i] = (float)pl.kb[i];
-    }
+// The tables of all plans of a context back to back, 256-byte aligned: added
+// one by one, then uploaded in one piece.
+struct TableImage {
+  std::vector<unsigned char> host;
+  template <typename T>
+  size_t add(const std::vector<T>& t) {
+    const size_t at = host.size();
+    host.resize((at + t.size() * sizeof(T) + 255) & ~(size_t)255, 0);
+    if (!t.empty()) std::memcpy(host.data() + at, t.data(), t.size() * sizeof(T));
+    return at;
   }
-  HIPCHECK(hipMalloc(&d.mem, off));
-  HIPCHECK(hipMemcpy(d.mem, host.data(), off, hipMemcpyHostToDevice));
-  unsigned char* b = static_cast<unsigned char*>(d.mem);
-  d.cstart = reinterpret_cast<const int*>(b + o_cs);
-  d.lu = reinterpret_cast<const double*>(b + o_lu);
-  d.rc = reinterpret_cast<const double*>(b + o_rc);
-  d.gsel = reinterpret_cast<const double*>(b + o_gs);
-  d.band = reinterpret_cast<const double*>(b + o_bd);
-  d.bcoef = reinterpret_cast<const double*>(b + o_bc);
-  d.bidx = reinterpret_cast<const short*>(b + o_bi);
-  d.bnt = reinterpret_cast<const int*>(b + o_bn);
-  d.lu32 = reinterpret_cast<const float*>(b + o_lu32);
-  d.rc32 = reinterpret_cast<const float*>(b + o_rc32);
-  d.gsel32 = reinterpret_cast<const float*>(b + o_gs32);
-  d.ntab = (int)(n * 9 + P * 16 * P);
-  if (nk) {
-    d.kf = reinterpret_cast<const double*>(b + o_kf);
-    d.kb = reinterpret_cast<const double*>(b + o_kb);
-    d.kf32 = reinterpret_cast<const float*>(b + o_kf32);
-    d.kb32 = reinterpret_cast<const float*>(b + o_kb32);
-  }
+};
+
+// adds the tables of a plan to the image; the addresses are offsets until
+// rebase() is called with the image's device address
+static void add_plan(TableImage& im, const OpPlan& pl, DevPlan& d) {
+  auto put = [&](const std::vector<double>& t) { return reinterpret_cast<const double*>(im.add(t)); };
+  d.wb = put(pl.wb);
+  d.kf = put(pl.kf);
+  d.kb = put(pl.kb);
+  d.tf = put(pl.tf);
+  d.tb = put(pl.tb);
+  d.tg = put(pl.tg);
+}
+static void add_plan(TableImage& im, const RefPlan& pl, DevRefPlan& d) {
+  if (pl.N == 0) return;
+  d.cls = reinterpret_cast<const float*>(im.add(pl.cls));
+  d.g = reinterpret_cast<const float*>(im.add(pl.g));
+  d.be = reinterpret_cast<const double*>(im.add(pl.be));
+  d.bcoef = reinterpret_cast<const double*>(im.add(pl.bcoef));
+  d.bidx = reinterpret_cast<const int*>(im.add(pl.bidx));
+}
+template <typename T>
+static void rebase(const T*& p, const unsigned char* base) {
+  p = reinterpret_cast<const T*>(base + reinterpret_cast<size_t>(p));
+}
+static void rebase(DevPlan& d, const unsigned char* base) {
+  for (const double** p : {&d.wb, &d.kf, &d.kb, &d.tf, &d.tb, &d.tg}) rebase(*p, base);
+}
+static void rebase(DevRefPlan& d, const unsigned char* base) {
+  rebase(d.cls, base);
+  rebase(d.g, base);
+  rebase(d.be, base);
+  rebase(d.bcoef, base);
+  rebase(d.bidx, base);
+}
+
+// every plan's tables onto the device: one allocation and one copy
+static int upload_plans(pyr_ctx* c) {
+  TableImage im;
+  auto each = [&](auto f) {
+    for (int op = 0; op < NOPS; ++op)
+      for (int d = 0; d < 3; ++d) {
+        f(c->plan[op][d], c->dplan[op][d]);
+        f(c->rplan[op][d], c->drplan[op][d]);
+        if (!c->has_anti[d]) continue;
+        f(c->plan_a[op][d], c->dplan_a[op][d]);
+        f(c->rplan_a[op][d], c->drplan_a[op][d]);
+      }
+  };
+  each([&](const auto& pl, auto& d) { add_plan(im, pl, d); });
+  if (im.host.empty()) return 0;
+  HIPCHECK(hipMalloc(&c->tables, im.host.size()));
+  HIPCHECK(hipMemcpy(c->tables, im.host.data(), im.host.size(), hipMemcpyHostToDevice));
+  each([&](const auto&, auto& d) { rebase(d, static_cast<const unsigned char*>(c->tables)); });
   return 0;
 }
 
 // host pointers of the same tables (host emulation)
-static void host_tables(const OpPlan& pl, DevPlan& d, std::vector<float>& lu32,
-                        std::vector<float>& rc32, std::vector<float>& gs32,
-                        std::vector<float>& kf32, std::vector<float>& kb32) {
-  lu32.assign(pl.lu.begin(), pl.lu.end());
-  rc32.assign(pl.rc.begin(), pl.rc.end());
-  gs32.assign(pl.gsel.begin(), pl.gsel.end());
-  kf32.assign(pl.kf.begin(), pl.kf.end());
-  kb32.assign(pl.kb.begin(), pl.kb.end());
-  d.kf = pl.kf.data();
-  d.kb = pl.kb.data();
-  d.kf32 = kf32.data();
-  d.kb32 = kb32.data();
-  d.cstart = pl.cstart.data();
-  d.lu = pl.lu.data();
-  d.rc = pl.rc.data();
-  d.gsel = pl.gsel.data();
-  d.band = pl.band.data();
+static void host_ref_tables(const RefPlan& pl, DevRefPlan& d) {
+  d.cls = pl.cls.data();
+  d.g = pl.g.data();
+  d.be = pl.be.data();
   d.bcoef = pl.bcoef.data();
   d.bidx = pl.bidx.data();
-  d.bnt = pl.bnt.data();
-  d.lu32 = lu32.data();
-  d.rc32 = rc32.data();
-  d.gsel32 = gs32.data();
+}
+static void host_tables(const OpPlan& pl, DevPlan& d) {
+  d.wb = pl.wb.data();
+  d.kf = pl.kf.data();
+  d.kb = pl.kb.data();
+  d.tf = pl.tf.data();
+  d.tb = pl.tb.data();
+  d.tg = pl.tg.data();
 }
 
 static LineArgs make_args(const pyr_ctx* c, const OpPlan& pl, const DevPlan& d, int dir, int epi,
@@ -1301,274 +977,186 @@ static LineArgs make_args(const pyr_ctx* c, const OpPlan& pl, const DevPlan& d, 
   a.epi = epi;
   a.scale = pl.scale;
   a.epi_c = ec;
-  for (int i = 0; i < 9; ++i) a.w[i] = pl.w[i];
-  a.cstart = d.cstart; a.lu = d.lu; a.rc = d.rc; a.gsel = d.gsel; a.band = d.band;
-  a.lu32 = d.lu32; a.rc32 = d.rc32; a.gsel32 = d.gsel32;
-  a.tab64 = d.lu; a.tab32 = d.lu32; a.ntab = d.ntab;
-  a.bcoef = d.bcoef; a.bidx = d.bidx; a.bnt = d.bnt;
-  a.p1 = pl.p1; a.p2 = pl.p2; a.invc = pl.invc;
-  a.p1f = (float)pl.p1; a.p2f = (float)pl.p2; a.invcf = (float)pl.invc;
-  for (int i = 0; i < 3; ++i) a.bd[i] = pl.bd[i];
-  a.kf = d.kf; a.kb = d.kb; a.kf32 = d.kf32; a.kb32 = d.kb32;
+  a.mb = pl.mb;
+  a.mx = pl.mx;
+  for (int i = 0; i < 4; ++i) a.w[i] = pl.w[i];
+  a.wb = d.wb;
+  a.p1 = pl.p1;
+  a.p2 = pl.p2;
+  a.W = pl.W;
+  a.kp = pl.kp;
+  a.kf = d.kf;
+  a.kb = d.kb;
+  a.tf = d.tf;
+  a.tb = d.tb;
+  a.tg = d.tg;
+  a.tlo = pl.tlo;
   return a;
 }
 
-// solve used for a plan: explicit, chunked LU, or circulant (periodic lines)
-static int plan_solve(const pyr_ctx* c, const OpPlan& pl) {
+// line arguments of the refined solve, from those of the same operator
+static RefArgs make_ref_args(const LineArgs& l, const RefPlan& pl, const DevRefPlan& d) {
+  RefArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.N = pl.N; a.P = pl.P; a.mb = pl.mb; a.mx = pl.mx;
+  a.nlines = l.nlines; a.nbytes = l.nbytes;
+  a.A = l.A; a.B = l.B; a.stride = l.stride;
+  a.addv = l.addv; a.epi = l.epi; a.epi_c = l.epi_c;
+  a.scale = pl.scale;
+  for (int i = 0; i < 9; ++i) a.w[i] = pl.w[i];
+  for (int i = 0; i < 5; ++i) a.bd[i] = pl.bd[i];
+  a.Wg = pl.Wg;
+  a.cls = d.cls; a.g = d.g; a.be = d.be; a.bcoef = d.bcoef; a.bidx = d.bidx;
+  return a;
+}
+
+// solve used for a plan: explicit, bounded lines, or periodic lines
+static int plan_solve(const OpPlan& pl) {
   if (!pl.implicit) return SOLVE_NONE;
-  if (pl.circ && c->periodic_solver == PYR_PSOLVE_CIRCULANT) return SOLVE_CIRC;
-  return SOLVE_LU;
+  return pl.periodic ? SOLVE_CIRC : SOLVE_BND;
 }
 
 // ---------------------------------------------------------------------------
 // launch
 // ---------------------------------------------------------------------------
-template <typename K>
-static int set_lds(K kernel, size_t bytes) {
-  if (bytes > 64 * 1024)
-    HIPCHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-  return 0;
+// LDS of a y/z workgroup of nthr chunk threads: two exchange buffers and one
+// flag per line.
+static size_t yz_lds(int nthr, int lines) { return 2 * (size_t)nthr * sizeof(D2) + (size_t)lines * sizeof(int); }
+
+// Lines per y/z workgroup (forced: the tuned value, 0 = none). At 256^3 32
+// lines measured fastest for FP64 fields (d1 y 54 us; 16 lines 58, 64 lines
+// 64: one workgroup of 16 waves fills a CU alone) and for FP32 y lines (33
+// us); FP32 z lines, whose rows are a plane apart, gain from 256-byte rows (64
+// lines 36 us, 32 lines 41). Lines of more than 32 chunks leave room for 16
+// in a workgroup. Fields too small to give every CU a workgroup take 16.
+static int yz_lines(int P, int nlines, int dir, int elem, int forced, int ncu) {
+  int ly = forced > 0 ? forced : (elem == 4 && dir == 2 ? 64 : 32);
+  while (ly > 16 && ly * P > WG_MAX) ly /= 2;
+  if (forced <= 0)
+    while (ly > 16 && nlines < ly * ncu) ly /= 2;
+  return ly;
 }
 
-template <typename TS, int KIND, int SOLVE, int MODE, int LY, bool FULL>
-static int launch_yz(pyr_ctx* c, int pre, dim3 grid, dim3 block, size_t shm, const LineArgs& a,
-                     const TS* in, TS* out) {
-  auto k = k_line_yz<TS, KIND, SOLVE, MODE, LY, FULL, PRE_NONE>;
-#if PYR_PREFETCH
-  // filters only exist for the r4 kind; accumulating epilogues for every kind
-  if (pre == PRE_V) {
-    if constexpr (KIND == K_R4) k = k_line_yz<TS, KIND, SOLVE, MODE, LY, FULL, PRE_V>;
-    else return fail("filter epilogue on a non-filter kernel");
-  } else if (pre == PRE_OLD) {
-    k = k_line_yz<TS, KIND, SOLVE, MODE, LY, FULL, PRE_OLD>;
-  }
-#else
-  if (pre != PRE_NONE) k = k_line_yz<TS, KIND, SOLVE, MODE, LY, FULL, PRE_LATE>;
-#endif
-  if (set_lds(k, shm)) return 1;
-  hipLaunchKernelGGL(k, grid, block, shm, c->stream, a, in, out);
-  return 0;
-}
-
-// Pipelined y/z launch when the line shape allows it (see k_line_yz_pipe);
-// returns 1 if launched, 0 if the caller should use k_line_yz, -1 on error.
-template <typename TS, int KIND, int SOLVE, int MODE>
-static int launch_yz_pipe(pyr_ctx* c, int pre, const LineArgs& a, const TS* in, TS* out) {
-  if constexpr (SOLVE != SOLVE_CIRC && SOLVE != SOLVE_NONE) {
-    return 0;
-  } else {
-    using CS = typename SolveT<MODE>::type;
-    constexpr int LG = 32;
-    // Measured on gfx950 at 256^3: with FP32 fields the pipelined kernel wins
-    // for the explicit filter (gbar y 54 -> 28 us) and the refined circulant
-    // solve (d1 y 51 -> 41 us), but not with accumulating epilogues; FP64
-    // fields leave too few waves per CU once two tiles fit in LDS.
-    if constexpr (sizeof(TS) != 4 || (SOLVE == SOLVE_CIRC && MODE != MODE_R32)) {
-      return 0;
-    } else {
-    if (pre == PRE_OLD) return 0;
-    if (LG * a.P > WG_MAX) return 0;
-    // whole waves (the copy loop strides by the wave count)
-    if (!c->yz_pipe || !a.periodic || a.N % CHUNK != 0 || (LG * a.P) % 64 != 0) return 0;
-    if (a.A % LG != 0 || a.nlines % LG != 0) return 0;
-    if ((uintptr_t)in % 16 != 0 || (a.stride * sizeof(TS)) % 16 != 0 || (a.B * sizeof(TS)) % 16 != 0) return 0;
-    constexpr int R = Halo<KIND>::R;
-    constexpr int RPI = 64 / (LG * (int)sizeof(TS) / 16);
-    // NT tile rows as in the kernel: N lines rows + 2R wrapped rows, in runs of RPI
-    const size_t tile_rows = (size_t)((a.N + 2 * R + RPI - 1) / RPI) * RPI;
-    const size_t tiles = align16(2 * tile_rows * LG * sizeof(TS));
-    // carry exchange and carry rows only for the circulant solve
-    const size_t shm = tiles + (SOLVE == SOLVE_CIRC ? (2 * (size_t)4 * a.P * LG + 2 * (size_t)4 * a.P * a.P) * sizeof(CS) : 0);
-    if (shm > 80 * 1024) return 0;
-    const int per_cu = (int)((160 * 1024) / shm);
-    const int ngroups = a.nlines / LG;
-    const int nblocks = std::min(ngroups, std::max(1, c->ncu * per_cu));
-    auto k = k_line_yz_pipe<TS, KIND, SOLVE, MODE, LG, PRE_NONE>;
-    if (pre == PRE_V) {
-      if constexpr (KIND == K_R4) k = k_line_yz_pipe<TS, KIND, SOLVE, MODE, LG, PRE_V>;
-      else return 0;
-    }
-    if (set_lds(k, shm)) return -1;
-    hipLaunchKernelGGL(k, dim3(nblocks), dim3(LG, a.P), shm, c->stream, a, in, out);
-    return 1;
-    }
-  }
-}
-
-template <typename TS, int KIND, int SOLVE, int MODE, bool FULL>
-static int launch_typed(pyr_ctx* c, int dir, LineArgs a, const TS* in, TS* out) {
-  using CS = typename SolveT<MODE>::type;
-  const int P = a.P;
-  // LU tables go to LDS unless they are too large (long lines): then the
-  // solve reads them from global memory (L2-resident, shared by all lines)
-  const size_t stage_full = SOLVE == SOLVE_LU ? stage_bytes<MODE>(a.ntab, a.N) : 0;
-  a.gtab = stage_full > STAGE_MAX_BYTES;
-  const size_t stage = a.gtab ? 0 : stage_full;
+template <typename TS, int KIND, int SOLVE, bool FULL>
+static int launch_typed(pyr_ctx* c, int dir, int forced, LineArgs a, const TS* in, TS* out) {
   if (dir == 0) {
-    constexpr int VW = Vec16<TS>::W;
-    a.vec = (a.N % VW == 0) && ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0);
-    a.pitch = a.vec ? a.N + VW : a.N + 1;
-    auto lds = [&](int lx) {
-      const size_t tile = align16((size_t)lx * a.pitch * sizeof(TS));
-      if (SOLVE == SOLVE_CIRC) return tile + 2 * align16((size_t)circ_words<MODE>() * P * lx * sizeof(CS));
-      if (SOLVE == SOLVE_LU) {
-        const size_t work = align16((size_t)4 * P * lx * sizeof(CS)) + stage;
-        return tile > work ? tile : work;
-      }
-      return tile;
-    };
-    if constexpr (FULL && SOLVE == SOLVE_NONE) {
-      // register-pipelined persistent kernel (yz_pipe 2 on x; explicit
-      // filters only: with a solve the prefetched rows and the solve's
-      // registers do not fit together without spills): one tile of LX lines
-      // with 16-byte aligned rows, LX * P threads in whole waves
-      const bool rok = c->yz_pipe == 2 && a.periodic && a.N % VW == 0 && ((uintptr_t)in % 16 == 0) &&
-                       ((uintptr_t)out % 16 == 0) && (!a.out32 || (uintptr_t)a.out32 % 8 == 0);
-      if (rok) {
-        a.pitch = a.N + VW;
-        a.vec = 1;
-        int lx = WG_MAX / P;
-        if (lx > 64) lx = 64;
-        while (lx > 1 && lds(lx) > (size_t)c->x_lds_kb * 1024) lx /= 2;
-        if ((lx * P) % 64 == 0) {
-          a.lx = lx;
-          const size_t shm = lds(lx);
-          const int ngroups = (a.nlines + lx - 1) / lx;
-          const int per_cu = std::max(1, (int)((160 * 1024) / shm));
-          const int nblocks = std::min(ngroups, c->ncu * per_cu);
-          auto k = k_line_x_rpipe<TS, KIND, SOLVE, MODE>;
-          if (set_lds(k, shm)) return 1;
-          hipLaunchKernelGGL(k, dim3(nblocks), dim3(lx * P), shm, c->stream, a, in, out);
-          HIPCHECK(hipGetLastError());
-          return 0;
-        }
-        a.pitch = a.vec ? a.N + VW : a.N + 1;
-      }
-    }
-    if constexpr (FULL && (SOLVE == SOLVE_CIRC || SOLVE == SOLVE_NONE)) {
-      // pipelined persistent kernel: two tiles of LX lines (16-byte aligned
-      // rows, whole KiB per line), LX * P threads in whole waves
-      const bool ok = c->yz_pipe == 1 && !a.out32 && a.periodic && (a.N * (int)sizeof(TS)) % 1024 == 0 &&
-                      ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0);
-      if (ok) {
-        const int pitch = a.N + VW;
-        auto lds2 = [&](int lx) {
-          size_t t = align16(2 * (size_t)lx * pitch * sizeof(TS));
-          if (SOLVE == SOLVE_CIRC) t += 2 * align16((size_t)4 * P * lx * sizeof(CS));
-          return t;
-        };
-        int lx = WG_MAX / P;
-        if (lx > 64) lx = 64;
-        while (lx > 1 && lds2(lx) > (size_t)c->x_lds_kb * 1024) lx /= 2;
-        if ((lx * P) % 64 == 0) {
-          a.lx = lx;
-          a.pitch = pitch;
-          a.vec = 1;
-          const size_t shm = lds2(lx);
-          const int ngroups = (a.nlines + lx - 1) / lx;
-          const int per_cu = std::max(1, (int)((160 * 1024) / shm));
-          const int nblocks = std::min(ngroups, c->ncu * per_cu);
-          auto k = k_line_x_pipe<TS, KIND, SOLVE, MODE>;
-          if (set_lds(k, shm)) return 1;
-          hipLaunchKernelGGL(k, dim3(nblocks), dim3(lx * P), shm, c->stream, a, in, out);
-          HIPCHECK(hipGetLastError());
-          return 0;
-        }
-      }
-    }
-    int lx = WG_MAX / P;
-    if (lx > 64) lx = 64;
-    // keep the workgroup's LDS within the budget so several workgroups share a CU
-    while (lx > 1 && lds(lx) > (size_t)c->x_lds_kb * 1024) lx /= 2;
-    a.lx = lx;
-    const size_t shm = lds(lx);
-    const dim3 grid((a.nlines + lx - 1) / lx), block(lx * P);
-    auto k = k_line_x<TS, KIND, SOLVE, MODE, FULL>;
-    if (set_lds(k, shm)) return 1;
-    hipLaunchKernelGGL(k, grid, block, shm, c->stream, a, in, out);
+    a.vec = ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0) && ((uintptr_t)a.out32 % 8 == 0);
+    a.lines = 64 / a.P;
+    const dim3 grid((unsigned)((a.nlines + a.lines - 1) / a.lines)), block(64);
+    hipLaunchKernelGGL((k_line_x<TS, KIND, SOLVE, FULL>), grid, block, 0, c->stream, a, in, out);
   } else {
-    // lines per workgroup: 64 x P chunk threads within WG_MAX (32 or 16 lines
-    // for longer lines); tuned: 32 or 16 lines (more, smaller workgroups per CU)
-    const int ly = c->yz_lines == 16 ? 16
-                 : ((P <= 8 && c->yz_lines != 32) ? 64 : (P <= WG_MAX / 32 ? 32 : 16));
-    const size_t ex = align16((size_t)4 * P * ly * sizeof(CS));
-    const size_t shm = SOLVE == SOLVE_CIRC ? 2 * ex : (SOLVE == SOLVE_LU ? ex + stage : 0);
-    const dim3 grid((a.nlines + ly - 1) / ly), block(ly, P);
-    const int pre = a.addv ? PRE_V : ((a.epi == EPI_ADD || a.epi == EPI_MAXABS) ? PRE_OLD : PRE_NONE);
-    if constexpr (FULL) {
-      // a filter with an accumulating epilogue keeps the plain kernel
-      if (!(a.addv && pre == PRE_V && (a.epi == EPI_ADD || a.epi == EPI_MAXABS))) {
-        const int r = launch_yz_pipe<TS, KIND, SOLVE, MODE>(c, pre, a, in, out);
-        if (r < 0) return 1;
-        if (r > 0) {
-          HIPCHECK(hipGetLastError());
-          return 0;
-        }
-      }
+    a.lines = yz_lines(a.P, a.nlines, dir, (int)sizeof(TS), forced, c->ncu);
+    const dim3 grid((unsigned)((a.nlines + a.lines - 1) / a.lines)), block(a.lines * a.P);
+    const size_t shm = SOLVE == SOLVE_NONE ? 0 : yz_lds(a.lines * a.P, a.lines);
+    auto k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_NONE>;
+    // filters only exist for the r4 kind; accumulating epilogues for every kind
+    if constexpr (KIND == K_R4) {
+      if (a.addv) k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_V>;
     }
-    if (ly == 64) {
-      if (launch_yz<TS, KIND, SOLVE, MODE, 64, FULL>(c, pre, grid, block, shm, a, in, out)) return 1;
-    } else if (ly == 32) {
-      if (launch_yz<TS, KIND, SOLVE, MODE, 32, FULL>(c, pre, grid, block, shm, a, in, out)) return 1;
-    } else {
-      if (launch_yz<TS, KIND, SOLVE, MODE, 16, FULL>(c, pre, grid, block, shm, a, in, out)) return 1;
+    if constexpr (SOLVE != SOLVE_NONE) {
+      if (!a.addv && (a.epi == EPI_ADD || a.epi == EPI_MAXABS)) k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_OLD>;
     }
+    hipLaunchKernelGGL(k, grid, block, shm, c->stream, a, in, out);
   }
   HIPCHECK(hipGetLastError());
   return 0;
 }
 
-template <typename TS, int MODE, bool FULL>
-int launch_kind(pyr_ctx* c, int dir, int kind, int sv, const LineArgs& a, const TS* in, TS* out) {
-  if constexpr (FULL && PYR_FULL_CHUNKS) {
-    switch (kind) {
-      case K_D1: return launch_typed<TS, K_D1, SOLVE_CIRC, MODE, true>(c, dir, a, in, out);
-      case K_R3: return launch_typed<TS, K_R3, SOLVE_CIRC, MODE, true>(c, dir, a, in, out);
-      default:
-        if (sv == SOLVE_CIRC) return launch_typed<TS, K_R4, SOLVE_CIRC, MODE, true>(c, dir, a, in, out);
-        return launch_typed<TS, K_R4, SOLVE_NONE, MODE, true>(c, dir, a, in, out);
-    }
-  } else if constexpr (!FULL) {
-    switch (kind) {
-      case K_D1:
-        return sv == SOLVE_CIRC ? launch_typed<TS, K_D1, SOLVE_CIRC, MODE, false>(c, dir, a, in, out)
-                                : launch_typed<TS, K_D1, SOLVE_LU, MODE, false>(c, dir, a, in, out);
-      case K_R3:
-        return sv == SOLVE_CIRC ? launch_typed<TS, K_R3, SOLVE_CIRC, MODE, false>(c, dir, a, in, out)
-                                : launch_typed<TS, K_R3, SOLVE_LU, MODE, false>(c, dir, a, in, out);
-      default:
-        if (sv == SOLVE_CIRC) return launch_typed<TS, K_R4, SOLVE_CIRC, MODE, false>(c, dir, a, in, out);
-        if (sv == SOLVE_LU) return launch_typed<TS, K_R4, SOLVE_LU, MODE, false>(c, dir, a, in, out);
-        return launch_typed<TS, K_R4, SOLVE_NONE, MODE, false>(c, dir, a, in, out);
-    }
+// CIRC: the periodic solve; otherwise bounded lines and the explicit filter
+template <typename TS, bool CIRC>
+int launch_kind(pyr_ctx* c, int dir, int kind, int sv, bool full, int forced, const LineArgs& a, const TS* in, TS* out) {
+  constexpr int SV = CIRC ? SOLVE_CIRC : SOLVE_BND;
+  switch (kind) {
+    case K_D1:
+      return full ? launch_typed<TS, K_D1, SV, true>(c, dir, forced, a, in, out)
+                  : launch_typed<TS, K_D1, SV, false>(c, dir, forced, a, in, out);
+    case K_R3:
+      return full ? launch_typed<TS, K_R3, SV, true>(c, dir, forced, a, in, out)
+                  : launch_typed<TS, K_R3, SV, false>(c, dir, forced, a, in, out);
+    default:
+      if constexpr (!CIRC) {
+        if (sv == SOLVE_NONE)
+          return full ? launch_typed<TS, K_R4, SOLVE_NONE, true>(c, dir, forced, a, in, out)
+                      : launch_typed<TS, K_R4, SOLVE_NONE, false>(c, dir, forced, a, in, out);
+      }
+      return full ? launch_typed<TS, K_R4, SV, true>(c, dir, forced, a, in, out)
+                  : launch_typed<TS, K_R4, SV, false>(c, dir, forced, a, in, out);
   }
-  return fail("full-chunk kernels are not built");
 }
 
-#define PYR_LAUNCH_KIND(TS, MODE, FULL) \
-  template int launch_kind<TS, MODE, FULL>(pyr_ctx*, int, int, int, const LineArgs&, const TS*, TS*);
+#define PYR_LAUNCH_KIND(TS, CIRC) \
+  template int launch_kind<TS, CIRC>(pyr_ctx*, int, int, int, bool, int, const LineArgs&, const TS*, TS*);
 #if PYR_PART == 1
-PYR_LAUNCH_KIND(double, MODE_F64, true)
-PYR_LAUNCH_KIND(double, MODE_F64, false)
+PYR_LAUNCH_KIND(double, true)
 #elif PYR_PART == 2
-PYR_LAUNCH_KIND(float, MODE_R32, true)
-PYR_LAUNCH_KIND(float, MODE_R32, false)
+PYR_LAUNCH_KIND(float, true)
 #elif PYR_PART == 3
-PYR_LAUNCH_KIND(float, MODE_S32, true)
-PYR_LAUNCH_KIND(float, MODE_S32, false)
-#else
-extern PYR_LAUNCH_KIND(double, MODE_F64, true)
-extern PYR_LAUNCH_KIND(double, MODE_F64, false)
-extern PYR_LAUNCH_KIND(float, MODE_R32, true)
-extern PYR_LAUNCH_KIND(float, MODE_R32, false)
-extern PYR_LAUNCH_KIND(float, MODE_S32, true)
-extern PYR_LAUNCH_KIND(float, MODE_S32, false)
+PYR_LAUNCH_KIND(double, false)
+#elif PYR_PART == 4
+PYR_LAUNCH_KIND(float, false)
+#elif PYR_PART == 0
+extern PYR_LAUNCH_KIND(double, true)
+extern PYR_LAUNCH_KIND(float, true)
+extern PYR_LAUNCH_KIND(double, false)
+extern PYR_LAUNCH_KIND(float, false)
 #endif
 #undef PYR_LAUNCH_KIND
 
+// lines per workgroup of P chunk threads: as many as fit, at most 64
+static int ref_lines(int P) {
+  int ly = 64;
+  while (ly * P > REF_THREADS) ly /= 2;
+  return ly;
+}
+
+#if PYR_PART == 7
+template <int KIND>
+static int launch_ref_kind(hipStream_t stream, int dir, RefArgs a, const float* in, float* out) {
+  if (dir == 0) {
+    a.vec = ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0);
+    a.lines = 64 / a.P;
+    const int per = a.lines * REF_X_WAVES;
+    hipLaunchKernelGGL((k_ref_x<KIND>), dim3((unsigned)((a.nlines + per - 1) / per)), dim3(64 * REF_X_WAVES), 0,
+                       stream, a, in, out);
+  } else {
+    a.lines = ref_lines(a.P);
+    while (a.lines > 16 && a.nlines < a.lines * 256) a.lines /= 2;  // small fields: more workgroups
+    auto k = k_ref_yz<KIND, PRE_NONE>;
+    if constexpr (KIND == K_R4) {
+      if (a.addv) k = k_ref_yz<KIND, PRE_V>;
+    }
+    if (!a.addv && (a.epi == EPI_ADD || a.epi == EPI_MAXABS)) k = k_ref_yz<KIND, PRE_OLD>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((a.nlines + a.lines - 1) / a.lines)), dim3(a.lines * a.P), 0, stream, a, in,
+                       out);
+  }
+  HIPCHECK(hipGetLastError());
+  return 0;
+}
+int launch_ref(hipStream_t stream, int dir, int kind, const RefArgs& a, const float* in, float* out) {
+  if (kind == K_D1) return launch_ref_kind<K_D1>(stream, dir, a, in, out);
+  if (kind == K_R3) return launch_ref_kind<K_R3>(stream, dir, a, in, out);
+  return launch_ref_kind<K_R4>(stream, dir, a, in, out);
+}
+#else
+int launch_ref(hipStream_t stream, int dir, int kind, const RefArgs& a, const float* in, float* out);
+#endif
+
 #if PYR_PART == 0
 
-template <typename TS, int MODE>
+// FP32 solve setting of one operator and direction: its tuned choice, else the
+// context's
+static int r32_mode(const pyr_ctx* c, int op, int dir) {
+  return c->tune_solve[op][dir] >= 0 ? c->tune_solve[op][dir] : c->r32_solve;
+}
+
+// bounded FP32 lines of a context in the refined mode keep the refined FP32
+// arithmetic; the FP64 recurrences serve every other line (periodic FP32 lines
+// in either mode: their refined solve agreed with one FP64 solve to the bit)
+static bool use_refined(const pyr_ctx* c, int op, int dir) {
+  return c->rplan[op][dir].N > 0 && r32_mode(c, op, dir) == PYR_R32_SOLVE_REFINED;
+}
+
+template <typename TS>
 static int launch_op(pyr_ctx* c, int op, int dir, const TS* in, TS* out, int epi, double ec, bool anti) {
   // anti: the antisymmetric member where the direction has a SYMM end, as
   // d1x/d8x(v, dv, bc=-1) select it (compact_operators.f90:300-303)
@@ -1583,7 +1171,7 @@ static int launch_op(pyr_ctx* c, int op, int dir, const TS* in, TS* out, int epi
     return 0;
   }
   LineArgs a = make_args(c, pl, ua ? c->dplan_a[op][dir] : c->dplan[op][dir], dir, epi, ec,
-                         MODE == MODE_F64 ? PYR_F64 : PYR_R32);
+                         sizeof(TS) == 8 ? PYR_F64 : PYR_R32);
   if (c->out32) {
     // the plain kernels of FP64 fields with the store epilogue write the
     // rounded copy
@@ -1591,37 +1179,24 @@ static int launch_op(pyr_ctx* c, int op, int dir, const TS* in, TS* out, int epi
     a.out32 = c->out32;
     a.only32 = c->only32;
   }
-  const int sv = plan_solve(c, pl);
-  // the balanced partition gives every chunk CHUNK rows exactly when CHUNK | N;
-  // the LU solve keeps runtime row counts (with compile-time counts the
-  // compiler hoists every table read of the chunk and runs out of registers)
-  const int sx = c->x_lds_kb, sp = c->yz_pipe, sl = c->yz_lines;
-  if (c->tune_xlds[op][dir][MODE] >= 0) c->x_lds_kb = c->tune_xlds[op][dir][MODE];
-  if (c->tune_pipe[op][dir][MODE] >= 0) c->yz_pipe = c->tune_pipe[op][dir][MODE];
-  else if (dir == 0) c->yz_pipe = 0;  // the pipelined x kernel only where tuning chose it
-  if (c->tune_ly[op][dir][MODE] >= 0) c->yz_lines = c->tune_ly[op][dir][MODE];
-  // yz_pipe 3 on y/z: the plain kernel with runtime row counts even when
-  // CHUNK | N (fewer registers, more waves per SIMD; the same results)
-  const bool full = PYR_FULL_CHUNKS && pl.N % CHUNK == 0 && sv != SOLVE_LU && !(dir != 0 && c->yz_pipe == 3);
-  const int r = full
-                    ? launch_kind<TS, MODE, true>(c, dir, pl.kind, sv, a, in, out)
-                    : launch_kind<TS, MODE, false>(c, dir, pl.kind, sv, a, in, out);
-  c->x_lds_kb = sx;
-  c->yz_pipe = sp;
-  c->yz_lines = sl;
-  return r;
+  if constexpr (sizeof(TS) == 4) {
+    if (use_refined(c, op, dir))
+      return launch_ref(c->stream, dir, pl.kind,
+                        make_ref_args(a, ua ? c->rplan_a[op][dir] : c->rplan[op][dir],
+                                      ua ? c->drplan_a[op][dir] : c->drplan[op][dir]), in, out);
+  }
+  const int sv = plan_solve(pl);
+  const int wd = sizeof(TS) == 8 ? 0 : 1;
+  const int forced = c->tune_ly[op][dir][wd] >= 0 ? c->tune_ly[op][dir][wd] : c->yz_lines;
+  const bool full = pl.N == pl.P * CHUNK && !(dir != 0 && c->tune_rt[op][dir][wd]);
+  return sv == SOLVE_CIRC ? launch_kind<TS, true>(c, dir, pl.kind, sv, full, forced, a, in, out)
+                          : launch_kind<TS, false>(c, dir, pl.kind, sv, full, forced, a, in, out);
 }
 
 static int check_ctx(pyr_ctx* c) {
   if (!c) return fail("null context");
   if (!c->device) return fail("context was set up host-only (pyr_setup_host)");
   return 0;
-}
-
-// FP32 solve arithmetic of one operator and direction: its tuned choice, else
-// the context's
-static int r32_mode(const pyr_ctx* c, int op, int dir) {
-  return c->tune_solve[op][dir] >= 0 ? c->tune_solve[op][dir] : c->r32_solve;
 }
 
 static int apply_any(pyr_ctx* c, int op, int dir, int prec, const void* in, void* out, int epi,
@@ -1634,12 +1209,9 @@ static int apply_any(pyr_ctx* c, int op, int dir, int prec, const void* in, void
   if (in == out || (void*)in == (void*)c->out32) return fail("input and output must not alias");
   if (only32 && prec != PYR_F64) return fail("an FP32-only result needs an FP64 sweep");
   if (prec == PYR_F64)
-    return launch_op<double, MODE_F64>(c, op, dir, (const double*)in, (double*)out, epi, ec, anti);
-  if (prec == PYR_R32) {
-    if (r32_mode(c, op, dir) == PYR_R32_SOLVE_FP64)
-      return launch_op<float, MODE_S32>(c, op, dir, (const float*)in, (float*)out, epi, ec, anti);
-    return launch_op<float, MODE_R32>(c, op, dir, (const float*)in, (float*)out, epi, ec, anti);
-  }
+    return launch_op<double>(c, op, dir, (const double*)in, (double*)out, epi, ec, anti);
+  if (prec == PYR_R32)
+    return launch_op<float>(c, op, dir, (const float*)in, (float*)out, epi, ec, anti);
   return fail("bad precision");
 }
 
@@ -1725,7 +1297,6 @@ static int setup_common(pyr_ctx** out, int nx, int ny, int nz, double x1, double
   if (!bc6) return fail("null bc array");
   std::unique_ptr<pyr_ctx> c(new pyr_ctx);
   c->n[0] = nx; c->n[1] = ny; c->n[2] = nz;
-  if (const char* e = std::getenv("PYRANDA_AMD_YZ_PIPE")) c->yz_pipe = std::atoi(e) != 0;
   if (const char* e = std::getenv("PYRANDA_AMD_X_LDS_KB")) {
     const int kb = std::atoi(e);
     if (kb >= 8 && kb <= 160) c->x_lds_kb = kb;
@@ -1752,12 +1323,17 @@ static int setup_common(pyr_ctx** out, int nx, int ny, int nz, double x1, double
       const int periodic = c->bc[2 * d] == PYR_BC_PERI;
       const int v1 = c->bc[2 * d] == PYR_BC_SYMM ? 1 : 0;
       const int v2 = c->bc[2 * d + 1] == PYR_BC_SYMM ? 1 : 0;
-      for (int op = 0; op < NOPS; ++op)
-        c->plan[op][d] = build_plan(op, c->n[d], periodic, v1, v2, c->dpatch[d]);
+      for (int op = 0; op < NOPS; ++op) {
+        c->plan[op][d] = build_plan(op, c->n[d], d, periodic, v1, v2, c->dpatch[d]);
+        if (!periodic && c->plan[op][d].implicit && !c->plan[op][d].null_op)
+          c->rplan[op][d] = build_ref_plan(op, c->n[d], v1, v2, c->dpatch[d]);
+      }
       c->has_anti[d] = !periodic && (v1 || v2) && c->n[d] >= 4;
       if (c->has_anti[d])
-        for (int op = 0; op < NOPS; ++op)
-          c->plan_a[op][d] = build_plan(op, c->n[d], periodic, -v1, -v2, c->dpatch[d]);
+        for (int op = 0; op < NOPS; ++op) {
+          c->plan_a[op][d] = build_plan(op, c->n[d], d, periodic, -v1, -v2, c->dpatch[d]);
+          if (c->plan_a[op][d].implicit) c->rplan_a[op][d] = build_ref_plan(op, c->n[d], -v1, -v2, c->dpatch[d]);
+        }
     }
   } catch (const std::exception& e) {
     return fail(std::string("setup: ") + e.what());
@@ -1770,11 +1346,10 @@ static int setup_common(pyr_ctx** out, int nx, int ny, int nz, double x1, double
       c->ncu = prop.multiProcessorCount;
     // once per GPU, with that GPU current: its copy of the scratch array
     if (noalloc_init(dev, &c->noalloc_tmp)) return 1;
-    for (int op = 0; op < NOPS; ++op)
-      for (int d = 0; d < 3; ++d) {
-        if (upload_plan(c->plan[op][d], c->dplan[op][d])) return 1;
-        if (c->has_anti[d] && upload_plan(c->plan_a[op][d], c->dplan_a[op][d])) return 1;
-      }
+    if (upload_plans(c.get())) {
+      if (c->tables) (void)hipFree(c->tables);
+      return 1;
+    }
     c->device = true;
   }
   *out = c.release();
@@ -1785,166 +1360,178 @@ static int setup_common(pyr_ctx** out, int nx, int ny, int nz, double x1, double
 // host emulation of the kernels (tests only): the same per-thread arithmetic,
 // chunk by chunk, with the LDS exchanges as plain arrays
 // ---------------------------------------------------------------------------
-template <typename TS, int KIND, int SOLVE, int MODE>
+template <typename TS, int KIND, int SOLVE>
 static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS* vout) {
   constexpr int R = Halo<KIND>::R;
-  using CS = typename SolveT<MODE>::type;
-  const int P = a.P, N = a.N;
   struct St {
-    TS win[CHUNK + 2 * 4];
-    double rhs[CHUNK];
-    CS x[CHUNK], d[CHUNK], z[4], zd[4];
+    TS win[CHUNK + 2 * R];
+    double x[CHUNK];
+    double e[2], b[2];
     int s, m;
   };
+  const int P = a.P, N = a.N;
   std::vector<St> st(P);
-  std::vector<CS> Y(4 * P), Yb(4 * P);
-  auto rd = [&](int i) { return vin[stride * i]; };
+  auto rows_of = [&](int p, auto f) {
+    if (SOLVE == SOLVE_BND && (p < a.tlo || p == P - 1)) f(TableRows{a.tf, a.tb, a.tg, P, p});
+    else f(ConstRows{a.p1, a.p2});
+  };
+  auto carry = [&](int p, int step, double& e0, double& e1) {
+    const double* K = step < 0 ? a.kf : a.kb;
+    e0 = e1 = 0.0;
+    int q = p;
+    for (int j = 0; j < a.W; ++j) {
+      q += step;
+      if (a.periodic) q = (q + P) % P;
+      if (q < 0 || q >= P) break;
+      const double* u = step < 0 ? st[q].e : st[q].b;
+      carry_add(K + 4 * (j * a.kp + (a.kp == 1 ? 0 : p)), u[0], u[1], e0, e1);
+    }
+  };
   for (int p = 0; p < P; ++p) {
     St& t = st[p];
-    t.s = a.cstart[p];
-    t.m = a.cstart[p + 1] - t.s;
+    t.s = chunk_start(a, p);
+    t.m = chunk_start(a, p + 1) - t.s;
     for (int w = 0; w < CHUNK + 2 * R; ++w) {
       int row = t.s - R + w;
       TS v = (TS)0;
-      if (w < t.m + 2 * R) {
-        if (a.periodic) {
-          row = row < 0 ? row + N : (row >= N ? row - N : row);
-          v = rd(row);
-        } else if (row >= 0 && row < N) {
-          v = rd(row);
-        }
+      if (w < t.m + 2 * R && (a.periodic || (row >= 0 && row < N))) {
+        row = row < 0 ? row + N : (row >= N ? row - N : row);
+        v = vin[stride * row];
       }
       t.win[w] = v;
     }
-    rhs_interior<KIND>(a, t.win, t.rhs, t.m);
-    rhs_boundary(a, t.s, t.m, t.rhs, rd);
+    rhs_interior<KIND>(a, t.win, t.x);
+    if (!a.periodic) rhs_boundary<KIND, false>(a, a.wb, p, t.win, t.x);
+    if (SOLVE == SOLVE_NONE) continue;
+    t.e[0] = t.e[1] = 0.0;
+    rows_of(p, [&](auto rows) { fwd_pass<false, false>(rows, t.x, t.m, t.e[0], t.e[1]); });
   }
-  // circulant solve of every chunk's vector `v` (without 1/c), as circ_solve
-  auto circ_all = [&](auto getv, const CS* kf, const CS* kb, CS p1, CS p2) {
-    for (int p = 0; p < P; ++p) circ_fwd_exit(getv(p), st[p].m, p1, p2, Y[2 * p], Y[2 * p + 1]);
-    for (int p = 0; p < P; ++p) {
-      CS e0, e1;
-      circ_carry(kf, p, P, [&](int cc) { return Y[cc]; }, e0, e1);
-      circ_fwd(getv(p), st[p].m, p1, p2, e0, e1);
-      circ_bwd_exit(getv(p), st[p].m, p1, p2, Yb[2 * p], Yb[2 * p + 1]);
-    }
-    for (int p = 0; p < P; ++p) {
-      CS e0, e1;
-      circ_carry(kb, p, P, [&](int cc) { return Yb[cc]; }, e0, e1);
-      circ_bwd(getv(p), st[p].m, p1, p2, e0, e1);
-    }
-  };
-  if (SOLVE == SOLVE_LU) {
-    const CS* G = MODE != MODE_R32 ? (const CS*)a.gsel : (const CS*)a.gsel32;
-    const CS* RC = MODE != MODE_R32 ? (const CS*)a.rc : (const CS*)a.rc32;
-    const CS* LU = MODE != MODE_R32 ? (const CS*)a.lu : (const CS*)a.lu32;
+  bool bad = false;
+  if (SOLVE != SOLVE_NONE)
     for (int p = 0; p < P; ++p) {
       St& t = st[p];
-      for (int k = 0; k < CHUNK; ++k) t.x[k] = (CS)t.rhs[k];
-      local_solve<CS>(LU, t.s, t.m, t.x);
-      CS e4[4];
-      edges(t.x, t.m, e4);
-      for (int q = 0; q < 4; ++q) Y[4 * p + q] = e4[q];
+      double e0, e1;
+      carry(p, -1, e0, e1);
+      t.b[0] = t.b[1] = 0.0;
+      rows_of(p, [&](auto rows) {
+        fwd_pass<false, true>(rows, t.x, t.m, e0, e1);
+        bwd_exit<false>(rows, t.x, t.m, t.b[0], t.b[1]);
+      });
+      bad = bad || !std::isfinite(t.b[0]) || !std::isfinite(t.b[1]);
     }
-    for (int p = 0; p < P; ++p) {
-      St& t = st[p];
-      neighbours<CS>(G, p, P, [&](int cc) { return Y[cc]; }, t.z);
-      spike_correct(RC, t.s, t.m, t.z, t.x);
-    }
-    if (MODE == MODE_R32) {
-      std::vector<CS> Yd(4 * P);
-      for (int p = 0; p < P; ++p) {
-        St& t = st[p];
-        double res[CHUNK];
-        residual64([&](int k) { return a.band + 5 * (t.s + k); }, t.m, t.rhs, (const float*)t.x,
-                   (const float*)t.z, res);
-        for (int k = 0; k < CHUNK; ++k) t.d[k] = (CS)res[k];
-        local_solve<CS>(LU, t.s, t.m, t.d);
-        CS f4[4];
-        edges(t.d, t.m, f4);
-        for (int q = 0; q < 4; ++q) Yd[4 * p + q] = f4[q];
-      }
-      for (int p = 0; p < P; ++p) {
-        St& t = st[p];
-        neighbours<CS>(G, p, P, [&](int cc) { return Yd[cc]; }, t.zd);
-        spike_correct(RC, t.s, t.m, t.zd, t.d);
-      }
-    }
-  } else if (SOLVE == SOLVE_CIRC) {
-    for (int p = 0; p < P; ++p)
-      for (int k = 0; k < CHUNK; ++k) st[p].x[k] = (CS)st[p].rhs[k];
-    auto gx = [&](int p) { return st[p].x; };
-    if (MODE != MODE_R32) {
-      circ_all(gx, (const CS*)a.kf, (const CS*)a.kb, (CS)a.p1, (CS)a.p2);
-      for (int p = 0; p < P; ++p)
-        for (int k = 0; k < CHUNK; ++k) st[p].x[k] *= (CS)a.invc;
-    } else {
-      const CS *kf = (const CS*)a.kf32, *kb = (const CS*)a.kb32;
-      const CS p1 = (CS)a.p1f, p2 = (CS)a.p2f, ic = (CS)a.invcf;
-      circ_all(gx, kf, kb, p1, p2);
-      std::vector<CS> E(4 * P);
-      for (int p = 0; p < P; ++p) {
-        for (int k = 0; k < CHUNK; ++k) st[p].x[k] *= ic;
-        edges(st[p].x, st[p].m, &E[4 * p]);
-      }
-      const double row[5] = {a.bd[0], a.bd[1], a.bd[2], a.bd[1], a.bd[0]};
-      for (int p = 0; p < P; ++p) {
-        St& t = st[p];
-        const int pm = (p - 1 + P) % P, pp = (p + 1) % P;
-        const float z[4] = {(float)E[4 * pm + 2], (float)E[4 * pm + 3], (float)E[4 * pp], (float)E[4 * pp + 1]};
-        double res[CHUNK];
-        residual64([&](int) { return row; }, t.m, t.rhs, (const float*)t.x, z, res);
-        for (int k = 0; k < CHUNK; ++k) t.d[k] = (CS)res[k];
-      }
-      circ_all([&](int p) { return st[p].d; }, kf, kb, p1, p2);
-      for (int p = 0; p < P; ++p)
-        for (int k = 0; k < CHUNK; ++k) st[p].d[k] *= ic;
-    }
-  }
   for (int p = 0; p < P; ++p) {
     St& t = st[p];
-    for (int k = 0; k < t.m; ++k) {
-      double y;
-      if (SOLVE == SOLVE_NONE) y = t.rhs[k];
-      else if (MODE != MODE_R32) y = (double)t.x[k];
-      else y = (double)t.x[k] + (double)t.d[k];
+    auto emit = [&](int k, double y) {
       double val = y * a.scale;
       if (a.addv) val += (double)t.win[k + R];
       vout[stride * (t.s + k)] = (TS)val;
+    };
+    if (SOLVE == SOLVE_NONE) {
+      for (int k = 0; k < t.m; ++k) emit(k, t.x[k]);
+      continue;
+    }
+    double b0, b1;
+    carry(p, 1, b0, b1);
+    if (bad) b0 = b1 = std::nan("");
+    rows_of(p, [&](auto rows) { bwd_sink<false>(rows, t.x, t.m, b0, b1, emit); });
+  }
+}
+
+template <int KIND>
+static void emulate_ref_line(const RefArgs& a, const float* vin, long long stride, float* vout) {
+  constexpr int R = Halo<KIND>::R;
+  struct St {
+    float win[RCHUNK + 2 * R];
+    double rhs[RCHUNK];
+    float x[RCHUNK], d[RCHUNK], z[4];
+    const float* t;
+    int s, m;
+  };
+  const int P = a.P, N = a.N;
+  std::vector<St> st(P);
+  std::vector<F4> Y(P), Yd(P);
+  auto rd = [&](int i) { return vin[stride * i]; };
+  for (int p = 0; p < P; ++p) {
+    St& t = st[p];
+    t.s = p * a.mb + std::min(p, a.mx);
+    t.m = a.mb + (p < a.mx ? 1 : 0);
+    t.t = a.cls + ref_class(p, P, a.mx) * (RCHUNK * CROW);
+    for (int w = 0; w < RCHUNK + 2 * R; ++w) {
+      const int row = t.s - R + w;
+      t.win[w] = w < t.m + 2 * R && row >= 0 && row < N ? rd(row) : 0.0f;
+    }
+    ref_rhs_interior<KIND>(a, t.win, t.rhs, t.m);
+    ref_rhs_boundary(a, p, t.rhs, [&](int slot) { return end_value(slot, N, rd); });
+    for (int k = 0; k < RCHUNK; ++k) t.x[k] = (float)t.rhs[k];
+    ref_local_solve(t.t, t.m, t.x);
+    ref_edges(t.x, t.m, &Y[p].x);
+  }
+  for (int p = 0; p < P; ++p) {
+    St& t = st[p];
+    ref_neighbours(a, p, [&](int q) { return Y[q]; }, t.z);
+    ref_spike(t.t, t.m, t.z, t.x);
+    ref_residual(a, p, t.m, t.rhs, t.x, t.z, t.d);
+    ref_local_solve(t.t, t.m, t.d);
+    ref_edges(t.d, t.m, &Yd[p].x);
+  }
+  for (int p = 0; p < P; ++p) {
+    St& t = st[p];
+    ref_neighbours(a, p, [&](int q) { return Yd[q]; }, t.z);
+    ref_spike(t.t, t.m, t.z, t.d);
+    for (int k = 0; k < t.m; ++k) {
+      double val = ((double)t.x[k] + (double)t.d[k]) * a.scale;
+      if (a.addv) val += (double)t.win[k + R];
+      vout[stride * (t.s + k)] = (float)val;
     }
   }
 }
 
-template <typename TS, int MODE>
-static int emulate(pyr_ctx* c, int op, int dir, const TS* in, TS* out) {
-  const OpPlan& pl = c->plan[op][dir];
+template <typename TS>
+static int emulate(pyr_ctx* c, int op, int dir, const TS* in, TS* out, bool anti) {
+  const bool ua = anti && c->has_anti[dir];
+  const OpPlan& pl = ua ? c->plan_a[op][dir] : c->plan[op][dir];
   const size_t n = c->npts();
   if (pl.null_op) {
     for (size_t i = 0; i < n; ++i) out[i] = pl.null_option == 1 ? in[i] : (TS)0;
     return 0;
   }
   DevPlan d;
-  std::vector<float> lu32, rc32, gs32, kf32, kb32;
-  host_tables(pl, d, lu32, rc32, gs32, kf32, kb32);
-  const LineArgs a = make_args(c, pl, d, dir, EPI_STORE, 0.0, MODE == MODE_F64 ? PYR_F64 : PYR_R32);
-  const int sv = plan_solve(c, pl);
+  host_tables(pl, d);
+  const LineArgs a = make_args(c, pl, d, dir, EPI_STORE, 0.0, sizeof(TS) == 8 ? PYR_F64 : PYR_R32);
+  const int sv = plan_solve(pl);
+  const bool refined = sizeof(TS) == 4 && use_refined(c, op, dir);
+  RefArgs ra;
+  if (refined) {
+    const RefPlan& rp = ua ? c->rplan_a[op][dir] : c->rplan[op][dir];
+    DevRefPlan rd;
+    host_ref_tables(rp, rd);
+    ra = make_ref_args(a, rp, rd);
+  }
   for (long long L = 0; L < a.nlines; ++L) {
     const long long base = (dir == 0) ? L * pl.N : (L % a.A) + a.B * (L / a.A);
     const TS* vi = in + base;
     TS* vo = out + base;
+    if constexpr (sizeof(TS) == 4) {
+      if (refined) {
+        if (pl.kind == K_D1) emulate_ref_line<K_D1>(ra, vi, a.stride, vo);
+        else if (pl.kind == K_R3) emulate_ref_line<K_R3>(ra, vi, a.stride, vo);
+        else emulate_ref_line<K_R4>(ra, vi, a.stride, vo);
+        continue;
+      }
+    }
     switch (pl.kind) {
       case K_D1:
-        if (sv == SOLVE_CIRC) emulate_line<TS, K_D1, SOLVE_CIRC, MODE>(a, vi, a.stride, vo);
-        else emulate_line<TS, K_D1, SOLVE_LU, MODE>(a, vi, a.stride, vo);
+        if (sv == SOLVE_CIRC) emulate_line<TS, K_D1, SOLVE_CIRC>(a, vi, a.stride, vo);
+        else emulate_line<TS, K_D1, SOLVE_BND>(a, vi, a.stride, vo);
         break;
       case K_R3:
-        if (sv == SOLVE_CIRC) emulate_line<TS, K_R3, SOLVE_CIRC, MODE>(a, vi, a.stride, vo);
-        else emulate_line<TS, K_R3, SOLVE_LU, MODE>(a, vi, a.stride, vo);
+        if (sv == SOLVE_CIRC) emulate_line<TS, K_R3, SOLVE_CIRC>(a, vi, a.stride, vo);
+        else emulate_line<TS, K_R3, SOLVE_BND>(a, vi, a.stride, vo);
         break;
       default:
-        if (sv == SOLVE_CIRC) emulate_line<TS, K_R4, SOLVE_CIRC, MODE>(a, vi, a.stride, vo);
-        else if (sv == SOLVE_LU) emulate_line<TS, K_R4, SOLVE_LU, MODE>(a, vi, a.stride, vo);
-        else emulate_line<TS, K_R4, SOLVE_NONE, MODE>(a, vi, a.stride, vo);
+        if (sv == SOLVE_CIRC) emulate_line<TS, K_R4, SOLVE_CIRC>(a, vi, a.stride, vo);
+        else if (sv == SOLVE_BND) emulate_line<TS, K_R4, SOLVE_BND>(a, vi, a.stride, vo);
+        else emulate_line<TS, K_R4, SOLVE_NONE>(a, vi, a.stride, vo);
     }
   }
   return 0;
@@ -1957,21 +1544,18 @@ static int emulate(pyr_ctx* c, int op, int dir, const TS* in, TS* out) {
 // ---------------------------------------------------------------------------
 // Members of a group are contexts of any grid sizes whose fields live in one
 // allocation (member m at off[m] elements). An operator along one direction
-// runs as ONE grouped launch over every member (workgroups shaped for the
-// member with the most chunks per line; threads without a chunk only take
-// the barriers), plus a k_null launch for a member whose direction is a null
-// operator. (Splitting the members by chunk count into separate launches
-// idles fewer threads but measured slower: the launches are latency-bound
-// and run one after another.) The per-member line arguments of a
-// launch are built once per (operator, direction, precision, epilogue) and
+// runs as ONE grouped launch over every member, plus a k_null launch for a
+// member whose direction is a null operator. The per-member line arguments of
+// a launch are built once per (operator, direction, precision, epilogue) and
 // kept on the device.
 struct GrpLaunch {
-  GrpEntry* dev = nullptr;
+  void* dev = nullptr;  // GrpEntry or, with refined, RefEntry per member
+  bool refined = false;
   int M = 0;
   long long nblocks = 0;
   dim3 block;
   size_t shm = 0;
-  int kind = 0, solve = 0, ly = 0, pre = 0;
+  int kind = 0, solve = 0, pre = 0;
   bool x = false;
 };
 struct GrpNull {
@@ -1983,20 +1567,15 @@ struct GrpPlan {
   std::vector<GrpLaunch> launches;
   std::vector<GrpNull> nulls;
 };
-// A plan depends on the solve arithmetic (carry types and LDS sizes) and on
-// the members' launch knobs at build time; all of them are part of the key so
-// that a change of tuning builds a new plan instead of reusing a stale one.
 struct GrpKey {
   int op, dir, prec, epi, power, aligned;
-  int mode, psolve, xlds;
+  int refined;  // FP32 solve arithmetic (a part of the plan)
   double ec;
   bool operator<(const GrpKey& o) const {
     if (op != o.op) return op < o.op;
     if (dir != o.dir) return dir < o.dir;
     if (prec != o.prec) return prec < o.prec;
-    if (mode != o.mode) return mode < o.mode;
-    if (psolve != o.psolve) return psolve < o.psolve;
-    if (xlds != o.xlds) return xlds < o.xlds;
+    if (refined != o.refined) return refined < o.refined;
     if (epi != o.epi) return epi < o.epi;
     if (power != o.power) return power < o.power;
     if (aligned != o.aligned) return aligned < o.aligned;
@@ -2016,10 +1595,8 @@ struct pyr_group {
 };
 
 #if PYR_PART == 0
-template <typename TS, int MODE>
+template <typename TS>
 static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
-  using CS = typename SolveT<MODE>::type;
-  constexpr int VW = Vec16<TS>::W;
   const int M = (int)g->mem.size();
   std::vector<int> ms;
   for (int m = 0; m < M; ++m) {
@@ -2031,171 +1608,171 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
   }
   if (ms.empty()) return 0;
   const OpPlan& pl0 = g->mem[ms[0]]->plan[key.op][key.dir];
-  const int sv = plan_solve(g->mem[ms[0]], pl0);
+  const int sv = plan_solve(pl0);
   std::vector<GrpEntry> all(ms.size());
   for (size_t j = 0; j < ms.size(); ++j) {
     pyr_ctx* c = g->mem[ms[j]];
     const OpPlan& pl = c->plan[key.op][key.dir];
-    if (plan_solve(c, pl) != sv || pl.kind != pl0.kind)
+    if (plan_solve(pl) != sv || pl.kind != pl0.kind)
       return fail("group members differ in boundary conditions along a direction");
     const double ec = key.ec * std::pow(c->dmesh[key.dir], (double)key.power);
     all[j].a = make_args(c, pl, c->dplan[key.op][key.dir], key.dir, key.epi, ec, key.prec);
-    // bounded lines: every member's LU tables are read from global memory
-    // (members differ in length; the workgroup's LDS holds the exchange only)
-    all[j].a.gtab = sv == SOLVE_LU;
     all[j].off = g->off[ms[j]];
   }
-  auto upload = [&](GrpLaunch& L, std::vector<GrpEntry>& host) -> int {
-    L.kind = pl0.kind;
-    L.solve = sv;
-    L.M = (int)host.size();
-    HIPCHECK(hipMalloc(&L.dev, host.size() * sizeof(GrpEntry)));
-    HIPCHECK(hipMemcpy(L.dev, host.data(), host.size() * sizeof(GrpEntry), hipMemcpyHostToDevice));
+  GrpLaunch L;
+  L.kind = pl0.kind;
+  L.solve = sv;
+  L.M = (int)all.size();
+  L.x = key.dir == 0;
+  auto upload = [&](const void* host, size_t bytes) -> int {
+    HIPCHECK(hipMalloc(&L.dev, bytes));
     gp.launches.push_back(L);
+    HIPCHECK(hipMemcpy(L.dev, host, bytes, hipMemcpyHostToDevice));
     return 0;
   };
-  if (key.dir == 0) {
-    // each member keeps its own lines per workgroup (its LDS within the
-    // budget), so lx * P stays near WG_MAX for every member; the launch
-    // takes the most threads and LDS of any member
-    GrpLaunch L;
-    L.x = true;
-    int nthr = 0;
-    size_t shm = 0;
-    long long blk = 0;
-    for (auto& e : all) {
-      const int P = e.a.P;
-      e.a.vec = key.aligned && (e.a.N % VW == 0) && ((e.off * (long long)sizeof(TS)) % 16 == 0);
-      e.a.pitch = e.a.vec ? e.a.N + VW : e.a.N + 1;
-      auto lds = [&](int lx) {
-        const size_t tile = align16((size_t)lx * e.a.pitch * sizeof(TS));
-        if (sv == SOLVE_CIRC) return tile + 2 * align16((size_t)4 * P * lx * sizeof(CS));
-        if (sv == SOLVE_LU) return std::max(tile, align16((size_t)4 * P * lx * sizeof(CS)));
-        return tile;
-      };
-      int lx = WG_MAX / P;
-      if (lx > 64) lx = 64;
-      while (lx > 1 && lds(lx) > (size_t)g->mem[0]->x_lds_kb * 1024) lx /= 2;
-      e.a.lx = lx;
-      e.blk0 = blk;
-      blk += (e.a.nlines + lx - 1) / lx;
-      nthr = std::max(nthr, lx * P);
-      shm = std::max(shm, lds(lx));
-    }
-    L.block = dim3(nthr);
-    L.shm = shm;
-    L.nblocks = blk;
-    return upload(L, all);
-  }
-  // y/z: workgroups are (ly lanes, P chunks) shaped for the longest member of
-  // the launch; members are split into launches by chunk count (<= 8, <= 16,
-  // <= 32) so that short lines do not run in workgroups shaped for 1024 points
   const int pre = all[0].a.addv ? PRE_V : ((key.epi == EPI_ADD || key.epi == EPI_MAXABS) ? PRE_OLD : PRE_NONE);
-  const int bounds[3] = {8, 16, 32};
-  for (int cl = 0; cl < 3; ++cl) {
-    std::vector<GrpEntry> host;
-    for (auto& e : all)
-      if (e.a.P <= bounds[cl] && (cl == 0 || e.a.P > bounds[cl - 1])) host.push_back(e);
-    if (host.empty()) continue;
-    int Pmax = 1;
-    for (auto& e : host) Pmax = std::max(Pmax, e.a.P);
-    const int ly = Pmax <= 8 ? 64 : (Pmax <= WG_MAX / 32 ? 32 : 16);
+  if (key.refined && sv == SOLVE_BND) {
+    std::vector<RefEntry> ref(all.size());
     long long blk = 0;
-    for (auto& e : host) {
-      e.blk0 = blk;
-      blk += (e.a.nlines + ly - 1) / ly;
+    for (size_t j = 0; j < all.size(); ++j) {
+      pyr_ctx* c = g->mem[ms[j]];
+      RefArgs& a = ref[j].a;
+      a = make_ref_args(all[j].a, c->rplan[key.op][key.dir], c->drplan[key.op][key.dir]);
+      a.vec = key.aligned && ((all[j].off * (long long)sizeof(float)) % 16 == 0);
+      a.lines = L.x ? 64 / a.P : ref_lines(a.P);
+      const int per = L.x ? a.lines * REF_X_WAVES : a.lines;
+      ref[j].off = all[j].off;
+      ref[j].blk0 = blk;
+      blk += (a.nlines + per - 1) / per;
     }
-    GrpLaunch L;
-    L.x = false;
-    L.ly = ly;
-    L.block = dim3(ly, Pmax);
-    const size_t ex = align16((size_t)4 * Pmax * ly * sizeof(CS));
-    L.shm = sv == SOLVE_CIRC ? 2 * ex : (sv == SOLVE_LU ? ex : 0);
+    L.refined = true;
     L.pre = pre;
+    L.block = dim3(L.x ? 64 * REF_X_WAVES : REF_THREADS);
     L.nblocks = blk;
-    if (upload(L, host)) return 1;
+    return upload(ref.data(), ref.size() * sizeof(RefEntry));
   }
-  return 0;
+  int nthr = 64;
+  if (!L.x) {
+    // 512 chunk threads a workgroup (64 lines of 8 chunks to 16 of 32), 1024
+    // where a member's lines have more than 32 chunks
+    int Pmax = 1;
+    for (auto& e : all) Pmax = std::max(Pmax, e.a.P);
+    nthr = Pmax > 32 ? WG_MAX : WG_MAX / 2;
+    L.shm = sv == SOLVE_NONE ? 0 : yz_lds(nthr, 128);
+    L.pre = pre;
+  }
+  L.block = dim3(nthr);
+  long long blk = 0;
+  for (auto& e : all) {
+    if (L.x) {
+      e.a.vec = key.aligned && ((e.off * (long long)sizeof(TS)) % 16 == 0);
+      e.a.lines = 64 / e.a.P;
+    } else {
+      e.a.lines = 128;
+      while (e.a.lines * e.a.P > nthr) e.a.lines /= 2;
+    }
+    e.blk0 = blk;
+    blk += (e.a.nlines + e.a.lines - 1) / e.a.lines;
+  }
+  L.nblocks = blk;
+  return upload(all.data(), all.size() * sizeof(GrpEntry));
 }
 
 #endif  // PYR_PART == 0
 
-template <typename TS, int KIND, int SOLVE, int MODE>
+template <typename TS, int KIND, int SOLVE>
 static int grp_launch_typed(pyr_group* g, const GrpLaunch& L, const TS* in, TS* out) {
   if (L.nblocks <= 0) return 0;
   const dim3 grid((unsigned)L.nblocks);
+  auto k = k_line_yz_grp<TS, KIND, SOLVE, PRE_NONE>;
   if (L.x) {
-    auto k = k_line_x_grp<TS, KIND, SOLVE, MODE>;
-    if (set_lds(k, L.shm)) return 1;
-    hipLaunchKernelGGL(k, grid, L.block, L.shm, g->stream, L.dev, L.M, in, out);
-  } else {
-    auto pick = [&](auto k64, auto k32, auto k16) {
-      return L.ly == 64 ? k64 : (L.ly == 32 ? k32 : k16);
-    };
-    auto k = pick(k_line_yz_grp<TS, KIND, SOLVE, MODE, 64, PRE_NONE>, k_line_yz_grp<TS, KIND, SOLVE, MODE, 32, PRE_NONE>,
-                  k_line_yz_grp<TS, KIND, SOLVE, MODE, 16, PRE_NONE>);
-    if (L.pre == PRE_OLD)
-      k = pick(k_line_yz_grp<TS, KIND, SOLVE, MODE, 64, PRE_OLD>, k_line_yz_grp<TS, KIND, SOLVE, MODE, 32, PRE_OLD>,
-               k_line_yz_grp<TS, KIND, SOLVE, MODE, 16, PRE_OLD>);
-    if (L.pre == PRE_V) {
-      if constexpr (KIND == K_R4)
-        k = pick(k_line_yz_grp<TS, KIND, SOLVE, MODE, 64, PRE_V>, k_line_yz_grp<TS, KIND, SOLVE, MODE, 32, PRE_V>,
-                 k_line_yz_grp<TS, KIND, SOLVE, MODE, 16, PRE_V>);
-      else
-        return fail("filter epilogue on a non-filter kernel");
-    }
-    if (set_lds(k, L.shm)) return 1;
-    hipLaunchKernelGGL(k, grid, L.block, L.shm, g->stream, L.dev, L.M, in, out);
+    k = k_line_x_grp<TS, KIND, SOLVE>;
+  } else if (L.pre == PRE_V) {
+    if constexpr (KIND == K_R4) k = k_line_yz_grp<TS, KIND, SOLVE, PRE_V>;
+    else return fail("filter epilogue on a non-filter kernel");
+  } else if (L.pre == PRE_OLD) {
+    k = k_line_yz_grp<TS, KIND, SOLVE, PRE_OLD>;
   }
+  hipLaunchKernelGGL(k, grid, L.block, L.shm, g->stream, (const GrpEntry*)L.dev, L.M, in, out);
   HIPCHECK(hipGetLastError());
   return 0;
 }
 
-template <typename TS, int MODE>
-int grp_launch_mode(pyr_group* g, const GrpLaunch& L, const TS* in, TS* out) {
+template <typename TS>
+int grp_launch(pyr_group* g, const GrpLaunch& L, const TS* in, TS* out) {
   switch (L.kind) {
     case K_D1:
-      return L.solve == SOLVE_CIRC ? grp_launch_typed<TS, K_D1, SOLVE_CIRC, MODE>(g, L, in, out)
-                                   : grp_launch_typed<TS, K_D1, SOLVE_LU, MODE>(g, L, in, out);
+      return L.solve == SOLVE_CIRC ? grp_launch_typed<TS, K_D1, SOLVE_CIRC>(g, L, in, out)
+                                   : grp_launch_typed<TS, K_D1, SOLVE_BND>(g, L, in, out);
     case K_R3:
-      return L.solve == SOLVE_CIRC ? grp_launch_typed<TS, K_R3, SOLVE_CIRC, MODE>(g, L, in, out)
-                                   : grp_launch_typed<TS, K_R3, SOLVE_LU, MODE>(g, L, in, out);
+      return L.solve == SOLVE_CIRC ? grp_launch_typed<TS, K_R3, SOLVE_CIRC>(g, L, in, out)
+                                   : grp_launch_typed<TS, K_R3, SOLVE_BND>(g, L, in, out);
     default:
-      if (L.solve == SOLVE_CIRC) return grp_launch_typed<TS, K_R4, SOLVE_CIRC, MODE>(g, L, in, out);
-      if (L.solve == SOLVE_LU) return grp_launch_typed<TS, K_R4, SOLVE_LU, MODE>(g, L, in, out);
-      return grp_launch_typed<TS, K_R4, SOLVE_NONE, MODE>(g, L, in, out);
+      if (L.solve == SOLVE_CIRC) return grp_launch_typed<TS, K_R4, SOLVE_CIRC>(g, L, in, out);
+      if (L.solve == SOLVE_BND) return grp_launch_typed<TS, K_R4, SOLVE_BND>(g, L, in, out);
+      return grp_launch_typed<TS, K_R4, SOLVE_NONE>(g, L, in, out);
   }
 }
 
-#define PYR_GRP_MODE(TS, MODE) template int grp_launch_mode<TS, MODE>(pyr_group*, const GrpLaunch&, const TS*, TS*);
-#if PYR_PART == 1
-PYR_GRP_MODE(double, MODE_F64)
-#elif PYR_PART == 2
-PYR_GRP_MODE(float, MODE_R32)
-#elif PYR_PART == 3
-PYR_GRP_MODE(float, MODE_S32)
+#if PYR_PART == 7
+template <int KIND>
+static int grp_launch_ref_kind(hipStream_t stream, const GrpLaunch& L, const float* in, float* out) {
+  if (L.nblocks <= 0) return 0;
+  auto k = k_ref_yz_grp<KIND, PRE_NONE>;
+  if (L.x) {
+    k = k_ref_x_grp<KIND>;
+  } else if (L.pre == PRE_V) {
+    if constexpr (KIND == K_R4) k = k_ref_yz_grp<KIND, PRE_V>;
+    else return fail("filter epilogue on a non-filter kernel");
+  } else if (L.pre == PRE_OLD) {
+    k = k_ref_yz_grp<KIND, PRE_OLD>;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)L.nblocks), L.block, 0, stream, (const RefEntry*)L.dev, L.M, in, out);
+  HIPCHECK(hipGetLastError());
+  return 0;
+}
+int grp_launch_ref(hipStream_t stream, const GrpLaunch& L, const float* in, float* out) {
+  if (L.kind == K_D1) return grp_launch_ref_kind<K_D1>(stream, L, in, out);
+  if (L.kind == K_R3) return grp_launch_ref_kind<K_R3>(stream, L, in, out);
+  return grp_launch_ref_kind<K_R4>(stream, L, in, out);
+}
 #else
-extern PYR_GRP_MODE(double, MODE_F64)
-extern PYR_GRP_MODE(float, MODE_R32)
-extern PYR_GRP_MODE(float, MODE_S32)
+int grp_launch_ref(hipStream_t stream, const GrpLaunch& L, const float* in, float* out);
 #endif
-#undef PYR_GRP_MODE
+
+#define PYR_GRP(TS) template int grp_launch<TS>(pyr_group*, const GrpLaunch&, const TS*, TS*);
+#if PYR_PART == 5
+PYR_GRP(double)
+#elif PYR_PART == 6
+PYR_GRP(float)
+#elif PYR_PART == 0
+extern PYR_GRP(double)
+extern PYR_GRP(float)
+#endif
+#undef PYR_GRP
 
 #if PYR_PART == 0
-template <typename TS, int MODE>
+template <typename TS>
 static int grp_apply(pyr_group* g, const GrpKey& key, const TS* in, TS* out) {
   auto it = g->plans.find(key);
   if (it == g->plans.end()) {
     GrpPlan gp;
-    if (grp_build<TS, MODE>(g, key, gp)) {
+    if (grp_build<TS>(g, key, gp)) {
       for (auto& l : gp.launches)
         if (l.dev) (void)hipFree(l.dev);
       return 1;
     }
     it = g->plans.emplace(key, std::move(gp)).first;
   }
-  for (const GrpLaunch& L : it->second.launches)
-    if (grp_launch_mode<TS, MODE>(g, L, in, out)) return 1;
+  for (const GrpLaunch& L : it->second.launches) {
+    if constexpr (sizeof(TS) == 4) {
+      if (L.refined) {
+        if (grp_launch_ref(g->stream, L, in, out)) return 1;
+        continue;
+      }
+    }
+    if (grp_launch<TS>(g, L, in, out)) return 1;
+  }
   for (const GrpNull& z : it->second.nulls) {
     const long long n = (long long)g->mem[z.member]->npts();
     const long long o = g->off[z.member];
@@ -2226,10 +1803,7 @@ int pyr_setup_host(pyr_ctx** ctx, int nx, int ny, int nz, double x1, double xn, 
 int pyr_destroy(pyr_ctx* c) {
   if (!c) return 0;
   if (c->device) {
-    for (int op = 0; op < NOPS; ++op)
-      for (int d = 0; d < 3; ++d)
-        for (DevPlan* dp : {&c->dplan[op][d], &c->dplan_a[op][d]})
-          if (dp->mem) (void)hipFree(dp->mem);
+    if (c->tables) (void)hipFree(c->tables);
     for (int i = 0; i < 2; ++i)
       if (c->field_tmp[i]) (void)hipFree(c->field_tmp[i]);
   }
@@ -2258,13 +1832,10 @@ int pyr_set_tuning(pyr_ctx* c, int op, int dir, int prec, int x_lds_kb, int yz_p
     return fail("yz_pipe must be 0, 1, 2 (x) or 3 (y/z) (or -1)");
   if (yz_lines >= 0 && yz_lines != 16 && yz_lines != 32 && yz_lines != 64)
     return fail("yz_lines must be 16, 32 or 64 (or -1)");
-  int mode;
-  if (prec == PYR_F64) mode = MODE_F64;
-  else if (prec == PYR_R32) mode = r32_mode(c, op, dir) == PYR_R32_SOLVE_FP64 ? MODE_S32 : MODE_R32;
-  else return fail("bad precision");
-  c->tune_xlds[op][dir][mode] = x_lds_kb < 0 ? -1 : x_lds_kb;
-  c->tune_pipe[op][dir][mode] = yz_pipe < 0 ? -1 : yz_pipe;
-  c->tune_ly[op][dir][mode] = yz_lines < 0 ? -1 : yz_lines;
+  if (prec != PYR_F64 && prec != PYR_R32) return fail("bad precision");
+  const int wd = prec == PYR_F64 ? 0 : 1;
+  c->tune_ly[op][dir][wd] = yz_lines < 0 ? -1 : yz_lines;
+  c->tune_rt[op][dir][wd] = yz_pipe == 3;
   return 0;
 }
 
@@ -2507,24 +2078,17 @@ int pyr_group_apply(pyr_group* g, int op, int dir, int prec, const void* in, voi
   key.power = mesh_power;
   key.aligned = ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0);
   key.ec = ec;
-  key.psolve = g->mem[0]->periodic_solver;
-  key.xlds = g->mem[0]->x_lds_kb;
   for (pyr_ctx* c : g->mem)
-    if (c->periodic_solver != key.psolve || c->x_lds_kb != key.xlds)
+    if (c->periodic_solver != g->mem[0]->periodic_solver || c->x_lds_kb != g->mem[0]->x_lds_kb)
       return fail("group members differ in their periodic solver or x-line LDS budget");
-  if (prec == PYR_F64) {
-    key.mode = MODE_F64;
-    return grp_apply<double, MODE_F64>(g, key, (const double*)in, (double*)out);
-  }
+  key.refined = 0;
+  if (prec == PYR_F64) return grp_apply<double>(g, key, (const double*)in, (double*)out);
   if (prec == PYR_R32) {
-    // the solve arithmetic of this operator and direction (per-operator
-    // tuning included), the same for every member
-    const int r = r32_mode(g->mem[0], op, dir);
     for (pyr_ctx* c : g->mem)
-      if (r32_mode(c, op, dir) != r) return fail("group members differ in their FP32 solve mode");
-    key.mode = r == PYR_R32_SOLVE_FP64 ? MODE_S32 : MODE_R32;
-    if (r == PYR_R32_SOLVE_FP64) return grp_apply<float, MODE_S32>(g, key, (const float*)in, (float*)out);
-    return grp_apply<float, MODE_R32>(g, key, (const float*)in, (float*)out);
+      if (r32_mode(c, op, dir) != r32_mode(g->mem[0], op, dir))
+        return fail("group members differ in their FP32 solve mode");
+    key.refined = r32_mode(g->mem[0], op, dir) == PYR_R32_SOLVE_REFINED;
+    return grp_apply<float>(g, key, (const float*)in, (float*)out);
   }
   return fail("bad precision");
 }
@@ -2546,12 +2110,11 @@ int pyr_host_weights(int op, double* ali, double* ari, double* alb1, double* alb
 
 int pyr_host_emulate(pyr_ctx* c, int op, int dir, int prec, const void* in, void* out) {
   if (!c) return fail("null context");
+  const bool anti = (op & PYR_OP_ANTISYM) != 0;
+  op &= ~PYR_OP_ANTISYM;
   if (op < 0 || op >= NOPS || dir < 0 || dir > 2) return fail("bad operator or direction");
-  if (prec == PYR_F64) return emulate<double, MODE_F64>(c, op, dir, (const double*)in, (double*)out);
-  if (prec == PYR_R32) {
-    if (r32_mode(c, op, dir) == PYR_R32_SOLVE_FP64) return emulate<float, MODE_S32>(c, op, dir, (const float*)in, (float*)out);
-    return emulate<float, MODE_R32>(c, op, dir, (const float*)in, (float*)out);
-  }
+  if (prec == PYR_F64) return emulate<double>(c, op, dir, (const double*)in, (double*)out, anti);
+  if (prec == PYR_R32) return emulate<float>(c, op, dir, (const float*)in, (float*)out, anti);
   return fail("bad precision");
 }
 

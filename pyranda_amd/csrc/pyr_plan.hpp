@@ -1,33 +1,37 @@
 // Host-side plan of one compact operator along one direction.
 //
 // The reference assembles a global band per direction (compact_basetype.f90:
-// 124-148) and factors it whole: a bordered cyclic LU for periodic lines
-// (pentadiagonal.f90:64-131) or a plain banded LU (:18-39). On the GPU each
-// line is instead split into P chunks of at most CHUNK rows; a thread keeps its
-// chunk in registers and solves it with the chunk's own banded LU. Chunks are
-// coupled only through the two rows at each end, so the exact solution is
-//     x = x_loc - rc(:,0..3) . (y[s-2], y[s-1], y[e], y[e+1])
-// where the four neighbour values come from a 4P x 4P reduced system whose
-// inverse G is identical for every line and is precomputed here. The same
-// construction handles the cyclic coupling of periodic lines (chunk 0's left
-// neighbour is chunk P-1), so no Sherman-Morrison step is needed.
+// 124-148), factors it whole (a bordered cyclic LU for periodic lines,
+// pentadiagonal.f90:64-131, or a plain banded LU, :18-39) and sweeps each line
+// sequentially. On the GPU a line is split into P chunks of at most CHUNK
+// rows, one thread per chunk, its rows in registers. A solve is a forward and
+// a backward second-order recurrence
+//     x_k = r_k - l1_k x_{k-1} - l2_k x_{k-2}
+//     y_k = g_k x_k - v1_k y_{k+1} - v2_k y_{k+2}
+// (y times 1/c is the solution). A chunk runs each recurrence from a zero
+// state to get its exit state; its true entry state is the sum over the chunks
+// before it (after it, backward) of their exits propagated through the chunks
+// between, and it re-runs the recurrence from there. The propagation matrices
+// decay geometrically with distance (the schemes' recurrences are strongly
+// damped), so only the W nearest chunks whose matrix is above CARRY_TOL enter.
 //
 // Periodic lines have a circulant LHS, which factors exactly as
 //     A = c Q^T Q,   Q = I + p1 S + p2 S^2   ((S x)_i = x_{i-1}, cyclic)
-// with both roots of 1 + p1 z + p2 z^2 outside the unit circle. A solve is then
-// a forward and a backward second-order recurrence with constant coefficients;
-// a chunk runs each recurrence from a zero state to get its exit state, the
-// true entry states of all chunks follow from a 2P x 2P carry system (rows
-// `kf`, `kb`), and the chunk re-runs the recurrence from its true entry. No
-// per-row tables are read.
+// with both roots of 1 + p1 z + p2 z^2 outside the unit circle: the
+// coefficients are constants (l = v = p, g = 1) and the carry wraps around.
+// Bounded lines take the LU factors of the assembled band row by row; away
+// from the lower end (and before the last four rows) they converge to the same
+// constants, and chunks whose rows have all converged use those.
 //
-// RHS rows: interior rows use the interior weights; the up-to-4 rows at each
-// end of a bounded line are stored as term lists coef*(v[a]-v[b]) that keep
-// the reference's difference forms (compact_d1.f90:113-207,
-// compact_r3.f90:97-157, compact_r4.f90:106-207).
+// RHS rows: interior rows use the interior weights; the four rows at each end
+// of a bounded line use rows of their own, in the difference form
+// sum_l c_l (v_{i+l} - v_i) + (sum_l c_l) v_i that the reference's forms
+// amount to (compact_d1.f90:113-207, compact_r3.f90:97-157,
+// compact_r4.f90:106-207); columns outside the line have no weight.
 #pragma once
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <complex>
 #include <stdexcept>
@@ -38,10 +42,13 @@
 
 namespace pyr {
 
-constexpr int CHUNK = 32;   // rows per thread (register-resident)
-constexpr int PMAX = 32;    // chunks per line -> N <= 1024
+// Rows per thread. 16 keeps an FP64 chunk with its halo in 75-110 VGPRs (five
+// waves per SIMD); measured at 256^3 on gfx950, FP64 d1 y: 54 us at 16 rows,
+// 57 at 32, 79 at 8 (a copy of the field: 50 us).
+constexpr int CHUNK = 16;
+constexpr int PMAX = 64;    // chunks per line -> N <= 1024
 constexpr int NB = 4;       // boundary rows per side with their own RHS forms
-constexpr int MAXT = 10;    // terms per boundary row
+constexpr int WBROW = 10;   // a boundary row: weights at offsets -4..4, their sum
 
 enum Kind { K_D1 = 0, K_R3 = 1, K_R4 = 2 };
 
@@ -51,142 +58,26 @@ inline int kind_halo(int kind) { return kind == K_R4 ? 4 : 3; }
 struct OpPlan {
   int op = 0, kind = 0, N = 0, P = 0, periodic = 0, implicit = 0, addv = 0;
   int null_op = 0, null_option = 0, R = 3;
-  double scale = 1.0;       // metric applied to the solve result
-  double w[9] = {};         // interior RHS weights, offsets -R..R
-  std::vector<int> cstart;  // P+1 chunk starts
-  std::vector<double> lu;   // N x 5: l(i-2), l(i-1), 1/u(i,i), u(i,i+1), u(i,i+2)
-  std::vector<double> rc;   // N x 4: spikes for y[s-2], y[s-1], y[e], y[e+1]
-  std::vector<double> gsel; // P x 4 x 4P: rows of G giving those four values
-  std::vector<double> band; // N x 5: full LHS band (refinement residual)
-  std::vector<double> bcoef;  // 2*NB x MAXT
-  std::vector<short> bidx;    // 2*NB x MAXT x 2 (a,b); -1 reads as 0
-  std::vector<int> bnt;       // 2*NB
-  // circulant solve of periodic implicit lines
-  int circ = 0;
-  double p1 = 0, p2 = 0, invc = 0;  // A = c Q^T Q, Q = I + p1 S + p2 S^2
-  double bd[3] = {};                // LHS row: A[i][i+-2], A[i][i+-1], A[i][i]
-  std::vector<double> kf, kb;       // P x 2 x 2P: entry states from all exit states
+  int mb = 0, mx = 0;         // chunk p has mb + (p < mx) rows
+  double scale = 1.0;         // metric (times 1/c of an implicit operator)
+  double w[4] = {};           // D1: weights at +1..+3; R3/R4: their tail sums (rhs_interior)
+  std::vector<double> wb;     // 2*NB x WBROW boundary rows of a bounded line
+  double p1 = 0, p2 = 0;      // limit coefficients
+  int W = 0;                  // chunks that enter a carry
+  int kp = 1;                 // 1: one set of carry matrices for all chunks, else P
+  std::vector<double> kf, kb; // W x kp x 4 carry matrices, forward and backward
+  // bounded lines: per-row factors, row k of chunk p at [k * P + p]
+  std::vector<double> tf, tb, tg;  // (l1, l2), (v1, v2), g
+  int tlo = 0;                // chunks p < tlo and p = P - 1 need the tables
 };
+
+// Propagation matrices below this are left out of the carries: relative to the
+// state they multiply it is under a thousandth of an FP64 rounding.
+constexpr long double CARRY_TOL = 1e-19L;
 
 namespace detail {
 
 using ld = long double;
-
-struct TermRow {
-  std::vector<double> c;
-  std::vector<int> a, b;
-  void add(double coef, int ia, int ib) {
-    if (coef == 0.0) return;
-    c.push_back(coef); a.push_back(ia); b.push_back(ib);
-  }
-};
-
-// Boundary-row RHS forms of a bounded line, 0-based rows; ar(l,i) is the
-// reference's (1-based l, 1-based i) weight. Ghost columns read 0.
-inline void boundary_terms(int kind, int n, int v1, int v2,
-                           const std::vector<std::vector<double>>& ar,
-                           TermRow lo[NB], TermRow hi[NB]) {
-  auto AR = [&](int l, int i1) { return ar[i1 - 1][l - 1]; };
-  auto sumr = [&](int i1, int nr) { double s = 0; for (int l = 1; l <= nr; ++l) s += AR(l, i1); return s; };
-  if (kind == K_D1) {
-    if (v1 == -1) {
-      for (int l = 4; l <= 7; ++l) lo[0].add(AR(l, 1), l - 4, -1);
-      for (int l = 3; l <= 7; ++l) lo[1].add(AR(l, 2), l - 3, -1);
-      for (int l = 2; l <= 7; ++l) lo[2].add(AR(l, 3), l - 2, -1);
-    } else {
-      for (int l = 5; l <= 7; ++l) lo[0].add(AR(l, 1), l - 4, 0);
-      for (int l = 4; l <= 7; ++l) lo[1].add(AR(l, 2), l - 3, 0);
-      lo[2].add(AR(5, 3), 3, 1); lo[2].add(AR(6, 3), 4, 0); lo[2].add(AR(7, 3), 5, 0);
-    }
-    // row 4 (1-based): interior antisymmetric form with its own weights
-    lo[3].add(AR(5, 4), 4, 2); lo[3].add(AR(6, 4), 5, 1); lo[3].add(AR(7, 4), 6, 0);
-    // row n-3 (1-based)
-    hi[0].add(AR(5, n - 3), n - 3, n - 5); hi[0].add(AR(6, n - 3), n - 2, n - 6);
-    hi[0].add(AR(7, n - 3), n - 1, n - 7);
-    if (v2 == -1) {
-      for (int l = 1; l <= 6; ++l) hi[1].add(AR(l, n - 2), n - 7 + l, -1);
-      for (int l = 1; l <= 5; ++l) hi[2].add(AR(l, n - 1), n - 6 + l, -1);
-      for (int l = 1; l <= 4; ++l) hi[3].add(AR(l, n), n - 5 + l, -1);
-    } else {
-      hi[1].add(AR(1, n - 2), n - 6, n - 1); hi[1].add(AR(2, n - 2), n - 5, n - 1);
-      hi[1].add(AR(3, n - 2), n - 4, n - 2);
-      for (int l = 1; l <= 4; ++l) hi[2].add(AR(l, n - 1), n - 6 + l, n - 1);
-      for (int l = 1; l <= 3; ++l) hi[3].add(AR(l, n), n - 5 + l, n - 1);
-    }
-  } else if (kind == K_R3) {
-    // ghosts are zero on a bounded end (compact_r3.f90:84-99)
-    for (int l = 1; l <= 3; ++l) lo[0].add(AR(l, 1), -1, 0);
-    for (int l = 4; l <= 7; ++l) lo[0].add(AR(l, 1), l - 4, 0);
-    for (int l = 1; l <= 2; ++l) lo[1].add(AR(l, 2), -1, 1);
-    for (int l = 3; l <= 7; ++l) lo[1].add(AR(l, 2), l - 3, 1);
-    lo[2].add(AR(1, 3), -1, 2);
-    for (int l = 2; l <= 7; ++l) lo[2].add(AR(l, 3), l - 2, 2);
-    for (int l = 1; l <= 7; ++l) lo[3].add(AR(l, 4), l - 1, 3);
-    if (v1 == -1)
-      for (int r = 0; r < 3; ++r) lo[r].add(sumr(r + 1, 7), r, -1);
-    for (int l = 1; l <= 7; ++l) hi[0].add(AR(l, n - 3), n - 8 + l, n - 4);
-    for (int l = 1; l <= 6; ++l) hi[1].add(AR(l, n - 2), n - 7 + l, n - 3);
-    hi[1].add(AR(7, n - 2), -1, n - 3);
-    for (int l = 1; l <= 5; ++l) hi[2].add(AR(l, n - 1), n - 6 + l, n - 2);
-    for (int l = 6; l <= 7; ++l) hi[2].add(AR(l, n - 1), -1, n - 2);
-    for (int l = 1; l <= 4; ++l) hi[3].add(AR(l, n), n - 5 + l, n - 1);
-    for (int l = 5; l <= 7; ++l) hi[3].add(AR(l, n), -1, n - 1);
-    if (v2 == -1)
-      for (int r = 1; r < 4; ++r) hi[r].add(sumr(n - 3 + r, 7), n - 4 + r, -1);
-  } else {
-    if (v1 == -1) {
-      for (int l = 5; l <= 9; ++l) lo[0].add(AR(l, 1), l - 5, -1);
-      for (int l = 4; l <= 9; ++l) lo[1].add(AR(l, 2), l - 4, -1);
-      for (int l = 3; l <= 9; ++l) lo[2].add(AR(l, 3), l - 3, -1);
-      for (int l = 2; l <= 9; ++l) lo[3].add(AR(l, 4), l - 2, -1);
-    } else {
-      for (int l = 6; l <= 9; ++l) lo[0].add(AR(l, 1), l - 5, 0);
-      for (int l = 5; l <= 9; ++l) lo[1].add(AR(l, 2), l - 4, 0);
-      for (int l = 4; l <= 9; ++l) lo[2].add(AR(l, 3), l - 3, 0);
-      for (int l = 3; l <= 9; ++l) lo[3].add(AR(l, 4), l - 2, 0);
-    }
-    if (v2 == -1) {
-      for (int l = 1; l <= 8; ++l) hi[0].add(AR(l, n - 3), n - 9 + l, -1);
-      for (int l = 1; l <= 7; ++l) hi[1].add(AR(l, n - 2), n - 8 + l, -1);
-      for (int l = 1; l <= 6; ++l) hi[2].add(AR(l, n - 1), n - 7 + l, -1);
-      for (int l = 1; l <= 5; ++l) hi[3].add(AR(l, n), n - 6 + l, -1);
-    } else {
-      for (int l = 1; l <= 7; ++l) hi[0].add(AR(l, n - 3), n - 9 + l, n - 1);
-      for (int l = 1; l <= 6; ++l) hi[1].add(AR(l, n - 2), n - 8 + l, n - 1);
-      for (int l = 1; l <= 5; ++l) hi[2].add(AR(l, n - 1), n - 7 + l, n - 1);
-      for (int l = 1; l <= 4; ++l) hi[3].add(AR(l, n), n - 6 + l, n - 1);
-    }
-  }
-}
-
-// Gauss-Jordan inverse with partial pivoting (small dense, long double)
-inline void invert(std::vector<ld>& a, int n) {
-  std::vector<ld> inv(size_t(n) * n, 0.0L);
-  for (int i = 0; i < n; ++i) inv[size_t(i) * n + i] = 1.0L;
-  for (int c = 0; c < n; ++c) {
-    int piv = c;
-    for (int r = c + 1; r < n; ++r)
-      if (std::fabs(a[size_t(r) * n + c]) > std::fabs(a[size_t(piv) * n + c])) piv = r;
-    if (a[size_t(piv) * n + c] == 0.0L) throw std::runtime_error("singular reduced system");
-    if (piv != c)
-      for (int k = 0; k < n; ++k) {
-        std::swap(a[size_t(c) * n + k], a[size_t(piv) * n + k]);
-        std::swap(inv[size_t(c) * n + k], inv[size_t(piv) * n + k]);
-      }
-    const ld d = 1.0L / a[size_t(c) * n + c];
-    for (int k = 0; k < n; ++k) { a[size_t(c) * n + k] *= d; inv[size_t(c) * n + k] *= d; }
-    for (int r = 0; r < n; ++r) {
-      if (r == c) continue;
-      const ld f = a[size_t(r) * n + c];
-      if (f == 0.0L) continue;
-      for (int k = 0; k < n; ++k) {
-        a[size_t(r) * n + k] -= f * a[size_t(c) * n + k];
-        inv[size_t(r) * n + k] -= f * inv[size_t(c) * n + k];
-      }
-    }
-  }
-  a.swap(inv);
-}
 
 // Spectral factor of the symmetric pentadiagonal symbol
 //   b/z^2 + a/z + d + a z + b z^2 = c (1 + p1 z + p2 z^2)(1 + p1/z + p2/z^2)
@@ -216,65 +107,58 @@ inline bool spectral_factor(ld b, ld a, ld d, ld& p1, ld& p2, ld& c) {
   return std::fabs(ed) <= 1e-14L * scale && std::fabs(ea) <= 1e-14L * scale;
 }
 
-// Carry rows of the circulant solve. Forward: chunk q entered with
-// (x[s_q-2], x[s_q-1]) leaves with its zero-entry exit e_q plus H_q times the
-// entry, and chunk q+1 (cyclic) is entered with that exit. Backward likewise
-// from the right with (u[e_q], u[e_q+1]). K maps the exits of all chunks
-// (layout 2q + i) to the entry of each chunk (rows 2p + i).
-inline void circ_carry_rows(int P, const std::vector<int>& cstart, ld p1, ld p2,
-                            std::vector<double>& kf, std::vector<double>& kb) {
-  const int n2 = 2 * P;
-  std::vector<ld> Mf(size_t(n2) * n2, 0.0L), Mb(size_t(n2) * n2, 0.0L);
-  for (int q = 0; q < P; ++q) {
-    const int m = cstart[q + 1] - cstart[q];
-    ld Hf[2][2], Hb[2][2];
-    for (int j = 0; j < 2; ++j) {
-      ld xm2 = j == 0, xm1 = j == 1;  // forward state (x[k-2], x[k-1])
-      for (int k = 0; k < m; ++k) {
-        const ld x = -p1 * xm1 - p2 * xm2;
-        xm2 = xm1;
-        xm1 = x;
-      }
-      Hf[0][j] = xm2;
-      Hf[1][j] = xm1;
-      ld u1 = j == 0, u2 = j == 1;  // backward state (u[k+1], u[k+2])
-      for (int k = m - 1; k >= 0; --k) {
-        const ld u = -p1 * u1 - p2 * u2;
-        u2 = u1;
-        u1 = u;
-      }
-      Hb[0][j] = u1;
-      Hb[1][j] = u2;
-    }
-    const int qn = (q + 1) % P, qp = (q - 1 + P) % P;
-    for (int i = 0; i < 2; ++i) {
-      Mf[size_t(2 * qn + i) * n2 + 2 * qn + i] += 1.0L;
-      Mb[size_t(2 * qp + i) * n2 + 2 * qp + i] += 1.0L;
-      for (int j = 0; j < 2; ++j) {
-        Mf[size_t(2 * qn + i) * n2 + 2 * q + j] -= Hf[i][j];
-        Mb[size_t(2 * qp + i) * n2 + 2 * q + j] -= Hb[i][j];
-      }
+using M2 = std::array<ld, 4>;  // 2x2, row-major
+
+inline M2 mul(const M2& x, const M2& y) {
+  return {x[0] * y[0] + x[1] * y[2], x[0] * y[1] + x[1] * y[3], x[2] * y[0] + x[3] * y[2], x[2] * y[1] + x[3] * y[3]};
+}
+inline ld norm(const M2& x) {
+  return std::max(std::max(std::fabs(x[0]), std::fabs(x[1])), std::max(std::fabs(x[2]), std::fabs(x[3])));
+}
+
+// Carry matrices of one direction. H[q] takes the entry state of chunk q to
+// the part of its exit state that depends on it; step is -1 forward (the carry
+// of chunk p comes from p-1, p-2, ...) or +1 backward. K[j][p] multiplies the
+// exit of chunk p + step (j+1); around a cyclic line the terms beyond one turn
+// fold onto the chunks they come from. Returns the terms per chunk.
+inline std::vector<std::vector<M2>> carry_matrices(const std::vector<M2>& H, int step, bool cyclic) {
+  const int P = (int)H.size();
+  std::vector<std::vector<M2>> K;
+  for (int p = 0; p < P; ++p) {
+    M2 acc = {1, 0, 0, 1};
+    for (int j = 0;; ++j) {
+      int q = p + step * (j + 1);
+      if (!cyclic && (q < 0 || q >= P)) break;
+      if (norm(acc) < CARRY_TOL) break;
+      q = ((q % P) + P) % P;
+      const int jj = j % P;
+      if ((int)K.size() <= jj) K.push_back(std::vector<M2>(P, M2{0, 0, 0, 0}));
+      for (int i = 0; i < 4; ++i) K[jj][p][i] += acc[i];
+      acc = mul(acc, H[q]);
     }
   }
-  invert(Mf, n2);
-  invert(Mb, n2);
-  // the exit of chunk q is the right-hand side of row block q+1 (forward) or
-  // q-1 (backward)
-  kf.assign(size_t(n2) * n2, 0.0);
-  kb.assign(size_t(n2) * n2, 0.0);
-  for (int r = 0; r < n2; ++r)
-    for (int q = 0; q < P; ++q)
-      for (int i = 0; i < 2; ++i) {
-        kf[size_t(r) * n2 + 2 * q + i] = (double)Mf[size_t(r) * n2 + 2 * ((q + 1) % P) + i];
-        kb[size_t(r) * n2 + 2 * q + i] = (double)Mb[size_t(r) * n2 + 2 * ((q - 1 + P) % P) + i];
-      }
+  return K;
+}
+
+// Chunks of a line of n rows along direction dir. x lines: one wave takes G
+// whole lines, so P is the most chunks that still leaves room for as many
+// lines as the fewest possible chunks would (n = 300: 19 chunks needed, 3
+// lines per wave, 21 chunks each). y/z lines: an even count, so that waves of
+// 32 lines hold two chunks each. Every chunk has at least 8 rows (n >= 8).
+inline int chunk_count(int n, int dir) {
+  const int need = (n + CHUNK - 1) / CHUNK;
+  if (n == need * CHUNK) return need;
+  if (dir == 0) return 64 / (64 / need);
+  return need > 2 ? need + (need & 1) : need;
 }
 
 }  // namespace detail
 
-// Build the plan. v1/v2 are the boundary variants (0 NONE, +1 SYMM).
-inline OpPlan build_plan(int op, int n, int periodic, int v1, int v2, double metric) {
+// Build the plan. v1/v2 are the boundary variants (0 NONE, +1 SYMM, -1 its
+// antisymmetric member).
+inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, double metric) {
   using detail::ld;
+  using detail::M2;
   OpPlan pl;
   const Scheme sc = make_scheme(op);
   pl.op = op;
@@ -288,192 +172,151 @@ inline OpPlan build_plan(int op, int n, int periodic, int v1, int v2, double met
   pl.null_op = (n < 4);  // compact_basetype.f90:86-90
   pl.scale = (op == OP_D1) ? 1.0 / metric : (op == OP_D2 ? 1.0 / (metric * metric) : 1.0);
   const int hr = sc.ncr / 2;
-  for (int l = -pl.R; l <= pl.R; ++l) pl.w[l + pl.R] = sc.ari[l + hr];
+  if (pl.kind == K_D1) {
+    for (int l = 1; l <= 3; ++l) pl.w[l - 1] = sc.ari[hr + l];
+  } else {
+    // symmetric rows of zero sum: sum_l w_l (v_{i+l} - v_i) = sum_m c_m
+    // (d_{i+m-1} - d_{i-m}) with d_j = v_{j+1} - v_j and c_m = w_m + w_{m+1} + ...
+    ld c = 0.0L;
+    for (int l = pl.R; l >= 1; --l) {
+      c += (ld)sc.ari[hr + l];
+      pl.w[l - 1] = (double)c;
+    }
+  }
   if (pl.null_op) return pl;
   // the reference's boundary forms read up to row 8 of a line (compact_r4.f90:
   // 117-120); shorter lines are outside what the schemes define
   if (n < 8) throw std::runtime_error("line length " + std::to_string(n) + " is below 8 (supported: 1-3 or 8-1024)");
   if (n > CHUNK * PMAX)
     throw std::runtime_error("line length " + std::to_string(n) + " exceeds " + std::to_string(CHUNK * PMAX));
-
-  // assembled rows (compact_basetype.f90:124-133), 0-based
-  std::vector<std::vector<double>> gal(n, std::vector<double>(5, 0.0));
-  std::vector<std::vector<double>> gar(n, std::vector<double>(9, 0.0));
-  for (int i = 0; i < n; ++i) {
-    for (int c = 0; c < sc.ncl; ++c) gal[i][c] = sc.ali[c];
-    for (int l = 0; l < sc.ncr; ++l) gar[i][l] = sc.ari[l];
-  }
-  if (!periodic) {
-    for (int j = 0; j < 4; ++j) {
-      for (int c = 0; c < sc.ncl; ++c) {
-        gal[j][c] = sc.alb1[v1 + 1][j][c];
-        gal[n - 4 + j][c] = sc.alb2[v2 + 1][j][c];
-      }
-      for (int l = 0; l < sc.ncr; ++l) {
-        gar[j][l] = sc.arb1[v1 + 1][j][l];
-        gar[n - 4 + j][l] = sc.arb2[v2 + 1][j][l];
-      }
-    }
-  }
-  // full LHS band as A[i][i-2..i+2] (explicit operators: identity)
-  pl.band.assign(size_t(n) * 5, 0.0);
-  for (int i = 0; i < n; ++i) {
-    if (sc.implicit)
-      for (int c = 0; c < 5; ++c) pl.band[size_t(i) * 5 + c] = gal[i][c];
-    else
-      pl.band[size_t(i) * 5 + 2] = 1.0;
-  }
-  // boundary RHS term lists
-  pl.bcoef.assign(2 * NB * MAXT, 0.0);
-  pl.bidx.assign(2 * NB * MAXT * 2, -1);
-  pl.bnt.assign(2 * NB, 0);
-  if (!periodic) {
-    detail::TermRow lo[NB], hi[NB];
-    detail::boundary_terms(pl.kind, n, v1, v2, gar, lo, hi);
-    for (int r = 0; r < 2 * NB; ++r) {
-      const detail::TermRow& t = r < NB ? lo[r] : hi[r - NB];
-      if ((int)t.c.size() > MAXT) throw std::runtime_error("boundary row has too many terms");
-      pl.bnt[r] = (int)t.c.size();
-      for (size_t q = 0; q < t.c.size(); ++q)
-        if (t.a[q] < -1 || t.a[q] >= n || t.b[q] < -1 || t.b[q] >= n)
-          throw std::runtime_error("boundary term outside the line");
-      for (size_t q = 0; q < t.c.size(); ++q) {
-        pl.bcoef[r * MAXT + q] = t.c[q];
-        pl.bidx[(r * MAXT + q) * 2 + 0] = (short)t.a[q];
-        pl.bidx[(r * MAXT + q) * 2 + 1] = (short)t.b[q];
-      }
-    }
-  }
-
-  // chunk partition: P = ceil(n/CHUNK), balanced lengths (all >= 4)
-  const int P = (n + CHUNK - 1) / CHUNK;
+  const int P = detail::chunk_count(n, dir);
   pl.P = P;
-  pl.cstart.resize(P + 1);
-  {
-    const int base = n / P, extra = n % P;
-    int s = 0;
-    for (int p = 0; p < P; ++p) { pl.cstart[p] = s; s += base + (p < extra ? 1 : 0); }
-    pl.cstart[P] = n;
+  pl.mb = n / P;
+  pl.mx = n % P;
+  auto start = [&](int p) { return p * pl.mb + std::min(p, pl.mx); };
+
+  // boundary rows of a bounded line (compact_basetype.f90:124-133)
+  if (!periodic) {
+    pl.wb.assign(2 * NB * WBROW, 0.0);
+    for (int j = 0; j < 2 * NB; ++j) {
+      const bool lo = j < NB;
+      const double* row = lo ? sc.arb1[v1 + 1][j] : sc.arb2[v2 + 1][j - NB];
+      double* o = &pl.wb[j * WBROW];
+      ld sum = 0.0L;
+      for (int l = -hr; l <= hr; ++l) {
+        if (std::abs(l) > 4) continue;
+        const int col = (lo ? j : n - 2 * NB + j) + l;
+        if (col < 0 || col >= n) continue;  // ghost columns read 0
+        sum += (ld)row[l + hr];
+        if (l != 0) o[l + 4] = row[l + hr];
+      }
+      // rows of the NONE and SYMM variants have zero sum
+      if ((lo ? v1 : v2) == -1) o[WBROW - 1] = (double)sum;
+    }
   }
-  pl.lu.assign(size_t(n) * 5, 0.0);
-  pl.rc.assign(size_t(n) * 4, 0.0);
-  pl.gsel.assign(size_t(P) * 4 * 4 * P, 0.0);
   if (!sc.implicit) return pl;
 
-  if (periodic && sc.ncl == 5 && sc.ali[0] == sc.ali[4] && sc.ali[1] == sc.ali[3]) {
-    ld p1, p2, cc;
-    if (detail::spectral_factor(sc.ali[0], sc.ali[1], sc.ali[2], p1, p2, cc)) {
-      pl.circ = 1;
-      pl.p1 = (double)p1;
-      pl.p2 = (double)p2;
-      pl.invc = (double)(1.0L / cc);
-      pl.bd[0] = sc.ali[0];
-      pl.bd[1] = sc.ali[1];
-      pl.bd[2] = sc.ali[2];
-      detail::circ_carry_rows(P, pl.cstart, p1, p2, pl.kf, pl.kb);
+  ld p1, p2, cc;
+  if (sc.ncl != 5 || sc.ali[0] != sc.ali[4] || sc.ali[1] != sc.ali[3] ||
+      !detail::spectral_factor(sc.ali[0], sc.ali[1], sc.ali[2], p1, p2, cc))
+    throw std::runtime_error("the scheme's left-hand side has no spectral factor");
+  pl.p1 = (double)p1;
+  pl.p2 = (double)p2;
+  pl.scale = (double)((ld)pl.scale / cc);
+
+  // per-row factors (constants for a periodic line)
+  std::vector<ld> l1(n, p1), l2(n, p2), u1(n, p1), u2(n, p2), g(n, 1.0L);
+  if (!periodic) {
+    std::vector<std::array<ld, 5>> A(n);
+    for (int i = 0; i < n; ++i)
+      for (int c = 0; c < 5; ++c) A[i][c] = (ld)sc.ali[c];
+    for (int j = 0; j < NB; ++j)
+      for (int c = 0; c < 5; ++c) {
+        A[j][c] = (ld)sc.alb1[v1 + 1][j][c];
+        A[n - NB + j][c] = (ld)sc.alb2[v2 + 1][j][c];
+      }
+    std::vector<ld> U0(n), U1(n), U2(n);
+    for (int i = 0; i < n; ++i) {
+      ld a0 = i >= 2 ? A[i][0] : 0.0L, a1 = i >= 1 ? A[i][1] : 0.0L, d = A[i][2];
+      ld b1 = i + 1 < n ? A[i][3] : 0.0L, b2 = i + 2 < n ? A[i][4] : 0.0L;
+      l1[i] = l2[i] = 0.0L;
+      if (i >= 2) {
+        l2[i] = a0 / U0[i - 2];
+        a1 -= l2[i] * U1[i - 2];
+        d -= l2[i] * U2[i - 2];
+      }
+      if (i >= 1) {
+        l1[i] = a1 / U0[i - 1];
+        d -= l1[i] * U1[i - 1];
+        b1 -= l1[i] * U2[i - 1];
+      }
+      if (d == 0.0L) throw std::runtime_error("zero pivot in the line factorization");
+      U0[i] = d; U1[i] = b1; U2[i] = b2;
+      u1[i] = b1 / d;
+      u2[i] = b2 / d;
+      g[i] = cc / d;
+    }
+    // rows that have converged take the limit exactly: a chunk of such rows
+    // then gives the same bits through the tables and through the constants
+    auto near = [](ld x, ld y) { return std::fabs(x - y) <= 1.2e-16L * std::fabs(y); };
+    std::vector<char> conv(n, 0);
+    for (int i = 0; i < n; ++i)
+      if (near(l1[i], p1) && near(l2[i], p2) && near(u1[i], p1) && near(u2[i], p2) && near(g[i], 1.0L)) {
+        conv[i] = 1;
+        l1[i] = u1[i] = p1;
+        l2[i] = u2[i] = p2;
+        g[i] = 1.0L;
+      }
+    pl.tf.assign((size_t)CHUNK * P * 2, 0.0);
+    pl.tb.assign((size_t)CHUNK * P * 2, 0.0);
+    pl.tg.assign((size_t)CHUNK * P, 0.0);
+    for (int p = 0; p < P; ++p) {
+      bool all = true;
+      for (int k = 0; start(p) + k < start(p + 1); ++k) {
+        const int i = start(p) + k;
+        const size_t e = (size_t)k * P + p;
+        all = all && conv[i];
+        pl.tf[2 * e] = (double)l1[i]; pl.tf[2 * e + 1] = (double)l2[i];
+        pl.tb[2 * e] = (double)u1[i]; pl.tb[2 * e + 1] = (double)u2[i];
+        pl.tg[e] = (double)g[i];
+      }
+      if (!all && p < P - 1) pl.tlo = p + 1;
     }
   }
 
-  auto Aent = [&](int i, int col) -> double {  // A[i][col], col may wrap
-    const int off = col - i;
-    if (periodic) {
-      int d = col - i;
-      // bring the offset into [-2,2] modulo n
-      if (d > 2) d -= n;
-      if (d < -2) d += n;
-      if (d < -2 || d > 2) return 0.0;
-      return gal[i][d + 2];
-    }
-    if (off < -2 || off > 2 || col < 0 || col >= n) return 0.0;
-    return gal[i][off + 2];
-  };
-
-  std::vector<ld> S(size_t(4 * P) * 4 * P, 0.0L);
-  for (int p = 0; p < P; ++p) {
-    const int s = pl.cstart[p], e = pl.cstart[p + 1], m = e - s;
-    // dense block, no pivoting LU (SPD-like blocks of the compact LHS)
-    std::vector<ld> blk(size_t(m) * m, 0.0L);
-    for (int i = 0; i < m; ++i)
-      for (int j = std::max(0, i - 2); j <= std::min(m - 1, i + 2); ++j)
-        blk[size_t(i) * m + j] = (ld)gal[s + i][j - i + 2];
-    std::vector<ld> L(size_t(m) * 3, 0.0L);  // multipliers for i-2, i-1
-    for (int k = 0; k < m; ++k) {
-      const ld piv = blk[size_t(k) * m + k];
-      if (piv == 0.0L) throw std::runtime_error("zero pivot in chunk LU");
-      for (int i = k + 1; i <= std::min(m - 1, k + 2); ++i) {
-        const ld f = blk[size_t(i) * m + k] / piv;
-        L[size_t(i) * 3 + (i - k == 2 ? 0 : 1)] = f;
-        for (int j = k; j <= std::min(m - 1, k + 2); ++j) blk[size_t(i) * m + j] -= f * blk[size_t(k) * m + j];
+  // carry matrices
+  std::vector<M2> Hf(P), Hb(P);
+  for (int p = 0; p < P; ++p)
+    for (int j = 0; j < 2; ++j) {
+      ld xm2 = j == 0, xm1 = j == 1;  // forward state (x[k-2], x[k-1])
+      for (int i = start(p); i < start(p + 1); ++i) {
+        const ld x = -l1[i] * xm1 - l2[i] * xm2;
+        xm2 = xm1;
+        xm1 = x;
       }
-    }
-    for (int i = 0; i < m; ++i) {
-      double* c = &pl.lu[size_t(s + i) * 5];
-      c[0] = (double)L[size_t(i) * 3 + 0];
-      c[1] = (double)L[size_t(i) * 3 + 1];
-      c[2] = (double)(1.0L / blk[size_t(i) * m + i]);
-      c[3] = (i + 1 < m) ? (double)blk[size_t(i) * m + i + 1] : 0.0;
-      c[4] = (i + 2 < m) ? (double)blk[size_t(i) * m + i + 2] : 0.0;
-    }
-    // solve with the long-double factors for the spike columns
-    auto solve = [&](std::vector<ld>& r) {
-      for (int i = 0; i < m; ++i) {
-        if (i >= 1) r[i] -= L[size_t(i) * 3 + 1] * r[i - 1];
-        if (i >= 2) r[i] -= L[size_t(i) * 3 + 0] * r[i - 2];
+      Hf[p][j] = xm2;
+      Hf[p][2 + j] = xm1;
+      ld b1 = j == 0, b2 = j == 1;  // backward state (y[k+1], y[k+2])
+      for (int i = start(p + 1) - 1; i >= start(p); --i) {
+        const ld y = -u1[i] * b1 - u2[i] * b2;
+        b2 = b1;
+        b1 = y;
       }
-      for (int i = m - 1; i >= 0; --i) {
-        ld v = r[i];
-        if (i + 1 < m) v -= blk[size_t(i) * m + i + 1] * r[i + 1];
-        if (i + 2 < m) v -= blk[size_t(i) * m + i + 2] * r[i + 2];
-        r[i] = v / blk[size_t(i) * m + i];
-      }
-    };
-    std::vector<ld> w0(m, 0.0L), w1(m, 0.0L), wm2(m, 0.0L), wm1(m, 0.0L);
-    w0[0] = 1; w1[1] = 1; wm2[m - 2] = 1; wm1[m - 1] = 1;
-    solve(w0); solve(w1); solve(wm2); solve(wm1);
-    const bool has_lo = periodic || p > 0, has_hi = periodic || p < P - 1;
-    // couplings to the previous chunk's last two unknowns (y[s-2], y[s-1])
-    const ld a_s_m2 = has_lo ? (ld)Aent(s, s - 2) : 0.0L;
-    const ld a_s_m1 = has_lo ? (ld)Aent(s, s - 1) : 0.0L;
-    const ld a_s1_m1 = has_lo ? (ld)Aent(s + 1, s - 1) : 0.0L;
-    // couplings to the next chunk's first two unknowns (y[e], y[e+1])
-    const ld a_e2_e = has_hi ? (ld)Aent(e - 2, e) : 0.0L;
-    const ld a_e1_e = has_hi ? (ld)Aent(e - 1, e) : 0.0L;
-    const ld a_e1_e1 = has_hi ? (ld)Aent(e - 1, e + 1) : 0.0L;
-    std::vector<ld> r0(m), r1(m), r2(m), r3(m);
-    for (int i = 0; i < m; ++i) {
-      r0[i] = a_s_m2 * w0[i];
-      r1[i] = a_s_m1 * w0[i] + a_s1_m1 * w1[i];
-      r2[i] = a_e2_e * wm2[i] + a_e1_e * wm1[i];
-      r3[i] = a_e1_e1 * wm1[i];
-      double* rr = &pl.rc[size_t(s + i) * 4];
-      rr[0] = (double)r0[i]; rr[1] = (double)r1[i]; rr[2] = (double)r2[i]; rr[3] = (double)r3[i];
+      Hb[p][j] = b1;
+      Hb[p][2 + j] = b2;
     }
-    // reduced-system rows for this chunk's four edge unknowns
-    const int pm = (p - 1 + P) % P, pp = (p + 1) % P;
-    const int edge[4] = {0, 1, m - 2, m - 1};
-    for (int q = 0; q < 4; ++q) {
-      const int row = 4 * p + q, li = edge[q];
-      S[size_t(row) * 4 * P + row] += 1.0L;
-      if (has_lo) {
-        S[size_t(row) * 4 * P + 4 * pm + 2] += r0[li];
-        S[size_t(row) * 4 * P + 4 * pm + 3] += r1[li];
+  const auto Kf = detail::carry_matrices(Hf, -1, periodic), Kb = detail::carry_matrices(Hb, 1, periodic);
+  pl.W = (int)std::max(Kf.size(), Kb.size());
+  pl.kp = (periodic && pl.mx == 0) ? 1 : P;
+  pl.kf.assign((size_t)pl.W * pl.kp * 4, 0.0);
+  pl.kb.assign((size_t)pl.W * pl.kp * 4, 0.0);
+  for (int j = 0; j < pl.W; ++j)
+    for (int p = 0; p < pl.kp; ++p)
+      for (int i = 0; i < 4; ++i) {
+        const size_t e = ((size_t)j * pl.kp + p) * 4 + i;
+        if (j < (int)Kf.size()) pl.kf[e] = (double)Kf[j][p][i];
+        if (j < (int)Kb.size()) pl.kb[e] = (double)Kb[j][p][i];
       }
-      if (has_hi) {
-        S[size_t(row) * 4 * P + 4 * pp + 0] += r2[li];
-        S[size_t(row) * 4 * P + 4 * pp + 1] += r3[li];
-      }
-    }
-  }
-  detail::invert(S, 4 * P);
-  for (int p = 0; p < P; ++p) {
-    const bool has_lo = periodic || p > 0, has_hi = periodic || p < P - 1;
-    const int pm = (p - 1 + P) % P, pp = (p + 1) % P;
-    const int rows[4] = {4 * pm + 2, 4 * pm + 3, 4 * pp + 0, 4 * pp + 1};
-    const bool use[4] = {has_lo, has_lo, has_hi, has_hi};
-    for (int q = 0; q < 4; ++q)
-      for (int c = 0; c < 4 * P; ++c)
-        pl.gsel[(size_t(p) * 4 + q) * 4 * P + c] = use[q] ? (double)S[size_t(rows[q]) * 4 * P + c] : 0.0;
-  }
   return pl;
 }
 

@@ -9,7 +9,8 @@ libpyranda_amd.so on torch's current stream and returns a freshly allocated
 output, like f2py's intent(out).
 
 Precision: fields of dtype float64 go through the FP64 kernels; float32 fields
-through the FP32-sweep + FP64-residual refinement kernels.
+are solved in FP64 registers along periodic lines and, by default, in FP32 with
+an FP64-residual refinement along bounded ones.
 """
 import ctypes
 
@@ -125,11 +126,10 @@ class ParcopContext:
                                                 -1 if name is None else _lib.R32_SOLVE[name]))
 
     def set_tuning(self, op, direction, dtype, x_lds_kb=-1, yz_pipe=-1, yz_lines=-1):
-        """Per-operator knobs (pyr_set_tuning): LDS budget of x-line
-        workgroups (KB), the pipelined kernels (y/z: 1; x: 1 with a second
-        LDS tile, 2 with the next tile prefetched into registers, explicit
-        filter only; y/z 3: the plain kernel with runtime row counts), lines per
-        plain y/z workgroup; -1 = default."""
+        """Per-operator knobs (pyr_set_tuning): lines per y/z workgroup
+        (yz_lines) and, with yz_pipe 3 on y/z, the kernel with runtime row
+        counts; x_lds_kb and the other values of yz_pipe are checked and change
+        nothing; -1 = default."""
         prec = _lib.F64 if dtype == torch.float64 else _lib.R32
         _lib.check(self._L.pyr_set_tuning(self._h, op, direction, prec, int(x_lds_kb), int(yz_pipe),
                                           int(yz_lines)))
@@ -137,16 +137,15 @@ class ParcopContext:
     def autotune(self, dtype, ops=None, reps=5, x_lds_kb=(8, 12, 16, 24, 40, 64, 80), seed=7, rounded=False,
                  solve_modes=False):
         """Time each operator and direction at this precision with every
-        candidate (x: LDS budget, hence lines per workgroup, and the pipelined
-        kernel or not; y/z: pipelined kernel or not) on random fields and keep
-        the fastest (x: the one-pass kernel or a pipelined one: 1, or for the
-        explicit filter also 2). The timed
+        candidate (y/z: 64, 32 or 16 lines per workgroup; x lines have one
+        shape, reported under the first of x_lds_kb) on random fields and keep
+        the fastest. The timed
         launches cycle through enough fields to exceed the device's 256 MB
         last-level cache, so every launch reads its input from HBM as the
         operators of a time step do. rounded: FP64
         z sweeps are timed storing the FP32 copy of their result as well (the
         last sweep of the filter of an FP32 run's FP64 state). solve_modes
-        (FP32 fields): the candidates also range over the solve arithmetic,
+        (FP32 fields): the candidates also range over the solve setting,
         refined FP32 or FP64 (("r32_solve", 0 or 1) in the choice); the two
         agree to the FP32 rounding of the result, so unlike the launch knobs
         this choice can change results in the last bits, and the FP64 solve
@@ -168,16 +167,9 @@ class ParcopContext:
                     continue
                 kw = {"out32": out32} if out32 is not None and d == 2 else {}
                 if d == 0:
-                    # the LDS budget (lines per workgroup) with the pipelined
-                    # persistent x kernel (yz_pipe=1, where the line shape
-                    # allows it) or the one-pass kernel
-                    # (2: the register-pipelined kernel of the explicit filter)
-                    pps = (0, 1, 2) if op == _lib.OP_GFILTER else (0, 1)
-                    cands = [(("x_lds_kb", kb), ("yz_pipe", pp)) for pp in pps for kb in x_lds_kb]
+                    cands = [(("x_lds_kb", next(iter(x_lds_kb))), ("yz_pipe", 0))]
                 else:
-                    cands = [(("yz_pipe", 1),), (("yz_pipe", 0), ("yz_lines", 64)),
-                             (("yz_pipe", 0), ("yz_lines", 32)), (("yz_pipe", 0), ("yz_lines", 16)),
-                             (("yz_pipe", 3), ("yz_lines", 64))]
+                    cands = [(("yz_pipe", 0), ("yz_lines", n)) for n in (64, 32, 16)]
                 if solve_modes and dtype == torch.float32:
                     cands = [(("r32_solve", m),) + c for m in (0, 1) for c in cands]
                 times = {}
