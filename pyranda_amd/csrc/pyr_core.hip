@@ -69,7 +69,7 @@ static int fail(const std::string& m) { return pyr::report_error(m); }
 enum Solve { SOLVE_NONE = 0, SOLVE_BND = 1, SOLVE_CIRC = 2 };
 
 // What the epilogue of a y/z row needs besides the solution, in registers
-// before the solve so that no store waits on a load: the input value (filters
+// before the backward pass so that no store waits on a load: the input value (filters
 // add v back) or the current output (accumulating epilogues).
 enum Pre { PRE_NONE = 0, PRE_V = 1, PRE_OLD = 2 };
 
@@ -104,43 +104,6 @@ __device__ __forceinline__ void buf_store(float v, __amdgpu_buffer_rsrc_t r, int
 // A pair of FP64 values moved as one 16-byte LDS or global access.
 using D2 = double __attribute__((ext_vector_type(2)));
 
-// Carry matrix of term j for chunk p (periodic lines of equal chunks share one
-// per term: kp = 1, which FULL lines know at compile time).
-template <bool SHARED>
-__device__ __forceinline__ const double* carry_row(const double* K, const LineArgs& a, int j, int p) {
-  return SHARED ? K + 4 * j : K + 4 * (j * a.kp + (a.kp > 1 ? p : 0));
-}
-
-// Entry state of chunk p: its carry matrices times the exit states of the
-// chunks that follow in direction `step` (-1: p-1, p-2, ...; +1: p+1, ...).
-// exit_of(q) reads the exit pair of chunk q.
-template <bool CYCLIC, bool SHARED, int STEP, typename ExitOf>
-__device__ __forceinline__ void carry_in(const LineArgs& a, const double* K, int p, ExitOf exit_of, double& e0,
-                                         double& e1) {
-  e0 = e1 = 0.0;
-  int q = p;
-  for (int j = 0; j < a.W; ++j) {
-    q += STEP;
-    if (CYCLIC) {
-      if (q < 0) q = a.P - 1;
-      if (q >= a.P) q = 0;
-    }
-    if (CYCLIC || (q >= 0 && q < a.P)) {
-      const D2 u = exit_of(q);
-      if (SHARED) {
-        const double* k = carry_row<SHARED>(K, a, j, p);
-        carry_add(k, u.x, u.y, e0, e1);
-      } else {
-        // the matrix rows as two 16-byte loads
-        const D2* k = reinterpret_cast<const D2*>(carry_row<SHARED>(K, a, j, p));
-        const D2 r0 = k[0], r1 = k[1];
-        const double kk[4] = {r0.x, r0.y, r1.x, r1.y};
-        carry_add(kk, u.x, u.y, e0, e1);
-      }
-    }
-  }
-}
-
 // The chunks of one wave that need the line's own factors (the wave then
 // takes them for all of its chunks: converged rows give the same bits).
 __device__ __forceinline__ bool wave_needs_tables(const LineArgs& a, int p) {
@@ -150,9 +113,46 @@ __device__ __forceinline__ bool wave_needs_tables(const LineArgs& a, int p) {
 // The passes of one chunk around its two exchanges. `rows` are ConstRows or
 // TableRows; the bounded solve picks one per wave.
 template <int SOLVE, typename F>
-__device__ __forceinline__ void with_rows(const LineArgs& a, bool tab, int p, F f) {
-  if (SOLVE == SOLVE_BND && tab) f(TableRows{a.tf, a.tb, a.tg, a.P, p});
+__device__ __forceinline__ void with_rows(const LineArgs& a, bool tab, const Tables& t, int slot, F f) {
+  if (SOLVE == SOLVE_BND && tab) f(TableRows{t, a.T, slot});
   else f(ConstRows{a.p1, a.p2});
+}
+
+// Carry of chunk p. Periodic lines: constant matrices from the kernel
+// arguments (FULL lines have chunks of one length); bounded lines: the table's.
+template <int SOLVE, bool FULL, int STEP, typename ExitOf>
+__device__ __forceinline__ void carry_of(const LineArgs& a, const Tables& t, int p, ExitOf exit_of, double& e0,
+                                         double& e1) {
+  auto read = [&](int q, double& u0, double& u1) {
+    const D2 u = exit_of(q);
+    u0 = u.x;
+    u1 = u.y;
+  };
+  if constexpr (SOLVE == SOLVE_BND) {
+    carry_in<false, STEP>(a, p, [&](int q) { return t.th + 8 * slot_of(a, q) + (STEP > 0 ? 4 : 0); }, read, e0, e1);
+  } else {
+    const double(*h)[4] = STEP < 0 ? a.hf : a.hb;
+    if constexpr (FULL) {
+      carry_in<true, STEP>(a, p, [&](int) { return h[1]; }, read, e0, e1);
+    } else {
+      double m[4];
+      carry_in<true, STEP>(a, p, [&](int q) {
+        const bool longer = q < a.mx;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[i] = longer ? h[0][i] : h[1][i];
+        return (const double*)m;
+      }, read, e0, e1);
+    }
+  }
+}
+
+// The tables of a bounded line into LDS: they are read row by row in the
+// solves' passes, each read a latency on the critical path of a workgroup
+// (from memory, the 2-D and ragged bounded sweeps took 28-36 us for fields
+// of a few MB).
+__device__ __forceinline__ void stage_tables(const LineArgs& a, double* tab) {
+  for (int e = threadIdx.x; e < a.ntab / 2; e += blockDim.x)
+    reinterpret_cast<D2*>(tab)[e] = reinterpret_cast<const D2*>(a.tab)[e];
 }
 
 // y/z lines. Thread (lane, p): line blk * lines + lane, chunk p; a.lines
@@ -183,6 +183,15 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
   const int m = FULL ? CHUNK : a.mb + (p < a.mx ? 1 : 0);
   const bool last = p == a.P - 1;
   const bool wrap = SOLVE == SOLVE_CIRC || (SOLVE == SOLVE_NONE && a.periodic);
+  const bool bounded = SOLVE == SOLVE_BND || (SOLVE == SOLVE_NONE && !a.periodic);
+  // LDS: two exchange buffers, a flag per line, the tables of a bounded line
+  const int nex = SOLVE == SOLVE_NONE ? 0 : (GRP ? (int)blockDim.x : a.P * LY);
+  D2* X0 = reinterpret_cast<D2*>(smem);
+  D2* X1 = X0 + nex;
+  double* tab = reinterpret_cast<double*>(X1 + nex);
+  int* bad = reinterpret_cast<int*>(tab + (bounded ? a.ntab : 0));
+  const Tables tabs(tab, a.T);
+  if (bounded) stage_tables(a, tab);
   const __amdgpu_buffer_rsrc_t rin = buf_rsrc(in, a.nbytes), rout = buf_rsrc(out, a.nbytes);
   // the FP32 copy of an FP64 result (LineArgs::out32), half the bytes per element
   [[maybe_unused]] const __amdgpu_buffer_rsrc_t rout32 = buf_rsrc(a.out32, a.nbytes / 2);
@@ -193,11 +202,6 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
   const int vhi = !act ? OOB : (!last ? vmid + CHUNK * rb : (wrap ? lane_off : OOB));  // FULL only
   auto row_off = [&](int k) { return (int)((unsigned)vmid + (unsigned)k * (unsigned)rb); };
   TS pre[PRE == PRE_OLD ? CHUNK : 1];
-  if constexpr (PRE == PRE_OLD) {
-#pragma unroll
-    for (int k = 0; k < CHUNK; ++k)
-      pre[k] = FULL ? buf_load(TS(), rout, vmid, k * rb) : buf_load(TS(), rout, k < m ? row_off(k) : OOB, 0);
-  }
   TS win[CHUNK + 2 * R];
 #pragma unroll
   for (int w = 0; w < CHUNK + 2 * R; ++w) {
@@ -217,9 +221,13 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
     }
   }
   double x[CHUNK];
+  B4 lo = {}, hi = {};
+  if (bounded) {
+    __syncthreads();  // tables visible
+    if (act) boundary_rows<KIND, FULL>(a, tabs.wb, p, win, lo, hi);
+  }
   rhs_interior<KIND>(a, win, x);
-  if (SOLVE == SOLVE_BND || (SOLVE == SOLVE_NONE && !a.periodic))
-    if (act) rhs_boundary<KIND, FULL>(a, a.wb, p, win, x);
+  if (bounded) put_boundary_rows<FULL>(a, p, lo, hi, x);
 
   // row k of the result: metric scale, filters add v back, fused epilogue, store
   auto emit = [&](int k, double y) {
@@ -245,24 +253,26 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
     for (int k = 0; k < CHUNK; ++k)
       if (FULL || k < m) emit(k, x[k]);
   } else {
-    constexpr bool CYC = SOLVE == SOLVE_CIRC;
-    constexpr bool SHARED = CYC && FULL;
-    const int nex = GRP ? (int)blockDim.x : a.P * LY;
-    D2* X0 = reinterpret_cast<D2*>(smem);
-    D2* X1 = X0 + nex;
-    int* bad = reinterpret_cast<int*>(X1 + nex);
-    const bool tab = SOLVE == SOLVE_BND && wave_needs_tables(a, p);
+    const bool own = SOLVE == SOLVE_BND && wave_needs_tables(a, p);
+    const int slot = SOLVE == SOLVE_BND ? slot_of(a, p) : 0;
     if (p == 0) bad[lane] = 0;
     double e0 = 0.0, e1 = 0.0;
     if (act) {
-      with_rows<SOLVE>(a, tab, p, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
+      with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
       X0[p * LY + lane] = D2{e0, e1};
     }
     __syncthreads();
+    // the current output, on its way while the recurrences run (the window's
+    // registers are free by now)
+    if constexpr (PRE == PRE_OLD) {
+#pragma unroll
+      for (int k = 0; k < CHUNK; ++k)
+        pre[k] = FULL ? buf_load(TS(), rout, vmid, k * rb) : buf_load(TS(), rout, k < m ? row_off(k) : OOB, 0);
+    }
     double b0 = 0.0, b1 = 0.0;
     if (act) {
-      carry_in<CYC, SHARED, -1>(a, a.kf, p, [&](int q) { return X0[q * LY + lane]; }, e0, e1);
-      with_rows<SOLVE>(a, tab, p, [&](auto rows) {
+      carry_of<SOLVE, FULL, -1>(a, tabs, p, [&](int q) { return X0[q * LY + lane]; }, e0, e1);
+      with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) {
         fwd_pass<FULL, true>(rows, x, m, e0, e1);
         bwd_exit<FULL>(rows, x, m, b0, b1);
       });
@@ -274,10 +284,10 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
     }
     __syncthreads();
     if (!act) return;
-    carry_in<CYC, SHARED, 1>(a, a.kb, p, [&](int q) { return X1[q * LY + lane]; }, b0, b1);
+    carry_of<SOLVE, FULL, 1>(a, tabs, p, [&](int q) { return X1[q * LY + lane]; }, b0, b1);
     if (bad[lane]) b0 = b1 = __builtin_nan("");
     if (!valid) return;
-    with_rows<SOLVE>(a, tab, p, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
+    with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
   }
 }
 
@@ -395,18 +405,34 @@ __device__ __forceinline__ unsigned long long line_lanes(int l, int P) {
 // fbar 84 -> 53 us, d1 79 -> 50 us, FP32 d1 47 -> 33 us; a copy takes 50 and
 // 25 us. A persistent variant that fetches its next lines into registers
 // while it solves measured slower (512^3 d1 408 us against 373).
+// Waves per workgroup: the waves of a bounded sweep share the line's tables.
+template <int SOLVE> struct XWaves { static constexpr int v = SOLVE == SOLVE_BND ? 4 : 1; };
+
 template <typename TS, int KIND, int SOLVE, bool FULL, bool GRP = false>
 __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, const TS* __restrict__ in,
                                             TS* __restrict__ out) {
   constexpr int R = Halo<KIND>::R;
   using T = XTile<TS, CHUNK, FULL>;
   constexpr int CP = T::CP;
-  __shared__ __align__(16) TS tile[T::SIZE];
-  __shared__ __align__(16) D2 ex[64];
+  constexpr int NW = XWaves<SOLVE>::v;
+  __shared__ __align__(16) TS tiles[NW][T::SIZE];
+  __shared__ __align__(16) D2 exits[NW][64];
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* tab = reinterpret_cast<double*>(smem);
+  const Tables tabs(tab, a.T);
+  const bool bounded = SOLVE == SOLVE_BND || (SOLVE == SOLVE_NONE && !a.periodic);
+  if (bounded) {
+    stage_tables(a, tab);
+    __syncthreads();
+  }
   const int N = a.N, P = a.P;
-  const int lane = threadIdx.x;
-  const long long L0 = blk * a.lines;
+  const int lane = threadIdx.x & 63;
+  const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  TS* tile = tiles[wave];
+  [[maybe_unused]] D2* ex = exits[wave];
+  const long long L0 = (blk * NW + wave) * a.lines;
   const long long rem = (long long)a.nlines - L0;
+  if (NW > 1 && rem <= 0) return;
   const int nval = (int)(rem < a.lines ? rem : a.lines);
   const long long E0 = L0 * N;
   const int sh = (!FULL && a.vec) ? (int)(E0 & (T::VW - 1)) : 0;
@@ -452,8 +478,10 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
     }
   }
   double x[CHUNK];
+  B4 lo = {}, hi = {};
+  if (bounded) boundary_rows<KIND, FULL>(a, tabs.wb, p, win, lo, hi);
   rhs_interior<KIND>(a, win, x);
-  if (SOLVE == SOLVE_BND || (SOLVE == SOLVE_NONE && !a.periodic)) rhs_boundary<KIND, FULL>(a, a.wb, p, win, x);
+  if (bounded) put_boundary_rows<FULL>(a, p, lo, hi, x);
   // filters add v back here, read from the tile before the result takes its place
   auto emit = [&](int k, double y) {
     if (act) {
@@ -468,16 +496,15 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
     for (int k = 0; k < CHUNK; ++k)
       if (FULL || k < m) emit(k, x[k]);
   } else {
-    constexpr bool CYC = SOLVE == SOLVE_CIRC;
-    constexpr bool SHARED = CYC && FULL;
     // lanes past the last whole line read some exit and drop the result
     auto exit_of = [&](int q) { return ex[l * P + q < 64 ? l * P + q : 0]; };
+    const int slot = SOLVE == SOLVE_BND ? slot_of(a, p) : 0;
     double e0 = 0.0, e1 = 0.0, b0 = 0.0, b1 = 0.0;
-    with_rows<SOLVE>(a, true, p, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
+    with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
     ex[lane] = D2{e0, e1};
     wave_fence();
-    carry_in<CYC, SHARED, -1>(a, a.kf, p, exit_of, e0, e1);
-    with_rows<SOLVE>(a, true, p, [&](auto rows) {
+    carry_of<SOLVE, FULL, -1>(a, tabs, p, exit_of, e0, e1);
+    with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) {
       fwd_pass<FULL, true>(rows, x, m, e0, e1);
       bwd_exit<FULL>(rows, x, m, b0, b1);
     });
@@ -486,9 +513,9 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
     wave_fence();
     ex[lane] = D2{b0, b1};
     wave_fence();
-    carry_in<CYC, SHARED, 1>(a, a.kb, p, exit_of, b0, b1);
+    carry_of<SOLVE, FULL, 1>(a, tabs, p, exit_of, b0, b1);
     if (bad & line_lanes(l, P)) b0 = b1 = __builtin_nan("");
-    with_rows<SOLVE>(a, true, p, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
+    with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
   }
   wave_fence();
   float* o32 = nullptr;
@@ -497,7 +524,7 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
 }
 
 template <typename TS, int KIND, int SOLVE, bool FULL>
-__global__ void __launch_bounds__(64) k_line_x(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
+__global__ void __launch_bounds__(64 * XWaves<SOLVE>::v) k_line_x(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
   line_x_body<TS, KIND, SOLVE, FULL>(a, blockIdx.x, in, out);
 }
 
@@ -527,7 +554,7 @@ __device__ __forceinline__ int grp_member(const Entry* __restrict__ g, int M, lo
 }
 
 template <typename TS, int KIND, int SOLVE>
-__global__ void __launch_bounds__(64) k_line_x_grp(const GrpEntry* __restrict__ g, int M, const TS* __restrict__ in,
+__global__ void __launch_bounds__(64 * XWaves<SOLVE>::v) k_line_x_grp(const GrpEntry* __restrict__ g, int M, const TS* __restrict__ in,
                                                    TS* __restrict__ out) {
   const int j = grp_member(g, M, blockIdx.x);
   // a private copy: its fields load once (wave-uniform) and no store of the
@@ -812,7 +839,7 @@ __global__ void k_rk_update(long long n, const TF* __restrict__ F, double* __res
 // Device addresses of a plan's tables, all inside the context's one table
 // allocation (pyr_ctx::tables).
 struct DevPlan {
-  const double *wb = nullptr, *kf = nullptr, *kb = nullptr, *tf = nullptr, *tb = nullptr, *tg = nullptr;
+  const double *tab = nullptr, *mw = nullptr;  // row tables with the boundary rows; remaining turns
 };
 
 struct DevRefPlan {
@@ -869,6 +896,13 @@ struct pyr_ctx {
   size_t npts() const { return (size_t)n[0] * n[1] * n[2]; }
 };
 
+// what a bounded sweep stages: the row tables, then the boundary rows
+static std::vector<double> with_boundary_rows(const OpPlan& pl) {
+  std::vector<double> t = pl.tab;
+  t.insert(t.end(), pl.wb.begin(), pl.wb.end());
+  return t;
+}
+
 // The tables of all plans of a context back to back, 256-byte aligned: added
 // one by one, then uploaded in one piece.
 struct TableImage {
@@ -885,13 +919,8 @@ struct TableImage {
 // adds the tables of a plan to the image; the addresses are offsets until
 // rebase() is called with the image's device address
 static void add_plan(TableImage& im, const OpPlan& pl, DevPlan& d) {
-  auto put = [&](const std::vector<double>& t) { return reinterpret_cast<const double*>(im.add(t)); };
-  d.wb = put(pl.wb);
-  d.kf = put(pl.kf);
-  d.kb = put(pl.kb);
-  d.tf = put(pl.tf);
-  d.tb = put(pl.tb);
-  d.tg = put(pl.tg);
+  d.tab = reinterpret_cast<const double*>(im.add(with_boundary_rows(pl)));
+  d.mw = reinterpret_cast<const double*>(im.add(pl.mw));
 }
 static void add_plan(TableImage& im, const RefPlan& pl, DevRefPlan& d) {
   if (pl.N == 0) return;
@@ -906,7 +935,7 @@ static void rebase(const T*& p, const unsigned char* base) {
   p = reinterpret_cast<const T*>(base + reinterpret_cast<size_t>(p));
 }
 static void rebase(DevPlan& d, const unsigned char* base) {
-  for (const double** p : {&d.wb, &d.kf, &d.kb, &d.tf, &d.tb, &d.tg}) rebase(*p, base);
+  for (const double** p : {&d.tab, &d.mw}) rebase(*p, base);
 }
 static void rebase(DevRefPlan& d, const unsigned char* base) {
   rebase(d.cls, base);
@@ -945,15 +974,6 @@ static void host_ref_tables(const RefPlan& pl, DevRefPlan& d) {
   d.bcoef = pl.bcoef.data();
   d.bidx = pl.bidx.data();
 }
-static void host_tables(const OpPlan& pl, DevPlan& d) {
-  d.wb = pl.wb.data();
-  d.kf = pl.kf.data();
-  d.kb = pl.kb.data();
-  d.tf = pl.tf.data();
-  d.tb = pl.tb.data();
-  d.tg = pl.tg.data();
-}
-
 static LineArgs make_args(const pyr_ctx* c, const OpPlan& pl, const DevPlan& d, int dir, int epi,
                           double ec, int prec) {
   LineArgs a;
@@ -980,17 +1000,16 @@ static LineArgs make_args(const pyr_ctx* c, const OpPlan& pl, const DevPlan& d, 
   a.mb = pl.mb;
   a.mx = pl.mx;
   for (int i = 0; i < 4; ++i) a.w[i] = pl.w[i];
-  a.wb = d.wb;
   a.p1 = pl.p1;
   a.p2 = pl.p2;
   a.W = pl.W;
-  a.kp = pl.kp;
-  a.kf = d.kf;
-  a.kb = d.kb;
-  a.tf = d.tf;
-  a.tb = d.tb;
-  a.tg = d.tg;
+  std::memcpy(a.hf, pl.hf, sizeof a.hf);
+  std::memcpy(a.hb, pl.hb, sizeof a.hb);
+  a.mw = pl.mw.empty() ? nullptr : d.mw;
+  a.tab = d.tab;
   a.tlo = pl.tlo;
+  a.T = pl.T;
+  a.ntab = (int)(pl.tab.size() + pl.wb.size());
   return a;
 }
 
@@ -1019,9 +1038,12 @@ static int plan_solve(const OpPlan& pl) {
 // ---------------------------------------------------------------------------
 // launch
 // ---------------------------------------------------------------------------
-// LDS of a y/z workgroup of nthr chunk threads: two exchange buffers and one
-// flag per line.
-static size_t yz_lds(int nthr, int lines) { return 2 * (size_t)nthr * sizeof(D2) + (size_t)lines * sizeof(int); }
+// LDS of a y/z workgroup of nthr chunk threads: two exchange buffers, one flag
+// per line, the tables of a bounded line.
+static size_t yz_lds(int solve, int nthr, int lines, int ntab) {
+  return (solve == SOLVE_NONE ? 0 : 2 * (size_t)nthr * sizeof(D2)) + (size_t)lines * sizeof(int) +
+         (size_t)ntab * sizeof(double);
+}
 
 // Lines per y/z workgroup (forced: the tuned value, 0 = none). At 256^3 32
 // lines measured fastest for FP64 fields (d1 y 54 us; 16 lines 58, 64 lines
@@ -1042,12 +1064,14 @@ static int launch_typed(pyr_ctx* c, int dir, int forced, LineArgs a, const TS* i
   if (dir == 0) {
     a.vec = ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0) && ((uintptr_t)a.out32 % 8 == 0);
     a.lines = 64 / a.P;
-    const dim3 grid((unsigned)((a.nlines + a.lines - 1) / a.lines)), block(64);
-    hipLaunchKernelGGL((k_line_x<TS, KIND, SOLVE, FULL>), grid, block, 0, c->stream, a, in, out);
+    const int per = a.lines * XWaves<SOLVE>::v;
+    const dim3 grid((unsigned)((a.nlines + per - 1) / per)), block(64 * XWaves<SOLVE>::v);
+    hipLaunchKernelGGL((k_line_x<TS, KIND, SOLVE, FULL>), grid, block, (size_t)a.ntab * sizeof(double), c->stream, a,
+                       in, out);
   } else {
     a.lines = yz_lines(a.P, a.nlines, dir, (int)sizeof(TS), forced, c->ncu);
     const dim3 grid((unsigned)((a.nlines + a.lines - 1) / a.lines)), block(a.lines * a.P);
-    const size_t shm = SOLVE == SOLVE_NONE ? 0 : yz_lds(a.lines * a.P, a.lines);
+    const size_t shm = yz_lds(SOLVE, a.lines * a.P, a.lines, a.ntab);
     auto k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_NONE>;
     // filters only exist for the r4 kind; accumulating epilogues for every kind
     if constexpr (KIND == K_R4) {
@@ -1371,21 +1395,22 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
   };
   const int P = a.P, N = a.N;
   std::vector<St> st(P);
+  const Tables tabs(a.tab, a.T);
   auto rows_of = [&](int p, auto f) {
-    if (SOLVE == SOLVE_BND && (p < a.tlo || p == P - 1)) f(TableRows{a.tf, a.tb, a.tg, P, p});
+    if (SOLVE == SOLVE_BND && (p < a.tlo || p == P - 1)) f(TableRows{tabs, a.T, slot_of(a, p)});
     else f(ConstRows{a.p1, a.p2});
   };
-  auto carry = [&](int p, int step, double& e0, double& e1) {
-    const double* K = step < 0 ? a.kf : a.kb;
-    e0 = e1 = 0.0;
-    int q = p;
-    for (int j = 0; j < a.W; ++j) {
-      q += step;
-      if (a.periodic) q = (q + P) % P;
-      if (q < 0 || q >= P) break;
-      const double* u = step < 0 ? st[q].e : st[q].b;
-      carry_add(K + 4 * (j * a.kp + (a.kp == 1 ? 0 : p)), u[0], u[1], e0, e1);
-    }
+  auto carry = [&](int p, auto step, double& e0, double& e1) {
+    constexpr int STEP = decltype(step)::value;
+    auto read = [&](int q, double& u0, double& u1) {
+      const double* u = STEP < 0 ? st[q].e : st[q].b;
+      u0 = u[0];
+      u1 = u[1];
+    };
+    if constexpr (SOLVE == SOLVE_BND)
+      carry_in<false, STEP>(a, p, [&](int q) { return tabs.th + 8 * slot_of(a, q) + (STEP > 0 ? 4 : 0); }, read, e0, e1);
+    else
+      carry_in<true, STEP>(a, p, [&](int q) { return (STEP < 0 ? a.hf : a.hb)[q < a.mx ? 0 : 1]; }, read, e0, e1);
   };
   for (int p = 0; p < P; ++p) {
     St& t = st[p];
@@ -1400,8 +1425,10 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
       }
       t.win[w] = v;
     }
+    B4 lo = {}, hi = {};
+    if (!a.periodic) boundary_rows<KIND, false>(a, tabs.wb, p, t.win, lo, hi);
     rhs_interior<KIND>(a, t.win, t.x);
-    if (!a.periodic) rhs_boundary<KIND, false>(a, a.wb, p, t.win, t.x);
+    if (!a.periodic) put_boundary_rows<false>(a, p, lo, hi, t.x);
     if (SOLVE == SOLVE_NONE) continue;
     t.e[0] = t.e[1] = 0.0;
     rows_of(p, [&](auto rows) { fwd_pass<false, false>(rows, t.x, t.m, t.e[0], t.e[1]); });
@@ -1411,7 +1438,7 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
     for (int p = 0; p < P; ++p) {
       St& t = st[p];
       double e0, e1;
-      carry(p, -1, e0, e1);
+      carry(p, std::integral_constant<int, -1>(), e0, e1);
       t.b[0] = t.b[1] = 0.0;
       rows_of(p, [&](auto rows) {
         fwd_pass<false, true>(rows, t.x, t.m, e0, e1);
@@ -1431,7 +1458,7 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
       continue;
     }
     double b0, b1;
-    carry(p, 1, b0, b1);
+    carry(p, std::integral_constant<int, 1>(), b0, b1);
     if (bad) b0 = b1 = std::nan("");
     rows_of(p, [&](auto rows) { bwd_sink<false>(rows, t.x, t.m, b0, b1, emit); });
   }
@@ -1495,8 +1522,10 @@ static int emulate(pyr_ctx* c, int op, int dir, const TS* in, TS* out, bool anti
     for (size_t i = 0; i < n; ++i) out[i] = pl.null_option == 1 ? in[i] : (TS)0;
     return 0;
   }
+  const std::vector<double> tab = with_boundary_rows(pl);
   DevPlan d;
-  host_tables(pl, d);
+  d.tab = tab.data();
+  d.mw = pl.mw.data();
   const LineArgs a = make_args(c, pl, d, dir, EPI_STORE, 0.0, sizeof(TS) == 8 ? PYR_F64 : PYR_R32);
   const int sv = plan_solve(pl);
   const bool refined = sizeof(TS) == 4 && use_refined(c, op, dir);
@@ -1651,14 +1680,18 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
     L.nblocks = blk;
     return upload(ref.data(), ref.size() * sizeof(RefEntry));
   }
-  int nthr = 64;
-  if (!L.x) {
+  int nthr = 64, ntab = 0;
+  for (auto& e : all) ntab = std::max(ntab, e.a.ntab);
+  if (L.x) {
+    nthr = 64 * (sv == SOLVE_BND ? XWaves<SOLVE_BND>::v : 1);
+    L.shm = (size_t)ntab * sizeof(double);
+  } else {
     // 512 chunk threads a workgroup (64 lines of 8 chunks to 16 of 32), 1024
     // where a member's lines have more than 32 chunks
     int Pmax = 1;
     for (auto& e : all) Pmax = std::max(Pmax, e.a.P);
     nthr = Pmax > 32 ? WG_MAX : WG_MAX / 2;
-    L.shm = sv == SOLVE_NONE ? 0 : yz_lds(nthr, 128);
+    L.shm = yz_lds(sv, nthr, 128, ntab);
     L.pre = pre;
   }
   L.block = dim3(nthr);
@@ -1671,8 +1704,9 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
       e.a.lines = 128;
       while (e.a.lines * e.a.P > nthr) e.a.lines /= 2;
     }
+    const int per = L.x ? e.a.lines * (nthr / 64) : e.a.lines;
     e.blk0 = blk;
-    blk += (e.a.nlines + e.a.lines - 1) / e.a.lines;
+    blk += (e.a.nlines + per - 1) / per;
   }
   L.nblocks = blk;
   return upload(all.data(), all.size() * sizeof(GrpEntry));

@@ -49,16 +49,13 @@ struct LineArgs {
   int addv, epi;
   double scale, epi_c;
   double w[4];             // interior right-hand side (rhs_interior)
-  const double* wb;        // boundary rows of a bounded line
   double p1, p2;           // recurrence constants
-  int W, kp;               // carry terms; carry matrices per term (1 or P)
-  const double* kf;
-  const double* kb;
-  // bounded lines: row factors of the chunks p < tlo and p = P - 1
-  const double* tf;
-  const double* tb;
-  const double* tg;
-  int tlo;
+  int W;                   // chunks that enter a carry
+  double hf[2][4], hb[2][4];  // H of constant chunks of mb + 1 and mb rows
+  const double* mw;        // remaining turns of a cyclic line (null: none matter)
+  // bounded lines: the tables of T slots (OpPlan::tab), then the boundary rows
+  const double* tab;
+  int tlo, T, ntab;
   int vec;                 // x lines: the pointers allow 16-byte accesses
   // FP64 sweeps with the store epilogue: when set, every stored value is also
   // written here rounded to FP32 (same element index as the output); with
@@ -115,32 +112,53 @@ PYR_HD double boundary_row(const double* c, const TW* v) {
   return acc;
 }
 
-// Replace the rows of a bounded line's ends by their own right-hand sides
-// (p: this chunk; every chunk has at least 2*NB rows).
+struct B4 { double a, b, c, d; };  // four values, never indexed at run time
+
+// The right-hand sides of a bounded line's end rows: into lo by the first
+// chunk, into hi by the last one (p: this chunk; every chunk has at least 2*NB
+// rows, the last one mb of them in every line). Taken before the interior rows,
+// while the window is all that is in registers.
 template <int KIND, bool FULL, typename TW>
-PYR_HD void rhs_boundary(const LineArgs& a, const double* wb, int p, const TW* win, double* rhs) {
+PYR_HD void boundary_rows(const LineArgs& a, const double* wb, int p, const TW* win, B4& lo, B4& hi) {
   constexpr int R = Halo<KIND>::R;
   if (p == 0) {
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      PYR_ROW_FENCE(k, 1);
-      rhs[k] = boundary_row<KIND>(wb + k * WBROW, win + k + R);
-    }
+    lo.a = boundary_row<KIND>(wb, win + R);
+    PYR_ROW_FENCE(0, 1);
+    lo.b = boundary_row<KIND>(wb + WBROW, win + 1 + R);
+    PYR_ROW_FENCE(0, 1);
+    lo.c = boundary_row<KIND>(wb + 2 * WBROW, win + 2 + R);
+    PYR_ROW_FENCE(0, 1);
+    lo.d = boundary_row<KIND>(wb + 3 * WBROW, win + 3 + R);
   }
   if (p == a.P - 1) {
-    if constexpr (FULL) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        PYR_ROW_FENCE(j, 1);
-        rhs[CHUNK - NB + j] = boundary_row<KIND>(wb + (NB + j) * WBROW, win + CHUNK - NB + j + R);
+    for (int k = FULL ? CHUNK - NB : NB; k < CHUNK; ++k) {
+      const int j = k - ((FULL ? CHUNK : a.mb) - NB);
+      if (j >= 0 && j < NB) {
+        PYR_ROW_FENCE(k, 1);
+        const double v = boundary_row<KIND>(wb + (NB + j) * WBROW, win + k + R);
+        hi.a = j == 0 ? v : hi.a;
+        hi.b = j == 1 ? v : hi.b;
+        hi.c = j == 2 ? v : hi.c;
+        hi.d = j == 3 ? v : hi.d;
       }
-    } else {
-      // the last chunk has mb rows in every line: the row is wave-uniform
+    }
+  }
+}
+// ... and into their rows of the chunk
+template <bool FULL>
+PYR_HD void put_boundary_rows(const LineArgs& a, int p, const B4& lo, const B4& hi, double* rhs) {
+  rhs[0] = p == 0 ? lo.a : rhs[0];
+  rhs[1] = p == 0 ? lo.b : rhs[1];
+  rhs[2] = p == 0 ? lo.c : rhs[2];
+  rhs[3] = p == 0 ? lo.d : rhs[3];
+  const double h0 = hi.a, h1 = hi.b, h2 = hi.c, h3 = hi.d;
 #pragma unroll
-      for (int k = NB; k < CHUNK; ++k) {
-        const int j = k - (a.mb - NB);
-        if (j >= 0 && j < NB) rhs[k] = boundary_row<KIND>(wb + (NB + j) * WBROW, win + k + R);
-      }
+  for (int k = FULL ? CHUNK - NB : NB; k < CHUNK; ++k) {
+    const int j = k - ((FULL ? CHUNK : a.mb) - NB);
+    if (j >= 0 && j < NB) {
+      const double v = j == 0 ? h0 : j == 1 ? h1 : j == 2 ? h2 : h3;
+      rhs[k] = p == a.P - 1 ? v : rhs[k];
     }
   }
 }
@@ -154,28 +172,31 @@ struct ConstRows {
   PYR_HD void bwd(int, double& c1, double& c2) const { c1 = p1; c2 = p2; }
   PYR_HD double diag(int, double x) const { return x; }
 };
+
+// Where the parts of a bounded line's tables sit (in LDS on the device).
+struct Tables {
+  const double *tf, *tb, *tg, *th, *wb;
+  PYR_HD Tables(const double* t, int T)
+      : tf(t), tb(t + 2 * CHUNK * T), tg(t + 4 * CHUNK * T), th(t + 5 * CHUNK * T), wb(t + 5 * CHUNK * T + 8 * T) {}
+};
+// table slot of chunk p
+PYR_HD int slot_of(const LineArgs& a, int p) {
+  if (p == a.P - 1) return a.T - 1;
+  return p < a.tlo ? p : a.tlo + (p < a.mx ? 0 : 1);
+}
 struct TableRows {
-  const double* tf;
-  const double* tb;
-  const double* tg;
-  int P, p;
+  Tables t;
+  int T, slot;
   PYR_HD static void fence([[maybe_unused]] int k) { PYR_ROW_FENCE(k, 4); }
-  struct alignas(16) D2 { double x, y; };
-  // row k of chunk p as a uniform row address plus the chunk's 32-bit offset
-  template <typename T>
-  PYR_HD T row(const double* t, int k) const {
-    const char* base = reinterpret_cast<const char*>(t) + (size_t)(unsigned)(k * P) * sizeof(T);
-    return *reinterpret_cast<const T*>(base + (unsigned)p * (unsigned)sizeof(T));
-  }
   PYR_HD void fwd(int k, double& c1, double& c2) const {
-    const D2 t = row<D2>(tf, k);
-    c1 = t.x; c2 = t.y;
+    const double* e = t.tf + 2 * (k * T + slot);
+    c1 = e[0]; c2 = e[1];
   }
   PYR_HD void bwd(int k, double& c1, double& c2) const {
-    const D2 t = row<D2>(tb, k);
-    c1 = t.x; c2 = t.y;
+    const double* e = t.tb + 2 * (k * T + slot);
+    c1 = e[0]; c2 = e[1];
   }
-  PYR_HD double diag(int k, double x) const { return x * row<double>(tg, k); }
+  PYR_HD double diag(int k, double x) const { return x * t.tg[k * T + slot]; }
 };
 
 // Forward recurrence entered with (x_{-2}, x_{-1}) = (e0, e1), which becomes
@@ -236,10 +257,35 @@ PYR_HD void bwd_sink(const Rows& rows, const double* x, int m, double b1, double
   }
 }
 
-// Add one chunk's exit (u0, u1) to an entry state through its carry matrix.
-PYR_HD void carry_add(const double* K, double u0, double u1, double& e0, double& e1) {
-  e0 += K[0] * u0 + K[1] * u1;
-  e1 += K[2] * u0 + K[3] * u1;
+// Entry state of chunk p from the exits of the W chunks on its near side
+// (STEP -1: forward, from p-W up to p-1; +1: backward, from p+W down to p+1):
+// E <- H_q E + e_q. exit_of(q, u0, u1) reads chunk q's exit, h(q) its matrix.
+// Beyond the ends of a bounded line nothing enters.
+template <bool CYCLIC, int STEP, typename H, typename ExitOf>
+PYR_HD void carry_in(const LineArgs& a, int p, H h, ExitOf exit_of, double& e0, double& e1) {
+  e0 = e1 = 0.0;
+  int q = p + STEP * a.W;
+  if (CYCLIC) q = q < 0 ? q + a.P : (q >= a.P ? q - a.P : q);
+#pragma unroll 2
+  for (int j = 0; j < a.W; ++j) {
+    const bool in = CYCLIC || (q >= 0 && q < a.P);
+    const int qq = in ? q : p;
+    double u0, u1;
+    exit_of(qq, u0, u1);
+    const double* m = h(qq);
+    const double s0 = (in ? u0 : 0.0) + m[1] * e1;
+    const double s1 = (in ? u1 : 0.0) + m[3] * e1;
+    e1 = s1 + m[2] * e0;
+    e0 = s0 + m[0] * e0;
+    q -= STEP;
+    if (CYCLIC) q = q < 0 ? a.P - 1 : (q >= a.P ? 0 : q);
+  }
+  if (CYCLIC && a.mw) {
+    const double* m = a.mw + 8 * p + (STEP > 0 ? 4 : 0);
+    const double t0 = m[0] * e0 + m[1] * e1;
+    e1 = m[2] * e0 + m[3] * e1;
+    e0 = t0;
+  }
 }
 
 template <typename TS>

@@ -9,11 +9,13 @@
 //     x_k = r_k - l1_k x_{k-1} - l2_k x_{k-2}
 //     y_k = g_k x_k - v1_k y_{k+1} - v2_k y_{k+2}
 // (y times 1/c is the solution). A chunk runs each recurrence from a zero
-// state to get its exit state; its true entry state is the sum over the chunks
-// before it (after it, backward) of their exits propagated through the chunks
-// between, and it re-runs the recurrence from there. The propagation matrices
-// decay geometrically with distance (the schemes' recurrences are strongly
-// damped), so only the W nearest chunks whose matrix is above CARRY_TOL enter.
+// state to get its exit state e; its true entry state follows from the chunks
+// before it (after it, backward) as E <- H_q E + e_q, with H_q the 2x2 matrix
+// that takes chunk q's entry to its exit, and it re-runs the recurrence from
+// there. Products of the H decay geometrically (the schemes' recurrences are
+// strongly damped), so the sum starts W chunks away, where they fall below
+// CARRY_TOL; around a cyclic line of fewer chunks it makes one turn and the
+// remaining turns are a matrix (I - H...H)^-1.
 //
 // Periodic lines have a circulant LHS, which factors exactly as
 //     A = c Q^T Q,   Q = I + p1 S + p2 S^2   ((S x)_i = x_{i-1}, cyclic)
@@ -64,14 +66,16 @@ struct OpPlan {
   std::vector<double> wb;     // 2*NB x WBROW boundary rows of a bounded line
   double p1 = 0, p2 = 0;      // limit coefficients
   int W = 0;                  // chunks that enter a carry
-  int kp = 1;                 // 1: one set of carry matrices for all chunks, else P
-  std::vector<double> kf, kb; // W x kp x 4 carry matrices, forward and backward
-  // bounded lines: per-row factors, row k of chunk p at [k * P + p]
-  std::vector<double> tf, tb, tg;  // (l1, l2), (v1, v2), g
-  int tlo = 0;                // chunks p < tlo and p = P - 1 need the tables
+  double hf[2][4] = {}, hb[2][4] = {};  // H of constant chunks of mb + 1 and mb rows
+  std::vector<double> mw;     // P x 8 remaining turns (forward, backward); empty if none matter
+  // bounded lines, for T slots (the chunks p < tlo, constant chunks of mb + 1
+  // and mb rows, the last chunk): CHUNK x T x (l1, l2), CHUNK x T x (v1, v2),
+  // CHUNK x T g, T x 8 H (forward, backward)
+  int tlo = 0, T = 0;
+  std::vector<double> tab;
 };
 
-// Propagation matrices below this are left out of the carries: relative to the
+// Propagation below this is left out of the carries: relative to the
 // state they multiply it is under a thousandth of an FP64 rounding.
 constexpr long double CARRY_TOL = 1e-19L;
 
@@ -116,28 +120,32 @@ inline ld norm(const M2& x) {
   return std::max(std::max(std::fabs(x[0]), std::fabs(x[1])), std::max(std::fabs(x[2]), std::fabs(x[3])));
 }
 
-// Carry matrices of one direction. H[q] takes the entry state of chunk q to
-// the part of its exit state that depends on it; step is -1 forward (the carry
-// of chunk p comes from p-1, p-2, ...) or +1 backward. K[j][p] multiplies the
-// exit of chunk p + step (j+1); around a cyclic line the terms beyond one turn
-// fold onto the chunks they come from. Returns the terms per chunk.
-inline std::vector<std::vector<M2>> carry_matrices(const std::vector<M2>& H, int step, bool cyclic) {
+// Chunks that enter the carries of one direction (step -1: chunk p takes from
+// p-1, p-2, ...; +1: from p+1, ...): the most, over p, whose propagation to p
+// is above CARRY_TOL.
+inline int carry_terms(const std::vector<M2>& H, int step, bool cyclic) {
   const int P = (int)H.size();
-  std::vector<std::vector<M2>> K;
+  int W = 0;
   for (int p = 0; p < P; ++p) {
     M2 acc = {1, 0, 0, 1};
-    for (int j = 0;; ++j) {
-      int q = p + step * (j + 1);
+    for (int j = 1;; ++j) {
+      const int q = p + step * j;
       if (!cyclic && (q < 0 || q >= P)) break;
       if (norm(acc) < CARRY_TOL) break;
-      q = ((q % P) + P) % P;
-      const int jj = j % P;
-      if ((int)K.size() <= jj) K.push_back(std::vector<M2>(P, M2{0, 0, 0, 0}));
-      for (int i = 0; i < 4; ++i) K[jj][p][i] += acc[i];
-      acc = mul(acc, H[q]);
+      W = std::max(W, j);
+      acc = mul(acc, H[((q % P) + P) % P]);
     }
   }
-  return K;
+  return W;
+}
+
+// (I - H around the whole line)^-1 for the entry of chunk p
+inline M2 turns(const std::vector<M2>& H, int p, int step) {
+  const int P = (int)H.size();
+  M2 acc = {1, 0, 0, 1};
+  for (int j = 1; j <= P; ++j) acc = mul(acc, H[(((p + step * j) % P) + P) % P]);
+  const ld a = 1 - acc[0], b = -acc[1], c = -acc[2], d = 1 - acc[3], det = a * d - b * c;
+  return {d / det, -b / det, -c / det, a / det};
 }
 
 // Chunks of a line of n rows along direction dir. x lines: one wave takes G
@@ -267,24 +275,12 @@ inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, d
         l2[i] = u2[i] = p2;
         g[i] = 1.0L;
       }
-    pl.tf.assign((size_t)CHUNK * P * 2, 0.0);
-    pl.tb.assign((size_t)CHUNK * P * 2, 0.0);
-    pl.tg.assign((size_t)CHUNK * P, 0.0);
-    for (int p = 0; p < P; ++p) {
-      bool all = true;
-      for (int k = 0; start(p) + k < start(p + 1); ++k) {
-        const int i = start(p) + k;
-        const size_t e = (size_t)k * P + p;
-        all = all && conv[i];
-        pl.tf[2 * e] = (double)l1[i]; pl.tf[2 * e + 1] = (double)l2[i];
-        pl.tb[2 * e] = (double)u1[i]; pl.tb[2 * e + 1] = (double)u2[i];
-        pl.tg[e] = (double)g[i];
-      }
-      if (!all && p < P - 1) pl.tlo = p + 1;
-    }
+    for (int p = 0; p < P - 1; ++p)
+      for (int i = start(p); i < start(p + 1); ++i)
+        if (!conv[i]) pl.tlo = p + 1;
   }
 
-  // carry matrices
+  // entry-to-exit matrices and carries
   std::vector<M2> Hf(P), Hb(P);
   for (int p = 0; p < P; ++p)
     for (int j = 0; j < 2; ++j) {
@@ -305,18 +301,53 @@ inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, d
       Hb[p][j] = b1;
       Hb[p][2 + j] = b2;
     }
-  const auto Kf = detail::carry_matrices(Hf, -1, periodic), Kb = detail::carry_matrices(Hb, 1, periodic);
-  pl.W = (int)std::max(Kf.size(), Kb.size());
-  pl.kp = (periodic && pl.mx == 0) ? 1 : P;
-  pl.kf.assign((size_t)pl.W * pl.kp * 4, 0.0);
-  pl.kb.assign((size_t)pl.W * pl.kp * 4, 0.0);
-  for (int j = 0; j < pl.W; ++j)
-    for (int p = 0; p < pl.kp; ++p)
+  const int need = std::max(detail::carry_terms(Hf, -1, periodic), detail::carry_terms(Hb, 1, periodic));
+  pl.W = std::min(need, periodic ? P : P - 1);
+  if (need > pl.W && periodic) {
+    pl.mw.resize((size_t)P * 8);
+    for (int p = 0; p < P; ++p) {
+      const M2 f = detail::turns(Hf, p, -1), b = detail::turns(Hb, p, 1);
       for (int i = 0; i < 4; ++i) {
-        const size_t e = ((size_t)j * pl.kp + p) * 4 + i;
-        if (j < (int)Kf.size()) pl.kf[e] = (double)Kf[j][p][i];
-        if (j < (int)Kb.size()) pl.kb[e] = (double)Kb[j][p][i];
+        pl.mw[p * 8 + i] = (double)f[i];
+        pl.mw[p * 8 + 4 + i] = (double)b[i];
       }
+    }
+  }
+  // constant chunks, from the limit coefficients
+  for (int w = 0; w < 2; ++w)
+    for (int j = 0; j < 2; ++j) {
+      ld a0 = j == 0, a1 = j == 1, b1 = j == 0, b2 = j == 1;
+      for (int k = 0; k < pl.mb + 1 - w; ++k) {
+        const ld x = -p1 * a1 - p2 * a0, y = -p1 * b1 - p2 * b2;
+        a0 = a1; a1 = x;
+        b2 = b1; b1 = y;
+      }
+      pl.hf[w][j] = (double)a0; pl.hf[w][2 + j] = (double)a1;
+      pl.hb[w][j] = (double)b1; pl.hb[w][2 + j] = (double)b2;
+    }
+  if (periodic) return pl;
+  const int T = pl.T = pl.tlo + 3;
+  pl.tab.assign((size_t)CHUNK * T * 5 + 8 * T, 0.0);
+  double* tf = pl.tab.data();
+  double* tb = tf + 2 * CHUNK * T;
+  double* tg = tb + 2 * CHUNK * T;
+  double* th = tg + CHUNK * T;
+  for (int t = 0; t < T; ++t) {
+    const bool chunk = t < pl.tlo || t == T - 1;  // else a constant slot
+    const int p = t == T - 1 ? P - 1 : t;
+    for (int k = 0; k < CHUNK; ++k) {
+      const int i = start(p) + k;
+      const bool own = chunk && i < start(p + 1);
+      const size_t e = (size_t)k * T + t;
+      tf[2 * e] = (double)(own ? l1[i] : p1); tf[2 * e + 1] = (double)(own ? l2[i] : p2);
+      tb[2 * e] = (double)(own ? u1[i] : p1); tb[2 * e + 1] = (double)(own ? u2[i] : p2);
+      tg[e] = own ? (double)g[i] : 1.0;
+    }
+    for (int i = 0; i < 4; ++i) {
+      th[8 * t + i] = chunk ? (double)Hf[p][i] : pl.hf[t - pl.tlo][i];
+      th[8 * t + 4 + i] = chunk ? (double)Hb[p][i] : pl.hb[t - pl.tlo][i];
+    }
+  }
   return pl;
 }
 
