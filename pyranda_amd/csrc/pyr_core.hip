@@ -110,6 +110,12 @@ __device__ __forceinline__ bool wave_needs_tables(const LineArgs& a, int p) {
   return __ballot(p < a.tlo || p == a.P - 1) != 0;
 }
 
+template <bool FULL>
+__device__ __forceinline__ auto rows_of_chunk(const LineArgs& a, int p) {
+  if constexpr (FULL) return AllRows{};
+  else return ChunkRows{a.mb, p < a.mx};
+}
+
 // The passes of one chunk around its two exchanges. `rows` are ConstRows or
 // TableRows; the bounded solve picks one per wave.
 template <int SOLVE, typename F>
@@ -181,6 +187,7 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
   const int rb = (int)(a.stride * (long long)sizeof(TS));
   const int s = FULL ? p * CHUNK : chunk_start(a, p);
   const int m = FULL ? CHUNK : a.mb + (p < a.mx ? 1 : 0);
+  const auto have = rows_of_chunk<FULL>(a, p);
   const bool last = p == a.P - 1;
   const bool wrap = SOLVE == SOLVE_CIRC || (SOLVE == SOLVE_NONE && a.periodic);
   const bool bounded = SOLVE == SOLVE_BND || (SOLVE == SOLVE_NONE && !a.periodic);
@@ -250,15 +257,14 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
   if constexpr (SOLVE == SOLVE_NONE) {
     if (!valid) return;
 #pragma unroll
-    for (int k = 0; k < CHUNK; ++k)
-      if (FULL || k < m) emit(k, x[k]);
+    for (int k = 0; k < CHUNK; ++k) have.row(k, [&] { emit(k, x[k]); });
   } else {
     const bool own = SOLVE == SOLVE_BND && wave_needs_tables(a, p);
     const int slot = SOLVE == SOLVE_BND ? slot_of(a, p) : 0;
     if (p == 0) bad[lane] = 0;
     double e0 = 0.0, e1 = 0.0;
     if (act) {
-      with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
+      with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) { fwd_pass<false>(have, rows, x, e0, e1); });
       X0[p * LY + lane] = D2{e0, e1};
     }
     __syncthreads();
@@ -267,14 +273,15 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
     if constexpr (PRE == PRE_OLD) {
 #pragma unroll
       for (int k = 0; k < CHUNK; ++k)
-        pre[k] = FULL ? buf_load(TS(), rout, vmid, k * rb) : buf_load(TS(), rout, k < m ? row_off(k) : OOB, 0);
+        if (FULL || k <= a.mb)
+          pre[k] = FULL ? buf_load(TS(), rout, vmid, k * rb) : buf_load(TS(), rout, k < m ? row_off(k) : OOB, 0);
     }
     double b0 = 0.0, b1 = 0.0;
     if (act) {
       carry_of<SOLVE, FULL, -1>(a, tabs, p, [&](int q) { return X0[q * LY + lane]; }, e0, e1);
       with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) {
-        fwd_pass<FULL, true>(rows, x, m, e0, e1);
-        bwd_exit<FULL>(rows, x, m, b0, b1);
+        fwd_pass<true>(have, rows, x, e0, e1);
+        bwd_exit(have, rows, x, b0, b1);
       });
       X1[p * LY + lane] = D2{b0, b1};
       // a NaN or infinity anywhere in a line spreads to all of it, as it does
@@ -287,7 +294,7 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
     carry_of<SOLVE, FULL, 1>(a, tabs, p, [&](int q) { return X1[q * LY + lane]; }, b0, b1);
     if (bad[lane]) b0 = b1 = __builtin_nan("");
     if (!valid) return;
-    with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
+    with_rows<SOLVE>(a, own, tabs, slot, [&](auto rows) { bwd_sink(have, rows, x, b0, b1, emit); });
   }
 }
 
@@ -443,6 +450,7 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   const bool act = l < nval;
   const int s = FULL ? p * CHUNK : chunk_start(a, p);
   const int m = FULL ? CHUNK : a.mb + (p < a.mx ? 1 : 0);
+  const auto have = rows_of_chunk<FULL>(a, p);
   const bool last = p == P - 1;
   const bool wrap = SOLVE == SOLVE_CIRC || (SOLVE == SOLVE_NONE && a.periodic);
   TS* row0 = tile + (act ? (FULL ? l * P * CP : sh + l * N) : (FULL ? 0 : sh));
@@ -493,20 +501,19 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   if constexpr (SOLVE == SOLVE_NONE) {
     wave_fence();  // every window is in registers
 #pragma unroll
-    for (int k = 0; k < CHUNK; ++k)
-      if (FULL || k < m) emit(k, x[k]);
+    for (int k = 0; k < CHUNK; ++k) have.row(k, [&] { emit(k, x[k]); });
   } else {
     // lanes past the last whole line read some exit and drop the result
     auto exit_of = [&](int q) { return ex[l * P + q < 64 ? l * P + q : 0]; };
     const int slot = SOLVE == SOLVE_BND ? slot_of(a, p) : 0;
     double e0 = 0.0, e1 = 0.0, b0 = 0.0, b1 = 0.0;
-    with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) { fwd_pass<FULL, false>(rows, x, m, e0, e1); });
+    with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) { fwd_pass<false>(have, rows, x, e0, e1); });
     ex[lane] = D2{e0, e1};
     wave_fence();
     carry_of<SOLVE, FULL, -1>(a, tabs, p, exit_of, e0, e1);
     with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) {
-      fwd_pass<FULL, true>(rows, x, m, e0, e1);
-      bwd_exit<FULL>(rows, x, m, b0, b1);
+      fwd_pass<true>(have, rows, x, e0, e1);
+      bwd_exit(have, rows, x, b0, b1);
     });
     // as in line_yz_body: a NaN or infinity spreads to the whole line
     const unsigned long long bad = __ballot(act && (!__builtin_isfinite(b0) || !__builtin_isfinite(b1)));
@@ -515,7 +522,7 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
     wave_fence();
     carry_of<SOLVE, FULL, 1>(a, tabs, p, exit_of, b0, b1);
     if (bad & line_lanes(l, P)) b0 = b1 = __builtin_nan("");
-    with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) { bwd_sink<FULL>(rows, x, m, b0, b1, emit); });
+    with_rows<SOLVE>(a, true, tabs, slot, [&](auto rows) { bwd_sink(have, rows, x, b0, b1, emit); });
   }
   wave_fence();
   float* o32 = nullptr;
@@ -531,8 +538,8 @@ __global__ void __launch_bounds__(64 * XWaves<SOLVE>::v) k_line_x(LineArgs a, co
 // Grouped launches: one launch applies the same operator to the fields of
 // several simulations (an ensemble's members, each at `off` elements into
 // one allocation), with lines of any lengths. Entry j covers workgroups
-// [blk0_j, blk0_{j+1}); a workgroup finds its member by binary search
-// (wave-uniform) and runs the single-field body with that member's line
+// [blk0_j, blk0_{j+1}); a workgroup reads its member from a map (one load; a
+// binary search over blk0 is a chain of them) and runs the single-field body with that member's line
 // arguments: every member has its own lines per workgroup (x: 64 / P, y/z: as
 // many as P chunk threads each leave room for), so one launch serves all
 // line lengths.
@@ -542,21 +549,10 @@ struct GrpEntry {
   long long blk0;
 };
 
-template <typename Entry>
-__device__ __forceinline__ int grp_member(const Entry* __restrict__ g, int M, long long b) {
-  int lo = 0, hi = M - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (g[mid].blk0 <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
 template <typename TS, int KIND, int SOLVE>
-__global__ void __launch_bounds__(64 * XWaves<SOLVE>::v) k_line_x_grp(const GrpEntry* __restrict__ g, int M, const TS* __restrict__ in,
+__global__ void __launch_bounds__(64 * XWaves<SOLVE>::v) k_line_x_grp(const GrpEntry* __restrict__ g, const int* __restrict__ member, const TS* __restrict__ in,
                                                    TS* __restrict__ out) {
-  const int j = grp_member(g, M, blockIdx.x);
+  const int j = member[blockIdx.x];
   // a private copy: its fields load once (wave-uniform) and no store of the
   // body can alias them
   const LineArgs a = g[j].a;
@@ -565,29 +561,32 @@ __global__ void __launch_bounds__(64 * XWaves<SOLVE>::v) k_line_x_grp(const GrpE
 }
 
 template <typename TS, int KIND, int SOLVE, int PRE>
-__global__ void __launch_bounds__(WG_MAX) k_line_yz_grp(const GrpEntry* __restrict__ g, int M,
+__global__ void __launch_bounds__(WG_MAX) k_line_yz_grp(const GrpEntry* __restrict__ g, const int* __restrict__ member,
                                                         const TS* __restrict__ in, TS* __restrict__ out) {
-  const int j = grp_member(g, M, blockIdx.x);
+  const int j = member[blockIdx.x];
   const LineArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
   line_yz_body<TS, KIND, SOLVE, false, PRE, true>(a, (long long)blockIdx.x - b0, in + off, out + off);
 }
 
 // --- refined FP32 solve of bounded lines (pyr_refined.hpp) -------------------
-// Threads are shaped as in the FP64 kernels above, with up to 32 rows each and
-// workgroups of 512 (x: four waves, each with its own lines and tile). What
-// bounds these kernels is the latency of one workgroup: the factors come from
-// the class tables in LDS (one 16-byte read per row and table quarter instead
-// of nine 4-byte loads from a whole-line table in memory), the reduced rows as
-// 16-byte loads of the chunks within reach, and the boundary rows' terms as
-// independent loads.
-constexpr int REF_THREADS = 512;
-constexpr int REF_X_WAVES = 4;
+// Threads are shaped as in the FP64 kernels above, with up to 32 rows each (two
+// waves per SIMD by registers) and workgroups of 256: as many lines as fit, any
+// number of them, so that few threads idle and an ensemble's sweep fits the
+// chip in one go (24 members, 3.7M points: 489 workgroups for 512 places; 512
+// threads and a power of two of lines gave 319 for 256). x: two waves, each
+// with its own lines and tile. What bounds these kernels is the latency of one
+// workgroup: the class tables and the reduced rows of the chunks within reach
+// are staged in LDS, and the boundary rows' terms are independent reads.
+constexpr int REF_THREADS = 256;
+constexpr int REF_X_WAVES = 2;
 
-// class tables into LDS
-__device__ __forceinline__ void ref_stage(const RefArgs& a, float* tab) {
+// class tables and reduced rows into LDS
+__device__ __forceinline__ void ref_stage(const RefArgs& a, float* tab, float* g) {
   for (int e = threadIdx.x; e < NCLS * RCHUNK * CROW / 4; e += blockDim.x)
     reinterpret_cast<F4*>(tab)[e] = reinterpret_cast<const F4*>(a.cls)[e];
+  for (int e = threadIdx.x; e < a.P * (2 * a.Wg + 1) * 4; e += blockDim.x)
+    reinterpret_cast<F4*>(g)[e] = reinterpret_cast<const F4*>(a.g)[e];
 }
 
 template <int KIND, int PRE>
@@ -598,10 +597,12 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, con
   __shared__ __align__(16) F4 Y0[REF_THREADS], Y1[REF_THREADS];
   __shared__ float ends[2 * (ENDS + 1) * 64];
   __shared__ int bad[64];
-  ref_stage(a, tab);
+  extern __shared__ __align__(16) unsigned char smem[];
+  float* g = reinterpret_cast<float*>(smem);
+  ref_stage(a, tab, g);
   const int LY = a.lines;
-  const int lane = threadIdx.x & (LY - 1);
-  const int p = (int)threadIdx.x >> __builtin_ctz(LY);
+  const int p = (int)((unsigned)threadIdx.x / (unsigned)LY);
+  const int lane = (int)threadIdx.x - p * LY;
   if (p == 0) bad[lane] = 0;
   const bool act = p < a.P;
   const long long L = blk * LY + lane;
@@ -612,20 +613,17 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, con
   const int m = a.mb + (p < a.mx ? 1 : 0);
   const __amdgpu_buffer_rsrc_t rin = buf_rsrc(in, a.nbytes), rout = buf_rsrc(out, a.nbytes);
   auto off_of = [&](int row) { return (int)((unsigned)lane_off + (unsigned)row * (unsigned)rb); };
-  float pre[PRE == PRE_OLD ? RCHUNK : 1];
-  if constexpr (PRE == PRE_OLD) {
-#pragma unroll
-    for (int k = 0; k < RCHUNK; ++k) pre[k] = buf_load(0.0f, rout, act && k < m ? off_of(s + k) : OOB, 0);
-  }
   // rows beyond the ends read 0
   float win[RCHUNK + 2 * R];
 #pragma unroll
   for (int w = 0; w < RCHUNK + 2 * R; ++w) {
     const int row = s - R + w;
-    win[w] = buf_load(0.0f, rin, act && w < m + 2 * R && row >= 0 && row < a.N ? off_of(row) : OOB, 0);
+    win[w] = 0.0f;
+    if (w <= a.mb + 2 * R)
+      win[w] = buf_load(0.0f, rin, act && w < m + 2 * R && row >= 0 && row < a.N ? off_of(row) : OOB, 0);
   }
   double rhs[RCHUNK];
-  ref_rhs_interior<KIND>(a, win, rhs, m);
+  ref_rhs_interior<KIND>(a, win, rhs);
   if (act && (p == 0 || p == a.P - 1)) {
     // the boundary rows name any of the eight rows at their end: this thread's
     // copy of them in LDS, indexed at run time (no other thread reads it)
@@ -646,40 +644,51 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, con
   }
   __syncthreads();  // class tables visible
   const float* t = tab + ref_class(p, a.P, a.mx) * (RCHUNK * CROW);
-  float x[RCHUNK], d[RCHUNK], z[4], e4[4];
+  float x[RCHUNK], d[RCHUNK], z[4];
+  const bool longer = p < a.mx;
 #pragma unroll
   for (int k = 0; k < RCHUNK; ++k) x[k] = (float)rhs[k];
   if (act) {
-    ref_local_solve(t, m, x);
-    ref_edges(x, m, e4);
-    Y0[p * LY + lane] = F4{e4[0], e4[1], e4[2], e4[3]};
+    ref_local_solve(a, t, x);
+    const F4 e = ref_edges(a, longer, x);
+    Y0[p * LY + lane] = e;
     // as in line_yz_body: a NaN or infinity spreads to the whole line
-    if (!__builtin_isfinite(e4[0]) || !__builtin_isfinite(e4[1])) bad[lane] = 1;
+    if (!__builtin_isfinite(e.x) || !__builtin_isfinite(e.y)) bad[lane] = 1;
   }
   __syncthreads();
   if (act) {
-    ref_neighbours(a, p, [&](int q) { return Y0[q * LY + lane]; }, z);
+    ref_neighbours(a, g, p, [&](int q) { return Y0[q * LY + lane]; }, z);
     if (bad[lane]) z[0] = z[1] = z[2] = z[3] = __builtin_nanf("");
-    ref_spike(t, m, z, x);
-    ref_residual(a, p, m, rhs, x, z, d);
-    ref_local_solve(t, m, d);
-    ref_edges(d, m, e4);
-    Y1[p * LY + lane] = F4{e4[0], e4[1], e4[2], e4[3]};
+    ref_spike(a, t, z, x);
+    ref_residual(a, p, longer, rhs, x, z, d);
+  }
+  // the filter's input or the current output, on its way while the correction
+  // is solved (the right-hand sides' registers are free by now)
+  float pre[PRE == PRE_NONE ? 1 : RCHUNK];
+  if constexpr (PRE != PRE_NONE) {
+#pragma unroll
+    for (int k = 0; k < RCHUNK; ++k)
+      if (k <= a.mb) pre[k] = buf_load(0.0f, PRE == PRE_V ? rin : rout, act && k < m ? off_of(s + k) : OOB, 0);
+  }
+  if (act) {
+    ref_local_solve(a, t, d);
+    Y1[p * LY + lane] = ref_edges(a, longer, d);
   }
   __syncthreads();
   if (!act || L >= a.nlines) return;
-  ref_neighbours(a, p, [&](int q) { return Y1[q * LY + lane]; }, z);
-  ref_spike(t, m, z, d);
+  ref_neighbours(a, g, p, [&](int q) { return Y1[q * LY + lane]; }, z);
+  ref_spike(a, t, z, d);
 #pragma unroll
   for (int k = 0; k < RCHUNK; ++k) {
-    if (k < m) {
+    if (k <= a.mb) {
       double val = ((double)x[k] + (double)d[k]) * a.scale;
-      if constexpr (PRE == PRE_V) val += (double)win[k + R];
+      const int off = k < m ? off_of(s + k) : OOB;
+      if constexpr (PRE == PRE_V) val += (double)pre[k];
       float old = 0.0f;
       if constexpr (PRE == PRE_OLD) old = pre[k];
       if constexpr (PRE == PRE_V)
-        if (a.epi == EPI_ADD || a.epi == EPI_MAXABS) old = buf_load(0.0f, rout, off_of(s + k), 0);
-      buf_store(epilogue<float>(a.epi, a.epi_c, val, old), rout, off_of(s + k), 0);
+        if (a.epi == EPI_ADD || a.epi == EPI_MAXABS) old = buf_load(0.0f, rout, off, 0);
+      buf_store(epilogue<float>(a.epi, a.epi_c, val, old), rout, off, 0);
     }
   }
 }
@@ -693,7 +702,9 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
   __shared__ __align__(16) float tab[NCLS * RCHUNK * CROW];
   __shared__ __align__(16) float tiles[NW][T::SIZE];
   __shared__ __align__(16) F4 ex[NW][64];
-  ref_stage(a, tab);
+  extern __shared__ __align__(16) unsigned char smem[];
+  float* g = reinterpret_cast<float*>(smem);
+  ref_stage(a, tab, g);
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -722,29 +733,30 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
     win[w] = ok ? v : 0.0f;
   }
   double rhs[RCHUNK];
-  ref_rhs_interior<KIND>(a, win, rhs, m);
+  ref_rhs_interior<KIND>(a, win, rhs);
   ref_rhs_boundary(a, p, rhs, [&](int slot) { return end_value(slot, N, [&](int i) { return row0[i]; }); });
   const float* t = tab + ref_class(p, P, a.mx) * (RCHUNK * CROW);
-  float x[RCHUNK], d[RCHUNK], z[4], e4[4];
+  float x[RCHUNK], d[RCHUNK], z[4];
+  const bool longer = p < a.mx;
 #pragma unroll
   for (int k = 0; k < RCHUNK; ++k) x[k] = (float)rhs[k];
   auto edges_of = [&](int q) { return ex[wave][l * P + q < 64 ? l * P + q : 0]; };
-  ref_local_solve(t, m, x);
-  ref_edges(x, m, e4);
-  ex[wave][lane] = F4{e4[0], e4[1], e4[2], e4[3]};
-  const unsigned long long bad = __ballot(act && (!__builtin_isfinite(e4[0]) || !__builtin_isfinite(e4[1])));
+  ref_local_solve(a, t, x);
+  const F4 e = ref_edges(a, longer, x);
+  ex[wave][lane] = e;
+  const unsigned long long bad = __ballot(act && (!__builtin_isfinite(e.x) || !__builtin_isfinite(e.y)));
   wave_fence();
-  ref_neighbours(a, p, edges_of, z);
+  ref_neighbours(a, g, p, edges_of, z);
   if (bad & line_lanes(l, P)) z[0] = z[1] = z[2] = z[3] = __builtin_nanf("");
-  ref_spike(t, m, z, x);
-  ref_residual(a, p, m, rhs, x, z, d);
-  ref_local_solve(t, m, d);
-  ref_edges(d, m, e4);
+  ref_spike(a, t, z, x);
+  ref_residual(a, p, longer, rhs, x, z, d);
+  ref_local_solve(a, t, d);
+  const F4 ed = ref_edges(a, longer, d);
   wave_fence();
-  ex[wave][lane] = F4{e4[0], e4[1], e4[2], e4[3]};
+  ex[wave][lane] = ed;
   wave_fence();
-  ref_neighbours(a, p, edges_of, z);
-  ref_spike(t, m, z, d);
+  ref_neighbours(a, g, p, edges_of, z);
+  ref_spike(a, t, z, d);
 #pragma unroll
   for (int k = 0; k < RCHUNK; ++k) {
     if (act && k < m) {
@@ -774,18 +786,18 @@ __global__ void __launch_bounds__(64 * REF_X_WAVES) __attribute__((amdgpu_waves_
   ref_x_body<KIND>(a, blockIdx.x, in, out);
 }
 template <int KIND, int PRE>
-__global__ void __launch_bounds__(REF_THREADS) k_ref_yz_grp(const RefEntry* __restrict__ g, int M,
+__global__ void __launch_bounds__(REF_THREADS) k_ref_yz_grp(const RefEntry* __restrict__ g, const int* __restrict__ member,
                                                             const float* __restrict__ in, float* __restrict__ out) {
-  const int j = grp_member(g, M, blockIdx.x);
+  const int j = member[blockIdx.x];
   const RefArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
   ref_yz_body<KIND, PRE>(a, (long long)blockIdx.x - b0, in + off, out + off);
 }
 template <int KIND>
-__global__ void __launch_bounds__(64 * REF_X_WAVES) __attribute__((amdgpu_waves_per_eu(2, 8))) k_ref_x_grp(const RefEntry* __restrict__ g, int M,
+__global__ void __launch_bounds__(64 * REF_X_WAVES) __attribute__((amdgpu_waves_per_eu(2, 8))) k_ref_x_grp(const RefEntry* __restrict__ g, const int* __restrict__ member,
                                                                 const float* __restrict__ in,
                                                                 float* __restrict__ out) {
-  const int j = grp_member(g, M, blockIdx.x);
+  const int j = member[blockIdx.x];
   const RefArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
   ref_x_body<KIND>(a, (long long)blockIdx.x - b0, in + off, out + off);
@@ -1126,12 +1138,10 @@ extern PYR_LAUNCH_KIND(float, false)
 #endif
 #undef PYR_LAUNCH_KIND
 
-// lines per workgroup of P chunk threads: as many as fit, at most 64
-static int ref_lines(int P) {
-  int ly = 64;
-  while (ly * P > REF_THREADS) ly /= 2;
-  return ly;
-}
+// lines per workgroup of P chunk threads: as many as fit, at most 64; LDS of
+// the reduced rows
+static int ref_lines(int P) { return std::min(64, REF_THREADS / P); }
+static size_t ref_lds(const RefArgs& a) { return (size_t)a.P * (2 * a.Wg + 1) * 16 * sizeof(float); }
 
 #if PYR_PART == 7
 template <int KIND>
@@ -1140,18 +1150,17 @@ static int launch_ref_kind(hipStream_t stream, int dir, RefArgs a, const float* 
     a.vec = ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0);
     a.lines = 64 / a.P;
     const int per = a.lines * REF_X_WAVES;
-    hipLaunchKernelGGL((k_ref_x<KIND>), dim3((unsigned)((a.nlines + per - 1) / per)), dim3(64 * REF_X_WAVES), 0,
-                       stream, a, in, out);
+    hipLaunchKernelGGL((k_ref_x<KIND>), dim3((unsigned)((a.nlines + per - 1) / per)), dim3(64 * REF_X_WAVES),
+                       ref_lds(a), stream, a, in, out);
   } else {
     a.lines = ref_lines(a.P);
-    while (a.lines > 16 && a.nlines < a.lines * 256) a.lines /= 2;  // small fields: more workgroups
     auto k = k_ref_yz<KIND, PRE_NONE>;
     if constexpr (KIND == K_R4) {
       if (a.addv) k = k_ref_yz<KIND, PRE_V>;
     }
     if (!a.addv && (a.epi == EPI_ADD || a.epi == EPI_MAXABS)) k = k_ref_yz<KIND, PRE_OLD>;
-    hipLaunchKernelGGL(k, dim3((unsigned)((a.nlines + a.lines - 1) / a.lines)), dim3(a.lines * a.P), 0, stream, a, in,
-                       out);
+    hipLaunchKernelGGL(k, dim3((unsigned)((a.nlines + a.lines - 1) / a.lines)), dim3(a.lines * a.P), ref_lds(a),
+                       stream, a, in, out);
   }
   HIPCHECK(hipGetLastError());
   return 0;
@@ -1431,7 +1440,7 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
     if (!a.periodic) put_boundary_rows<false>(a, p, lo, hi, t.x);
     if (SOLVE == SOLVE_NONE) continue;
     t.e[0] = t.e[1] = 0.0;
-    rows_of(p, [&](auto rows) { fwd_pass<false, false>(rows, t.x, t.m, t.e[0], t.e[1]); });
+    rows_of(p, [&](auto rows) { fwd_pass<false>(ChunkRows{a.mb, p < a.mx}, rows, t.x, t.e[0], t.e[1]); });
   }
   bool bad = false;
   if (SOLVE != SOLVE_NONE)
@@ -1441,8 +1450,8 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
       carry(p, std::integral_constant<int, -1>(), e0, e1);
       t.b[0] = t.b[1] = 0.0;
       rows_of(p, [&](auto rows) {
-        fwd_pass<false, true>(rows, t.x, t.m, e0, e1);
-        bwd_exit<false>(rows, t.x, t.m, t.b[0], t.b[1]);
+        fwd_pass<true>(ChunkRows{a.mb, p < a.mx}, rows, t.x, e0, e1);
+        bwd_exit(ChunkRows{a.mb, p < a.mx}, rows, t.x, t.b[0], t.b[1]);
       });
       bad = bad || !std::isfinite(t.b[0]) || !std::isfinite(t.b[1]);
     }
@@ -1460,7 +1469,7 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
     double b0, b1;
     carry(p, std::integral_constant<int, 1>(), b0, b1);
     if (bad) b0 = b1 = std::nan("");
-    rows_of(p, [&](auto rows) { bwd_sink<false>(rows, t.x, t.m, b0, b1, emit); });
+    rows_of(p, [&](auto rows) { bwd_sink(ChunkRows{a.mb, p < a.mx}, rows, t.x, b0, b1, emit); });
   }
 }
 
@@ -1487,24 +1496,24 @@ static void emulate_ref_line(const RefArgs& a, const float* vin, long long strid
       const int row = t.s - R + w;
       t.win[w] = w < t.m + 2 * R && row >= 0 && row < N ? rd(row) : 0.0f;
     }
-    ref_rhs_interior<KIND>(a, t.win, t.rhs, t.m);
+    ref_rhs_interior<KIND>(a, t.win, t.rhs);
     ref_rhs_boundary(a, p, t.rhs, [&](int slot) { return end_value(slot, N, rd); });
     for (int k = 0; k < RCHUNK; ++k) t.x[k] = (float)t.rhs[k];
-    ref_local_solve(t.t, t.m, t.x);
-    ref_edges(t.x, t.m, &Y[p].x);
+    ref_local_solve(a, t.t, t.x);
+    Y[p] = ref_edges(a, p < a.mx, t.x);
   }
   for (int p = 0; p < P; ++p) {
     St& t = st[p];
-    ref_neighbours(a, p, [&](int q) { return Y[q]; }, t.z);
-    ref_spike(t.t, t.m, t.z, t.x);
-    ref_residual(a, p, t.m, t.rhs, t.x, t.z, t.d);
-    ref_local_solve(t.t, t.m, t.d);
-    ref_edges(t.d, t.m, &Yd[p].x);
+    ref_neighbours(a, a.g, p, [&](int q) { return Y[q]; }, t.z);
+    ref_spike(a, t.t, t.z, t.x);
+    ref_residual(a, p, p < a.mx, t.rhs, t.x, t.z, t.d);
+    ref_local_solve(a, t.t, t.d);
+    Yd[p] = ref_edges(a, p < a.mx, t.d);
   }
   for (int p = 0; p < P; ++p) {
     St& t = st[p];
-    ref_neighbours(a, p, [&](int q) { return Yd[q]; }, t.z);
-    ref_spike(t.t, t.m, t.z, t.d);
+    ref_neighbours(a, a.g, p, [&](int q) { return Yd[q]; }, t.z);
+    ref_spike(a, t.t, t.z, t.d);
     for (int k = 0; k < t.m; ++k) {
       double val = ((double)t.x[k] + (double)t.d[k]) * a.scale;
       if (a.addv) val += (double)t.win[k + R];
@@ -1580,7 +1589,7 @@ static int emulate(pyr_ctx* c, int op, int dir, const TS* in, TS* out, bool anti
 struct GrpLaunch {
   void* dev = nullptr;  // GrpEntry or, with refined, RefEntry per member
   bool refined = false;
-  int M = 0;
+  const int* member = nullptr;  // member of each workgroup, after the entries in dev
   long long nblocks = 0;
   dim3 block;
   size_t shm = 0;
@@ -1651,33 +1660,42 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
   GrpLaunch L;
   L.kind = pl0.kind;
   L.solve = sv;
-  L.M = (int)all.size();
   L.x = key.dir == 0;
+  std::vector<int> member;  // of each workgroup
   auto upload = [&](const void* host, size_t bytes) -> int {
-    HIPCHECK(hipMalloc(&L.dev, bytes));
+    std::vector<unsigned char> image(bytes + member.size() * sizeof(int));
+    std::memcpy(image.data(), host, bytes);
+    std::memcpy(image.data() + bytes, member.data(), member.size() * sizeof(int));
+    HIPCHECK(hipMalloc(&L.dev, image.size()));
+    L.member = reinterpret_cast<const int*>(static_cast<unsigned char*>(L.dev) + bytes);
+    L.nblocks = (long long)member.size();
     gp.launches.push_back(L);
-    HIPCHECK(hipMemcpy(L.dev, host, bytes, hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(L.dev, image.data(), image.size(), hipMemcpyHostToDevice));
     return 0;
+  };
+  auto add_blocks = [&](size_t j, int nlines, int per) {
+    const long long blk0 = (long long)member.size();
+    member.insert(member.end(), (size_t)((nlines + per - 1) / per), (int)j);
+    return blk0;
   };
   const int pre = all[0].a.addv ? PRE_V : ((key.epi == EPI_ADD || key.epi == EPI_MAXABS) ? PRE_OLD : PRE_NONE);
   if (key.refined && sv == SOLVE_BND) {
     std::vector<RefEntry> ref(all.size());
-    long long blk = 0;
+    size_t lds = 0;
     for (size_t j = 0; j < all.size(); ++j) {
       pyr_ctx* c = g->mem[ms[j]];
       RefArgs& a = ref[j].a;
       a = make_ref_args(all[j].a, c->rplan[key.op][key.dir], c->drplan[key.op][key.dir]);
       a.vec = key.aligned && ((all[j].off * (long long)sizeof(float)) % 16 == 0);
       a.lines = L.x ? 64 / a.P : ref_lines(a.P);
-      const int per = L.x ? a.lines * REF_X_WAVES : a.lines;
       ref[j].off = all[j].off;
-      ref[j].blk0 = blk;
-      blk += (a.nlines + per - 1) / per;
+      ref[j].blk0 = add_blocks(j, a.nlines, L.x ? a.lines * REF_X_WAVES : a.lines);
+      lds = std::max(lds, ref_lds(a));
     }
+    L.shm = lds;
     L.refined = true;
     L.pre = pre;
     L.block = dim3(L.x ? 64 * REF_X_WAVES : REF_THREADS);
-    L.nblocks = blk;
     return upload(ref.data(), ref.size() * sizeof(RefEntry));
   }
   int nthr = 64, ntab = 0;
@@ -1695,8 +1713,8 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
     L.pre = pre;
   }
   L.block = dim3(nthr);
-  long long blk = 0;
-  for (auto& e : all) {
+  for (size_t j = 0; j < all.size(); ++j) {
+    GrpEntry& e = all[j];
     if (L.x) {
       e.a.vec = key.aligned && ((e.off * (long long)sizeof(TS)) % 16 == 0);
       e.a.lines = 64 / e.a.P;
@@ -1704,11 +1722,8 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
       e.a.lines = 128;
       while (e.a.lines * e.a.P > nthr) e.a.lines /= 2;
     }
-    const int per = L.x ? e.a.lines * (nthr / 64) : e.a.lines;
-    e.blk0 = blk;
-    blk += (e.a.nlines + per - 1) / per;
+    e.blk0 = add_blocks(j, e.a.nlines, L.x ? e.a.lines * (nthr / 64) : e.a.lines);
   }
-  L.nblocks = blk;
   return upload(all.data(), all.size() * sizeof(GrpEntry));
 }
 
@@ -1727,7 +1742,7 @@ static int grp_launch_typed(pyr_group* g, const GrpLaunch& L, const TS* in, TS* 
   } else if (L.pre == PRE_OLD) {
     k = k_line_yz_grp<TS, KIND, SOLVE, PRE_OLD>;
   }
-  hipLaunchKernelGGL(k, grid, L.block, L.shm, g->stream, (const GrpEntry*)L.dev, L.M, in, out);
+  hipLaunchKernelGGL(k, grid, L.block, L.shm, g->stream, (const GrpEntry*)L.dev, L.member, in, out);
   HIPCHECK(hipGetLastError());
   return 0;
 }
@@ -1761,7 +1776,7 @@ static int grp_launch_ref_kind(hipStream_t stream, const GrpLaunch& L, const flo
   } else if (L.pre == PRE_OLD) {
     k = k_ref_yz_grp<KIND, PRE_OLD>;
   }
-  hipLaunchKernelGGL(k, dim3((unsigned)L.nblocks), L.block, 0, stream, (const RefEntry*)L.dev, L.M, in, out);
+  hipLaunchKernelGGL(k, dim3((unsigned)L.nblocks), L.block, L.shm, stream, (const RefEntry*)L.dev, L.member, in, out);
   HIPCHECK(hipGetLastError());
   return 0;
 }

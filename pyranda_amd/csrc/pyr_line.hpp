@@ -199,14 +199,31 @@ struct TableRows {
   PYR_HD double diag(int k, double x) const { return x * t.tg[k * T + slot]; }
 };
 
+// Which rows a chunk has: mb of them, the same in every chunk of the line (so
+// the test is wave-uniform), and one more where `longer`. Every chunk has at
+// least 2*NB rows.
+struct ChunkRows {
+  int mb;
+  bool longer;
+  template <typename F>
+  PYR_HD void row(int k, F f) const {
+    if (k < 2 * NB || k < mb) f();
+    else if (k == mb && longer) f();
+  }
+};
+struct AllRows {
+  template <typename F>
+  PYR_HD void row(int, F f) const { f(); }
+};
+
 // Forward recurrence entered with (x_{-2}, x_{-1}) = (e0, e1), which becomes
 // the exit state; STORE keeps the rows. The older state is subtracted first,
 // so one FMA per row is on the dependent chain.
-template <bool FULL, bool STORE, typename Rows>
-PYR_HD void fwd_pass(const Rows& rows, double* x, int m, double& e0, double& e1) {
+template <bool STORE, typename Have, typename Rows>
+PYR_HD void fwd_pass(const Have& have, const Rows& rows, double* x, double& e0, double& e1) {
 #pragma unroll
   for (int k = 0; k < CHUNK; ++k) {
-    if (FULL || k < m) {
+    have.row(k, [&] {
       double c1, c2;
       rows.fence(k);
       rows.fwd(k, c1, c2);
@@ -215,17 +232,17 @@ PYR_HD void fwd_pass(const Rows& rows, double* x, int m, double& e0, double& e1)
       if (STORE) x[k] = v;
       e0 = e1;
       e1 = v;
-    }
+    });
   }
 }
 
 // Diagonal and exit state of the backward recurrence entered with zeros; the
 // rows are scaled by the diagonal in place.
-template <bool FULL, typename Rows>
-PYR_HD void bwd_exit(const Rows& rows, double* x, int m, double& b1, double& b2) {
+template <typename Have, typename Rows>
+PYR_HD void bwd_exit(const Have& have, const Rows& rows, double* x, double& b1, double& b2) {
 #pragma unroll
   for (int k = CHUNK - 1; k >= 0; --k) {
-    if (FULL || k < m) {
+    have.row(k, [&] {
       double c1, c2;
       rows.fence(k);
       rows.bwd(k, c1, c2);
@@ -234,17 +251,17 @@ PYR_HD void bwd_exit(const Rows& rows, double* x, int m, double& b1, double& b2)
       const double v = t - c1 * b1;
       b2 = b1;
       b1 = v;
-    }
+    });
   }
 }
 
 // Backward recurrence entered with (y_m, y_{m+1}) = (b1, b2); row k goes to
 // sink(k, y_k).
-template <bool FULL, typename Rows, typename Sink>
-PYR_HD void bwd_sink(const Rows& rows, const double* x, int m, double b1, double b2, Sink sink) {
+template <typename Have, typename Rows, typename Sink>
+PYR_HD void bwd_sink(const Have& have, const Rows& rows, const double* x, double b1, double b2, Sink sink) {
 #pragma unroll
   for (int k = CHUNK - 1; k >= 0; --k) {
-    if (FULL || k < m) {
+    have.row(k, [&] {
       double c1, c2;
       rows.fence(k);
       rows.bwd(k, c1, c2);
@@ -253,7 +270,7 @@ PYR_HD void bwd_sink(const Rows& rows, const double* x, int m, double b1, double
       b2 = b1;
       b1 = v;
       sink(k, v);
-    }
+    });
   }
 }
 

@@ -26,7 +26,7 @@ constexpr int RCHUNK = 32;  // rows per thread
 constexpr int MAXT = 10;    // terms per boundary row
 constexpr int ENDS = 16;    // rows the terms name: slot i < 8 is row i, i < 16 row N - 16 + i, 16 reads 0
 constexpr int NCLS = 4;     // first, interior (mb + 1 rows), interior (mb), last
-constexpr int CROW = 12;    // floats per table row: 5 of the factors, 4 spikes, padding
+constexpr int CROW = 12;    // floats per table row: 4 spikes | 1/u, u1, u2, 0 | l2, l1, 0, 0
 
 struct RefPlan {
   int N = 0, P = 0, mb = 0, mx = 0;
@@ -35,7 +35,8 @@ struct RefPlan {
   double w[9] = {};         // interior weights at offsets -R..R
   double bd[5] = {};        // interior row of the left-hand side
   std::vector<float> cls;   // NCLS x RCHUNK x CROW
-  std::vector<float> g;     // P x 4P x 4: reduced-system rows of the four neighbour values
+  std::vector<float> g;     // P x (2 Wg + 1) x 4 x 4: reduced-system rows of the four neighbour values,
+                            // for the chunks within reach (0 beyond the line's ends)
   std::vector<double> be;   // 2*NB x 5: left-hand rows at the ends
   std::vector<double> bcoef;  // 2*NB x MAXT terms coef * (v[a] - v[b])
   std::vector<int> bidx;      // 2*NB x MAXT x 2: slots of a and b among the line's end rows
@@ -260,7 +261,8 @@ inline RefPlan build_ref_plan(int op, int n, int v1, int v2, double metric) {
                            (double)(1.0L / blk[size_t(i) * m + i]),
                            (i + 1 < m) ? (double)blk[size_t(i) * m + i + 1] : 0.0,
                            (i + 2 < m) ? (double)blk[size_t(i) * m + i + 2] : 0.0};
-      for (int q = 0; q < 5; ++q) tab[i * CROW + q] = (float)c[q];
+      const int at[5] = {8, 9, 4, 5, 6};
+      for (int q = 0; q < 5; ++q) tab[i * CROW + at[q]] = (float)c[q];
     }
     // solve with the long-double factors for the spike columns
     auto solve = [&](std::vector<ld>& r) {
@@ -294,7 +296,7 @@ inline RefPlan build_ref_plan(int op, int n, int v1, int v2, double metric) {
       r2[i] = a_e2_e * wm2[i] + a_e1_e * wm1[i];
       r3[i] = a_e1_e1 * wm1[i];
       const ld r[4] = {r0[i], r1[i], r2[i], r3[i]};
-      for (int q = 0; q < 4; ++q) tab[i * CROW + 5 + q] = (float)(double)r[q];
+      for (int q = 0; q < 4; ++q) tab[i * CROW + q] = (float)(double)r[q];
     }
     float* have_tab = &pl.cls[cl * RCHUNK * CROW];
     if (!have[cl]) std::memcpy(have_tab, tab.data(), tab.size() * sizeof(float));
@@ -318,18 +320,24 @@ inline RefPlan build_ref_plan(int op, int n, int v1, int v2, double metric) {
     }
   }
   detail::invert(S, 4 * P);
-  pl.g.assign((size_t)P * 4 * P * 4, 0.0f);
-  for (int p = 0; p < P; ++p) {
-    const int pm = p - 1, pp = p + 1;
-    const int rows[4] = {4 * pm + 2, 4 * pm + 3, 4 * pp + 0, 4 * pp + 1};
-    const bool use[4] = {p > 0, p > 0, p < P - 1, p < P - 1};
+  auto row_of = [&](int p, int q, int c) -> double {
+    const int rows[4] = {4 * (p - 1) + 2, 4 * (p - 1) + 3, 4 * (p + 1) + 0, 4 * (p + 1) + 1};
+    if (q < 2 ? p == 0 : p == P - 1) return 0.0;
+    return (double)S[size_t(rows[q]) * 4 * P + c];
+  };
+  for (int p = 0; p < P; ++p)
     for (int c = 0; c < 4 * P; ++c)
-      for (int q = 0; q < 4; ++q) {
-        const double v = use[q] ? (double)S[size_t(rows[q]) * 4 * P + c] : 0.0;
-        pl.g[((size_t)p * 4 * P + c) * 4 + q] = (float)v;
-        if (std::fabs(v) > 1e-17) pl.Wg = std::max(pl.Wg, std::abs(c / 4 - p));
-      }
-  }
+      for (int q = 0; q < 4; ++q)
+        if (std::fabs(row_of(p, q, c)) > 1e-17) pl.Wg = std::max(pl.Wg, std::abs(c / 4 - p));
+  const int K = 2 * pl.Wg + 1;
+  pl.g.assign((size_t)P * K * 16, 0.0f);
+  for (int p = 0; p < P; ++p)
+    for (int j = 0; j < K; ++j) {
+      const int qc = p - pl.Wg + j;
+      if (qc < 0 || qc >= P) continue;
+      for (int i = 0; i < 4; ++i)
+        for (int q = 0; q < 4; ++q) pl.g[(((size_t)p * K + j) * 4 + i) * 4 + q] = (float)row_of(p, q, 4 * qc + i);
+    }
   return pl;
 }
 
@@ -349,29 +357,43 @@ struct RefArgs {
   const int* bidx;
 };
 
+// A chunk has mb or mb + 1 rows, mb the same in all chunks of a line, so a
+// group of four rows is skipped or taken as a whole by a wave-uniform test and
+// nothing else depends on the row count: past a chunk's end the tables hold
+// zeros, which make the rows there 0 and leave the others alone.
+constexpr int RGROUP = 4;
+
 // --- right-hand side ------------------------------------------------------
-// win[w] holds v[s - R + w]; rows k >= m get 0.
+// win[w] holds v[s - R + w]; rows of skipped groups get 0.
 template <int KIND, typename TW>
-PYR_HD void ref_rhs_interior(const RefArgs& a, const TW* win, double* rhs, int m) {
+PYR_HD void ref_rhs_interior(const RefArgs& a, const TW* win, double* rhs) {
   constexpr int R = Halo<KIND>::R;
 #pragma unroll
-  for (int k = 0; k < RCHUNK; ++k) {
-    double acc;
-    if (KIND == K_D1) {
-      // antisymmetric pairs (compact_d1.f90:156)
-      acc = a.w[4] * ((double)win[k + R + 1] - (double)win[k + R - 1]) +
-            a.w[5] * ((double)win[k + R + 2] - (double)win[k + R - 2]) +
-            a.w[6] * ((double)win[k + R + 3] - (double)win[k + R - 3]);
-    } else {
-      // difference form sum_l w_l (v_{i+l} - v_i) (compact_r3.f90:124-132,
-      // compact_r4.f90:144-156)
-      const double vc = (double)win[k + R];
-      acc = 0.0;
+  for (int g = 0; g < RCHUNK; g += RGROUP) {
+    if (g <= a.mb) {
 #pragma unroll
-      for (int l = -R; l <= R; ++l)
-        if (l != 0) acc += ((double)win[k + R + l] - vc) * a.w[l + R];
+      for (int k = g; k < g + RGROUP; ++k) {
+        double acc;
+        if (KIND == K_D1) {
+          // antisymmetric pairs (compact_d1.f90:156)
+          acc = a.w[4] * ((double)win[k + R + 1] - (double)win[k + R - 1]) +
+                a.w[5] * ((double)win[k + R + 2] - (double)win[k + R - 2]) +
+                a.w[6] * ((double)win[k + R + 3] - (double)win[k + R - 3]);
+        } else {
+          // difference form sum_l w_l (v_{i+l} - v_i) (compact_r3.f90:124-132,
+          // compact_r4.f90:144-156)
+          const double vc = (double)win[k + R];
+          acc = 0.0;
+#pragma unroll
+          for (int l = -R; l <= R; ++l)
+            if (l != 0) acc += ((double)win[k + R + l] - vc) * a.w[l + R];
+        }
+        rhs[k] = acc;
+      }
+    } else {
+#pragma unroll
+      for (int k = g; k < g + RGROUP; ++k) rhs[k] = 0.0;
     }
-    rhs[k] = (k < m) ? acc : 0.0;
   }
 }
 
@@ -399,6 +421,9 @@ PYR_HD float end_value(int slot, int N, Row row) {
   return slot < ENDS ? v : 0.0f;
 }
 
+struct alignas(16) F4 { float x, y, z, w; };
+struct alignas(8) F2 { float x, y; };
+
 // Replace the rows of the line's ends by their own right-hand sides.
 template <typename Reader>
 PYR_HD void ref_rhs_boundary(const RefArgs& a, int p, double* rhs, Reader rd) {
@@ -416,118 +441,138 @@ PYR_HD void ref_rhs_boundary(const RefArgs& a, int p, double* rhs, Reader rd) {
       PYR_ROW_FENCE(j, 1);
       g[j] = ref_boundary_row(a, NB + j, rd);
     }
+    const double g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3];
 #pragma unroll
     for (int k = NB; k < RCHUNK; ++k) {
       const int j = k - (a.mb - NB);  // the last chunk has mb rows in every line
-      if (j >= 0 && j < NB) rhs[k] = (j == 0) ? g[0] : (j == 1) ? g[1] : (j == 2) ? g[2] : g[3];
+      if (j >= 0 && j < NB) rhs[k] = (j == 0) ? g0 : (j == 1) ? g1 : (j == 2) ? g2 : g3;
     }
   }
 }
 
 // --- chunk solve ------------------------------------------------------------
 // t: the table of this chunk's class
-PYR_HD void ref_local_solve(const float* t, int m, float* x) {
+PYR_HD void ref_local_solve(const RefArgs& a, const float* t, float* x) {
 #pragma unroll
-  for (int k = 0; k < RCHUNK; ++k) {
-    if (k < m) {
-      PYR_ROW_FENCE(k, 4);
-      const float* c = t + k * CROW;
-      float v = x[k];
-      if (k >= 1) v -= c[1] * x[k - 1];
-      if (k >= 2) v -= c[0] * x[k - 2];
-      x[k] = v;
+  for (int g = 0; g < RCHUNK; g += RGROUP) {
+    if (g <= a.mb) {
+      PYR_ROW_FENCE(g, RGROUP);
+#pragma unroll
+      for (int k = g; k < g + RGROUP; ++k) {
+        const F2 l = *reinterpret_cast<const F2*>(t + k * CROW + 8);
+        float v = x[k];
+        if (k >= 1) v -= l.y * x[k - 1];
+        if (k >= 2) v -= l.x * x[k - 2];
+        x[k] = v;
+      }
     }
   }
 #pragma unroll
-  for (int k = RCHUNK - 1; k >= 0; --k) {
-    if (k < m) {
-      PYR_ROW_FENCE(k, 4);
-      const float* c = t + k * CROW;
-      float v = x[k];
-      if (k + 1 < RCHUNK) v -= c[3] * x[k + 1];
-      if (k + 2 < RCHUNK) v -= c[4] * x[k + 2];
-      x[k] = v * c[2];
+  for (int g = RCHUNK - RGROUP; g >= 0; g -= RGROUP) {
+    if (g <= a.mb) {
+      PYR_ROW_FENCE(g, RGROUP);
+#pragma unroll
+      for (int k = g + RGROUP - 1; k >= g; --k) {
+        const F4 u = *reinterpret_cast<const F4*>(t + k * CROW + 4);
+        float v = x[k];
+        if (k + 1 < RCHUNK) v -= u.y * x[k + 1];
+        if (k + 2 < RCHUNK) v -= u.z * x[k + 2];
+        x[k] = v * u.x;
+      }
     }
   }
 }
 
-PYR_HD void ref_edges(const float* x, int m, float* e4) {
-  e4[0] = x[0];
-  e4[1] = x[1];
-  float a = 0, b = 0;
+// The chunk's first two and last two values (longer: it has mb + 1 rows).
+PYR_HD F4 ref_edges(const RefArgs& a, bool longer, const float* x) {
+  float l0 = 0, l1 = 0, l2 = 0;  // rows mb - 2, mb - 1, mb
 #pragma unroll
-  for (int k = 2; k < RCHUNK; ++k) {
-    if (k == m - 2) a = x[k];
-    if (k == m - 1) b = x[k];
+  for (int k = 2 * NB - 2; k < RCHUNK; ++k) {
+    if (k == a.mb - 2) l0 = x[k];
+    if (k == a.mb - 1) l1 = x[k];
+    if (k == a.mb) l2 = x[k];
   }
-  e4[2] = a;
-  e4[3] = b;
+  return F4{x[0], x[1], longer ? l1 : l0, longer ? l2 : l1};
 }
 
-struct alignas(16) F4 { float x, y, z, w; };
-
-// z = the four values next to chunk p: rows of the reduced inverse times the
+// z = the four values next to chunk p: rows g of the reduced inverse times the
 // edge values of the chunks within reach; yr(q) returns those of chunk q
 template <typename YR>
-PYR_HD void ref_neighbours(const RefArgs& a, int p, YR yr, float* z) {
-  const F4* g = reinterpret_cast<const F4*>(a.g) + (size_t)p * 4 * a.P;
+PYR_HD void ref_neighbours(const RefArgs& a, const float* g, int p, YR yr, float* z) {
+  const int K = 2 * a.Wg + 1;
+  const F4* c = reinterpret_cast<const F4*>(g) + (size_t)p * K * 4;
   float z0 = 0, z1 = 0, z2 = 0, z3 = 0;
-  const int q1 = p + a.Wg < a.P - 1 ? p + a.Wg : a.P - 1;
-  for (int q = p > a.Wg ? p - a.Wg : 0; q <= q1; ++q) {
-    const F4 e = yr(q);
+#pragma unroll 3
+  for (int j = 0; j < K; ++j) {
+    const int q = p - a.Wg + j;
+    const F4 e = yr(q < 0 ? 0 : (q >= a.P ? a.P - 1 : q));
     const float y[4] = {e.x, e.y, e.z, e.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const F4 c = g[4 * q + i];
-      z0 += c.x * y[i];
-      z1 += c.y * y[i];
-      z2 += c.z * y[i];
-      z3 += c.w * y[i];
+      const F4 r = c[4 * j + i];
+      z0 += r.x * y[i];
+      z1 += r.y * y[i];
+      z2 += r.z * y[i];
+      z3 += r.w * y[i];
     }
   }
   z[0] = z0; z[1] = z1; z[2] = z2; z[3] = z3;
 }
 
-PYR_HD void ref_spike(const float* t, int m, const float* z, float* x) {
+PYR_HD void ref_spike(const RefArgs& a, const float* t, const float* z, float* x) {
 #pragma unroll
-  for (int k = 0; k < RCHUNK; ++k) {
-    if (k < m) {
-      PYR_ROW_FENCE(k, 4);
-      const float* r = t + k * CROW + 5;
-      x[k] -= r[0] * z[0] + r[1] * z[1] + r[2] * z[2] + r[3] * z[3];
+  for (int g = 0; g < RCHUNK; g += RGROUP) {
+    if (g <= a.mb) {
+      PYR_ROW_FENCE(g, RGROUP);
+#pragma unroll
+      for (int k = g; k < g + RGROUP; ++k) {
+        const F4 r = *reinterpret_cast<const F4*>(t + k * CROW);
+        x[k] -= r.x * z[0] + r.y * z[1] + r.z * z[2] + r.w * z[3];
+      }
     }
   }
 }
 
-// FP64 residual r = rhs - A y of row k of the chunk; y outside the chunk comes
-// from z = (y[s-2], y[s-1], y[e], y[e+1]); b: the row's five band entries.
-PYR_HD double ref_residual_row(const double* b, int k, int m, double rhs, const float* y, const float* z) {
-  double yy[5];
+// d = the FP32 rounding of the FP64 residual rhs - A y of every row, with
+// z = (y[s-2], y[s-1], y[e], y[e+1]) the values of y outside the chunk. What
+// lands past the chunk's end is finite and the solve that follows drops it.
+PYR_HD void ref_residual(const RefArgs& a, int p, bool longer, const double* rhs, const float* y, const float* z,
+                         float* d) {
+  // rows m and m + 1 of y are the next chunk's
+  const float z0 = z[0], z1 = z[1], z2 = z[2], z3 = z[3];
+  const float n1 = longer ? z2 : z3;  // row mb + 1
+  float ye[RCHUNK + 2];
 #pragma unroll
-  for (int o = -2; o <= 2; ++o) {
-    const int kk = k + o;
-    double v;
-    if (kk < 0) v = (kk == -2) ? (double)z[0] : (double)z[1];
-    else if (kk < RCHUNK) v = (kk < m) ? (double)y[kk] : ((kk == m) ? (double)z[2] : (double)z[3]);
-    else v = (kk == m) ? (double)z[2] : (double)z[3];
-    yy[o + 2] = v;
+  for (int k = 0; k < RCHUNK + 2; ++k) {
+    const float v = k < RCHUNK ? y[k] : 0.0f;
+    const float v0 = longer ? v : z2, v2 = longer ? z3 : v;
+    ye[k] = k == a.mb ? v0 : (k == a.mb + 1 ? n1 : (k == a.mb + 2 ? v2 : v));
   }
-  return rhs - (b[0] * yy[0] + b[1] * yy[1] + b[2] * yy[2] + b[3] * yy[3] + b[4] * yy[4]);
-}
-
-// d = the FP32 rounding of the residual of every row (0 past the chunk's end)
-PYR_HD void ref_residual(const RefArgs& a, int p, int m, const double* rhs, const float* y, const float* z, float* d) {
+  auto row = [&](const double* b, int k) {
+    const double y0 = k >= 2 ? (double)ye[k >= 2 ? k - 2 : 0] : (k == 0 ? (double)z0 : (double)z1);
+    const double y1 = k >= 1 ? (double)ye[k >= 1 ? k - 1 : 0] : (double)z1;
+    return (float)(rhs[k] - (b[0] * y0 + b[1] * y1 + b[2] * (double)ye[k] + b[3] * (double)ye[k + 1] +
+                             b[4] * (double)ye[k + 2]));
+  };
 #pragma unroll
-  for (int k = 0; k < RCHUNK; ++k) d[k] = k < m ? (float)ref_residual_row(a.bd, k, m, rhs[k], y, z) : 0.0f;
+  for (int g = 0; g < RCHUNK; g += RGROUP) {
+    if (g <= a.mb) {
+#pragma unroll
+      for (int k = g; k < g + RGROUP; ++k) d[k] = row(a.bd, k);
+    } else {
+#pragma unroll
+      for (int k = g; k < g + RGROUP; ++k) d[k] = 0.0f;
+    }
+  }
   if (p == 0) {
 #pragma unroll
-    for (int k = 0; k < NB; ++k) d[k] = (float)ref_residual_row(a.be + 5 * k, k, m, rhs[k], y, z);
+    for (int k = 0; k < NB; ++k) d[k] = row(a.be + 5 * k, k);
   }
   if (p == a.P - 1) {
 #pragma unroll
     for (int k = NB; k < RCHUNK; ++k) {
       const int j = k - (a.mb - NB);
-      if (j >= 0 && j < NB) d[k] = (float)ref_residual_row(a.be + 5 * (NB + j), k, m, rhs[k], y, z);
+      if (j >= 0 && j < NB) d[k] = row(a.be + 5 * (NB + j), k);
     }
   }
 }
