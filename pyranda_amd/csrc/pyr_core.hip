@@ -178,8 +178,15 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
   extern __shared__ __align__(16) unsigned char smem[];
   const int LY = a.lines;
   const int lane = threadIdx.x & (LY - 1);
-  const int p = (int)threadIdx.x >> __builtin_ctz(LY);
-  const bool act = !GRP || p < a.P;
+  int p = (int)threadIdx.x >> __builtin_ctz(LY);
+  if constexpr (SOLVE == SOLVE_NONE) {
+    // chunks of the explicit filter are independent: a workgroup takes some of
+    // a line group's chunks
+    const int per = (int)blockDim.x >> __builtin_ctz(LY), groups = (a.P + per - 1) / per;
+    p += (int)(blk % groups) * per;
+    blk /= groups;
+  }
+  const bool act = (!GRP && SOLVE != SOLVE_NONE) || p < a.P;
   const long long L = blk * LY + lane;
   const bool valid = act && L < a.nlines;
   const long long Lc = L < a.nlines ? L : (long long)a.nlines - 1;
@@ -318,27 +325,46 @@ __device__ __forceinline__ void wave_fence() {
 // Moves the lines of one wave between HBM and its LDS tile. `end` elements
 // from src on (element 0 is the first of the 16-byte vector that holds the
 // lines' first element, `sh` the offset of that element in it); CH rows per
-// chunk, at most 64 chunks. PAD: one extra vector after every CH elements of
-// the tile (lines of whole chunks), which spreads the lanes' window reads over
-// the banks; other lines sit in the tile as in memory.
-template <typename TS, int CH, bool PAD>
+// chunk, at most 64 chunks. One extra vector after every CH elements of the
+// tile spreads the lanes' reads, a chunk apart, over the banks (without it 16
+// lanes share one bank; gbar on 1000-point FP32 lines 53 -> 41 us). Elements
+// from -CH on may be addressed and, past the lines, 2 CH more: a window can be
+// read whole where part of it is not used.
+template <typename TS, int CH>
 struct XTile {
   using V = typename Vec16<TS>::type;
   static constexpr int VW = Vec16<TS>::W;
-  static constexpr int CP = PAD ? CH + VW : CH;              // tile elements per chunk
-  static constexpr int SIZE = 64 * CP + (PAD ? 0 : 2 * VW);
-  static constexpr int NV = CH / VW + (PAD ? 0 : 1);          // vectors per lane
-  static __device__ __forceinline__ int at(int i) { return PAD ? i + i / CH * VW : i; }
+  static constexpr int CP = CH + VW;                 // tile elements per chunk
+  static constexpr int ORIGIN = CP;
+  static constexpr int SIZE = 64 * CP + 4 * CP;
+  static __device__ __forceinline__ int at(int i) { return i + (i >= 0 ? i / CH : -1) * VW; }
+
+  // Positions of elements i0, i0 + 1, ... for compile-time steps w < 2 CH: a
+  // run of CH elements crosses one boundary, which a comparison finds.
+  struct Run {
+    int b0, f;
+    __device__ __forceinline__ explicit Run(int i0) {
+      const int c = i0 >= 0 ? i0 / CH : -1;
+      b0 = i0 + c * VW;
+      f = i0 - c * CH;
+    }
+    __device__ __forceinline__ int operator()(int w) const {
+      return b0 + w + (f >= CH - w ? VW : 0) + (w > CH && f >= 2 * CH - w ? VW : 0);
+    }
+  };
 
   // avail: elements from src to the end of the field
+  // WHOLE: the lines are whole vectors from an aligned start, CH elements a lane
+  template <bool WHOLE>
   static __device__ __forceinline__ void load(TS* tile, const TS* src, int end, long long avail, int vec, int lane) {
+    constexpr int NV = CH / VW + (WHOLE ? 0 : 1);  // vectors per lane
     if (!vec) {
       for (int e = lane; e < end; e += 64) tile[at(e)] = src[e];
       return;
     }
     // whole vectors that lie inside the field, then the rest one by one
     int nv = (end + VW - 1) / VW;
-    if (!PAD && (long long)nv * VW > avail) --nv;
+    if (!WHOLE && (long long)nv * VW > avail) --nv;
     V t[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
@@ -350,13 +376,15 @@ struct XTile {
       const int e = lane + 64 * j;
       if (e < nv) *reinterpret_cast<V*>(tile + at(e * VW)) = t[j];
     }
-    if (!PAD && nv * VW + lane < end) tile[nv * VW + lane] = src[nv * VW + lane];
+    if (!WHOLE && nv * VW + lane < end) tile[at(nv * VW + lane)] = src[nv * VW + lane];
   }
 
   // the results, with the epilogue; dst as src, o32 (if not null) the FP32
   // copy of FP64 results, only32 instead of them
+  template <bool WHOLE>
   static __device__ __forceinline__ void store(const TS* tile, TS* dst, int sh, int end, int vec, int lane, int epi,
                                                double epi_c, float* o32, int only32) {
+    constexpr int NV = CH / VW + (WHOLE ? 0 : 1);
     const bool need_old = epi == EPI_ADD || epi == EPI_MAXABS;
     auto put = [&](int e) {
       TS r = tile[at(e)];
@@ -389,7 +417,7 @@ struct XTile {
         }
       }
     }
-    if constexpr (!PAD) {
+    if constexpr (!WHOLE) {
       if (lane >= sh && lane < v0 * VW && lane < end) put(lane);
       const int tail = v1 * VW + lane;
       if (lane < VW && tail >= v0 * VW && tail < end) put(tail);
@@ -419,7 +447,7 @@ template <typename TS, int KIND, int SOLVE, bool FULL, bool GRP = false>
 __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, const TS* __restrict__ in,
                                             TS* __restrict__ out) {
   constexpr int R = Halo<KIND>::R;
-  using T = XTile<TS, CHUNK, FULL>;
+  using T = XTile<TS, CHUNK>;
   constexpr int CP = T::CP;
   constexpr int NW = XWaves<SOLVE>::v;
   __shared__ __align__(16) TS tiles[NW][T::SIZE];
@@ -435,7 +463,7 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   const int N = a.N, P = a.P;
   const int lane = threadIdx.x & 63;
   const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  TS* tile = tiles[wave];
+  TS* tile = tiles[wave] + T::ORIGIN;
   [[maybe_unused]] D2* ex = exits[wave];
   const long long L0 = (blk * NW + wave) * a.lines;
   const long long rem = (long long)a.nlines - L0;
@@ -444,7 +472,7 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   const long long E0 = L0 * N;
   const int sh = (!FULL && a.vec) ? (int)(E0 & (T::VW - 1)) : 0;
   const int end = sh + nval * N;
-  T::load(tile, in + (E0 - sh), end, (long long)a.nlines * N - (E0 - sh), a.vec, lane);
+  T::template load<FULL>(tile, in + (E0 - sh), end, (long long)a.nlines * N - (E0 - sh), a.vec, lane);
   wave_fence();
   const int l = lane / P, p = lane - l * P;
   const bool act = l < nval;
@@ -453,16 +481,18 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   const auto have = rows_of_chunk<FULL>(a, p);
   const bool last = p == P - 1;
   const bool wrap = SOLVE == SOLVE_CIRC || (SOLVE == SOLVE_NONE && a.periodic);
-  TS* row0 = tile + (act ? (FULL ? l * P * CP : sh + l * N) : (FULL ? 0 : sh));
-  TS* mo = row0 + (FULL ? p * CP : s);
+  const int i0 = sh + (act ? l : 0) * N;  // the line's first element in the tile
+  const typename T::Run run(i0 + s - R);
+  auto own = [&](int k) -> TS& { return tile[FULL ? (i0 / CHUNK + p) * CP + k : run(k + R)]; };
   TS win[CHUNK + 2 * R];
   if constexpr (FULL) {
+    const TS* row0 = tile + i0 / CHUNK * CP;
     const TS* lo = row0 + (p == 0 ? P - 1 : p - 1) * CP;
     const TS* hi = row0 + (last ? 0 : p + 1) * CP;
 #pragma unroll
     for (int w = 0; w < CHUNK + 2 * R; ++w) {
       if (w < R) win[w] = lo[CHUNK - R + w];
-      else if (w < CHUNK + R) win[w] = mo[w - R];
+      else if (w < CHUNK + R) win[w] = own(w - R);
       else win[w] = hi[w - CHUNK - R];
     }
     if (!wrap) {
@@ -473,16 +503,21 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
       }
     }
   } else {
+    // the rows as they lie in the tile, then the halos beyond the line's ends
+    // (the last chunk has mb rows); what is read past a chunk's own halo is
+    // not used
 #pragma unroll
-    for (int w = 0; w < CHUNK + 2 * R; ++w) {
-      int row = s - R + w;
-      bool ok = w < m + 2 * R;
-      if (row < 0 || row >= N) {
-        ok = ok && wrap;
-        row = row < 0 ? row + N : row - N;
+    for (int w = 0; w < CHUNK + 2 * R; ++w) win[w] = tile[run(w)];
+    if (p == 0) {
+#pragma unroll
+      for (int w = 0; w < R; ++w) win[w] = wrap ? tile[T::at(i0 + N - R + w)] : (TS)0;
+    }
+    if (last) {
+#pragma unroll
+      for (int w = 2 * NB + R; w < CHUNK + 2 * R; ++w) {
+        const int j = w - R - a.mb;
+        if (j >= 0 && j < R) win[w] = wrap ? tile[T::at(i0 + j)] : (TS)0;
       }
-      const TS v = row0[ok ? row : 0];
-      win[w] = ok ? v : (TS)0;
     }
   }
   double x[CHUNK];
@@ -494,8 +529,9 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   auto emit = [&](int k, double y) {
     if (act) {
       double val = y * a.scale;
-      if (a.addv) val += (double)mo[k];
-      mo[k] = (TS)val;
+      TS& o = own(k);
+      if (a.addv) val += (double)o;
+      o = (TS)val;
     }
   };
   if constexpr (SOLVE == SOLVE_NONE) {
@@ -527,7 +563,7 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   wave_fence();
   float* o32 = nullptr;
   if constexpr (sizeof(TS) == 8 && !GRP) o32 = a.out32 ? a.out32 + (E0 - sh) : nullptr;
-  T::store(tile, out + (E0 - sh), sh, end, a.vec, lane, a.epi, a.epi_c, o32, GRP ? 0 : a.only32);
+  T::template store<FULL>(tile, out + (E0 - sh), sh, end, a.vec, lane, a.epi, a.epi_c, o32, GRP ? 0 : a.only32);
 }
 
 template <typename TS, int KIND, int SOLVE, bool FULL>
@@ -698,7 +734,7 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
                                            float* __restrict__ out) {
   constexpr int R = Halo<KIND>::R;
   constexpr int NW = REF_X_WAVES;
-  using T = XTile<float, RCHUNK, false>;
+  using T = XTile<float, RCHUNK>;
   __shared__ __align__(16) float tab[NCLS * RCHUNK * CROW];
   __shared__ __align__(16) float tiles[NW][T::SIZE];
   __shared__ __align__(16) F4 ex[NW][64];
@@ -708,7 +744,7 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  float* tile = tiles[wave];
+  float* tile = tiles[wave] + T::ORIGIN;
   const int N = a.N, P = a.P;
   const long long L0 = (blk * NW + wave) * a.lines;
   const long long rem = (long long)a.nlines - L0;
@@ -717,24 +753,30 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
   const long long E0 = L0 * N;
   const int sh = a.vec ? (int)(E0 & (T::VW - 1)) : 0;
   const int end = sh + nval * N;
-  T::load(tile, in + (E0 - sh), end, (long long)a.nlines * N - (E0 - sh), a.vec, lane);
+  T::load<false>(tile, in + (E0 - sh), end, (long long)a.nlines * N - (E0 - sh), a.vec, lane);
   wave_fence();
   const int l = lane / P, p = lane - l * P;
   const bool act = l < nval;
   const int s = p * a.mb + (p < a.mx ? p : a.mx);
   const int m = a.mb + (p < a.mx ? 1 : 0);
-  float* row0 = tile + sh + (act ? l * N : 0);
+  const int i0 = sh + (act ? l : 0) * N;
+  const T::Run run(i0 + s - R);
+  // the rows as they lie in the tile; beyond the line's ends 0
   float win[RCHUNK + 2 * R];
 #pragma unroll
-  for (int w = 0; w < RCHUNK + 2 * R; ++w) {
-    const int row = s - R + w;
-    const bool ok = w < m + 2 * R && row >= 0 && row < N;
-    const float v = row0[ok ? row : 0];
-    win[w] = ok ? v : 0.0f;
+  for (int w = 0; w < RCHUNK + 2 * R; ++w) win[w] = w < m + 2 * R ? tile[run(w)] : 0.0f;
+  if (p == 0) {
+#pragma unroll
+    for (int w = 0; w < R; ++w) win[w] = 0.0f;
+  }
+  if (p == P - 1) {
+#pragma unroll
+    for (int w = 2 * NB + R; w < RCHUNK + 2 * R; ++w)
+      if (w >= a.mb + R) win[w] = 0.0f;
   }
   double rhs[RCHUNK];
   ref_rhs_interior<KIND>(a, win, rhs);
-  ref_rhs_boundary(a, p, rhs, [&](int slot) { return end_value(slot, N, [&](int i) { return row0[i]; }); });
+  ref_rhs_boundary(a, p, rhs, [&](int slot) { return end_value(slot, N, [&](int i) { return tile[T::at(i0 + i)]; }); });
   const float* t = tab + ref_class(p, P, a.mx) * (RCHUNK * CROW);
   float x[RCHUNK], d[RCHUNK], z[4];
   const bool longer = p < a.mx;
@@ -762,11 +804,11 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
     if (act && k < m) {
       double val = ((double)x[k] + (double)d[k]) * a.scale;
       if (a.addv) val += (double)win[k + R];
-      row0[s + k] = (float)val;
+      tile[run(k + R)] = (float)val;
     }
   }
   wave_fence();
-  T::store(tile, out + (E0 - sh), sh, end, a.vec, lane, a.epi, a.epi_c, nullptr, 0);
+  T::store<false>(tile, out + (E0 - sh), sh, end, a.vec, lane, a.epi, a.epi_c, nullptr, 0);
 }
 
 struct RefEntry {
@@ -1057,6 +1099,11 @@ static size_t yz_lds(int solve, int nthr, int lines, int ntab) {
          (size_t)ntab * sizeof(double);
 }
 
+// Workgroups of the explicit filter per line group: its chunks need no
+// exchange, so a workgroup is 64 lines by as many chunks as 256 threads hold.
+constexpr int NONE_THREADS = 256;
+static int explicit_groups(int P, int nthr, int lines) { return (P + nthr / lines - 1) / (nthr / lines); }
+
 // Lines per y/z workgroup (forced: the tuned value, 0 = none). At 256^3 32
 // lines measured fastest for FP64 fields (d1 y 54 us; 16 lines 58, 64 lines
 // 64: one workgroup of 16 waves fills a CU alone) and for FP32 y lines (33
@@ -1081,9 +1128,15 @@ static int launch_typed(pyr_ctx* c, int dir, int forced, LineArgs a, const TS* i
     hipLaunchKernelGGL((k_line_x<TS, KIND, SOLVE, FULL>), grid, block, (size_t)a.ntab * sizeof(double), c->stream, a,
                        in, out);
   } else {
-    a.lines = yz_lines(a.P, a.nlines, dir, (int)sizeof(TS), forced, c->ncu);
-    const dim3 grid((unsigned)((a.nlines + a.lines - 1) / a.lines)), block(a.lines * a.P);
-    const size_t shm = yz_lds(SOLVE, a.lines * a.P, a.lines, a.ntab);
+    a.lines = SOLVE == SOLVE_NONE && forced <= 0 ? 64 : yz_lines(a.P, a.nlines, dir, (int)sizeof(TS), forced, c->ncu);
+    unsigned nblk = (unsigned)((a.nlines + a.lines - 1) / a.lines);
+    int nthr = a.lines * a.P;
+    if (SOLVE == SOLVE_NONE) {
+      nthr = std::min(nthr, NONE_THREADS);
+      nblk *= (unsigned)explicit_groups(a.P, nthr, a.lines);
+    }
+    const dim3 grid(nblk), block(nthr);
+    const size_t shm = yz_lds(SOLVE, nthr, a.lines, a.ntab);
     auto k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_NONE>;
     // filters only exist for the r4 kind; accumulating epilogues for every kind
     if constexpr (KIND == K_R4) {
@@ -1673,9 +1726,9 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
     HIPCHECK(hipMemcpy(L.dev, image.data(), image.size(), hipMemcpyHostToDevice));
     return 0;
   };
-  auto add_blocks = [&](size_t j, int nlines, int per) {
+  auto add_blocks = [&](size_t j, int nlines, int per, int times = 1) {
     const long long blk0 = (long long)member.size();
-    member.insert(member.end(), (size_t)((nlines + per - 1) / per), (int)j);
+    member.insert(member.end(), (size_t)((nlines + per - 1) / per) * times, (int)j);
     return blk0;
   };
   const int pre = all[0].a.addv ? PRE_V : ((key.epi == EPI_ADD || key.epi == EPI_MAXABS) ? PRE_OLD : PRE_NONE);
@@ -1708,7 +1761,7 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
     // where a member's lines have more than 32 chunks
     int Pmax = 1;
     for (auto& e : all) Pmax = std::max(Pmax, e.a.P);
-    nthr = Pmax > 32 ? WG_MAX : WG_MAX / 2;
+    nthr = sv == SOLVE_NONE ? NONE_THREADS : (Pmax > 32 ? WG_MAX : WG_MAX / 2);
     L.shm = yz_lds(sv, nthr, 128, ntab);
     L.pre = pre;
   }
@@ -1719,10 +1772,11 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
       e.a.vec = key.aligned && ((e.off * (long long)sizeof(TS)) % 16 == 0);
       e.a.lines = 64 / e.a.P;
     } else {
-      e.a.lines = 128;
-      while (e.a.lines * e.a.P > nthr) e.a.lines /= 2;
+      e.a.lines = sv == SOLVE_NONE ? 64 : 128;
+      while (sv != SOLVE_NONE && e.a.lines * e.a.P > nthr) e.a.lines /= 2;
     }
-    e.blk0 = add_blocks(j, e.a.nlines, L.x ? e.a.lines * (nthr / 64) : e.a.lines);
+    e.blk0 = add_blocks(j, e.a.nlines, L.x ? e.a.lines * (nthr / 64) : e.a.lines,
+                        !L.x && sv == SOLVE_NONE ? explicit_groups(e.a.P, nthr, e.a.lines) : 1);
   }
   return upload(all.data(), all.size() * sizeof(GrpEntry));
 }
