@@ -38,6 +38,7 @@
 namespace pyr {
 
 enum Epi { EPI_STORE = 0, EPI_ADD = 1, EPI_ABS = 2, EPI_MAXABS = 3 };
+PYR_HD bool reads_out(int epi) { return epi == EPI_ADD || epi == EPI_MAXABS; }
 
 // Everything a kernel needs about one operator/direction, passed by value.
 struct LineArgs {
@@ -52,7 +53,8 @@ struct LineArgs {
   double p1, p2;           // recurrence constants
   int W;                   // chunks that enter a carry
   double hf[2][4], hb[2][4];  // H of constant chunks of mb + 1 and mb rows
-  const double* mw;        // remaining turns of a cyclic line (null: none matter)
+  int turns;               // cyclic lines: the turns beyond the first matter
+  double tf[4], tb[4];     // their sum, (I - H of the line)^-1, forward and backward
   // bounded lines: the tables of T slots (OpPlan::tab), then the boundary rows
   const double* tab;
   int tlo, T, ntab;
@@ -297,8 +299,8 @@ PYR_HD void carry_in(const LineArgs& a, int p, H h, ExitOf exit_of, double& e0, 
     q -= STEP;
     if (CYCLIC) q = q < 0 ? a.P - 1 : (q >= a.P ? 0 : q);
   }
-  if (CYCLIC && a.mw) {
-    const double* m = a.mw + 8 * p + (STEP > 0 ? 4 : 0);
+  if (CYCLIC && a.turns) {
+    const double* m = STEP > 0 ? a.tb : a.tf;
     const double t0 = m[0] * e0 + m[1] * e1;
     e1 = m[2] * e0 + m[3] * e1;
     e0 = t0;

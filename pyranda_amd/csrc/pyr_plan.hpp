@@ -67,7 +67,8 @@ struct OpPlan {
   double p1 = 0, p2 = 0;      // limit coefficients
   int W = 0;                  // chunks that enter a carry
   double hf[2][4] = {}, hb[2][4] = {};  // H of constant chunks of mb + 1 and mb rows
-  std::vector<double> mw;     // P x 8 remaining turns (forward, backward); empty if none matter
+  int turns = 0;              // turns of a cyclic line beyond the first matter
+  double tf[4] = {0, 0, 0, 0}, tb[4] = {0, 0, 0, 0};  // their sum (forward, backward)
   // bounded lines, for T slots (the chunks p < tlo, constant chunks of mb + 1
   // and mb rows, the last chunk): CHUNK x T x (l1, l2), CHUNK x T x (v1, v2),
   // CHUNK x T g, T x 8 H (forward, backward)
@@ -139,11 +140,11 @@ inline int carry_terms(const std::vector<M2>& H, int step, bool cyclic) {
   return W;
 }
 
-// (I - H around the whole line)^-1 for the entry of chunk p
-inline M2 turns(const std::vector<M2>& H, int p, int step) {
+// (I - H around a whole cyclic line)^-1 for the entry of a chunk
+inline M2 turns(const std::vector<M2>& H, int step) {
   const int P = (int)H.size();
   M2 acc = {1, 0, 0, 1};
-  for (int j = 1; j <= P; ++j) acc = mul(acc, H[(((p + step * j) % P) + P) % P]);
+  for (int j = 1; j <= P; ++j) acc = mul(acc, H[(((step * j) % P) + P) % P]);
   const ld a = 1 - acc[0], b = -acc[1], c = -acc[2], d = 1 - acc[3], det = a * d - b * c;
   return {d / det, -b / det, -c / det, a / det};
 }
@@ -304,13 +305,12 @@ inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, d
   const int need = std::max(detail::carry_terms(Hf, -1, periodic), detail::carry_terms(Hb, 1, periodic));
   pl.W = std::min(need, periodic ? P : P - 1);
   if (need > pl.W && periodic) {
-    pl.mw.resize((size_t)P * 8);
-    for (int p = 0; p < P; ++p) {
-      const M2 f = detail::turns(Hf, p, -1), b = detail::turns(Hb, p, 1);
-      for (int i = 0; i < 4; ++i) {
-        pl.mw[p * 8 + i] = (double)f[i];
-        pl.mw[p * 8 + 4 + i] = (double)b[i];
-      }
+    // every H is a power of one matrix, so the sum is the same for each chunk
+    pl.turns = 1;
+    const M2 f = detail::turns(Hf, -1), b = detail::turns(Hb, 1);
+    for (int i = 0; i < 4; ++i) {
+      pl.tf[i] = (double)f[i];
+      pl.tb[i] = (double)b[i];
     }
   }
   // constant chunks, from the limit coefficients

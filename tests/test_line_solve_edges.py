@@ -131,3 +131,46 @@ def test_nonfinite_values_spread_over_their_line(kind, dtype):
                 b[tuple(line)] = a[tuple(line)]
                 assert torch.equal(a, b), (d, op, row)
         ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nn", [(40, 33, 1), (40, 1, 33), (1, 33, 40), (64, 3, 2), (2, 64, 1), (1, 3, 64), (2, 1, 3)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_null_directions_of_composites(nn, dtype):
+    """Filters, ring, Laplacian and divergence on grids with directions too
+    short for the operators: equal to the sweeps of all three directions one
+    by one (a null direction copies or adds zero), NaN and infinity included."""
+    from pyranda_amd import _lib as amd
+    print("null directions", nn, dtype, flush=True)
+    kinds = ["PERI" if n % 2 else "NONE" for n in nn]
+    ctx = _ctx(nn, kinds, [(0.0, 1.0, n) for n in nn])
+    g = torch.Generator(device="cuda").manual_seed(2)
+    f = [torch.randn(tuple(reversed(nn)), generator=g, device="cuda", dtype=dtype).permute(2, 1, 0) for _ in range(3)]
+    bad = f[0].clone()
+    bad[0, 0, 0], bad[-1, -1, -1] = float("nan"), float("inf")
+    for v in (f[0], bad):
+        for name, op in (("sfilter", amd.OP_SFILTER), ("gfilter", amd.OP_GFILTER)):
+            ref = v
+            for d in range(3):
+                ref = ctx.apply(op, d, ref)
+            assert torch.equal(getattr(ctx, name)(v).nan_to_num(7.0), ref.nan_to_num(7.0)), name
+            if name == "sfilter" and dtype == torch.float64:
+                out, out32 = ctx.sfilter_rounded(v)
+                assert torch.equal(out.nan_to_num(7.0), ref.nan_to_num(7.0))
+                assert torch.equal(out32.nan_to_num(7.0), ref.float().nan_to_num(7.0))
+        ref = None
+        for d in range(3):
+            ref = ctx.apply(amd.OP_D8, d, v, out=ref, epi=amd.EPI_MAXABS_SCALED if d else amd.EPI_ABS_SCALED,
+                            epi_scale=ctx.dmesh[d] ** 2)
+        assert torch.equal(ctx.pring(v).nan_to_num(7.0), ref.nan_to_num(7.0)), "ring"
+        for name, op, fs in (("plaplacian", amd.OP_D2, (v, v, v)), ("divergence", amd.OP_D1, (v, f[1], f[2]))):
+            ref = None
+            for d in range(3):
+                ref = ctx.apply(op, d, fs[d], out=ref, epi=amd.EPI_ADD if d else amd.EPI_STORE)
+            got = ctx.plaplacian(v) if name == "plaplacian" else ctx.divergence(*fs)
+            assert torch.equal(got.nan_to_num(7.0), ref.nan_to_num(7.0)), name
+    # the refusals of the whole call hold for a direction that is not swept
+    for call in ("pyr_plaplacian_f64", "pyr_sfilter_f64", "pyr_pring_f64"):
+        p = ctypes.c_void_p(f[0].data_ptr())
+        assert getattr(ctx._L, call)(ctx._h, p, p) != 0, call
+    ctx.close()
