@@ -68,10 +68,22 @@ static int fail(const std::string& m) { return pyr::report_error(m); }
 // ---------------------------------------------------------------------------
 enum Solve { SOLVE_NONE = 0, SOLVE_BND = 1, SOLVE_CIRC = 2 };
 
-// What the epilogue of a y/z row needs besides the solution, in registers
-// before the backward pass so that no store waits on a load: the input value (filters
-// add v back) or the current output (accumulating epilogues).
-enum Pre { PRE_NONE = 0, PRE_V = 1, PRE_OLD = 2 };
+// What a y/z row's epilogue does and needs besides the solution, in registers
+// before the backward pass so that no store waits on a load: store it
+// (PRE_NONE), add the input back and store (PRE_V, filters), or join the
+// current output (PRE_OLD: the maximum for the r4 kind's ring, the sum for the
+// others). These are the composites' own sweeps, with nothing to decide per
+// row: the branches over the epilogue and the FP32 copy, taken for each of the
+// 16 rows, had cut the backward pass and its stores into pieces (256^3 FP64
+// gradient 165 -> 155 us, filter 145 -> 137, FP32 ring 102 -> 98; bounded
+// Laplacian on 192^3 118 -> 112). PRE_ANY takes every other epilogue and the
+// FP32 copy, read from the arguments row by row.
+enum Pre { PRE_NONE = 0, PRE_V = 1, PRE_OLD = 2, PRE_ANY = 3 };
+constexpr int joined_epi(int kind) { return kind == K_R4 ? EPI_MAXABS : EPI_ADD; }
+static int pre_of(int kind, bool addv, int epi, bool out32) {
+  if (epi == EPI_STORE && !out32) return addv ? PRE_V : PRE_NONE;
+  return !addv && epi == joined_epi(kind) ? PRE_OLD : PRE_ANY;
+}
 
 constexpr int WG_MAX = 1024;
 
@@ -249,17 +261,18 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
     if constexpr (PRE == PRE_V) val += (double)win[k + R];
     const int off = FULL ? vmid : row_off(k);
     const int soff = FULL ? k * rb : 0;
-    TS old = (TS)0;
-    if constexpr (PRE == PRE_OLD) old = pre[k];
-    // a filter with an accumulating epilogue (only through pyr_apply) reads
-    // the output in place
-    if constexpr (PRE == PRE_V)
-      if (reads_out(a.epi)) old = buf_load(TS(), rout, off, soff);
-    const TS r = epilogue<TS>(a.epi, a.epi_c, val, old);
-    if (sizeof(TS) != 8 || GRP || !a.only32) buf_store(r, rout, off, soff);
-    // (store epilogues only: the accumulating variants keep their registers)
-    if constexpr (sizeof(TS) == 8 && PRE != PRE_OLD && !GRP)
-      if (a.out32) buf_store((float)r, rout32, off / 2, soff / 2);
+    if constexpr (PRE == PRE_ANY) {
+      if (KIND == K_R4 && a.addv) val += (double)win[k + R];
+      const TS old = reads_out(a.epi) ? buf_load(TS(), rout, off, soff) : (TS)0;
+      const TS r = epilogue<TS>(a.epi, a.epi_c, val, old);
+      if (sizeof(TS) != 8 || GRP || !a.only32) buf_store(r, rout, off, soff);
+      if constexpr (sizeof(TS) == 8 && !GRP)
+        if (a.out32) buf_store((float)r, rout32, off / 2, soff / 2);
+    } else if constexpr (PRE == PRE_OLD) {
+      buf_store(epilogue<TS>(joined_epi(KIND), a.epi_c, val, pre[k]), rout, off, soff);
+    } else {
+      buf_store((TS)val, rout, off, soff);
+    }
   };
   if constexpr (SOLVE == SOLVE_NONE) {
     if (!valid) return;
@@ -702,9 +715,10 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, con
   // is solved (the right-hand sides' registers are free by now)
   float pre[PRE == PRE_NONE ? 1 : RCHUNK];
   if constexpr (PRE != PRE_NONE) {
+    const bool v = PRE == PRE_V || (PRE == PRE_ANY && a.addv);
 #pragma unroll
     for (int k = 0; k < RCHUNK; ++k)
-      if (k <= a.mb) pre[k] = buf_load(0.0f, PRE == PRE_V ? rin : rout, act && k < m ? off_of(s + k) : OOB, 0);
+      if (k <= a.mb) pre[k] = buf_load(0.0f, v ? rin : rout, act && k < m ? off_of(s + k) : OOB, 0);
   }
   if (act) {
     ref_local_solve(a, t, d);
@@ -720,11 +734,18 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, con
       double val = ((double)x[k] + (double)d[k]) * a.scale;
       const int off = k < m ? off_of(s + k) : OOB;
       if constexpr (PRE == PRE_V) val += (double)pre[k];
-      float old = 0.0f;
-      if constexpr (PRE == PRE_OLD) old = pre[k];
-      if constexpr (PRE == PRE_V)
-        if (reads_out(a.epi)) old = buf_load(0.0f, rout, off, 0);
-      buf_store(epilogue<float>(a.epi, a.epi_c, val, old), rout, off, 0);
+      if constexpr (PRE == PRE_ANY) {
+        float old = pre[k];
+        if (a.addv) {
+          val += (double)pre[k];
+          if (reads_out(a.epi)) old = buf_load(0.0f, rout, off, 0);
+        }
+        buf_store(epilogue<float>(a.epi, a.epi_c, val, old), rout, off, 0);
+      } else if constexpr (PRE == PRE_OLD) {
+        buf_store(epilogue<float>(joined_epi(KIND), a.epi_c, val, pre[k]), rout, off, 0);
+      } else {
+        buf_store((float)val, rout, off, 0);
+      }
     }
   }
 }
@@ -1138,13 +1159,15 @@ static int launch_typed(pyr_ctx* c, int dir, int forced, LineArgs a, const TS* i
     }
     const dim3 grid(nblk), block(nthr);
     const size_t shm = yz_lds(SOLVE, nthr, a.lines, a.ntab);
-    auto k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_NONE>;
-    // filters only exist for the r4 kind; accumulating epilogues for every kind
+    const int pre = pre_of(KIND, a.addv, a.epi, a.out32 != nullptr);
+    auto k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_ANY>;
+    // filters only exist for the r4 kind, the explicit operator is one
     if constexpr (KIND == K_R4) {
-      if (a.addv) k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_V>;
+      if (pre == PRE_V) k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_V>;
     }
     if constexpr (SOLVE != SOLVE_NONE) {
-      if (!a.addv && reads_out(a.epi)) k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_OLD>;
+      if (pre == PRE_NONE) k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_NONE>;
+      if (pre == PRE_OLD) k = k_line_yz<TS, KIND, SOLVE, FULL, PRE_OLD>;
     }
     hipLaunchKernelGGL(k, grid, block, shm, c->stream, a, in, out);
   }
@@ -1208,11 +1231,13 @@ static int launch_ref_kind(hipStream_t stream, int dir, RefArgs a, const float* 
                        ref_lds(a), stream, a, in, out);
   } else {
     a.lines = ref_lines(a.P);
-    auto k = k_ref_yz<KIND, PRE_NONE>;
+    const int pre = pre_of(KIND, a.addv, a.epi, false);
+    auto k = k_ref_yz<KIND, PRE_ANY>;
     if constexpr (KIND == K_R4) {
-      if (a.addv) k = k_ref_yz<KIND, PRE_V>;
+      if (pre == PRE_V) k = k_ref_yz<KIND, PRE_V>;
     }
-    if (!a.addv && reads_out(a.epi)) k = k_ref_yz<KIND, PRE_OLD>;
+    if (pre == PRE_NONE) k = k_ref_yz<KIND, PRE_NONE>;
+    if (pre == PRE_OLD) k = k_ref_yz<KIND, PRE_OLD>;
     hipLaunchKernelGGL(k, dim3((unsigned)((a.nlines + a.lines - 1) / a.lines)), dim3(a.lines * a.P), ref_lds(a),
                        stream, a, in, out);
   }
@@ -1783,7 +1808,7 @@ static int grp_build(pyr_group* g, const GrpKey& key, GrpPlan& gp) {
     member.insert(member.end(), (size_t)((nlines + per - 1) / per) * times, (int)j);
     return blk0;
   };
-  const int pre = all[0].a.addv ? PRE_V : (reads_out(key.epi) ? PRE_OLD : PRE_NONE);
+  const int pre = pre_of(pl0.kind, all[0].a.addv, key.epi, false);
   if (key.refined && sv == SOLVE_BND) {
     std::vector<RefEntry> ref(all.size());
     size_t lds = 0;
@@ -1839,15 +1864,15 @@ template <typename TS, int KIND, int SOLVE>
 static int grp_launch_typed(pyr_group* g, const GrpLaunch& L, const TS* in, TS* out) {
   if (L.nblocks <= 0) return 0;
   const dim3 grid((unsigned)L.nblocks);
-  auto k = k_line_yz_grp<TS, KIND, SOLVE, PRE_NONE>;
-  if (L.x) {
-    k = k_line_x_grp<TS, KIND, SOLVE>;
-  } else if (L.pre == PRE_V) {
-    if constexpr (KIND == K_R4) k = k_line_yz_grp<TS, KIND, SOLVE, PRE_V>;
-    else return fail("filter epilogue on a non-filter kernel");
-  } else if (L.pre == PRE_OLD) {
-    k = k_line_yz_grp<TS, KIND, SOLVE, PRE_OLD>;
+  auto k = k_line_yz_grp<TS, KIND, SOLVE, PRE_ANY>;
+  if constexpr (KIND == K_R4) {
+    if (L.pre == PRE_V) k = k_line_yz_grp<TS, KIND, SOLVE, PRE_V>;
   }
+  if constexpr (SOLVE != SOLVE_NONE) {
+    if (L.pre == PRE_NONE) k = k_line_yz_grp<TS, KIND, SOLVE, PRE_NONE>;
+    if (L.pre == PRE_OLD) k = k_line_yz_grp<TS, KIND, SOLVE, PRE_OLD>;
+  }
+  if (L.x) k = k_line_x_grp<TS, KIND, SOLVE>;
   hipLaunchKernelGGL(k, grid, L.block, L.shm, g->stream, (const GrpEntry*)L.dev, L.member, in, out);
   HIPCHECK(hipGetLastError());
   return 0;
@@ -1873,15 +1898,13 @@ int grp_launch(pyr_group* g, const GrpLaunch& L, const TS* in, TS* out) {
 template <int KIND>
 static int grp_launch_ref_kind(hipStream_t stream, const GrpLaunch& L, const float* in, float* out) {
   if (L.nblocks <= 0) return 0;
-  auto k = k_ref_yz_grp<KIND, PRE_NONE>;
-  if (L.x) {
-    k = k_ref_x_grp<KIND>;
-  } else if (L.pre == PRE_V) {
-    if constexpr (KIND == K_R4) k = k_ref_yz_grp<KIND, PRE_V>;
-    else return fail("filter epilogue on a non-filter kernel");
-  } else if (L.pre == PRE_OLD) {
-    k = k_ref_yz_grp<KIND, PRE_OLD>;
+  auto k = k_ref_yz_grp<KIND, PRE_ANY>;
+  if constexpr (KIND == K_R4) {
+    if (L.pre == PRE_V) k = k_ref_yz_grp<KIND, PRE_V>;
   }
+  if (L.pre == PRE_NONE) k = k_ref_yz_grp<KIND, PRE_NONE>;
+  if (L.pre == PRE_OLD) k = k_ref_yz_grp<KIND, PRE_OLD>;
+  if (L.x) k = k_ref_x_grp<KIND>;
   hipLaunchKernelGGL(k, dim3((unsigned)L.nblocks), L.block, L.shm, stream, (const RefEntry*)L.dev, L.member, in, out);
   HIPCHECK(hipGetLastError());
   return 0;

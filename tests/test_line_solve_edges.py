@@ -174,3 +174,35 @@ def test_null_directions_of_composites(nn, dtype):
         p = ctypes.c_void_p(f[0].data_ptr())
         assert getattr(ctx._L, call)(ctx._h, p, p) != 0, call
     ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["PERI", "NONE"])
+@pytest.mark.parametrize("n", [64, 71])
+def test_every_epilogue_of_every_operator(n, kind):
+    """Each operator and direction with each epilogue and with the FP32 copy,
+    whole and ragged chunks: the epilogue of the stored result, to one rounding
+    of the stored type (the fused forms round the result once, not twice)."""
+    from pyranda_amd import _lib as amd
+    print("epilogues", n, kind, flush=True)
+    nn = (n, n, n)
+    ctx = _ctx(nn, [kind] * 3, [(0.0, 1.0, n)] * 3)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    for dtype in (torch.float64, torch.float32):
+        eps = torch.finfo(dtype).eps
+        v, old = [torch.randn(nn, generator=g, device="cuda", dtype=dtype).permute(2, 1, 0) for _ in range(2)]
+        for op in range(5):
+            for d in range(3):
+                y = ctx.apply(op, d, v)
+                for epi, want in ((amd.EPI_ADD, old.double() + y.double()),
+                                  (amd.EPI_ABS_SCALED, 0.75 * y.double().abs()),
+                                  (amd.EPI_MAXABS_SCALED, torch.maximum(old.double(), 0.75 * y.double().abs()))):
+                    out = old.permute(2, 1, 0).clone().permute(2, 1, 0)
+                    got = ctx.apply(op, d, v, out=out, epi=epi, epi_scale=0.75).double()
+                    bar = 2 * eps * (old.double().abs() + y.double().abs())
+                    assert ((got - want).abs() <= bar).all(), (op, d, epi, dtype)
+                if dtype == torch.float64:
+                    o32 = torch.empty(nn, device="cuda", dtype=torch.float32).permute(2, 1, 0)
+                    assert torch.equal(ctx.apply(op, d, v, out32=o32), y) and torch.equal(o32, y.float()), (op, d)
+                    assert torch.equal(ctx.apply_to32(op, d, v), y.float()), (op, d)
+    ctx.close()
