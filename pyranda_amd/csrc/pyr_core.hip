@@ -168,6 +168,15 @@ __device__ __forceinline__ void carry_of(const LineArgs& a, const Tables& t, int
 // solves' passes, each read a latency on the critical path of a workgroup
 // (from memory, the 2-D and ragged bounded sweeps took 28-36 us for fields
 // of a few MB).
+// First element of y/z line L (the last line for L past it): 32-bit division,
+// the lines and elements of a field are fewer than 2^28.
+template <typename Args>
+__device__ __forceinline__ int line_offset(const Args& a, int L) {
+  const unsigned l = (unsigned)(L < a.nlines ? L : a.nlines - 1), n = (unsigned)a.A;
+  const unsigned q = l / n;
+  return (int)(l - q * n + (unsigned)a.B * q);
+}
+
 __device__ __forceinline__ void stage_tables(const LineArgs& a, double* tab) {
   for (int e = threadIdx.x; e < a.ntab / 2; e += blockDim.x)
     reinterpret_cast<D2*>(tab)[e] = reinterpret_cast<const D2*>(a.tab)[e];
@@ -184,7 +193,7 @@ __device__ __forceinline__ void stage_tables(const LineArgs& a, double* tab) {
 // The body takes the workgroup's line-group index `blk` (blockIdx.x for one
 // field, the member-local index for a grouped launch over several fields).
 template <typename TS, int KIND, int SOLVE, bool FULL, int PRE, bool GRP = false>
-__device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, const TS* __restrict__ in,
+__device__ __forceinline__ void line_yz_body(const LineArgs& a, int blk, const TS* __restrict__ in,
                                              TS* __restrict__ out) {
   constexpr int R = Halo<KIND>::R;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -195,14 +204,13 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, long long blk, c
     // chunks of the explicit filter are independent: a workgroup takes some of
     // a line group's chunks
     const int per = (int)blockDim.x >> __builtin_ctz(LY), groups = (a.P + per - 1) / per;
-    p += (int)(blk % groups) * per;
-    blk /= groups;
+    p += (int)((unsigned)blk % (unsigned)groups) * per;
+    blk = (int)((unsigned)blk / (unsigned)groups);
   }
   const bool act = (!GRP && SOLVE != SOLVE_NONE) || p < a.P;
-  const long long L = blk * LY + lane;
+  const int L = blk * LY + lane;
   const bool valid = act && L < a.nlines;
-  const long long Lc = L < a.nlines ? L : (long long)a.nlines - 1;
-  const int lane_off = (int)(((Lc % a.A) + a.B * (Lc / a.A)) * (long long)sizeof(TS));
+  const int lane_off = line_offset(a, L) * (int)sizeof(TS);
   const int rb = (int)(a.stride * (long long)sizeof(TS));
   const int s = FULL ? p * CHUNK : chunk_start(a, p);
   const int m = FULL ? CHUNK : a.mb + (p < a.mx ? 1 : 0);
@@ -624,7 +632,7 @@ __global__ void __launch_bounds__(WG_MAX) k_line_yz_grp(const GrpEntry* __restri
   const int j = member[blockIdx.x];
   const LineArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
-  line_yz_body<TS, KIND, SOLVE, false, PRE, true>(a, (long long)blockIdx.x - b0, in + off, out + off);
+  line_yz_body<TS, KIND, SOLVE, false, PRE, true>(a, (int)(blockIdx.x - b0), in + off, out + off);
 }
 
 // --- refined FP32 solve of bounded lines (pyr_refined.hpp) -------------------
@@ -659,7 +667,7 @@ __device__ __forceinline__ void ref_stage(const RefArgs& a, float* tab, float* g
 }
 
 template <int KIND, int PRE>
-__device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, const float* __restrict__ in,
+__device__ __forceinline__ void ref_yz_body(const RefArgs& a, int blk, const float* __restrict__ in,
                                             float* __restrict__ out) {
   constexpr int R = Halo<KIND>::R;
   __shared__ __align__(16) float tab[NCLS * RCHUNK * CROW];
@@ -668,15 +676,13 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, con
   __shared__ int bad[64];
   extern __shared__ __align__(16) unsigned char smem[];
   float* g = reinterpret_cast<float*>(smem);
-  ref_stage(a, tab, g);
   const int LY = a.lines;
   const int p = (int)((unsigned)threadIdx.x / (unsigned)LY);
   const int lane = (int)threadIdx.x - p * LY;
   if (p == 0) bad[lane] = 0;
   const bool act = p < a.P;
-  const long long L = blk * LY + lane;
-  const long long Lc = L < a.nlines ? L : (long long)a.nlines - 1;
-  const int lane_off = (int)(((Lc % a.A) + a.B * (Lc / a.A)) * (long long)sizeof(float));
+  const int L = blk * LY + lane;
+  const int lane_off = line_offset(a, L) * (int)sizeof(float);
   const int rb = (int)(a.stride * (long long)sizeof(float));
   const int s = p * a.mb + (p < a.mx ? p : a.mx);
   const int m = a.mb + (p < a.mx ? 1 : 0);
@@ -691,6 +697,7 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, long long blk, con
     if (w <= a.mb + 2 * R)
       win[w] = buf_load(0.0f, rin, act && w < m + 2 * R && row >= 0 && row < a.N ? off_of(row) : OOB, 0);
   }
+  ref_stage(a, tab, g);  // behind the window's loads
   double rhs[RCHUNK];
   ref_rhs_interior<KIND>(a, win, rhs);
   if (act && (p == 0 || p == a.P - 1)) {
@@ -880,7 +887,7 @@ __global__ void __launch_bounds__(REF_THREADS) k_ref_yz_grp(const RefEntry* __re
   const int j = member[blk];
   const RefArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
-  ref_yz_body<KIND, PRE>(a, blk - b0, in + off, out + off);
+  ref_yz_body<KIND, PRE>(a, (int)(blk - b0), in + off, out + off);
 }
 template <int KIND, int PRE>
 __global__ void __launch_bounds__(64 * REF_X_WAVES) __attribute__((amdgpu_waves_per_eu(2, 8))) k_ref_x_grp(const RefEntry* __restrict__ g, const int* __restrict__ member,
