@@ -6,6 +6,8 @@ loudly if it is missing: there is no CPU fallback for the operators.
 import ctypes
 import os
 
+import torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 # PYRANDA_AMD_LIB selects another in-tree build of the same library (tuning
 # variants built by _build.build(out=..., defines=...))
@@ -106,6 +108,18 @@ def lib():
             fn.argtypes = args
         _LIB = L
     return _LIB
+
+
+# torch.cuda.current_stream builds a Stream object on each call (2 us of a
+# launch's host time); the handle alone is what a launch needs
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def stream_of(device):
+    """Handle of torch's current stream on a device, for a c_void_p argument."""
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def check(status):

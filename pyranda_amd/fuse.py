@@ -252,11 +252,11 @@ def _expand_members(vals, shape):
 def _field_ok(t, shape):
     if not torch.is_tensor(t) or t.dtype not in (torch.float64, torch.float32) or not t.is_cuda:
         return False
-    if tuple(t.shape) != shape:
+    if t.shape != shape:
         return False
     nx, ny, nz = shape
     want = (1, nx, nx * ny)
-    return all(s == w or n == 1 for s, w, n in zip(t.stride(), want, shape))
+    return t.stride() == want or all(s == w or n == 1 for s, w, n in zip(t.stride(), want, shape))
 
 
 class FusedSubtree:
@@ -422,6 +422,14 @@ class FusedSubtree:
         nfield = 0
         dev = None
         for v in vals:
+            if torch.is_tensor(v) and v.dim() == 3 and _field_ok(v, shape):
+                f64 = v.dtype == torch.float64
+                sig.append("T64" if f64 else "T32")
+                any64 |= f64
+                fields.append(v)
+                nfield += 1
+                dev = v.device
+                continue
             if torch.is_tensor(v) and v.dim() == 0 and not _device_scalar(v):
                 v = v.item()
             if isinstance(v, (int, float)) or (hasattr(v, "dtype") and not torch.is_tensor(v)
@@ -438,12 +446,6 @@ class FusedSubtree:
                 # one value per member of a group (read per point by member)
                 sig.append("G64" if v.dtype == torch.float64 else "G32")
                 fields.append(v)
-            elif _field_ok(v, shape):
-                sig.append("T64" if v.dtype == torch.float64 else "T32")
-                any64 |= v.dtype == torch.float64
-                fields.append(v)
-                nfield += 1
-                dev = v.device
             else:
                 return self._py(*_expand_members(vals, shape))
         if not nfield or self.is_bool:
@@ -475,11 +477,11 @@ class FusedSubtree:
             return DeferredF(self, sig, out_dt, fields, scalars, tuple(shape), dev)
         fn = self.kernel(sig, out_dt)
         nx, ny, nz = shape
-        out = torch.empty((nz, ny, nx), dtype=torch.float64 if out_dt == "f64" else torch.float32,
-                          device=dev).permute(2, 1, 0)
+        out = torch.empty_strided((nx, ny, nz), (1, nx, nx * ny),
+                                  dtype=torch.float64 if out_dt == "f64" else torch.float32, device=dev)
         ptrs = (ctypes.c_void_p * (len(fields) + 1))(*[f.data_ptr() for f in fields], out.data_ptr())
         sc = (ctypes.c_double * max(1, len(scalars)))(*scalars)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        stream = _lib.stream_of(dev)
         _lib.check_pw(_lib.lib().pyr_pw_launch(fn, stream, nx * ny * nz, len(fields) + 1, ptrs,
                                                len(scalars), sc))
         if decide:
@@ -579,6 +581,12 @@ class FusedGroup:
         is64 = []
         dev = None
         for v in vals:
+            if torch.is_tensor(v) and v.dim() == 3 and _field_ok(v, shape):
+                sig.append("T64" if v.dtype == torch.float64 else "T32")
+                is64.append(sig[-1] == "T64")
+                fields.append(v)
+                dev = v.device
+                continue
             if torch.is_tensor(v) and v.dim() == 0 and not _device_scalar(v):
                 v = v.item()
             if isinstance(v, (int, float)) or (hasattr(v, "dtype") and not torch.is_tensor(v)
@@ -591,10 +599,6 @@ class FusedGroup:
             elif _member_scalar(v, shape):
                 sig.append("G64" if v.dtype == torch.float64 else "G32")
                 fields.append(v)
-            elif _field_ok(v, shape):
-                sig.append("T64" if v.dtype == torch.float64 else "T32")
-                fields.append(v)
-                dev = v.device
             else:
                 return self._separate(shape, vals)
             is64.append(sig[-1] == "T64")
@@ -621,12 +625,13 @@ class FusedGroup:
             return self._separate(shape, vals)
         fn = self.kernel(tuple(sig), tuple(out_dts))
         nx, ny, nz = shape
-        outs = [torch.empty((nz, ny, nx), dtype=torch.float64 if dt == "f64" else torch.float32,
-                            device=dev).permute(2, 1, 0) for dt in out_dts]
+        outs = [torch.empty_strided((nx, ny, nz), (1, nx, nx * ny),
+                                    dtype=torch.float64 if dt == "f64" else torch.float32, device=dev)
+                for dt in out_dts]
         ptrs = (ctypes.c_void_p * (len(fields) + nout))(*[f.data_ptr() for f in fields],
                                                          *[o.data_ptr() for o in outs])
         sc = (ctypes.c_double * max(1, len(scalars)))(*scalars)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        stream = _lib.stream_of(dev)
         _lib.check_pw(_lib.lib().pyr_pw_launch(fn, stream, nx * ny * nz, len(fields) + nout, ptrs,
                                                len(scalars), sc))
         if decide:
@@ -752,10 +757,10 @@ class DeferredF:
     def materialize(self):
         fn = self.sub.kernel(self.sig, self.out_dt)
         nx, ny, nz = self.shape
-        out = torch.empty((nz, ny, nx), dtype=self.dtype, device=self.device).permute(2, 1, 0)
+        out = torch.empty_strided((nx, ny, nz), (1, nx, nx * ny), dtype=self.dtype, device=self.device)
         ptrs = (ctypes.c_void_p * (len(self.fields) + 1))(*[f.data_ptr() for f in self.fields], out.data_ptr())
         sc = (ctypes.c_double * max(1, len(self.scalars)))(*self.scalars)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+        stream = _lib.stream_of(self.device)
         _lib.check_pw(_lib.lib().pyr_pw_launch(fn, stream, nx * ny * nz, len(self.fields) + 1, ptrs,
                                                len(self.scalars), sc))
         return out
@@ -776,7 +781,7 @@ class DeferredF:
         nx, ny, nz = self.shape
         pp = (ctypes.c_void_p * len(ptrs))(*[t.data_ptr() for t in ptrs])
         sc = (ctypes.c_double * len(scal))(*scal)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+        stream = _lib.stream_of(self.device)
         _lib.check_pw(_lib.lib().pyr_pw_launch(fn, stream, nx * ny * nz, len(ptrs), pp, len(scal), sc))
         return True
 
@@ -904,7 +909,7 @@ class FusedReduce:
         part = torch.empty(blocks, dtype=torch.float64, device=dev)
         ptrs = (ctypes.c_void_p * (len(fields) + 1))(*[f.data_ptr() for f in fields], part.data_ptr())
         sc = (ctypes.c_double * max(1, len(scalars)))(*[float(x) for x in scalars])
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        stream = _lib.stream_of(dev)
         _lib.check_pw(_lib.lib().pyr_pw_launch_blocks(fn, stream, n, blocks, len(fields) + 1, ptrs,
                                                       len(scalars), sc))
         return part
@@ -1000,7 +1005,7 @@ class SegmentedReduce:
         ptrs = (ctypes.c_void_p * (len(fields) + 4))(*[f.data_ptr() for f in fields], part.data_ptr(),
                                                      seg.seg.data_ptr(), seg.blk.data_ptr(), sc.data_ptr())
         one = (ctypes.c_double * 1)(0.0)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        stream = _lib.stream_of(dev)
         L = _lib.lib()
         _lib.check_pw(L.pyr_pw_launch_blocks(fn, stream, seg.nmem, seg.nblocks, len(fields) + 4, ptrs, 0, one))
         # second pass: member m reduces its partials blk[m] .. blk[m+1]
@@ -1282,12 +1287,13 @@ class PointwiseRun:
                 raise _lib.PyrandaAMDError(L.pyr_pw_last_error().decode())
             fn = self._kernels[key] = h
         nx, ny, nz = shape
-        outs = [torch.empty((nz, ny, nx), dtype=torch.float64 if t == "f64" else torch.float32,
-                            device=dev).permute(2, 1, 0) for t in types]
+        outs = [torch.empty_strided((nx, ny, nz), (1, nx, nx * ny),
+                                    dtype=torch.float64 if t == "f64" else torch.float32, device=dev)
+                for t in types]
         ptrs = (ctypes.c_void_p * (len(fields) + len(outs)))(*[f.data_ptr() for f in fields],
                                                              *[o.data_ptr() for o in outs])
         sc = (ctypes.c_double * max(1, len(scalars)))(*scalars)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        stream = _lib.stream_of(dev)
         _lib.check_pw(_lib.lib().pyr_pw_launch(fn, stream, nx * ny * nz, len(fields) + len(outs), ptrs,
                                                len(scalars), sc))
         for lhs, o in zip(self.outputs, outs):

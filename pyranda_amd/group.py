@@ -87,10 +87,10 @@ class GroupContext:
         v = self._prep(v)
         if out is None:
             out = self._out(v)
-        self._L.pyr_group_set_stream(self._h, ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream))
+        self._L.pyr_group_set_stream(self._h, _lib.stream_of(self.device))
         prec = _lib.F64 if v.dtype == torch.float64 else _lib.R32
-        _lib.check(self._L.pyr_group_apply(self._h, op, d, prec, ctypes.c_void_p(v.data_ptr()),
-                                           ctypes.c_void_p(out.data_ptr()), epi, float(scale), int(power)))
+        _lib.check(self._L.pyr_group_apply(self._h, op, d, prec, v.data_ptr(), out.data_ptr(), epi, float(scale),
+                                           int(power)))
         return out
 
     # -- parcop names -------------------------------------------------------------
@@ -528,7 +528,7 @@ class pyrandaGroupSim(pyrandaSim):
         out = torch.empty(self.mesh.shape, dtype=self.dtype, device=u.device)
         shadow = self._shadow[U].data_ptr() if fp32 and self._shadow[U] is not None else None
         dt64 = dt.to(torch.float64).contiguous()
-        stream = ctypes.c_void_p(torch.cuda.current_stream(u.device).cuda_stream)
+        stream = _lib.stream_of(u.device)
         _lib.check(_lib.lib().pyr_rk_update_member_dt(
             stream, _lib.R32 if fp32 else _lib.F64, self.npts, ctypes.c_void_p(F.contiguous().data_ptr()),
             ctypes.c_void_p(PHI[U].data_ptr()), ctypes.c_void_p(u.contiguous().data_ptr()),

@@ -22,7 +22,10 @@ from . import _lib
 def empty_field(shape, dtype, device):
     """(nx,ny,nz) tensor with Fortran strides (x fastest)."""
     nx, ny, nz = shape
-    return torch.empty((nz, ny, nx), dtype=dtype, device=device).permute(2, 1, 0)
+    return torch.empty_strided((nx, ny, nz), (1, nx, nx * ny), dtype=dtype, device=device)
+
+
+_FIELD_TYPES = (torch.float64, torch.float32)
 
 
 def is_fortran(t):
@@ -94,6 +97,7 @@ class ParcopContext:
                                x1[2], xn[2], bc6))
         self._h = h
         self._L = L
+        self._strides = (1, self.nn[0], self.nn[0] * self.nn[1])
         dp = (ctypes.c_double * 3)()
         dm = (ctypes.c_double * 3)()
         gl = ctypes.c_double()
@@ -216,6 +220,12 @@ class ParcopContext:
 
     # -- helpers ------------------------------------------------------------
     def _prep(self, v, dtype=None):
+        # a field as the kernels take it, as in nearly every call: small fields
+        # are bound by this host path (with the stream handle and the strided
+        # allocation: fbar on 32^3 17.1 -> 13.2 us, gradient on 64^3 22.7 -> 16.1)
+        if (torch.is_tensor(v) and v.shape == self.nn and v.stride() == self._strides
+                and v.dtype in _FIELD_TYPES and (dtype is None or v.dtype == dtype) and v.device == self.device):
+            return v
         if not torch.is_tensor(v):
             v = torch.full(self.nn, float(v), dtype=dtype or torch.float64, device=self.device)
         if v.device != self.device:
@@ -231,10 +241,10 @@ class ParcopContext:
         return v
 
     def _stream(self):
-        self._L.pyr_set_stream(self._h, ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream))
+        self._L.pyr_set_stream(self._h, _lib.stream_of(self.device))
 
     def _out(self, like):
-        return empty_field(self.nn, like.dtype, self.device)
+        return torch.empty_strided(self.nn, self._strides, dtype=like.dtype, device=self.device)
 
     @staticmethod
     def _ptr(t):
@@ -257,7 +267,8 @@ class ParcopContext:
                                   or tuple(out32.shape) != self.nn):
             raise ValueError("out32: an FP32 field for the store epilogue of an FP64 sweep")
         self._stream()
-        tkey = self._timed((op, direction, str(v.dtype) + ("+float32" if out32 is not None else "")))
+        tkey = self.timing is not None and self._timed(
+            (op, direction, str(v.dtype) + ("+float32" if out32 is not None else ""))) or None
         if tkey is not None:
             ev0 = torch.cuda.Event(enable_timing=True)
             ev1 = torch.cuda.Event(enable_timing=True)
@@ -266,7 +277,7 @@ class ParcopContext:
             _lib.check(self._L.pyr_apply_rounded(self._h, op, direction, self._ptr(v), self._ptr(out),
                                                  self._ptr(out32)))
         else:
-            _lib.check(self._L.pyr_apply(self._h, op, direction, prec, self._ptr(v), self._ptr(out), epi,
+            _lib.check(self._L.pyr_apply(self._h, op, direction, prec, v.data_ptr(), out.data_ptr(), epi,
                                          float(epi_scale)))
         if tkey is not None:
             ev1.record()
@@ -313,12 +324,12 @@ class ParcopContext:
         return out
 
     def _unary(self, name, v):
-        if name in _COMPOSITE and self._split_composite(_COMPOSITE_OP[name]):
+        if self.timing is not None and name in _COMPOSITE and self._split_composite(_COMPOSITE_OP[name]):
             return _COMPOSITE[name](self, v)
         v = self._prep(v)
         out = self._out(v)
         self._stream()
-        _lib.check(getattr(self._L, "pyr_%s_%s" % (name, self._suffix(v)))(self._h, self._ptr(v), self._ptr(out)))
+        _lib.check(getattr(self._L, "pyr_%s_%s" % (name, self._suffix(v)))(self._h, v.data_ptr(), out.data_ptr()))
         return out
 
     # -- parcop names (parcop.f90:202-379) ----------------------------------
@@ -379,7 +390,7 @@ class ParcopContext:
         outs = [self._out(v) for _ in range(3)]
         self._stream()
         _lib.check(getattr(self._L, "pyr_grads_%s" % self._suffix(v))(
-            self._h, self._ptr(v), *[self._ptr(o) for o in outs]))
+            self._h, v.data_ptr(), *[o.data_ptr() for o in outs]))
         return outs
 
     def divergence(self, fx, fy, fz):
@@ -389,5 +400,5 @@ class ParcopContext:
         out = self._out(fx)
         self._stream()
         _lib.check(getattr(self._L, "pyr_divergence_%s" % self._suffix(fx))(
-            self._h, self._ptr(fx), self._ptr(fy), self._ptr(fz), self._ptr(out)))
+            self._h, fx.data_ptr(), fy.data_ptr(), fz.data_ptr(), out.data_ptr()))
         return out
