@@ -168,6 +168,20 @@ __device__ __forceinline__ void carry_of(const LineArgs& a, const Tables& t, int
 // solves' passes, each read a latency on the critical path of a workgroup
 // (from memory, the 2-D and ragged bounded sweeps took 28-36 us for fields
 // of a few MB).
+// The work item of this workgroup when neighbouring items share cache lines:
+// consecutive workgroups start on the 8 XCDs in turn, each with an L2 of its
+// own, so each XCD takes a run of consecutive items. A refined y/z group of
+// 256 threads is 8 lines of 32 chunks, 32-byte rows of the same 128-byte lines
+// as three neighbours': in an ensemble of 24 members (3.7M points) d1 30.2 ->
+// 27.2 us, the filter 44.3 -> 35.4, the ring's maximum 40.2 -> 34.2.
+// The explicit filter's groups along a line share halo rows, of which each XCD
+// fetched its own copy (20% more bytes at 256^3 in FP64): y sweep 43.3 -> 38.4
+// us, 1000x301x53 in FP32 91.4 -> 82.7 us for the three sweeps.
+__device__ __forceinline__ int xcd_order() {
+  const int n = (int)gridDim.x, b = (int)blockIdx.x, x = b & 7, q = n >> 3, r = n & 7;
+  return x * q + (x < r ? x : r) + (b >> 3);
+}
+
 // First element of y/z line L (the last line for L past it): 32-bit division,
 // the lines and elements of a field are fewer than 2^28.
 template <typename Args>
@@ -328,7 +342,7 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, int blk, const T
 
 template <typename TS, int KIND, int SOLVE, bool FULL, int PRE>
 __global__ void __launch_bounds__(WG_MAX) k_line_yz(LineArgs a, const TS* __restrict__ in, TS* __restrict__ out) {
-  line_yz_body<TS, KIND, SOLVE, FULL, PRE>(a, blockIdx.x, in, out);
+  line_yz_body<TS, KIND, SOLVE, FULL, PRE>(a, SOLVE == SOLVE_NONE ? xcd_order() : (int)blockIdx.x, in, out);
 }
 
 // 16-byte vector of the storage type
@@ -629,10 +643,11 @@ __global__ void __launch_bounds__(64 * XWaves<SOLVE>::v) k_line_x_grp(const GrpE
 template <typename TS, int KIND, int SOLVE, int PRE>
 __global__ void __launch_bounds__(WG_MAX) k_line_yz_grp(const GrpEntry* __restrict__ g, const int* __restrict__ member,
                                                         const TS* __restrict__ in, TS* __restrict__ out) {
-  const int j = member[blockIdx.x];
+  const int blk = SOLVE == SOLVE_NONE ? xcd_order() : (int)blockIdx.x;
+  const int j = member[blk];
   const LineArgs a = g[j].a;
   const long long off = g[j].off, b0 = g[j].blk0;
-  line_yz_body<TS, KIND, SOLVE, false, PRE, true>(a, (int)(blockIdx.x - b0), in + off, out + off);
+  line_yz_body<TS, KIND, SOLVE, false, PRE, true>(a, (int)(blk - b0), in + off, out + off);
 }
 
 // --- refined FP32 solve of bounded lines (pyr_refined.hpp) -------------------
@@ -646,17 +661,6 @@ __global__ void __launch_bounds__(WG_MAX) k_line_yz_grp(const GrpEntry* __restri
 // are staged in LDS, and the boundary rows' terms are independent reads.
 constexpr int REF_THREADS = 256;
 constexpr int REF_X_WAVES = 2;
-
-// The work item of this workgroup when neighbouring items share cache lines:
-// consecutive workgroups start on the 8 XCDs in turn, each with an L2 of its
-// own, so each XCD takes a run of consecutive items. A refined y/z group of
-// 256 threads is 8 lines of 32 chunks, 32-byte rows of the same 128-byte lines
-// as three neighbours': in an ensemble of 24 members (3.7M points) d1 30.2 ->
-// 27.2 us, the filter 44.3 -> 35.4, the ring's maximum 40.2 -> 34.2.
-__device__ __forceinline__ int xcd_order() {
-  const int n = (int)gridDim.x, b = (int)blockIdx.x, x = b & 7, q = n >> 3, r = n & 7;
-  return x * q + (x < r ? x : r) + (b >> 3);
-}
 
 // class tables and reduced rows into LDS
 __device__ __forceinline__ void ref_stage(const RefArgs& a, float* tab, float* g) {
