@@ -6,8 +6,9 @@ on the conserved variables after every stage) with Mach 0.1
 (p0 = 1/(gamma*0.1^2)), CFL 0.5 from the initial state, run through
 pyranda_amd.pyrandaSim with every field resident in HBM.
 
-The headline value is FP32-refined point-updates/s (FP32 fields and sweeps,
-one FP64-residual refinement in every operator, FP64 RK4 state, FP64
+The headline value is FP32 point-updates/s (FP32 fields; operators on them in
+FP64 registers along periodic lines, all lines of this workload, and in FP32
+with one FP64-residual refinement along bounded ones; FP64 RK4 state, FP64
 storage of the offset-dominated fields). The FP64 path is timed beside it on
 the same steps, and every conserved variable of the FP32 run is compared
 with the FP64 run after the same steps (rel_max / rel_L2, bar 1e-6).
@@ -40,17 +41,18 @@ HBM_PEAK_GBS = 8000.0
 # commands are in profiles/line_ops_hbm_traffic_pmc.md. Key: (op, direction,
 # field dtype) of the circulant solve.
 MEASURED_TRAFFIC = {
-    ("d1", "x", "torch.float64"): (131472 + 131072) * 1024,
-    ("d1", "x", "torch.float32"): (65959 + 65536) * 1024,
-    ("d1", "y", "torch.float64"): (131687 + 131072) * 1024,
-    ("d1", "y", "torch.float32"): (65845 + 65536) * 1024,
-    ("fbar", "y", "torch.float64"): (131510 + 131072) * 1024,
-    ("fbar", "y", "torch.float32"): (65952 + 65536) * 1024,
-    ("gbar", "y", "torch.float64"): (140248 + 131072) * 1024,
-    ("gbar", "y", "torch.float32"): (65844 + 65536) * 1024,
-    ("fbar", "x", "torch.float64"): (131496 + 131072) * 1024,
-    # FP64 fbar z sweep that also stores the FP32 rounding (20 B/pt)
-    ("fbar", "z", "torch.float64+float32"): (131502 + 196608) * 1024,
+    ("d1", "x", "torch.float64"): (131175 + 131072) * 1024,
+    ("d1", "x", "torch.float32"): (65630 + 65536) * 1024,
+    ("d1", "y", "torch.float64"): (133307 + 131072) * 1024,
+    ("d1", "y", "torch.float32"): (65611 + 65536) * 1024,
+    ("d1", "z", "torch.float64"): (133050 + 131072) * 1024,
+    ("fbar", "y", "torch.float64"): (131605 + 131072) * 1024,
+    ("fbar", "y", "torch.float32"): (65629 + 65536) * 1024,
+    ("gbar", "y", "torch.float64"): (132632 + 131072) * 1024,
+    ("gbar", "y", "torch.float32"): (65620 + 65536) * 1024,
+    ("fbar", "x", "torch.float64"): (131183 + 131072) * 1024,
+    # FP64 fbar sweep that also stores the FP32 rounding (20 B/pt)
+    ("fbar", "z", "torch.float64+float32"): (131222 + 196608) * 1024,
 }
 OPS = ["d1", "d2", "d8", "fbar", "gbar"]
 CONSERVED = ("rho", "rhou", "rhov", "rhow", "Et")
@@ -353,7 +355,8 @@ def ensemble_bench(args, dev):
         "value": out[best]["value"], "unit": "point-updates/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": out[best]["ms_per_step"], "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None,
-        "dtype": {"fp32": "f32 fields and sweeps, f64 residual refinement, f64 RK4 state",
+        "dtype": {"fp32": "f32 fields, f32 sweeps with f64 residual refinement along bounded lines, f64 "
+                          "sweeps along periodic ones, f64 RK4 state",
                   "fp32-fp64solve": "f32 fields, f64 sweeps, f64 RK4 state",
                   "fp64": "f64"}[args.ens_precision],
         "data": ("synthetic (wall-bounded KH layer, seeded multimode perturbation, on each member grid)" if wall
@@ -491,8 +494,8 @@ def main():
                     help="--ops: arithmetic of the solves on FP32 fields")
     ap.add_argument("--precision", default="fp64,fp32,fp32-offset",
                     help="comma-separated pyrandaSim precisions to time (the headline is fp32: FP32 "
-                         "storage where it keeps 1e-6 (pyrandaSim wide_fields='auto'), FP32 sweeps plus "
-                         "one FP64-residual refinement in every FP32 operator; fp32-offset stores only the "
+                         "storage where it keeps 1e-6 (pyrandaSim wide_fields='auto'), bounded FP32 lines "
+                         "with FP32 sweeps plus one FP64-residual refinement; fp32-offset stores only the "
                          "offset-dominated fields in FP64 (faster, less accurate); fp32-fp64solve solves "
                          "in FP64 on FP32 fields; fp32-rounded-state is fp32 without the FP64 state through "
                          "the filter; fp32-all-f32 stores every field in FP32)")
@@ -649,9 +652,8 @@ def main():
         "vs_baseline": None,
         "dtype": "f32 storage for operator results (derivatives, LAD ring and filters) and what is "
                  "computed from them, f64 storage for offset-dominated fields, for values computed from "
-                 "f64 values only and for flux arguments with f64 inputs; f32 sweeps plus one "
-                 "f64-residual refinement in every operator on f32 fields, f64 sweeps on f64 fields; "
-                 "f64 RK4 state",
+                 "f64 values only and for flux arguments with f64 inputs; every sweep solved in "
+                 "f64 registers; f64 RK4 state",
         "data": "synthetic (Taylor-Green initial condition)",
         "config": {"workload": "taylor_green_euler_lad_%d^3" % n, "grid": [n, n, n], "gamma": gamma,
                    "mach": 0.1, "cfl": 0.5, "dt": dt, "rk_stages": 5, "lad": True,

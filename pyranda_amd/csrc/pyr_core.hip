@@ -164,10 +164,6 @@ __device__ __forceinline__ void carry_of(const LineArgs& a, const Tables& t, int
   }
 }
 
-// The tables of a bounded line into LDS: they are read row by row in the
-// solves' passes, each read a latency on the critical path of a workgroup
-// (from memory, the 2-D and ragged bounded sweeps took 28-36 us for fields
-// of a few MB).
 // The work item of this workgroup when neighbouring items share cache lines:
 // consecutive workgroups start on the 8 XCDs in turn, each with an L2 of its
 // own, so each XCD takes a run of consecutive items. A refined y/z group of
@@ -191,6 +187,10 @@ __device__ __forceinline__ int line_offset(const Args& a, int L) {
   return (int)(l - q * n + (unsigned)a.B * q);
 }
 
+// The tables of a bounded line into LDS: they are read row by row in the
+// solves' passes, each read a latency on the critical path of a workgroup
+// (from memory, the 2-D and ragged bounded sweeps took 28-36 us for fields
+// of a few MB).
 __device__ __forceinline__ void stage_tables(const LineArgs& a, double* tab) {
   for (int e = threadIdx.x; e < a.ntab / 2; e += blockDim.x)
     reinterpret_cast<D2*>(tab)[e] = reinterpret_cast<const D2*>(a.tab)[e];
