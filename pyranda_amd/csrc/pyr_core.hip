@@ -726,10 +726,8 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, int blk, const flo
   const float* t = tab + ref_class(p, a.P, a.mx) * (RCHUNK * CROW);
   float x[RCHUNK], d[RCHUNK], z[4];
   const bool longer = p < a.mx;
-#pragma unroll
-  for (int k = 0; k < RCHUNK; ++k) x[k] = (float)rhs[k];
   if (act) {
-    ref_local_solve(a, t, x);
+    ref_local_solve(a, longer, t, rhs, x);
     const F4 e = ref_edges(a, longer, x);
     Y0[p * LY + lane] = e;
     // as in line_yz_body: a NaN or infinity spreads to the whole line
@@ -752,7 +750,7 @@ __device__ __forceinline__ void ref_yz_body(const RefArgs& a, int blk, const flo
       if (k <= a.mb) pre[k] = buf_load(0.0f, v ? rin : rout, act && k < m ? off_of(s + k) : OOB, 0);
   }
   if (act) {
-    ref_local_solve(a, t, d);
+    ref_local_solve(a, longer, t, d, d);
     Y1[p * LY + lane] = ref_edges(a, longer, d);
   }
   __syncthreads();
@@ -832,10 +830,8 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
   const float* t = tab + ref_class(p, P, a.mx) * (RCHUNK * CROW);
   float x[RCHUNK], d[RCHUNK], z[4];
   const bool longer = p < a.mx;
-#pragma unroll
-  for (int k = 0; k < RCHUNK; ++k) x[k] = (float)rhs[k];
   auto edges_of = [&](int q) { return ex[wave][l * P + q < 64 ? l * P + q : 0]; };
-  ref_local_solve(a, t, x);
+  ref_local_solve(a, longer, t, rhs, x);
   const F4 e = ref_edges(a, longer, x);
   ex[wave][lane] = e;
   const unsigned long long bad = __ballot(act && (!__builtin_isfinite(e.x) || !__builtin_isfinite(e.y)));
@@ -844,7 +840,7 @@ __device__ __forceinline__ void ref_x_body(const RefArgs& a, long long blk, cons
   if (bad & line_lanes(l, P)) z[0] = z[1] = z[2] = z[3] = __builtin_nanf("");
   ref_spike(a, t, z, x);
   ref_residual(a, p, longer, rhs, x, z, d);
-  ref_local_solve(a, t, d);
+  ref_local_solve(a, longer, t, d, d);
   const F4 ed = ref_edges(a, longer, d);
   wave_fence();
   ex[wave][lane] = ed;
@@ -1685,8 +1681,7 @@ static void emulate_ref_line(const RefArgs& a, const float* vin, long long strid
     }
     ref_rhs_interior<KIND>(a, t.win, t.rhs);
     ref_rhs_boundary(a, p, t.rhs, [&](int slot) { return end_value(slot, N, rd); });
-    for (int k = 0; k < RCHUNK; ++k) t.x[k] = (float)t.rhs[k];
-    ref_local_solve(a, t.t, t.x);
+    ref_local_solve(a, p < a.mx, t.t, t.rhs, t.x);
     Y[p] = ref_edges(a, p < a.mx, t.x);
   }
   for (int p = 0; p < P; ++p) {
@@ -1694,7 +1689,7 @@ static void emulate_ref_line(const RefArgs& a, const float* vin, long long strid
     ref_neighbours(a, a.g, p, [&](int q) { return Y[q]; }, t.z);
     ref_spike(a, t.t, t.z, t.x);
     ref_residual(a, p, p < a.mx, t.rhs, t.x, t.z, t.d);
-    ref_local_solve(a, t.t, t.d);
+    ref_local_solve(a, p < a.mx, t.t, t.d, t.d);
     Yd[p] = ref_edges(a, p < a.mx, t.d);
   }
   for (int p = 0; p < P; ++p) {

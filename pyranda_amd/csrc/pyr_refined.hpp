@@ -358,9 +358,9 @@ struct RefArgs {
 };
 
 // A chunk has mb or mb + 1 rows, mb the same in all chunks of a line, so a
-// group of four rows is skipped or taken as a whole by a wave-uniform test and
-// nothing else depends on the row count: past a chunk's end the tables hold
-// zeros, which make the rows there 0 and leave the others alone.
+// group of four rows is skipped or taken as a whole by a wave-uniform test.
+// Past a chunk's end the solve starts from zeros, and the zeros of its tables
+// keep the rows there at 0 and out of the others.
 constexpr int RGROUP = 4;
 
 // --- right-hand side ------------------------------------------------------
@@ -451,11 +451,20 @@ PYR_HD void ref_rhs_boundary(const RefArgs& a, int p, double* rhs, Reader rd) {
 }
 
 // --- chunk solve ------------------------------------------------------------
-// t: the table of this chunk's class
-PYR_HD void ref_local_solve(const RefArgs& a, const float* t, float* x) {
+// t: the table of this chunk's class; r: the right-hand sides, whose rows past
+// the chunk's end (longer: it has mb + 1) are sums over part of their points and
+// can overflow FP32 where no whole row does (constant fields above 5e36)
+template <typename T>
+PYR_HD void ref_local_solve(const RefArgs& a, bool longer, const float* t, const T* r, float* x) {
 #pragma unroll
   for (int g = 0; g < RCHUNK; g += RGROUP) {
+#pragma unroll
+    for (int k = g; k < g + RGROUP; ++k) x[k] = g <= a.mb ? (float)r[k] : 0.0f;
     if (g <= a.mb) {
+      if (a.mb < g + RGROUP) {
+#pragma unroll
+        for (int k = g; k < g + RGROUP; ++k) x[k] = k < a.mb || (k == a.mb && longer) ? x[k] : 0.0f;
+      }
       PYR_ROW_FENCE(g, RGROUP);
 #pragma unroll
       for (int k = g; k < g + RGROUP; ++k) {
@@ -534,8 +543,8 @@ PYR_HD void ref_spike(const RefArgs& a, const float* t, const float* z, float* x
 }
 
 // d = the FP32 rounding of the FP64 residual rhs - A y of every row, with
-// z = (y[s-2], y[s-1], y[e], y[e+1]) the values of y outside the chunk. What
-// lands past the chunk's end is finite and the solve that follows drops it.
+// z = (y[s-2], y[s-1], y[e], y[e+1]) the values of y outside the chunk. The
+// solve that follows drops what lands past the chunk's end.
 PYR_HD void ref_residual(const RefArgs& a, int p, bool longer, const double* rhs, const float* y, const float* z,
                          float* d) {
   // rows m and m + 1 of y are the next chunk's

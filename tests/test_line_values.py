@@ -1,0 +1,86 @@
+"""Line operators on values near the ends of the number formats."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+BOUNDED = [("NONE", "NONE"), ("SYMM", "SYMM"), ("NONE", "SYMM")]
+# whole and ragged chunks of up to 16 and 32 rows, one of them and several
+LENGTHS = [8, 9, 16, 31, 32, 33, 37, 48, 64, 65, 100, 257]
+
+
+class Host:
+    """The kernels' arithmetic along direction d on host arrays."""
+
+    def __init__(self, nn, d, faces):
+        from pyranda_amd import _lib as amd
+        self.amd, self.L, self.d = amd, amd.lib(), d
+        self.h = ctypes.c_void_p()
+        kinds = ["PERI"] * 6
+        kinds[2 * d:2 * d + 2] = faces
+        bc6 = (ctypes.c_int * 6)(*[amd.BC[k] for k in kinds])
+        amd.check(self.L.pyr_setup_host(ctypes.byref(self.h), *nn, 0.0, 1.0, 0.0, 1.0, 0.0, 1.0, bc6))
+
+    def __call__(self, op, v):
+        out = np.full(v.shape, 7.0, dtype=v.dtype, order="F")
+        prec = self.amd.F64 if v.dtype == np.float64 else self.amd.R32
+        self.amd.check(self.L.pyr_host_emulate(self.h, op, self.d, prec, v.ctypes.data, out.ctypes.data))
+        return out
+
+    def close(self):
+        self.L.pyr_destroy(self.h)
+
+
+class Device:
+    """The same through the kernels."""
+
+    def __init__(self, nn, d, faces):
+        from pyranda_amd.parcop import ParcopContext
+        kinds = ["PERI"] * 6
+        kinds[2 * d:2 * d + 2] = faces
+        self.d, self.ctx = d, ParcopContext(nn, (0.0,) * 3, (1.0,) * 3, kinds)
+
+    def __call__(self, op, v):
+        vd = torch.from_numpy(np.ascontiguousarray(v.transpose(2, 1, 0))).cuda().permute(2, 1, 0)
+        return self.ctx.apply(op, self.d, vd).cpu().numpy()
+
+    def close(self):
+        self.ctx.close()
+
+
+def _dims(n, d):
+    nn = [2, 3, 2]
+    nn[d] = n
+    return tuple(nn)
+
+
+def _each(run, lengths, faces):
+    for n in lengths:
+        for d in range(3):
+            f = run(_dims(n, d), d, faces)
+            yield n, d, f
+            f.close()
+
+
+def _constants_of_any_size(run, faces):
+    # rows are sums of differences of the field's values: a derivative of a
+    # constant is 0 and a filter returns the constant, whatever its size
+    for n, d, f in _each(run, LENGTHS, faces):
+        for c in (1.0, 1e36, 3.4e38):
+            v = np.full(_dims(n, d), c, dtype=np.float32, order="F")
+            for op in range(5):
+                want = v if op > 2 else np.zeros_like(v)
+                assert np.array_equal(f(op, v), want), (n, d, op, c)
+
+
+@pytest.mark.parametrize("faces", BOUNDED)
+def test_emulated_constants_of_any_size(faces):
+    _constants_of_any_size(Host, faces)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("faces", BOUNDED)
+def test_device_constants_of_any_size(faces):
+    print("constants", faces, flush=True)
+    _constants_of_any_size(Device, faces)
