@@ -68,6 +68,12 @@ static int fail(const std::string& m) { return pyr::report_error(m); }
 // ---------------------------------------------------------------------------
 enum Solve { SOLVE_NONE = 0, SOLVE_BND = 1, SOLVE_CIRC = 2 };
 
+template <int KIND, int SOLVE, typename TW>
+PYR_HD void right_hand_side(const LineArgs& a, const TW* win, double* rhs) {
+  if constexpr (SOLVE == SOLVE_NONE) rhs_explicit(a, win, rhs);
+  else rhs_interior<KIND>(a, win, rhs);
+}
+
 // What a y/z row's epilogue does and needs besides the solution, in registers
 // before the backward pass so that no store waits on a load: store it
 // (PRE_NONE), add the input back and store (PRE_V, filters), or join the
@@ -272,9 +278,9 @@ __device__ __forceinline__ void line_yz_body(const LineArgs& a, int blk, const T
   B4 lo = {}, hi = {};
   if (bounded) {
     __syncthreads();  // tables visible
-    if (act) boundary_rows<KIND, FULL>(a, tabs.wb, p, win, lo, hi);
+    if (act) boundary_rows<KIND, SOLVE == SOLVE_NONE, FULL>(a, tabs.wb, p, win, lo, hi);
   }
-  rhs_interior<KIND>(a, win, x);
+  right_hand_side<KIND, SOLVE>(a, win, x);
   if (bounded) put_boundary_rows<FULL>(a, p, lo, hi, x);
 
   // row k of the result: metric scale, filters add v back, fused epilogue, store
@@ -563,8 +569,8 @@ __device__ __forceinline__ void line_x_body(const LineArgs& a, long long blk, co
   }
   double x[CHUNK];
   B4 lo = {}, hi = {};
-  if (bounded) boundary_rows<KIND, FULL>(a, tabs.wb, p, win, lo, hi);
-  rhs_interior<KIND>(a, win, x);
+  if (bounded) boundary_rows<KIND, SOLVE == SOLVE_NONE, FULL>(a, tabs.wb, p, win, lo, hi);
+  right_hand_side<KIND, SOLVE>(a, win, x);
   if (bounded) put_boundary_rows<FULL>(a, p, lo, hi, x);
   // filters add v back here, read from the tile before the result takes its place
   auto emit = [&](int k, double y) {
@@ -1618,8 +1624,8 @@ static void emulate_line(const LineArgs& a, const TS* vin, long long stride, TS*
       t.win[w] = v;
     }
     B4 lo = {}, hi = {};
-    if (!a.periodic) boundary_rows<KIND, false>(a, tabs.wb, p, t.win, lo, hi);
-    rhs_interior<KIND>(a, t.win, t.x);
+    if (!a.periodic) boundary_rows<KIND, SOLVE == SOLVE_NONE, false>(a, tabs.wb, p, t.win, lo, hi);
+    right_hand_side<KIND, SOLVE>(a, t.win, t.x);
     if (!a.periodic) put_boundary_rows<false>(a, p, lo, hi, t.x);
     if (SOLVE == SOLVE_NONE) continue;
     t.e[0] = t.e[1] = 0.0;

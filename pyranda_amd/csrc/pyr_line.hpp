@@ -49,7 +49,7 @@ struct LineArgs {
   int lines;               // lines per workgroup (y/z: a power of two)
   int addv, epi;
   double scale, epi_c;
-  double w[4];             // interior right-hand side (rhs_interior)
+  double w[4];             // interior right-hand side (rhs_interior, rhs_explicit)
   double p1, p2;           // recurrence constants
   int W;                   // chunks that enter a carry
   double hf[2][4], hb[2][4];  // H of constant chunks of mb + 1 and mb rows
@@ -102,6 +102,26 @@ PYR_HD void rhs_interior(const LineArgs& a, const TW* win, double* rhs) {
   }
 }
 
+// The explicit filter's rows, sum_l w_l (v_{i+l} - v_i) as it stands: first
+// differences of an infinity hold both signs of it and give NaN for neighbours
+// whose value is that infinity. Those are fewer operations (y sweep of 256^3 in
+// FP32 25.9 us against 26.4, bounded x sweep of 1000x301x53 35.3 against 39.0,
+// with the end rows below), but a second look at rows that are not finite costs
+// more than it saves (29.6 us for the first).
+template <typename TW>
+PYR_HD void rhs_explicit(const LineArgs& a, const TW* win, double* rhs) {
+  constexpr int R = Halo<K_R4>::R;
+#pragma unroll
+  for (int k = 0; k < CHUNK; ++k) {
+    const double vc = (double)win[k + R];
+    double acc = 0.0;
+#pragma unroll
+    for (int l = -R; l <= R; ++l)
+      if (l != 0) acc += a.w[(l < 0 ? -l : l) - 1] * ((double)win[k + R + l] - vc);
+    rhs[k] = acc;
+  }
+}
+
 // One boundary row: c points at its weights, v at the row itself in the window.
 template <int KIND, typename TW>
 PYR_HD double boundary_row(const double* c, const TW* v) {
@@ -114,31 +134,63 @@ PYR_HD double boundary_row(const double* c, const TW* v) {
   return acc;
 }
 
+// ... of the explicit filter, `in` rows from the line's end, which lies at
+// offset -in (SIDE -1) or in (+1) and has the value e: sum_l c_l (v_{i+l} - e),
+// or sum_l c_l v_{i+l} where the last weight is not 0 (compact_r4.f90:106-207).
+// Points that are not in the sum are left out and not multiplied by 0: e may be
+// infinite.
+template <int SIDE, typename TW>
+PYR_HD double explicit_row(const double* c, const TW* v, int in, double e) {
+  constexpr int R = Halo<K_R4>::R;
+  const bool plain = c[WBROW - 1] != 0.0;
+  if (plain) e = 0.0;
+  double acc = 0.0;
+#pragma unroll
+  for (int l = -R; l <= R; ++l) {
+    const int to_end = SIDE * l;  // rows towards the end
+    if (to_end > NB - 1) continue;
+    const double t = (double)v[l] - e;
+    if (to_end < 0) acc += c[l + 4] * t;
+    else acc += c[l + 4] * (to_end < in || (to_end == in && plain) ? t : 0.0);
+  }
+  return acc;
+}
+
 struct B4 { double a, b, c, d; };  // four values, never indexed at run time
 
 // The right-hand sides of a bounded line's end rows: into lo by the first
 // chunk, into hi by the last one (p: this chunk; every chunk has at least 2*NB
 // rows, the last one mb of them in every line). Taken before the interior rows,
 // while the window is all that is in registers.
-template <int KIND, bool FULL, typename TW>
+template <int KIND, bool EXPLICIT, bool FULL, typename TW>
 PYR_HD void boundary_rows(const LineArgs& a, const double* wb, int p, const TW* win, B4& lo, B4& hi) {
   constexpr int R = Halo<KIND>::R;
   if (p == 0) {
-    lo.a = boundary_row<KIND>(wb, win + R);
-    PYR_ROW_FENCE(0, 1);
-    lo.b = boundary_row<KIND>(wb + WBROW, win + 1 + R);
-    PYR_ROW_FENCE(0, 1);
-    lo.c = boundary_row<KIND>(wb + 2 * WBROW, win + 2 + R);
-    PYR_ROW_FENCE(0, 1);
-    lo.d = boundary_row<KIND>(wb + 3 * WBROW, win + 3 + R);
+    [[maybe_unused]] const double e = (double)win[R];
+    auto row = [&](int k) {
+      PYR_ROW_FENCE(0, 1);
+      if constexpr (EXPLICIT) return explicit_row<-1>(wb + k * WBROW, win + k + R, k, e);
+      else return boundary_row<KIND>(wb + k * WBROW, win + k + R);
+    };
+    lo.a = row(0);
+    lo.b = row(1);
+    lo.c = row(2);
+    lo.d = row(3);
   }
   if (p == a.P - 1) {
+    [[maybe_unused]] double e = (double)win[CHUNK - 1 + R];
+    if (EXPLICIT && !FULL) {
+#pragma unroll
+      for (int k = 2 * NB - 1; k < CHUNK; ++k) e = k == a.mb - 1 ? (double)win[k + R] : e;
+    }
 #pragma unroll
     for (int k = FULL ? CHUNK - NB : NB; k < CHUNK; ++k) {
       const int j = k - ((FULL ? CHUNK : a.mb) - NB);
       if (j >= 0 && j < NB) {
         PYR_ROW_FENCE(k, 1);
-        const double v = boundary_row<KIND>(wb + (NB + j) * WBROW, win + k + R);
+        double v;
+        if constexpr (EXPLICIT) v = explicit_row<1>(wb + (NB + j) * WBROW, win + k + R, NB - 1 - j, e);
+        else v = boundary_row<KIND>(wb + (NB + j) * WBROW, win + k + R);
         hi.a = j == 0 ? v : hi.a;
         hi.b = j == 1 ? v : hi.b;
         hi.c = j == 2 ? v : hi.c;

@@ -62,7 +62,7 @@ struct OpPlan {
   int null_op = 0, null_option = 0, R = 3;
   int mb = 0, mx = 0;         // chunk p has mb + (p < mx) rows
   double scale = 1.0;         // metric (times 1/c of an implicit operator)
-  double w[4] = {};           // D1: weights at +1..+3; R3/R4: their tail sums (rhs_interior)
+  double w[4] = {};           // D1, explicit R4: weights at +1, +2, ...; R3/R4: their tail sums (rhs_interior)
   std::vector<double> wb;     // 2*NB x WBROW boundary rows of a bounded line
   double p1 = 0, p2 = 0;      // limit coefficients
   int W = 0;                  // chunks that enter a carry
@@ -181,8 +181,8 @@ inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, d
   pl.null_op = (n < 4);  // compact_basetype.f90:86-90
   pl.scale = (op == OP_D1) ? 1.0 / metric : (op == OP_D2 ? 1.0 / (metric * metric) : 1.0);
   const int hr = sc.ncr / 2;
-  if (pl.kind == K_D1) {
-    for (int l = 1; l <= 3; ++l) pl.w[l - 1] = sc.ari[hr + l];
+  if (pl.kind == K_D1 || !sc.implicit) {
+    for (int l = 1; l <= pl.R; ++l) pl.w[l - 1] = sc.ari[hr + l];
   } else {
     // symmetric rows of zero sum: sum_l w_l (v_{i+l} - v_i) = sum_m c_m
     // (d_{i+m-1} - d_{i-m}) with d_j = v_{j+1} - v_j and c_m = w_m + w_{m+1} + ...
@@ -217,7 +217,7 @@ inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, d
         const int col = (lo ? j : n - 2 * NB + j) + l;
         if (col < 0 || col >= n) continue;  // ghost columns read 0
         sum += (ld)row[l + hr];
-        if (l != 0) o[l + 4] = row[l + hr];
+        if (l != 0 || !sc.implicit) o[l + 4] = row[l + hr];
       }
       // rows of the NONE and SYMM variants have zero sum
       if ((lo ? v1 : v2) == -1) o[WBROW - 1] = (double)sum;

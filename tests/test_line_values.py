@@ -84,3 +84,44 @@ def test_emulated_constants_of_any_size(faces):
 def test_device_constants_of_any_size(faces):
     print("constants", faces, flush=True)
     _constants_of_any_size(Device, faces)
+
+
+def _explicit_filter_of_infinities(run, faces, oracle_mod):
+    # a row next to an infinity is that infinity, the infinity's own row is NaN
+    # and no other row is touched, rows at the ends and their antisymmetric
+    # variants included; finite values to a few roundings of the largest one
+    rng = np.random.default_rng(5)
+    with np.errstate(invalid="ignore"):
+        for n, d, f in _each(run, LENGTHS, faces):
+            nn = _dims(n, d)
+            P = oracle_mod.Oracle(nn, (1.0,) * 3, [faces[0] == "PERI" if e == d else True for e in range(3)],
+                                  symmetric=[[e == d and k == "SYMM" for k in faces] for e in range(3)])
+            v0 = rng.standard_normal(nn)
+            for dtype in (np.float64, np.float32):
+                for row in sorted({0, 1, 3, 4, n // 2, n - 5, n - 4, n - 1}):
+                    for bad in (np.inf, -np.inf):
+                        v = np.asfortranarray(v0.astype(dtype))
+                        idx = [1, 1, 1]
+                        idx[d] = row
+                        v[tuple(idx)] = bad
+                        w = np.asfortranarray(v.astype(np.float64))
+                        for anti in ((0, 1) if "SYMM" in faces else (0,)):
+                            want = P.apply_sym(4, d, -1, w) if anti else P.apply(4, d, w)
+                            got = f(4 | (0x10 if anti else 0), v)
+                            where = (n, d, dtype, row, bad, anti)
+                            for kind in (np.isnan, np.isposinf, np.isneginf):
+                                assert np.array_equal(kind(got), kind(want)), where
+                            ok = np.isfinite(want)
+                            assert np.abs(got[ok] - want[ok]).max() <= 8 * np.finfo(dtype).eps * np.abs(w[np.isfinite(w)]).max(), where
+
+
+@pytest.mark.parametrize("faces", BOUNDED + [("PERI", "PERI")])
+def test_emulated_explicit_filter_of_infinities(oracle_mod, faces):
+    _explicit_filter_of_infinities(Host, faces, oracle_mod)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("faces", BOUNDED + [("PERI", "PERI")])
+def test_device_explicit_filter_of_infinities(oracle_mod, faces):
+    print("explicit filter of infinities", faces, flush=True)
+    _explicit_filter_of_infinities(Device, faces, oracle_mod)
