@@ -232,6 +232,15 @@ inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, d
   pl.p1 = (double)p1;
   pl.p2 = (double)p2;
   pl.scale = (double)((ld)pl.scale / cc);
+  if (!periodic) {
+    // The recurrences solve for c times the result (d2: c = 1e4). By a power of
+    // two next to c, which changes no bit, the right-hand sides leave them as
+    // much room below the largest number as the result has.
+    const int k = std::ilogb((double)cc);
+    for (double& w : pl.w) w = std::ldexp(w, -k);
+    for (double& w : pl.wb) w = std::ldexp(w, -k);
+    pl.scale = std::ldexp(pl.scale, k);
+  }
 
   // per-row factors (constants for a periodic line)
   std::vector<ld> l1(n, p1), l2(n, p2), u1(n, p1), u2(n, p2), g(n, 1.0L);

@@ -125,3 +125,33 @@ def test_emulated_explicit_filter_of_infinities(oracle_mod, faces):
 def test_device_explicit_filter_of_infinities(oracle_mod, faces):
     print("explicit filter of infinities", faces, flush=True)
     _explicit_filter_of_infinities(Device, faces, oracle_mod)
+
+
+# bounds on the right-hand side's partial sums, in units of the largest value
+RHS_GAIN = (16.0, 57400.0, 11200.0, 4.0, 4.0)
+
+
+def _fields_near_overflow(run, faces):
+    # a field times a power of two gives the result times that power, up to
+    # where the result or a row's right-hand side leaves the FP64 range
+    rng = np.random.default_rng(6)
+    for n, d, f in _each(run, LENGTHS, faces):
+        v = np.asfortranarray(rng.uniform(-1.0, 1.0, _dims(n, d)))
+        for op in range(5):
+            for anti in ((0, 0x10) if "SYMM" in faces else (0,)):
+                out = f(op | anti, v)
+                top = max(np.abs(out).max(), RHS_GAIN[op])
+                s = 2.0 ** np.floor(np.log2(np.finfo(float).max / top) - 2.0)
+                assert np.array_equal(f(op | anti, np.asfortranarray(v * s)), out * s), (n, d, op, anti)
+
+
+@pytest.mark.parametrize("faces", BOUNDED)
+def test_emulated_fields_near_overflow(faces):
+    _fields_near_overflow(Host, faces)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("faces", BOUNDED)
+def test_device_fields_near_overflow(faces):
+    print("fields near overflow", faces, flush=True)
+    _fields_near_overflow(Device, faces)
