@@ -1676,6 +1676,7 @@ static void emulate_ref_line(const RefArgs& a, const float* vin, long long strid
   std::vector<St> st(P);
   std::vector<F4> Y(P), Yd(P);
   auto rd = [&](int i) { return vin[stride * i]; };
+  bool bad = false;
   for (int p = 0; p < P; ++p) {
     St& t = st[p];
     t.s = p * a.mb + std::min(p, a.mx);
@@ -1689,10 +1690,12 @@ static void emulate_ref_line(const RefArgs& a, const float* vin, long long strid
     ref_rhs_boundary(a, p, t.rhs, [&](int slot) { return end_value(slot, N, rd); });
     ref_local_solve(a, p < a.mx, t.t, t.rhs, t.x);
     Y[p] = ref_edges(a, p < a.mx, t.x);
+    bad = bad || !std::isfinite(Y[p].x) || !std::isfinite(Y[p].y);
   }
   for (int p = 0; p < P; ++p) {
     St& t = st[p];
     ref_neighbours(a, a.g, p, [&](int q) { return Y[q]; }, t.z);
+    if (bad) t.z[0] = t.z[1] = t.z[2] = t.z[3] = std::nanf("");
     ref_spike(a, t.t, t.z, t.x);
     ref_residual(a, p, p < a.mx, t.rhs, t.x, t.z, t.d);
     ref_local_solve(a, p < a.mx, t.t, t.d, t.d);

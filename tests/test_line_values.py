@@ -155,3 +155,25 @@ def test_emulated_fields_near_overflow(faces):
 def test_device_fields_near_overflow(faces):
     print("fields near overflow", faces, flush=True)
     _fields_near_overflow(Device, faces)
+
+
+@pytest.mark.parametrize("faces", BOUNDED + [("PERI", "PERI")])
+def test_emulated_nonfinite_values_spread_over_their_line(faces):
+    # as in the kernels (test_line_solve_edges.py)
+    rng = np.random.default_rng(7)
+    with np.errstate(invalid="ignore"):
+        for n, d, f in _each(Host, [9, 65, 257, 1000], faces):
+            for dtype in (np.float64, np.float32):
+                for row, bad in ((0, np.nan), (n - 1, -np.inf), (n // 2, np.inf)):
+                    v = np.asfortranarray(rng.standard_normal(_dims(n, d)).astype(dtype))
+                    line = [1, 1, 1]
+                    line[d] = slice(None)
+                    clean = [f(op, v) for op in range(4)]
+                    line[d] = row
+                    v[tuple(line)] = bad
+                    line[d] = slice(None)
+                    for op in range(4):
+                        got = f(op, v)
+                        assert not np.isfinite(got[tuple(line)]).any(), (n, d, op, dtype, row)
+                        got[tuple(line)] = clean[op][tuple(line)]
+                        assert np.array_equal(got, clean[op]), (n, d, op, dtype, row)
