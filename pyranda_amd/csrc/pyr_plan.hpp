@@ -232,14 +232,14 @@ inline OpPlan build_plan(int op, int n, int dir, int periodic, int v1, int v2, d
   pl.p1 = (double)p1;
   pl.p2 = (double)p2;
   pl.scale = (double)((ld)pl.scale / cc);
-  if (!periodic) {
-    // The recurrences solve for c times the result (d2: c = 1e4). By a power of
-    // two next to c, which changes no bit, the right-hand sides leave them as
-    // much room below the largest number as the result has.
-    const int k = std::ilogb((double)cc);
-    for (double& w : pl.w) w = std::ldexp(w, -k);
-    for (double& w : pl.wb) w = std::ldexp(w, -k);
-    pl.scale = std::ldexp(pl.scale, k);
+  if (!periodic && op == OP_D2) {
+    // The recurrences solve for c times the result, c = 1e4, which next to a
+    // bounded end reaches eight times the largest right-hand side before the
+    // scale takes c back. This factor changes no bit and keeps it below the
+    // largest number wherever the right-hand sides are.
+    for (double& w : pl.w) w *= 0.125;
+    for (double& w : pl.wb) w *= 0.125;
+    pl.scale *= 8.0;
   }
 
   // per-row factors (constants for a periodic line)
