@@ -1,0 +1,91 @@
+"""Bounded lines in the default solve modes: the refined FP32 solve at the
+lengths where its chunks of up to 32 rows split in every way."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from test_line_solve_edges import LENGTHS
+
+FACES = [("NONE", "NONE"), ("SYMM", "SYMM"), ("NONE", "SYMM"), ("SYMM", "NONE")]
+
+
+def _bounded(oracle_mod, run, others, faces, lengths, dtype):
+    """Each implicit operator on smooth fields with 5% noise, against the oracle
+    on the same values: the repository's bars, 1e-12 of max|ref| in FP64 and 1e-6
+    for FP32 fields. The antisymmetric member gets fields that are odd about the
+    faces."""
+    bar = 1e-12 if dtype == np.float64 else 1e-6
+    from meshgen import mesh
+    rng = np.random.default_rng(8)
+    for n in lengths:
+        for d in range(3):
+            nn = list(others)
+            nn[d] = n
+            dom = [(0.0, 1.0, m) for m in nn]
+            _, dd = mesh(dom)
+            P = oracle_mod.Oracle(tuple(nn), dd, [e != d for e in range(3)],
+                                  symmetric=[[e == d and k == "SYMM" for k in faces] for e in range(3)])
+            s = [((np.arange(m) + 0.5) / m).reshape([-1 if e == i else 1 for i in range(3)]) for e, m in enumerate(nn)]
+            noise = 0.05 * rng.standard_normal(nn)
+            cross = np.cos(s[(d + 1) % 3] + 2.0 * s[(d + 2) % 3])
+            even = (2.0 + np.cos(3.0 * s[d]) * cross + noise).astype(dtype)
+            odd = (np.sin(2.0 * np.pi * s[d]) * (cross + noise)).astype(dtype)
+            kinds = ["PERI"] * 6
+            kinds[2 * d:2 * d + 2] = faces
+            apply, close = run(tuple(nn), kinds, d)
+            for op in range(4):
+                for anti in ((0, 1) if "SYMM" in faces else (0,)):
+                    v = np.asfortranarray(odd if anti else even)
+                    w = np.asfortranarray(v.astype(np.float64))
+                    ref = P.apply_sym(op, d, -1, w) if anti else P.apply(op, d, w)
+                    got = apply(op | (0x10 if anti else 0), v)
+                    assert np.abs(got - ref).max() <= bar * np.abs(ref).max(), (n, d, op, anti)
+            close()
+
+
+@pytest.mark.parametrize("faces", FACES)
+def test_emulated_refined_lines_match_oracle(oracle_mod, faces):
+    from pyranda_amd import _lib as amd
+    L = amd.lib()
+
+    def run(nn, kinds, d):
+        h = ctypes.c_void_p()
+        bc6 = (ctypes.c_int * 6)(*[amd.BC[k] for k in kinds])
+        amd.check(L.pyr_setup_host(ctypes.byref(h), *nn, 0.0, 1.0, 0.0, 1.0, 0.0, 1.0, bc6))
+
+        def apply(op, v):
+            out = np.zeros(nn, dtype=np.float32, order="F")
+            amd.check(L.pyr_host_emulate(h, op, d, amd.R32, v.ctypes.data, out.ctypes.data))
+            return out
+        return apply, lambda: L.pyr_destroy(h)
+    _bounded(oracle_mod, run, (2, 3, 2), faces, LENGTHS, np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", LENGTHS)
+def test_device_bounded_lines_match_oracle(oracle_mod, n, dtype):
+    """Line counts that leave the last wave or workgroup partly filled, on
+    fields whose first element is 16-byte aligned and on ones off by one, which
+    give the same bits."""
+    from pyranda_amd.parcop import ParcopContext
+    print("bounded lines of", n, dtype, flush=True)
+
+    def run(nn, kinds, d):
+        ctx = ParcopContext(nn, (0.0,) * 3, (1.0,) * 3, kinds)
+
+        def apply(op, v):
+            flat = torch.from_numpy(np.ascontiguousarray(v.transpose(2, 1, 0))).reshape(-1).cuda()
+            got = []
+            for off in (0, 1):
+                buf, out = [torch.empty(flat.numel() + off, dtype=flat.dtype, device="cuda") for _ in range(2)]
+                buf[off:] = flat
+                vd, od = [b[off:].view(nn[2], nn[1], nn[0]).permute(2, 1, 0) for b in (buf, out)]
+                got.append(ctx.apply(op, d, vd, out=od))
+            assert torch.equal(*got), (nn, d, op)
+            return got[0].cpu().numpy()
+        return apply, ctx.close
+    for faces in FACES:
+        _bounded(oracle_mod, run, (9, 11, 10), faces, [n], dtype)
