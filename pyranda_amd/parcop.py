@@ -93,6 +93,8 @@ class ParcopContext:
         L = _lib.lib()
         h = ctypes.c_void_p()
         bc6 = (ctypes.c_int * 6)(*[_lib.BC[b] for b in bcs])
+        self._bounded = tuple(_lib.BC[b] != _lib.BC["PERI"] for b in list(bcs)[::2])
+        self._r32_solve, self._solve_tuned = "refined", {}
         _lib.check(L.pyr_setup(ctypes.byref(h), *self.nn, x1[0], xn[0], x1[1], xn[1],
                                x1[2], xn[2], bc6))
         self._h = h
@@ -118,9 +120,11 @@ class ParcopContext:
     def set_r32_solve(self, name):
         """'refined' (default) or 'fp64': arithmetic of the solves on FP32 fields."""
         _lib.check(self._L.pyr_set_r32_solve(self._h, _lib.R32_SOLVE[name]))
+        self._r32_solve = name
 
     def set_periodic_solver(self, name):
-        """'circulant' (default) or 'lu': solver of periodic implicit lines."""
+        """'circulant' (default) or 'lu': periodic implicit lines take the
+        circulant solve in either setting; members of a group agree on it."""
         _lib.check(self._L.pyr_set_periodic_solver(self._h, _lib.PSOLVE[name]))
 
     def set_solve_tuning(self, op, direction, name=None):
@@ -128,6 +132,12 @@ class ParcopContext:
         (pyr_set_solve_tuning): 'refined', 'fp64', or None for the context's."""
         _lib.check(self._L.pyr_set_solve_tuning(self._h, op, direction,
                                                 -1 if name is None else _lib.R32_SOLVE[name]))
+        self._solve_tuned[op, direction] = name
+
+    def _two_solves(self, op, direction):
+        """Whether FP32 fields have two solves to choose from here: bounded
+        implicit lines (every other line is solved in FP64 in both modes)."""
+        return self._bounded[direction] and op != _lib.OP_GFILTER
 
     def set_tuning(self, op, direction, dtype, x_lds_kb=-1, yz_pipe=-1, yz_lines=-1):
         """Per-operator knobs (pyr_set_tuning): lines per y/z workgroup
@@ -141,19 +151,21 @@ class ParcopContext:
     def autotune(self, dtype, ops=None, reps=5, x_lds_kb=(8, 12, 16, 24, 40, 64, 80), seed=7, rounded=False,
                  solve_modes=False):
         """Time each operator and direction at this precision with every
-        candidate (y/z: 64, 32 or 16 lines per workgroup; x lines have one
-        shape, reported under the first of x_lds_kb) on random fields and keep
-        the fastest. The timed
+        candidate (y/z: 64, 32 or 16 lines per workgroup; x lines and the
+        refined FP32 solve of y/z lines have one shape, reported under the
+        first of x_lds_kb and the default yz_lines, -1) on random fields and
+        keep the fastest. The timed
         launches cycle through enough fields to exceed the device's 256 MB
         last-level cache, so every launch reads its input from HBM as the
         operators of a time step do. rounded: FP64
         z sweeps are timed storing the FP32 copy of their result as well (the
         last sweep of the filter of an FP32 run's FP64 state). solve_modes
-        (FP32 fields): the candidates also range over the solve setting,
-        refined FP32 or FP64 (("r32_solve", 0 or 1) in the choice); the two
-        agree to the FP32 rounding of the result, so unlike the launch knobs
-        this choice can change results in the last bits, and the FP64 solve
-        is taken only when it is faster by SOLVE_MODE_MARGIN or more. Returns
+        (FP32 fields): where there are two solves (bounded implicit lines) the
+        candidates also range over the solve setting, refined FP32 or FP64
+        (("r32_solve", 0 or 1) in the choice, 0 elsewhere); the two agree to
+        the FP32 rounding of the result, so unlike the launch knobs this choice
+        can change results in the last bits, and the FP64 solve is taken only
+        when it is faster by SOLVE_MODE_MARGIN or more. Returns
         {(op, dir): (choice, {choice: mean ms})}."""
         ops = ops if ops is not None else (_lib.OP_D1, _lib.OP_D2, _lib.OP_D8, _lib.OP_SFILTER, _lib.OP_GFILTER)
         g = torch.Generator(device=self.device).manual_seed(seed)
@@ -170,12 +182,19 @@ class ParcopContext:
                 if self.nn[d] <= 3:
                     continue
                 kw = {"out32": out32} if out32 is not None and d == 2 else {}
-                if d == 0:
-                    cands = [(("x_lds_kb", next(iter(x_lds_kb))), ("yz_pipe", 0))]
-                else:
-                    cands = [(("yz_pipe", 0), ("yz_lines", n)) for n in (64, 32, 16)]
+                two = dtype == torch.float32 and self._two_solves(op, d)
                 if solve_modes and dtype == torch.float32:
-                    cands = [(("r32_solve", m),) + c for m in (0, 1) for c in cands]
+                    solves = [((("r32_solve", m),), name) for m, name in enumerate(("refined", "fp64")[:1 + two])]
+                else:
+                    solves = [((), self._solve_tuned.get((op, d)) or self._r32_solve)]
+                cands = []
+                for pre, name in solves:
+                    if d == 0:
+                        shapes = [(("x_lds_kb", next(iter(x_lds_kb))), ("yz_pipe", 0))]
+                    else:
+                        lines = (-1,) if two and name == "refined" else (64, 32, 16)
+                        shapes = [(("yz_pipe", 0), ("yz_lines", n)) for n in lines]
+                    cands += [pre + c for c in shapes]
                 times = {}
                 for cand in cands:
                     self._set_choice(op, d, dtype, cand)
@@ -203,7 +222,6 @@ class ParcopContext:
     def _set_choice(self, op, d, dtype, choice):
         kw = dict(choice)
         if "r32_solve" in kw:
-            # the solve mode first: the launch knobs are kept per solve mode
             self.set_solve_tuning(op, d, ("refined", "fp64")[kw.pop("r32_solve")])
         self.set_tuning(op, d, dtype, **kw)
 

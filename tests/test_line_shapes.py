@@ -1,5 +1,6 @@
 """Bounded lines in the default solve modes: the refined FP32 solve at the
-lengths where its chunks of up to 32 rows split in every way."""
+lengths where its chunks of up to 32 rows split in every way, and the autotuner's
+choice of launch shapes and solve modes."""
 import ctypes
 
 import numpy as np
@@ -89,3 +90,47 @@ def test_device_bounded_lines_match_oracle(oracle_mod, n, dtype):
         return apply, ctx.close
     for faces in FACES:
         _bounded(oracle_mod, run, (9, 11, 10), faces, [n], dtype)
+
+
+def _ctx(nn, kinds):
+    from pyranda_amd.parcop import ParcopContext
+    return ParcopContext(nn, (0.0,) * 3, (1.0,) * 3, [k for k in kinds for _ in (0, 1)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["refined", "fp64"])
+def test_autotune_of_bounded_fp32_lines(mode):
+    """One candidate where one launch exists (the refined solve), which leaves
+    the FP64 solve's lines per workgroup at their default; results unchanged."""
+    from pyranda_amd import _lib
+    print("autotune of bounded lines", mode, flush=True)
+    ctx = _ctx((40, 48, 33), ("PERI", "NONE", "SYMM"))
+    ctx.set_r32_solve(mode)
+    v = torch.rand((33, 48, 40), device="cuda", dtype=torch.float32).permute(2, 1, 0)
+    before = {(op, d): ctx.apply(op, d, v) for op in range(5) for d in range(3)}
+    rep = ctx.autotune(torch.float32, reps=2)
+    for (op, d), (best, times) in rep.items():
+        one = d == 0 or (mode == "refined" and op != _lib.OP_GFILTER)
+        assert len(times) == (1 if one else 3) and best in times, (op, d)
+        assert torch.equal(ctx.apply(op, d, v), before[op, d]), (op, d)
+    ctx.close()
+
+
+@pytest.mark.gpu
+def test_autotune_solve_modes_of_bounded_lines():
+    """Bounded implicit lines range over both solves, every other line keeps
+    the one it has; each result is that of a context in the chosen mode."""
+    from pyranda_amd import _lib
+    print("autotune of solve modes", flush=True)
+    nn, kinds = (40, 48, 33), ("NONE", "NONE", "PERI")
+    ctx, ref = _ctx(nn, kinds), [_ctx(nn, kinds) for _ in range(2)]
+    ref[1].set_r32_solve("fp64")
+    v = torch.rand(tuple(reversed(nn)), device="cuda", dtype=torch.float32).permute(2, 1, 0)
+    rep = ctx.autotune(torch.float32, reps=2, solve_modes=True)
+    for (op, d), (best, times) in rep.items():
+        modes = {c[0] for c in times}
+        both = d < 2 and op != _lib.OP_GFILTER
+        assert modes == {("r32_solve", m) for m in range(1 + both)}, (op, d)
+        assert torch.equal(ctx.apply(op, d, v), ref[best[0][1]].apply(op, d, v)), (op, d)
+    for c in [ctx] + ref:
+        c.close()
