@@ -177,8 +177,8 @@ __device__ __forceinline__ void carry_of(const LineArgs& a, const Tables& t, int
 // as three neighbours': in an ensemble of 24 members (3.7M points) d1 30.2 ->
 // 27.2 us, the filter 44.3 -> 35.4, the ring's maximum 40.2 -> 34.2.
 // The explicit filter's groups along a line share halo rows, of which each XCD
-// fetched its own copy (20% more bytes at 256^3 in FP64): y sweep 43.3 -> 38.4
-// us, 1000x301x53 in FP32 91.4 -> 82.7 us for the three sweeps.
+// fetched its own copy (20% more bytes at 256^3 in FP64): y sweep 47.0 -> 44.8
+// us, 1000x301x53 in FP32 94.3 -> 89.5 us for the three sweeps.
 __device__ __forceinline__ int xcd_order() {
   const int n = (int)gridDim.x, b = (int)blockIdx.x, x = b & 7, q = n >> 3, r = n & 7;
   return x * q + (x < r ? x : r) + (b >> 3);
@@ -991,11 +991,11 @@ struct pyr_ctx {
   int yz_lines = 0;
   int tune_ly[NOPS][3][2];
   int tune_rt[NOPS][3][2] = {};
-  // settings that no longer change a launch, kept as group members must agree
-  // on them: the x-line LDS budget, the periodic solver (above) and the solve
-  // arithmetic of FP32 fields per operator and direction (-1 = r32_solve)
-  int x_lds_kb = 40;
+  // FP32 solve mode per operator and direction (-1 = r32_solve; r32_mode)
   int tune_solve[NOPS][3];
+  // settings that change no launch, kept as group members have to agree on
+  // them: the x-line LDS budget and the periodic solver (above)
+  int x_lds_kb = 40;
   pyr_ctx() {
     for (int o = 0; o < NOPS; ++o)
       for (int d = 0; d < 3; ++d) {
@@ -1321,7 +1321,8 @@ static int r32_mode(const pyr_ctx* c, int op, int dir) {
 
 // bounded FP32 lines of a context in the refined mode keep the refined FP32
 // arithmetic; the FP64 recurrences serve every other line (periodic FP32 lines
-// in either mode: their refined solve agreed with one FP64 solve to the bit)
+// in either mode: one FP64 solve is closer to exact than the refined one they
+// had, whose rounded results it leaves but for the last bit of some points)
 static bool use_refined(const pyr_ctx* c, int op, int dir) {
   return c->rplan[op][dir].N > 0 && r32_mode(c, op, dir) == PYR_R32_SOLVE_REFINED;
 }

@@ -9,9 +9,11 @@
 //   C  entry state from the chunks after it and the backward recurrence,
 //      whose rows go straight to the epilogue.
 // All array indices are compile-time after unrolling, so the chunk lives in
-// VGPRs. FP32 fields are solved in FP64 as well: an FP64 FMA issues at the rate
-// of an FP32 one on CDNA3/4, and one FP64 solve is less work than an FP32 solve
-// refined with an FP64 residual (256^3 d8 y: 65 -> 33 us) and closer to exact.
+// VGPRs. Periodic lines of FP32 fields, and bounded ones in the FP64 solve mode,
+// are solved in FP64 as well: an FP64 FMA issues at the rate of an FP32 one on
+// CDNA3/4, and one FP64 solve is less work than an FP32 solve refined with an
+// FP64 residual (256^3 d8 y: 65 -> 33 us) and closer to exact. Bounded FP32 lines
+// in the default mode take that refined solve (pyr_refined.hpp).
 #pragma once
 
 #include "pyr_plan.hpp"

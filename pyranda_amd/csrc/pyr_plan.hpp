@@ -76,8 +76,10 @@ struct OpPlan {
   std::vector<double> tab;
 };
 
-// Propagation below this is left out of the carries: relative to the
-// state they multiply it is under a thousandth of an FP64 rounding.
+// Propagation below this is left out of the carries. Relative to the state it
+// multiplies, and so to the largest value of the line, that is under a
+// thousandth of an FP64 rounding; a point W chunks away from values 1e16 times
+// its own no longer gets their decayed share, which could have been its size.
 constexpr long double CARRY_TOL = 1e-19L;
 
 namespace detail {

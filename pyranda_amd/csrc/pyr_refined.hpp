@@ -328,6 +328,7 @@ inline RefPlan build_ref_plan(int op, int n, int v1, int v2, double metric) {
   for (int p = 0; p < P; ++p)
     for (int c = 0; c < 4 * P; ++c)
       for (int q = 0; q < 4; ++q)
+        // (as CARRY_TOL: 1e-10 of an FP32 rounding of the values they multiply)
         if (std::fabs(row_of(p, q, c)) > 1e-17) pl.Wg = std::max(pl.Wg, std::abs(c / 4 - p));
   const int K = 2 * pl.Wg + 1;
   pl.g.assign((size_t)P * K * 16, 0.0f);
