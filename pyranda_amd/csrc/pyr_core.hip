@@ -1321,8 +1321,8 @@ static int r32_mode(const pyr_ctx* c, int op, int dir) {
 
 // bounded FP32 lines of a context in the refined mode keep the refined FP32
 // arithmetic; the FP64 recurrences serve every other line (periodic FP32 lines
-// in either mode: one FP64 solve is closer to exact than the refined one they
-// had, whose rounded results it leaves but for the last bit of some points)
+// in either mode: a refined solve of them rounds to another last bit at about 1
+// point in 30 000)
 static bool use_refined(const pyr_ctx* c, int op, int dir) {
   return c->rplan[op][dir].N > 0 && r32_mode(c, op, dir) == PYR_R32_SOLVE_REFINED;
 }
