@@ -134,3 +134,40 @@ def test_autotune_solve_modes_of_bounded_lines():
         assert torch.equal(ctx.apply(op, d, v), ref[best[0][1]].apply(op, d, v)), (op, d)
     for c in [ctx] + ref:
         c.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("kinds", [("PERI", "PERI", "PERI"), ("NONE", "NONE", "PERI"), ("PERI", "NONE", "NONE")])
+def test_grouped_launches_equal_single_ones(kinds, dtype):
+    """Members of very different line lengths, a null direction and starts that
+    are not 16-byte aligned among them, in one launch: each member's result is
+    its own sweep's, bit for bit, for every operator and epilogue, and nothing
+    between the members is written."""
+    from pyranda_amd import _lib
+    print("grouped launches", kinds, dtype, flush=True)
+    sizes = [(8, 9, 10), (64, 40, 16), (1000, 12, 8), (33, 1024, 1), (17, 31, 129), (256, 16, 3), (9, 700, 8)]
+    ctxs = [_ctx(n, kinds) for n in sizes]
+    offs, at = [], 0
+    for i, n in enumerate(sizes):
+        offs.append(at)
+        at += n[0] * n[1] * n[2] + (16, 1, 3)[i % 3]
+    L, h = _lib.lib(), ctypes.c_void_p()
+    _lib.check(L.pyr_group_create(ctypes.byref(h), len(ctxs), (ctypes.c_void_p * len(ctxs))(*[c._h.value for c in ctxs]),
+                                  (ctypes.c_longlong * len(ctxs))(*offs)))
+    _lib.check(L.pyr_group_set_stream(h, _lib.stream_of(torch.device("cuda", torch.cuda.current_device()))))
+    g = torch.Generator(device="cuda").manual_seed(9)
+    src, old = [torch.randn(at, generator=g, device="cuda", dtype=dtype) for _ in range(2)]
+    prec = _lib.F64 if dtype == torch.float64 else _lib.R32
+    for op in range(5):
+        for d in range(3):
+            for epi in (_lib.EPI_STORE, _lib.EPI_ADD, _lib.EPI_ABS_SCALED, _lib.EPI_MAXABS_SCALED):
+                got, want = old.clone(), old.clone()
+                _lib.check(L.pyr_group_apply(h, op, d, prec, src.data_ptr(), got.data_ptr(), epi, 0.75, 2))
+                for c, n, o in zip(ctxs, sizes, offs):
+                    v, w = [t[o:o + n[0] * n[1] * n[2]].view(n[2], n[1], n[0]).permute(2, 1, 0) for t in (src, want)]
+                    c.apply(op, d, v, out=w, epi=epi, epi_scale=0.75 * c.dmesh[d] ** 2)
+                assert torch.equal(got, want), (op, d, epi)
+    _lib.check(L.pyr_group_destroy(h))
+    for c in ctxs:
+        c.close()
